@@ -424,7 +424,7 @@ class GpuParallelSweep:
 
     def debug_regions(self):
         """Mailbox words of the persistent apply's regions, (regions, 6):
-        parity counters, probe counter, staged, passes published, waits passed."""
+        passes finished, launch tag, probe counter, three unused words."""
         st = self.stats()
         cap = 6 * max(st["regions"], 1)
         out = np.zeros(cap, np.uint32)
@@ -501,9 +501,9 @@ class GpuParallelSweep:
 
 
 def debug_math(kind, x, device=0):
-    kinds = {"cbrt": 0, "log": 1, "exp": 2, "sqrt": 3, "div": 4, "sin": 5, "cos": 6}
+    kinds = {"cbrt": 0, "log": 1, "exp": 2, "sqrt": 3, "div": 4, "sin": 5, "cos": 6, "div_const": 7}
     x = np.ascontiguousarray(x, np.float64)
-    n = x.size // 2 if kind == "div" else x.size
+    n = x.size // 2 if kind in ("div", "div_const") else x.size
     out = np.zeros(n)
     rc = lib().hmc_debug_math(device, kinds[kind], _p(x), _p(out), n)
     if rc != HMC_OK:

@@ -1,6 +1,7 @@
 // The C ABI of a batch of replicas: creation, state, hipGraph-captured
 // steps, SDF and the tile autotuner.
 #include "host.hpp"
+#include "persist.hpp"
 #include <algorithm>
 
 namespace {
@@ -38,10 +39,11 @@ void launch_batch_step(hmc_batch* b, int from_args, int advance, uint32_t launch
       // the persistent applies stage their sites from the FP64 copies: one
       // cooperative launch runs every cycle of every replica, round by round
       k_place<PREC, false><<<grid_for(b->n_total, kBlock), kBlock, 0, s>>>(b->gtot, b->bodies, b->cells, b->w);
-      uint32_t nrounds = (uint32_t)b->grp_tile0.size(), nwg = b->nwg, chunk = (nwg + 7) / 8, probe = 0;
+      uint32_t nrounds = (uint32_t)b->grp_tile0.size(), nwg = b->nwg, chunk = (nwg + 7) / 8, probe = 0,
+               tag = ++b->sync_tag;
       void* args[] = {(void*)&b->reps, (void*)&b->dptcs, (void*)&b->dptoff, (void*)&b->dptrep, (void*)&b->sts,
                       (void*)&b->drt0, (void*)&b->drn,   (void*)&nrounds,   (void*)&nwg,       (void*)&chunk,
-                      (void*)&probe,   (void*)&b->bodies, (void*)&b->cells, (void*)&b->w};
+                      (void*)&probe,   (void*)&tag,      (void*)&b->bodies, (void*)&b->cells, (void*)&b->w};
       const hipError_t e = hipLaunchCooperativeKernel((const void*)k_bapply_tile<3>, dim3(chunk * 8),
                                                       dim3(b->pthreads), args, b->plds, s);
       if (e != hipSuccess && b->launch_err == hipSuccess) b->launch_err = e;
@@ -241,7 +243,7 @@ bool batch_regions(hmc_batch* b, int cus) {
         ntiles *= tc.nt[a];
       }
       const uint32_t EL = 2 * T + 2, rows = ncell / EL;
-      if (rows > 64u * kRowsPerLane || rows * (EL + 2) > threads * kValsPerThread) ok = false;
+      if (rows > kMaxRegionRows) ok = false;
       const double occ = (double)g.n_bodies / (double)g.n_spaces;
       tc.trials = trials;
       tc.ncell = ncell;
@@ -256,17 +258,11 @@ bool batch_regions(hmc_batch* b, int cus) {
                       : (uint32_t)std::ceil(1.1 * occ * ncell) + 64;
       tc.ntiles = ntiles;
       tc.xcd_chunk = (ntiles + 7) / 8;
-      const size_t lr = ((16 * ((size_t)rows + 1) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
-                        (size_t)tc.maxb * sizeof(float4);
+      fill_halo_lists(&tc, D);
+      const size_t lr = ((region_head_bytes(rows, tc.hoff[kHaloLists]) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
+                        (size_t)(tc.maxb + kTilePad) * sizeof(float4);
       if (lr > cap || lr > kTileLds) ok = false;
       tc.lds_bytes = (uint32_t)lr;
-      uint32_t q = threads;
-      for (int a = D - 1; a > 0; --a) {
-        const uint32_t rad = a == D - 1 ? EL + 2 : tc.E[a];
-        tc.step[a] = q % rad;
-        q /= rad;
-      }
-      tc.step[0] = q;
       // the persistent layout's band, as for a context
       const double sigma = g.sigma;
       double lmax = 0.0, Rb = 0.0;
@@ -379,10 +375,10 @@ bool batch_regions(hmc_batch* b, int cus) {
       hipMemset(b->sts, 0, (R + 1) * sizeof(ApplyState)) != hipSuccess)
     return false;
   {
-    uint32_t nrounds = nr, nwg = b->nwg, chunk = (nwg + 7) / 8, probe = 1;
+    uint32_t nrounds = nr, nwg = b->nwg, chunk = (nwg + 7) / 8, probe = 1, tag = 0;
     void* args[] = {(void*)&b->reps, (void*)&b->dptcs, (void*)&b->dptoff, (void*)&b->dptrep, (void*)&b->sts,
                     (void*)&b->drt0, (void*)&b->drn,   (void*)&nrounds,   (void*)&nwg,       (void*)&chunk,
-                    (void*)&probe,   (void*)&b->bodies, (void*)&b->cells, (void*)&b->w};
+                    (void*)&probe,   (void*)&tag,      (void*)&b->bodies, (void*)&b->cells, (void*)&b->w};
     if (hipLaunchCooperativeKernel(fn, dim3(chunk * 8), dim3(best_threads), args, best_lds, b->stream) !=
             hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)

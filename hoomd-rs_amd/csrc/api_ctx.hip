@@ -1,6 +1,7 @@
 // The C ABI of one context (include/hmc.h): creation, state, applies and
 // runs, traces, statistics and profiling.
 #include "host.hpp"
+#include "persist.hpp"
 
 namespace hmc {
 
@@ -61,6 +62,7 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
       (void)hipEventRecord(p0, s);
     }
     ApplyState* stp = c->st;
+    c->pc.tag += 1;
     void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&c->pc};
     const void* fn = is_isotropic(g.model) ? (const void*)k_apply_lj<D> : (const void*)k_apply_tile<D>;
     const hipError_t le =
@@ -286,8 +288,25 @@ bool choose_tiles(const Geometry& g, int D, double occ, size_t vt, int cus, Tile
 // so a shape qualifies only if all its workgroups fit on the device (LDS: the
 // box's offsets and a site capacity of 1.1x its expected count plus 64).
 // Among those the fewest lanes per workgroup win -- a colour pass lasts as
-// long as one workgroup's trials -- then the most trials on those lanes, then
-// the least staging.
+// long as one workgroup's trials -- then the least staging (C2: 500 regions of
+// 5 x 5 x 10 colour spaces; 510 of 3 x 5 x 17, whose boxes and halos are a
+// tenth larger, took 7% longer).
+void fill_halo_lists(TileCfg* tc, int D) {
+  int32_t rl[3] = {1, 1, 1};
+  for (int a = 0; a < D; ++a) rl[a] = (int32_t)(2 * tc->T[a]);
+  uint32_t cnt[kHaloLists] = {};
+  const int32_t z1 = D == 3 ? rl[2] : -1;
+  for (int32_t x = -1; x <= rl[0]; ++x)
+    for (int32_t y = -1; y <= rl[1]; ++y)
+      for (int32_t z = -1; z <= z1; ++z) {
+        const int32_t lc[3] = {x, y, z};
+        const uint32_t q = D == 3 ? halo_list<3>(lc, rl) : halo_list<2>(lc, rl);
+        if (q != UINT32_MAX) ++cnt[q];
+      }
+  tc->hoff[0] = 0;
+  for (int q = 0; q < kHaloLists; ++q) tc->hoff[q + 1] = tc->hoff[q] + cnt[q];
+}
+
 bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out) {
   uint32_t lim[3] = {1, 1, 1};
   const uint32_t cap[3] = {16, 16, 32};
@@ -298,7 +317,7 @@ bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out)
   const size_t static_lds = 2 * 257 * sizeof(double) + 64;
   const size_t cu_lds = 160 * 1024;
   const uint32_t cu_waves = 8;  // two waves per SIMD at the kernel's register use
-  uint32_t best_threads = 0, best_trials = 0;
+  uint32_t best_threads = 0;
   double best_work = 0.0;
   bool found = false;
   for (uint32_t t0 = 1; t0 <= lim[0]; ++t0)
@@ -308,26 +327,25 @@ bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out)
         const uint32_t trials = T[0] * T[1] * T[2];
         if (trials > (uint32_t)kTileThreads) continue;
         const uint32_t threads = ((trials + 63) / 64) * 64;
-        uint32_t ncell = 1, ntiles = 1;
+        uint32_t ncell = 1, ntiles = 1, own = 1;
         for (int a = 0; a < D; ++a) {
           ncell *= 2 * T[a] + 2;
+          own *= 2 * T[a];
           ntiles *= (g.half_shape[a] + T[a] - 1) / T[a];
         }
         const uint32_t EL = 2 * T[D - 1] + 2, rows = ncell / EL;
-        if (rows > 64u * kRowsPerLane || rows * (EL + 2) > threads * kValsPerThread) continue;
+        if (rows > kMaxRegionRows) continue;
         const uint32_t maxb = (uint32_t)std::ceil(1.1 * occ * ncell) + 64;
-        const size_t lds = ((16 * ((size_t)rows + 1) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
-                           (size_t)maxb * sizeof(float4);
+        const size_t lds = ((region_head_bytes(rows, ncell - own) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
+                           (size_t)(maxb + kTilePad) * sizeof(float4);
         if (lds > kTileLds) continue;
         const uint32_t per_cu = std::min<uint32_t>((uint32_t)(cu_lds / (lds + static_lds)), cu_waves / (threads / 64));
         const uint32_t grid = ((ntiles + 7) / 8) * 8;
         if (per_cu == 0 || grid > per_cu * (uint32_t)cus) continue;
         const double work = (double)ntiles * ncell;
-        if (!found || threads < best_threads || (threads == best_threads && trials > best_trials) ||
-            (threads == best_threads && trials == best_trials && work < best_work)) {
+        if (!found || threads < best_threads || (threads == best_threads && work < best_work)) {
           found = true;
           best_threads = threads;
-          best_trials = trials;
           best_work = work;
           for (int a = 0; a < 3; ++a) {
             out->T[a] = a < D ? T[a] : 1;
@@ -341,14 +359,6 @@ bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out)
           out->ntiles = ntiles;
           out->xcd_chunk = (ntiles + 7) / 8;
           out->lds_bytes = (uint32_t)lds;
-          uint32_t r = threads;
-          for (int a = D - 1; a > 0; --a) {
-            const uint32_t rad = a == D - 1 ? EL + 2 : out->E[a];
-            out->step[a] = r % rad;
-            r /= rad;
-          }
-          out->step[0] = r;
-          for (int a = D; a < 3; ++a) out->step[a] = 0;
         }
       }
   return found;
@@ -390,7 +400,7 @@ static uint32_t lj_region_threads(uint32_t trials) { return trials <= 2 ? 64u : 
 
 // Region shape of the persistent isotropic apply (k_apply_lj): as
 // choose_regions, with at most 12 trials (half-wavefronts taking one or two
-// each), at most 128 cells of a colour's halo, and a site capacity of 1.1x
+// each) and a site capacity of 1.1x
 // the box's expected count plus 128.  Among the shapes whose workgroups all
 // fit on the device at once (two waves per SIMD, the kernel's register
 // budget; the host checks the real occupancy): the least staging over all
@@ -401,9 +411,9 @@ bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* o
     if (g.shape[a] < 6 || g.reach[a] != 1) return false;
     lim[a] = std::min<uint32_t>(std::min<uint32_t>(g.half_shape[a], 8u), (uint32_t)(g.shape[a] - 4) / 2);
   }
-  // ziggurat tables, halo lists, 12 proposals of 160 bytes, the shared
-  // trials' partial sums (2 x 8 x 11 floats)
-  const size_t static_lds = 2 * 257 * sizeof(double) + (2 * 128 + 1) * sizeof(uint32_t) + 12 * 160 + 2 * 8 * 11 * 4 + 64;
+  // ziggurat tables, 12 proposals of 160 bytes, the shared trials' partial
+  // sums (2 x 8 x 11 floats), the halo lists' counts
+  const size_t static_lds = 2 * 257 * sizeof(double) + 12 * 160 + 2 * 8 * 11 * 4 + kHaloLists * 4 + 64;
   const size_t cu_lds = 160 * 1024;
   const uint32_t cu_waves = 8;
   bool found = false;
@@ -416,17 +426,16 @@ bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* o
         const uint32_t trials = T[0] * T[1] * T[2];
         if (trials > 12) continue;
         const uint32_t threads = lj_region_threads(trials);
-        uint32_t ncell = 1, ntiles = 1, halo = 1;
+        uint32_t ncell = 1, ntiles = 1, own = 1;
         for (int a = 0; a < D; ++a) {
           ncell *= 2 * T[a] + 2;
+          own *= 2 * T[a];
           ntiles *= (g.half_shape[a] + T[a] - 1) / T[a];
-          halo *= T[a] + 1;
         }
-        if (halo > 128) continue;
         const uint32_t EL = 2 * T[D - 1] + 2, rows = ncell / EL;
-        if (rows > 64u * kRowsPerLane || rows * (EL + 2) > threads * kValsPerThread) continue;
+        if (rows > kMaxRegionRows) continue;
         const uint32_t maxb = (uint32_t)std::ceil(1.1 * occ * ncell) + 128;  // >= 96: the overflow path's tables
-        const size_t lds = ((16 * ((size_t)rows + 1) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
+        const size_t lds = ((region_head_bytes(rows, ncell - own) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
                            (size_t)maxb * sizeof(float4);
         if (lds + static_lds > cu_lds) continue;
         const uint32_t per_cu = std::min<uint32_t>((uint32_t)(cu_lds / (lds + static_lds)), cu_waves / (threads / 64));
@@ -449,14 +458,6 @@ bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* o
           out->ntiles = ntiles;
           out->xcd_chunk = (ntiles + 7) / 8;
           out->lds_bytes = (uint32_t)lds;
-          uint32_t r = threads;
-          for (int a = D - 1; a > 0; --a) {
-            const uint32_t rad = a == D - 1 ? EL + 2 : out->E[a];
-            out->step[a] = r % rad;
-            r /= rad;
-          }
-          out->step[0] = r;
-          for (int a = D; a < 3; ++a) out->step[a] = 0;
         }
       }
   return found;
@@ -656,6 +657,8 @@ int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_
     g.shape[a] = (int32_t)inside;
     g.half_shape[a] = (uint32_t)(inside / 2);
     g.width[a] = L / (double)inside;
+    g.inv_L[a] = inv_const(L);
+    g.inv_width[a] = inv_const(g.width[a]);
     // a pair closer than sigma lies in neighbouring spaces unless the width is
     // within rounding of sigma; then the scan reaches two spaces out
     g.reach[a] = g.width[a] > sigma * (1.0 + 1e-9) ? 1 : 2;
@@ -818,6 +821,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop) {
       TileCfg pc{};
       if (choose_regions(g, D, (double)cfg->n_bodies / (double)spaces, cus, &pc)) {
+        fill_halo_lists(&pc, D);
         // Band of the persistent layout, whose LDS entries are the FP64
         // box-relative positions rounded once to FP32.  Per axis: that
         // rounding for the site and for the trial site (2^-24 R each, R the
@@ -829,7 +833,11 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         for (int a = 0; a < D; ++a) R = std::max(R, 0.5 * pc.E[a] * g.width[a] + g.width[a]);
         const double Et = (0x1p-24 * (2.0 * R + 2.0 * sigma) + 0x1p-53 * (4.0 * lmax + 2.0 * sigma)) * 1.01;
         const void* fn = D == 2 ? (const void*)k_apply_tile<2> : (const void*)k_apply_tile<3>;
-        const uint32_t threads = ((pc.trials + 63) / 64) * 64;
+        // one lane per trial, and where the regions leave compute units to
+        // spare, wavefronts that only stage and reload (a small system's box of
+        // 1000 cells staged by one wavefront took 40 us of a 200 us apply)
+        uint32_t threads = ((pc.trials + 63) / 64) * 64;
+        if (pc.xcd_chunk * 8u <= (uint32_t)cus) threads = kTileThreads;
         int per_cu = 0;
         if (contact_band(Et, sigma, g.sigma2, g.edge2, D, &pc.band_lo, &pc.band_hi) &&
             hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pc.lds_bytes) == hipSuccess &&
@@ -858,6 +866,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
         choose_regions_lj(g, D, (double)cfg->n_bodies / (double)spaces, cus, &pc)) {
+      fill_halo_lists(&pc, D);
       // Per-axis bound E on the FP32 displacement of two staged entries
       // against the reference's FP64 displacement: the rounding of each
       // box-relative coordinate to FP32 (2^-24 R, R the largest), the FP64
@@ -1503,7 +1512,7 @@ int hmc_profile_read(hmc_ctx* c, double* pass_ms_total, uint64_t* pass_launches,
 int hmc_debug_math(int device, int kind, const double* in, double* out, uint64_t n) {
   if (hipSetDevice(device) != hipSuccess) return HMC_ERR_DEVICE;
   if (n == 0) return HMC_OK;
-  uint64_t nin = kind == 4 ? 2 * n : n;
+  uint64_t nin = kind == 4 || kind == 7 ? 2 * n : n;
   double *din = nullptr, *dout = nullptr;
   if (dalloc(&din, nin) != hipSuccess || dalloc(&dout, n) != hipSuccess) {
     (void)hipFree(din);

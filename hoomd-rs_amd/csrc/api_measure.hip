@@ -32,6 +32,7 @@ Geometry sdf_geometry(const Geometry& g, double xmax) {
     s.shape[a] = (int32_t)k;
     s.half_shape[a] = (uint32_t)std::max<int64_t>(1, k / 2);
     s.width[a] = g.L[a] / (double)k;
+    s.inv_width[a] = inv_const(s.width[a]);
     spaces *= (uint64_t)k;
   }
   uint32_t str = 1;

@@ -22,12 +22,10 @@ struct Sfc64 {
   __device__ __forceinline__ uint64_t next() {
     uint64_t out = a + b + ctr;
     a = b ^ (b >> 11);
-    // c + 8c as a shift and an add: folded into a multiply it would read an
+    // c + 8c in one instruction: folded into a multiply it would read an
     // unused high half from whatever register holds it, and a register with a
     // load in flight makes the wave wait for that load
-    uint64_t c8 = c << 3;
-    asm("" : "+v"(c8));
-    b = c + c8;
+    asm("v_lshl_add_u64 %0, %1, 3, %1" : "=v"(b) : "v"(c));
     c = ((c << 24) | (c >> 40)) + out;
     ctr += 1;
     return out;
@@ -35,11 +33,20 @@ struct Sfc64 {
   __device__ __forceinline__ uint32_t next_u32() { return (uint32_t)next(); }
 };
 
-// Counter(step, substep, seed).index(index).make_rng()
+// Counter(step, substep, seed).index(index).make_rng().  FLAT: the twelve
+// rounds without a loop, for kernels that draw many times per launch (a taken
+// branch costs a third of a round); a kernel that draws once is faster with the
+// loop, which is less code to fetch.
+template <bool FLAT = false>
 __device__ __forceinline__ Sfc64 counter_rng(uint64_t step, uint32_t substep, uint32_t seed, uint64_t index) {
   Sfc64 r{step, ((uint64_t)substep << 32) | (uint64_t)seed, index, 0};
+  if constexpr (FLAT) {
+#pragma unroll
+    for (int i = 0; i < 12; ++i) r.next();
+  } else {
 #pragma unroll 1
-  for (int i = 0; i < 12; ++i) r.next();
+    for (int i = 0; i < 12; ++i) r.next();
+  }
   return r;
 }
 
@@ -98,7 +105,13 @@ __device__ __forceinline__ double standard_normal(G& r, const double* zx, const 
     }
     double f0 = zf[i], f1 = zf[i + 1];
     double lhs = f1 + (f0 - f1) * uniform01(r);
-    if (lhs < glibc_exp(-x * x / 2.0)) return x;
+    // exp(-x^2 / 2) from the hardware's FP32 exp2 first: x^2 / 2 < 7, so its
+    // relative error (the argument's roundings and 1 ulp) stays below 2^-19.
+    // Only a value within 2^-16 of it needs the library's exp (which a
+    // wavefront would otherwise run for one of its lanes in every other draw).
+    const double ex = (double)__builtin_amdgcn_exp2f((float)(-x * x / 2.0) * 1.44269504f);
+    if (lhs < ex * (1.0 - 0x1p-16)) return x;
+    if (lhs < ex * (1.0 + 0x1p-16) && lhs < glibc_exp(-x * x / 2.0)) return x;
   }
 }
 

@@ -93,6 +93,7 @@ struct hmc_batch {
   uint32_t* drt0 = nullptr;                     // the rounds' first regions and sizes (device)
   uint32_t* drn = nullptr;
   uint32_t nwg = 0;                             // workgroups of the launch: the largest round
+  uint32_t sync_tag = 0;                        // persistent launches so far (their progress words' tag)
   uint32_t pper_cu = 0, pregions = 0;           // resident regions per CU; all regions
   std::vector<TileCfg> hptcs;                   // the replicas' region shapes (host copy)
   // per replica and region shape T (index T): the largest body count of a
@@ -134,6 +135,8 @@ void collect_events(hmc_ctx* c, std::vector<std::pair<hipEvent_t, hipEvent_t>>& 
 int read_state(hmc_ctx* c, ApplyState* out, bool check_errors = true);
 bool contact_band(double E, double sigma, double sigma2, double edge2, int D, float* lo, float* hi);
 bool choose_tiles(const Geometry& g, int D, double occ, size_t vt, int cus, TileCfg* out);
+// The places of the halo lists (TileCfg::hoff) of a full region of shape T.
+void fill_halo_lists(TileCfg* tc, int D);
 bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out);
 bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* out);
 int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_out, double* lmax_out);

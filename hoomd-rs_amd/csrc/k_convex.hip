@@ -25,13 +25,13 @@ __device__ void trial_convex(const Geometry& g, const ApplyState* st, const Bodi
   } else {
     q = qmul(versor_displacement(rng, st->max_move, zx, zf), q);
   }
-  for (int a = 0; a < 3; ++a) x[a] = wrap1(x[a], g.L[a]);  // wrap(propose(..))
+  for (int a = 0; a < 3; ++a) x[a] = wrap1(g, a, x[a]);  // wrap(propose(..))
   bool accept = false;
   if (space_of<3>(g, st->origin, x) == s) {
     // the trial site: wrap(x + rotate(q, 0)) with orientation q * identity
     // (property/oriented_point.rs:107-113)
     const v3 r0 = qrotate(q, v3{0.0, 0.0, 0.0});
-    const double t[3] = {wrap1(x[0] + r0.x, g.L[0]), wrap1(x[1] + r0.y, g.L[1]), wrap1(x[2] + r0.z, g.L[2])};
+    const double t[3] = {wrap1(g, 0, x[0] + r0.x), wrap1(g, 1, x[1] + r0.y), wrap1(g, 2, x[2] + r0.z)};
     const quat qt = qmul(q, quat{1.0, {0.0, 0.0, 0.0}});
     const v3 tv = {t[0], t[1], t[2]};
     uint32_t nb[3][5];
@@ -68,9 +68,9 @@ __device__ void trial_convex(const Geometry& g, const ApplyState* st, const Bodi
       // update_body_properties (microstate.rs:985-1034): body = wrap(props),
       // site = wrap(body.transform(site))
       double nb3[3], ns3[3];
-      for (int a = 0; a < 3; ++a) nb3[a] = wrap1(x[a], g.L[a]);
+      for (int a = 0; a < 3; ++a) nb3[a] = wrap1(g, a, x[a]);
       const double r0a[3] = {r0.x, r0.y, r0.z};
-      for (int a = 0; a < 3; ++a) ns3[a] = wrap1(nb3[a] + r0a[a], g.L[a]);
+      for (int a = 0; a < 3; ++a) ns3[a] = wrap1(g, a, nb3[a] + r0a[a]);
       const uint32_t fl = ghost_flags<3>(g, ns3);
       B.bpos[body] = make_double4(nb3[0], nb3[1], nb3[2], move_stamp(st->epoch));
       B.bquat[body] = make_double4(q.s, q.v.x, q.v.y, q.v.z);
@@ -473,7 +473,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
     } else {
       q = qmul(dq, q);
     }
-    for (int a = 0; a < 3; ++a) x[a] = wrap1(x[a], g.L[a]);  // wrap(propose(..))
+    for (int a = 0; a < 3; ++a) x[a] = wrap1(g, a, x[a]);  // wrap(propose(..))
     active = space_of<3>(g, st->origin, x) == s;
   }
   if (!active) tot = 0;  // a trial outside its space is rejected without pair tests
@@ -482,9 +482,9 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
   const v3 r0 = qrotate(q, v3{0.0, 0.0, 0.0});
   const quat qt = qmul(q, quat{1.0, {0.0, 0.0, 0.0}});
   if (active && kl == 0) {
-    W.t[k][0] = wrap1(x[0] + r0.x, g.L[0]);
-    W.t[k][1] = wrap1(x[1] + r0.y, g.L[1]);
-    W.t[k][2] = wrap1(x[2] + r0.z, g.L[2]);
+    W.t[k][0] = wrap1(g, 0, x[0] + r0.x);
+    W.t[k][1] = wrap1(g, 1, x[1] + r0.y);
+    W.t[k][2] = wrap1(g, 2, x[2] + r0.z);
     W.qt[k][0] = qt.s;
     W.qt[k][1] = qt.v.x;
     W.qt[k][2] = qt.v.y;
@@ -580,9 +580,9 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
       // update_body_properties (microstate.rs:985-1034): body = wrap(props),
       // site = wrap(body.transform(site))
       double nb3[3], ns3[3];
-      for (int a = 0; a < 3; ++a) nb3[a] = wrap1(x[a], g.L[a]);
+      for (int a = 0; a < 3; ++a) nb3[a] = wrap1(g, a, x[a]);
       const double r0a[3] = {r0.x, r0.y, r0.z};
-      for (int a = 0; a < 3; ++a) ns3[a] = wrap1(nb3[a] + r0a[a], g.L[a]);
+      for (int a = 0; a < 3; ++a) ns3[a] = wrap1(g, a, nb3[a] + r0a[a]);
       const uint32_t fl = ghost_flags<3>(g, ns3);
       B.bpos[body] = make_double4(nb3[0], nb3[1], nb3[2], move_stamp(st->epoch));
       B.bquat[body] = make_double4(q.s, q.v.x, q.v.y, q.v.z);
@@ -675,10 +675,10 @@ __global__ void __launch_bounds__(256) k_tune_eval_convex(Geometry g, const Appl
   } else {
     q = qmul(versor_displacement(r, size, zx, zf), q);  // rotate/versor.rs:111-122
   }
-  for (int a = 0; a < 3; ++a) x[a] = wrap1(x[a], g.L[a]);  // wrap(propose(..))
+  for (int a = 0; a < 3; ++a) x[a] = wrap1(g, a, x[a]);  // wrap(propose(..))
   // the trial site: wrap(x + rotate(q, 0)), orientation q * identity
   const v3 r0 = qrotate(q, v3{0.0, 0.0, 0.0});
-  const double t[3] = {wrap1(x[0] + r0.x, g.L[0]), wrap1(x[1] + r0.y, g.L[1]), wrap1(x[2] + r0.z, g.L[2])};
+  const double t[3] = {wrap1(g, 0, x[0] + r0.x), wrap1(g, 1, x[1] + r0.y), wrap1(g, 2, x[2] + r0.z)};
   const quat qt = qmul(q, quat{1.0, {0.0, 0.0, 0.0}});
   const v3 tv = {t[0], t[1], t[2]};
   bool hit = false, outside = false;

@@ -71,14 +71,14 @@ __device__ __forceinline__ void trial(const Geometry& g, const ApplyState* st, c
   }
   double x[3] = {bp.x, bp.y, bp.z};
   for (int a = 0; a < D; ++a) x[a] += v[a];
-  for (int a = 0; a < D; ++a) x[a] = wrap1(x[a], g.L[a]);  // generate_trial_moves: wrap(propose(..))
+  for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a]);  // generate_trial_moves: wrap(propose(..))
 
   bool accept = false;
   if (space_of<D>(g, st->origin, x) == s) {
     // trial site: wrap(body.transform(site)) = wrap(x + 0) (pairwise_cutoff.rs:436);
     // x + 0.0 differs from x only for -0.0, which wraps to the same value
     double t[3] = {0.0, 0.0, 0.0};
-    for (int a = 0; a < D; ++a) t[a] = wrap1(x[a], g.L[a]);
+    for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a]);
     float t32[3] = {0.0f, 0.0f, 0.0f};
     for (int a = 0; a < D; ++a) t32[a] = (float)t[a];
     bool hit = false;
@@ -140,7 +140,7 @@ __device__ __forceinline__ void trial(const Geometry& g, const ApplyState* st, c
       // update_body_properties (microstate.rs:985-1034): body = wrap(props),
       // which is t; site = wrap(body + 0)
       double nsp[3] = {0.0, 0.0, 0.0};
-      for (int a = 0; a < D; ++a) nsp[a] = wrap1(t[a] + 0.0, g.L[a]);
+      for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
       const uint32_t fl = ghost_flags<D>(g, nsp);
       B.bpos[body] = make_double4(t[0], t[1], t[2], move_stamp(st->epoch));
       const double4 sp = pack_site(nsp, fl);
@@ -501,14 +501,14 @@ __device__ __forceinline__ void pass_tile(const Geometry& g, ApplyState* st, con
     const uint32_t slot = s0 + pick;
     double x[3] = {bp.x, bp.y, bp.z};
     for (int a = 0; a < D; ++a) x[a] += v[a];
-    for (int a = 0; a < D; ++a) x[a] = wrap1(x[a], g.L[a]);  // generate_trial_moves: wrap(propose(..))
+    for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a]);  // generate_trial_moves: wrap(propose(..))
 
     bool accept = false;
     if (space_of<D>(g, st->origin, x) == s) {
       // the trial site wrap(x + 0) (pairwise_cutoff.rs:436); x + 0.0 differs
       // from x only for -0.0, which wraps to the same value
       double t[3] = {0.0, 0.0, 0.0};
-      for (int a = 0; a < D; ++a) t[a] = wrap1(x[a], g.L[a]);
+      for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a]);
       bool hit = false;
       unsigned retests = 0;
       uint32_t rounds = 0;
@@ -571,7 +571,7 @@ __device__ __forceinline__ void pass_tile(const Geometry& g, ApplyState* st, con
         // update_body_properties (microstate.rs:985-1034): body = wrap(x),
         // which is t; site = wrap(body + 0)
         double nsp[3] = {0.0, 0.0, 0.0};
-        for (int a = 0; a < D; ++a) nsp[a] = wrap1(t[a] + 0.0, g.L[a]);
+        for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
         const uint32_t fl = ghost_flags<D>(g, nsp);
         B.bpos[body] = make_double4(t[0], t[1], t[2], move_stamp(st->epoch));
         const double4 sp = pack_site(nsp, fl);

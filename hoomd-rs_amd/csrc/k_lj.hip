@@ -169,11 +169,11 @@ __device__ void trial_lj(const Geometry& g, const ApplyState* st, const Bodies& 
   ball_sample<D>(rng, st->max_move, zx, zf, v);
   double x[3] = {bp.x, bp.y, bp.z};
   for (int a = 0; a < D; ++a) x[a] += v[a];
-  for (int a = 0; a < D; ++a) x[a] = wrap1(x[a], g.L[a]);  // generate_trial_moves: wrap(propose(..))
+  for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a]);  // generate_trial_moves: wrap(propose(..))
   bool accept = false;
   if (space_of<D>(g, st->origin, x) == s) {
     double t[3] = {0.0, 0.0, 0.0};  // wrap(x + 0) == wrap(x)
-    for (int a = 0; a < D; ++a) t[a] = wrap1(x[a], g.L[a]);
+    for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a]);
     const double xi[3] = {sp.x, sp.y, sp.z};
     const uint32_t* tb = tabbed ? tab : nullptr;
     const uint32_t total = base;
@@ -224,7 +224,7 @@ __device__ void trial_lj(const Geometry& g, const ApplyState* st, const Bodies& 
     if (accept && lane == 0) {
       // update_body_properties (microstate.rs:985-1034)
       double nsp[3] = {0.0, 0.0, 0.0};
-      for (int a = 0; a < D; ++a) nsp[a] = wrap1(t[a] + 0.0, g.L[a]);
+      for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
       const uint32_t fl = ghost_flags<D>(g, nsp);
       B.bpos[body] = make_double4(t[0], t[1], t[2], move_stamp(st->epoch));
       const double4 nspk = pack_site(nsp, fl);

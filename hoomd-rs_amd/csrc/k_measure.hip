@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(kEnergyBlock) k_insert_energy(Geometry g, cons
   const uint32_t k = blockIdx.x * kEnergyBlock + threadIdx.x;
   if (k >= n) return;
   double t[3] = {0.0, 0.0, 0.0};
-  for (int a = 0; a < D; ++a) t[a] = wrap1(cand[(size_t)k * D + a] + 0.0, g.L[a]);
+  for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, cand[(size_t)k * D + a] + 0.0);
   const uint32_t s = space_of<D>(g, st->origin, t);
   if (s == UINT32_MAX) {  // outside the checkerboard: reported as an error by the host
     atomicOr(outside, 1u);

@@ -17,7 +17,7 @@ __global__ void k_init_sites(Geometry g, Bodies B, int have_sites) {
     s[1] = sp.y;
     s[2] = sp.z;
   } else {
-    for (int a = 0; a < D; ++a) s[a] = wrap1(x[a] + 0.0, g.L[a]);
+    for (int a = 0; a < D; ++a) s[a] = wrap1(g, a, x[a] + 0.0);
   }
   B.spos[e] = pack_site(s, ghost_flags<D>(g, s));
 }
@@ -48,8 +48,8 @@ __global__ void k_map_bodies(Geometry g, double3 lold, const double4* __restrict
   }
   if (!inside) atomicOr(outside, 1u);
   double s[3] = {0.0, 0.0, 0.0};
-  for (int a = 0; a < D; ++a) p[a] = wrap1(p[a], g.L[a]);
-  for (int a = 0; a < D; ++a) s[a] = wrap1(p[a] + 0.0, g.L[a]);
+  for (int a = 0; a < D; ++a) p[a] = wrap1(g, a, p[a]);
+  for (int a = 0; a < D; ++a) s[a] = wrap1(g, a, p[a] + 0.0);
   B.bpos[e] = make_double4(p[0], p[1], p[2], 0.0);
   B.spos[e] = pack_site(s, ghost_flags<D>(g, s));
 }
@@ -113,6 +113,11 @@ __global__ void k_debug_math(int kind, const double* in, double* out, uint64_t n
     case 1: r = glibc_log(in[i]); break;
     case 2: r = glibc_exp(in[i]); break;
     case 3: r = sqrt(in[i]); break;
+    case 7: {
+      const double a = in[2 * i], b = in[2 * i + 1], y = inv_const(b), m = fabs(a);
+      r = y > 0.0 && m >= 0x1p-900 && m <= 0x1p900 ? div_const_fast(a, b, y) : a / b;
+      break;
+    }
     case 5: {
       double c;
       glibc_sincos(in[i], &r, &c);

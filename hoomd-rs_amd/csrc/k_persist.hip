@@ -36,11 +36,11 @@ __device__ __noinline__ TrialOut trial_global_dev(const Geometry* gp, ApplyState
   const double4 bp = bpos[body];
   double x[3] = {bp.x, bp.y, bp.z};
   for (int a = 0; a < D; ++a) x[a] += v[a];
-  for (int a = 0; a < D; ++a) x[a] = wrap1(x[a], g.L[a]);
+  for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a]);
   bool accept = false;
   if (space_of<D>(g, st->origin, x) == s) {
     double t[3] = {0.0, 0.0, 0.0};
-    for (int a = 0; a < D; ++a) t[a] = wrap1(x[a], g.L[a]);
+    for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a]);
     bool hit = false;
     for (int i0 = -1; i0 <= 1 && !hit; ++i0)
       for (int i1 = -1; i1 <= 1 && !hit; ++i1)
@@ -62,7 +62,7 @@ __device__ __noinline__ TrialOut trial_global_dev(const Geometry* gp, ApplyState
     accept = !hit;
     if (accept) {
       double nsp[3] = {0.0, 0.0, 0.0};
-      for (int a = 0; a < D; ++a) nsp[a] = wrap1(t[a] + 0.0, g.L[a]);
+      for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
       const uint32_t fl = ghost_flags<D>(g, nsp);
       bpos[body] = make_double4(t[0], t[1], t[2], move_stamp(st->epoch));
       st_dev_d4(&spos[body], pack_site(nsp, fl));
@@ -85,10 +85,163 @@ __device__ __noinline__ TrialOut trial_global_dev(const Geometry* gp, ApplyState
   return o;
 }
 
+// FP32 squared distance of a staged site from the trial site (fused: three
+// roundings, within the band's 4 u relative term).
+template <int D>
+__device__ __forceinline__ float tile_dist2(const float4& q, const float* tr) {
+  const float dx = q.x - tr[0], dy = q.y - tr[1];
+  if (D == 3) {
+    const float dz = q.z - tr[2];
+    return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+  }
+  return fmaf(dx, dx, dy * dy);
+}
+
+// The rows of a trial: the 3^D cells around the trial's own are 3^(D-1) rows
+// of three cells, contiguous among the staged sites.  key[r] = the row's
+// length << 16 | its first entry, longest first.
+//
+// A cell whose nearest point is a diameter away holds nothing to test: rows
+// and row ends are cut by the distance from the trial site (box-relative, tr)
+// to the faces of its cell cb (27 cells become 20 on average).  Spaces are
+// exact in FP64 and a body stays in its space for the whole apply, so the
+// cut's margin of 10^-4 covers every rounding (coordinates of some tens of
+// diameters in FP32).
+//
+// Sorted by length so that the walk below runs as many slots as the
+// wavefront's fullest lanes have sites: on C2 32 for 27 candidates a lane,
+// where rounds over all rows in place took 71.
+template <int D>
+__device__ __forceinline__ void tile_rows(GeoPtr g, const TileCfg& tc, const uint16_t* coff,
+                                          const uint32_t* cb, const float* tr, uint32_t* key) {
+  constexpr int AL = D - 1, NR = D == 3 ? 9 : 3;
+  const float cut = tc.band_hi * (1.0f + 1e-4f);
+  // squared distance from the trial site to the lower and upper face of its cell
+  float flo[3] = {0.0f, 0.0f, 0.0f}, fhi[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const float wd = (float)g->width[a];
+    const float u = tr[a] - ((float)cb[a] - 0.5f * (float)tc.E[a]) * wd;
+    const float dl = fmaxf(u, 0.0f), dh = fmaxf(wd - u, 0.0f);
+    flo[a] = dl * dl;
+    fhi[a] = dh * dh;
+  }
+  const uint32_t s1 = tc.E[AL] + 1, s0 = D == 3 ? tc.E[1] * s1 : s1;  // cells between neighbouring rows
+  const uint32_t c0 = D == 3 ? cb[0] * s0 + cb[1] * s1 + cb[2] : cb[0] * s0 + cb[1];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int i0 = D == 3 ? r / 3 : r, i1 = D == 3 ? r % 3 : 1;
+    float d = i0 == 0 ? flo[0] : i0 == 2 ? fhi[0] : 0.0f;
+    if (D == 3) d += i1 == 0 ? flo[1] : i1 == 2 ? fhi[1] : 0.0f;
+    const uint32_t c = c0 + (uint32_t)(i0 - 1) * s0 + (D == 3 ? (uint32_t)(i1 - 1) * s1 : 0u);
+    const uint32_t b = coff[c - (d + flo[AL] < cut ? 1u : 0u)];
+    const uint32_t e = coff[c + (d + fhi[AL] < cut ? 2u : 1u)];
+    key[r] = d < cut ? ((e - b) << 16) | b : 0u;
+  }
+  auto order = [&](int i, int j) {
+    const uint32_t hi = max(key[i], key[j]), lo = min(key[i], key[j]);
+    key[i] = hi;
+    key[j] = lo;
+  };
+  if (D == 3) {
+    // Floyd's 25-comparator network for nine elements
+    order(0, 3), order(1, 7), order(2, 5), order(4, 8);
+    order(0, 7), order(2, 4), order(3, 8), order(5, 6);
+    order(0, 2), order(1, 3), order(4, 5), order(7, 8);
+    order(1, 4), order(3, 6), order(5, 7);
+    order(0, 1), order(2, 4), order(3, 5), order(6, 8);
+    order(2, 3), order(4, 5), order(6, 7);
+    order(1, 2), order(3, 4), order(5, 6);
+  } else {
+    order(0, 2), order(0, 1), order(1, 2);
+  }
+}
+
+// Does the trial site (FP64 t, box-relative FP32 tr) overlap a staged site of
+// its rows other than its own, entry `self` (value old) of lb?
+//
+// Three rows at a time, one site of each per round, while any lane has a site
+// left in the longest of them.  A lane past the end of its row reads on into
+// the sites that follow: they are sites of the box too, either in the trial's
+// neighbourhood or a space's width or more away (a site's FP32 coordinates
+// never leave its space by more than rounding, also while another trial moves
+// it), and at the end of the box kTilePad entries out of reach.  So no slot
+// needs a validity test; the own entry is moved out of reach for the walk.
+// (The 12-byte LDS reads at scattered entries bound the walk.)
+//
+// Pairs inside the band are re-tested in FP64 after the walk when no certain
+// overlap was found.  `odd`: the box holds a site without images, whose entry
+// is NaN and which is always re-tested; such a box, and a row longer than
+// kTilePad, is walked one site at a time.  lb[self] holds `old` again on
+// return.
+template <int D>
+__device__ __forceinline__ bool tile_overlaps(const Geometry& g, const TileCfg& tc, float4* lb, const double4* spos,
+                                              const double* t, const float* tr, uint32_t* key, uint32_t self,
+                                              float4 old, bool odd, unsigned* retests) {
+  constexpr int NR = D == 3 ? 9 : 3;
+  const float lo = tc.band_lo, hi = tc.band_hi;
+  lb[self] = make_float4(kTileFar, 0.0f, 0.0f, 0.0f);
+  bool hit = false, walk = __any(odd || (key[0] >> 16) > (uint32_t)kTilePad);
+  if (!walk) {  // uniform
+    const float4* p[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) p[r] = lb + (key[r] & 0xffffu);
+    float near2 = kTileFar;
+    auto slots = [&](int r0, uint32_t k) {
+      const float4 a = p[r0][k], b = p[r0 + 1][k], c = p[r0 + 2][k];
+      near2 = fminf(near2, tile_dist2<D>(a, tr));
+      near2 = fminf(near2, fminf(tile_dist2<D>(b, tr), tile_dist2<D>(c, tr)));
+    };
+    for (uint32_t k = 0; __any(!(near2 < lo) && (key[0] >> 16) > k); ++k) {
+      slots(0, k);
+      if (D == 3) {
+        if (!__any((key[3] >> 16) > k)) continue;
+        slots(3, k);
+        if (!__any((key[6] >> 16) > k)) continue;
+        slots(6, k);
+      }
+    }
+    hit = near2 < lo;
+    walk = near2 < hi && !hit;
+  }
+  if (walk) {
+#pragma unroll 1
+    for (int r = 0; r < NR && !hit; ++r) {
+      const uint32_t b = key[0] & 0xffffu, n = key[0] >> 16;
+#pragma unroll
+      for (int i = 0; i + 1 < NR; ++i) key[i] = key[i + 1];
+#pragma unroll 1
+      for (uint32_t k = 0; k < n && !hit; ++k) {
+        const float4 q = lb[b + k];
+        const float d2 = tile_dist2<D>(q, tr);
+        if (d2 < lo) hit = true;
+        if (d2 < lo || d2 >= hi) continue;
+        ++*retests;
+        hit = retest64_body<D>(g.self, spos, (uint32_t)__float_as_int(q.w), t[0], t[1], t[2]);
+      }
+    }
+  }
+  lb[self] = old;
+  return hit;
+}
+
 // Every cycle and colour of one apply for region `tile` of the system (g, st,
 // w.start, w.mbox); the region's accepted moves are added to *acc.  zx, zf:
 // the ziggurat layers (an LDS copy, or the constant tables).
-template <int D>
+//
+// A pass is a chain of latencies (two wavefronts per SIMD: one lane per trial
+// of a colour fills the chip no further), so what a pass does not need from
+// its neighbours is taken off the chain.  After the trials of pass i:
+//   publish (stores acknowledged, progress word);
+//   the draws of pass i + 1: random numbers, chosen body, displacement;
+//   each wavefront polls the progress words it needs (usually there by now)
+//   and issues the loads of its halo entries;
+//   the rest of the proposal while they are in flight: wrapped positions,
+//   space test, the entries an acceptance writes, the rows to walk;
+//   the halo entries into LDS, a barrier, the trials.
+// None of the proposal reads what pass i or a neighbour changed: a trial's
+// body belongs to its own colour's cell, and cells' offsets are static.
+template <int D, int CELLS>
 __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st, const Bodies& B, const Cells& C,
                                                const Work& w, const TileCfg& tc, uint32_t tile,
                                                unsigned long long* acc, const double* zx, const double* zf) {
@@ -100,8 +253,9 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
   const uint16_t* coff = l.coff;
   float4* lb = l.lb;
   __shared__ unsigned blk_acc;
+  __shared__ uint32_t hcnt[kHaloLists];
+  __shared__ uint32_t odd;  // the box holds (or held) a site without images
   const uint32_t tid = threadIdx.x;
-  const uint32_t wid = tid >> 6, lane = tid & 63u;
   const uint32_t cycles = st->cycles, substep0 = st->substep0;
   const uint64_t step = st->step;
   const uint32_t seed = st->seed;
@@ -123,84 +277,93 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
     }
   }
   const bool has_trial = tid < tc.trials;
-  // wave 0's lane l < nnb notifies neighbour region l after each pass
-  const uint32_t nnb = D == 3 ? 26u : 8u;
-  const uint32_t nbt = wid == 0 && lane < nnb ? region_neighbour<D>(tc, rg, lane) : tile;
 
-  if (tid == 0) blk_acc = 0;
-  const bool overflow = region_stage<D>(g, tc, rg, B, C, w, l);
+  if (tid == 0) blk_acc = odd = 0;
+  if (tid < (uint32_t)kHaloLists) hcnt[tid] = 0;
+  const bool overflow = region_stage<D, kTilePad>(g, tc, rg, B, C, w, l, &odd);
 
   unsigned retests = 0;
-  // The proposal of pass i (cycle i / 2^D, colour i mod 2^D) depends only on
-  // the counter, the space's body count and the chosen body's position, which
-  // no other colour changes; it is drawn while the neighbour regions finish
-  // the previous pass, and with it everything of the trial that depends on
-  // the proposal alone: the wrapped trial position and its space test, its
-  // FP32 image, and the site and LDS entry an acceptance writes.
+  // the proposal of this thread's trial
   bool pgo = false, pin = false;
-  uint32_t ps = 0, pcrow = 0, pe0 = 0, pn = 0, ppick = 0, pbody = 0;
-  uint32_t pcb[3] = {0, 0, 0};
-  double pt[3] = {0.0, 0.0, 0.0};
+  uint32_t ps = 0, self = 0, body = 0;
+  uint32_t pcb[3] = {0, 0, 0}, key[9];
+  double v[3] = {0.0, 0.0, 0.0}, pt[3] = {0.0, 0.0, 0.0};
   float ptr[3] = {0.0f, 0.0f, 0.0f};
-  double4 psp = make_double4(0.0, 0.0, 0.0, 0.0);
-  float4 pent = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  auto propose = [&](uint32_t i) {
+  double4 bp = make_double4(0.0, 0.0, 0.0, 0.0), psp = bp;
+  float4 pent = make_float4(0.0f, 0.0f, 0.0f, 0.0f), pold = pent;
+  for (int r = 0; r < 9; ++r) key[r] = 0;
+  // the draws of pass i (cycle i / 2^D, colour i mod 2^D)
+  auto draw = [&](uint32_t i) {
     const uint32_t colour = i & (NCOL - 1), substep = substep0 + (i >> D);
     bool active = has_trial && !overflow;
     uint32_t s = 0;
     for (int a = 0; a < D; ++a) {
-      const uint32_t l = 2 * hh[a] + ((colour >> (D - 1 - a)) & 1u);
-      if ((int32_t)l >= rl[a]) active = false;
-      s += (uint32_t)(org[a] + (int32_t)l) * g.stride[a];
-      pcb[a] = l + 1;
+      const uint32_t h = 2 * hh[a] + ((colour >> (D - 1 - a)) & 1u);
+      if ((int32_t)h >= rl[a]) active = false;
+      s += (uint32_t)(org[a] + (int32_t)h) * g.stride[a];
+      pcb[a] = h + 1;
     }
     ps = s;
     pgo = false;
     if (!active) return;
-    pcrow = D == 3 ? pcb[0] * tc.E[1] + pcb[1] : pcb[0];
-    pe0 = coff[pcrow * CW + pcb[AL]];
-    pn = coff[pcrow * CW + pcb[AL] + 1] - pe0;
-    if (!pn) return;
+    const uint32_t c = (D == 3 ? pcb[0] * tc.E[1] + pcb[1] : pcb[0]) * CW + pcb[AL];
+    const uint32_t e0 = coff[c], n = coff[c + 1] - e0;
+    if (!n) return;
     pgo = true;
     // the choice first (a few draws), then the chosen body's position in
     // flight during the displacement draw
-    Sfc64 rng = counter_rng(step, substep, seed, s);
-    ppick = choose_index(rng, pn);
-    pbody = (uint32_t)__float_as_int(lb[pe0 + ppick].w);
-    const double4 bp = B.bpos[pbody];
-    double v[3] = {0.0, 0.0, 0.0};
+    Sfc64 rng = counter_rng<true>(step, substep, seed, s);
+    self = e0 + choose_index(rng, n);
+    pold = lb[self];
+    body = (uint32_t)__float_as_int(pold.w);
+    bp = B.bpos[body];
     ball_sample<D>(rng, max_move, zx, zf, v);
-    double x[3] = {bp.x, bp.y, bp.z};
-    for (int a = 0; a < D; ++a) x[a] += v[a];
-    for (int a = 0; a < D; ++a) x[a] = wrap1(x[a], g.L[a]);  // generate_trial_moves: wrap(propose(..))
-    pin = space_of<D>(g, origin, x) == s;
-    for (int a = 0; a < D; ++a) pt[a] = wrap1(x[a], g.L[a]);
-    const float4 te = stage_entry64<D>(g, c64, make_double4(pt[0], pt[1], D == 3 ? pt[2] : 0.0, 0.0), 0u);
-    ptr[0] = te.x;
-    ptr[1] = te.y;
-    ptr[2] = te.z;
-    // update_body_properties (microstate.rs:985-1034): site = wrap(body + 0)
-    double nsp[3] = {0.0, 0.0, 0.0};
-    for (int a = 0; a < D; ++a) nsp[a] = wrap1(pt[a] + 0.0, g.L[a]);
-    psp = pack_site(nsp, ghost_flags<D>(g, nsp));
-    pent = stage_entry64<D>(g, c64, psp, pbody);
+  };
+  // the rest of the proposal: everything of the trial that depends on it alone
+  auto finish = [&]() {
+    if (!pgo) return;
+    const GeoPtr gp = geo_ptr(g.self);
+    const double x[3] = {bp.x + v[0], bp.y + v[1], bp.z + v[2]};
+    uint32_t own[3];
+    for (int a = 0; a < D; ++a) own[a] = (uint32_t)org[a] + pcb[a] - 1u;
+    const TrialSite<D> ts = trial_site<D>(gp, st, origin, x, own, ps);
+    pin = ts.in;
+    for (int a = 0; a < D; ++a) pt[a] = ts.t[a];
+    psp = pack_site(ts.n, ts.flags);
+    box_relative64<D>(gp, c64, ts.t, ptr);
+    float e[3] = {0.0f, 0.0f, 0.0f};
+    box_relative64<D>(gp, c64, ts.n, e);
+    pent = make_float4(ts.flags == kNoImages ? __int_as_float(0x7fc00000) : e[0], e[1], e[2], __int_as_float((int)body));
+    tile_rows<D>(gp, tc, coff, pcb, ptr, key);
   };
 
   const uint32_t npass = cycles * NCOL;
-  if (npass) propose(0);
   for (uint32_t i = 0; i < npass; ++i) {
+    // (one copy of the proposal and of the reload for every pass)
     const uint32_t colour = i & (NCOL - 1), substep = substep0 + (i >> D);
+    if (i) region_publish(w.mbox, tile, tc.tag, i);
+    draw(i);
+    if (i) region_wait<D>(st, w.mbox, tc, rg, tile, i);
+    // the body's position is here before the halo loads are issued: the
+    // compiler cannot count those, and would wait for them all to use it
+    asm volatile("" : "+v"(bp.x), "+v"(bp.y), "+v"(bp.z));
+    RegionReload<D, 1, CELLS, 3> reload(g, tc, rg, B, l, hcnt, i);
+    if (i && !overflow) reload.issue();
+    finish();
+    if (i && !overflow) reload.commit(&odd);
+    if (i == 0) region_halo_lists<D>(tc, rg, l, hcnt);  // (read after the next barrier)
+    if (i) __syncthreads();
     unsigned accepted = 0;
     if (has_trial && overflow) {
       bool active = true;
       uint32_t s = 0;
       for (int a = 0; a < D; ++a) {
-        const uint32_t l = 2 * hh[a] + ((colour >> (D - 1 - a)) & 1u);
-        if ((int32_t)l >= rl[a]) active = false;
-        s += (uint32_t)(org[a] + (int32_t)l) * g.stride[a];
+        const uint32_t h = 2 * hh[a] + ((colour >> (D - 1 - a)) & 1u);
+        if ((int32_t)h >= rl[a]) active = false;
+        s += (uint32_t)(org[a] + (int32_t)h) * g.stride[a];
       }
-      const uint32_t s0 = w.start[s], n = w.start[s + 1] - s0;
-      if (active && n) {
+      const uint32_t s0 = active ? w.start[s] : 0u, n = active ? w.start[s + 1] - s0 : 0u;
+      if (n) {
         const TrialOut o = trial_global_dev<D>(g.self, st, B.bpos, B.spos, C.body, w.start,
                                                w.tracing ? w.trace : nullptr, w.trace_cap, zx, zf, s, s0, n,
                                                colour, substep);
@@ -209,71 +372,13 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
       }
     } else if (pgo) {
       // ---- the trial of this pass from LDS
-      const uint32_t s = ps, self = pe0 + ppick, body = pbody;
-      if (pin) {
-        constexpr int NR = D == 3 ? 9 : 3;
-        uint32_t rlo[NR], rhi[NR];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          const int i0 = D == 3 ? r / 3 : r;
-          const int i1 = D == 3 ? r % 3 : 0;
-          const uint32_t row = D == 3 ? (pcb[0] + i0 - 1) * tc.E[1] + (pcb[1] + i1 - 1) : pcb[0] + i0 - 1;
-          rlo[r] = coff[row * CW + pcb[AL] - 1];
-          rhi[r] = coff[row * CW + pcb[AL] + 2];
-        }
-        const double* t = pt;
-        bool hit = false;
-        uint32_t rounds = 0;
-#pragma unroll
-        for (int r = 0; r < NR; ++r) rounds = max(rounds, rhi[r] - rlo[r]);
-        const float* tr = ptr;
-        const float lo = tc.band_lo, hi = tc.band_hi;
-        // rows of three cells; only the centre row (the trial's own cell in
-        // its middle) can hold the trial's own site.  Two rounds per step:
-        // 2 NR LDS reads in flight together.  The FP32 distance is fused
-        // (three roundings, within the band's 4 u relative term).
-        constexpr int RC = NR / 2;
-        uint32_t len[NR];
-#pragma unroll
-        for (int r = 0; r < NR; ++r) len[r] = rhi[r] - rlo[r];
-        for (uint32_t kk = 0; kk < rounds && !hit; kk += 2) {
-          uint32_t amb = 0;
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-              const uint32_t k2 = kk + (uint32_t)h;
-              const uint32_t idx = rlo[r] + k2;
-              const bool valid = k2 < len[r] && (r != RC || idx != self);
-              const float4 q = lb[valid ? idx : self];
-              const float dx = q.x - tr[0], dy = q.y - tr[1];
-              float d2;
-              if (D == 3) {
-                const float dz = q.z - tr[2];
-                d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-              } else {
-                d2 = fmaf(dx, dx, dy * dy);
-              }
-              hit |= valid && d2 < lo;
-              if (valid && !(d2 < lo) && !(d2 >= hi)) amb |= 1u << (h * NR + r);
-            }
-          }
-          while (amb && !hit) {
-            const int b2 = __ffs(amb) - 1;
-            amb &= amb - 1;
-            const int h = b2 / NR, r = b2 % NR;
-            const float4 q = lb[rlo[r] + kk + (uint32_t)h];
-            ++retests;
-            hit |= retest64_body<D>(g.self, B.spos, (uint32_t)__float_as_int(q.w), t[0], t[1], t[2]);
-          }
-        }
-        if (!hit) {
-          // update_body_properties (microstate.rs:985-1034), formed with the proposal
-          B.bpos[body] = make_double4(t[0], t[1], t[2], stamp);
-          st_dev_d4(&B.spos[body], psp);
-          lb[self] = pent;
-          accepted = 1;
-        }
+      if (pin && !tile_overlaps<D>(g, tc, lb, B.spos, pt, ptr, key, self, pold, odd != 0, &retests)) {
+        // update_body_properties (microstate.rs:985-1034), formed with the proposal
+        B.bpos[body] = make_double4(pt[0], pt[1], pt[2], stamp);
+        st_dev_d4(&B.spos[body], psp);
+        lb[self] = pent;
+        if (!(pent.x == pent.x)) odd = 1;
+        accepted = 1;
       }
       if (w.tracing) {
         unsigned long long ti = atomicAdd((unsigned long long*)&st->trace_n, 1ull);
@@ -281,7 +386,7 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
           hmc_trace_record rec;
           rec.substep = substep;
           rec.color = colour;
-          rec.space = s;
+          rec.space = ps;
           rec.body = (int64_t)body;
           rec.status = (int32_t)accepted;
           rec.pad = 0;
@@ -291,17 +396,6 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
     }
     const unsigned long long mk = __ballot(accepted != 0);
     if (__lane_id() == 0 && mk) atomicAdd(&blk_acc, (unsigned)__popcll(mk));
-    if (i + 1 == npass) break;  // no later pass reads the halo
-    region_publish(w.mbox, nbt, nnb, i & 1u);
-    // the next proposal reads only static cell data and this region's own
-    // bodies, none of which pass i changed: drawn while the neighbours finish
-    propose(i + 1);
-    region_wait(st, w.mbox, tile, nnb, i);
-    // ---- reload the halo cells of this colour
-    if (!overflow)
-      region_reload<D>(g, tc, rg, B, l, colour);
-    else
-      __syncthreads();
   }
   lane_add(&st->band_retests, retests);
   if (tid == 0 && overflow) atomicAdd(&st->tile_overflows, 1ull);
@@ -321,7 +415,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_apply_tile(Geometry g, Appl
   }
   __shared__ double zx[257], zf[257];
   if (D == 3) stage_zig(zx, zf);  // (read after region_stage's barriers)
-  apply_tile_run<D>(g, st, B, C, w, tc, tile, &w.acc_slots[b & (kAccSlots - 1)], zx, zf);
+  apply_tile_run<D, 2>(g, st, B, C, w, tc, tile, &w.acc_slots[b & (kAccSlots - 1)], zx, zf);
 }
 
 // The persistent applies of every replica of a batch in one cooperative
@@ -341,8 +435,8 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_bapply_tile(const BatchRep*
                                                               const uint32_t* toff, const uint32_t* trep,
                                                               ApplyState* sts, const uint32_t* rt0,
                                                               const uint32_t* rn, uint32_t nrounds, uint32_t nwg,
-                                                              uint32_t xcd_chunk, uint32_t probe, Bodies B,
-                                                              Cells C, Work w) {
+                                                              uint32_t xcd_chunk, uint32_t probe, uint32_t tag,
+                                                              Bodies B, Cells C, Work w) {
   __shared__ Geometry sg;
   __shared__ TileCfg stc;
   const uint32_t b = blockIdx.x;
@@ -358,7 +452,8 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_bapply_tile(const BatchRep*
     const uint32_t* gsrc = (const uint32_t*)&reps[r].g;
     for (uint32_t i = threadIdx.x; i < sizeof(Geometry) / 4; i += blockDim.x) ((uint32_t*)&sg)[i] = gsrc[i];
     const uint32_t* tsrc = (const uint32_t*)&tcs[r];
-    for (uint32_t i = threadIdx.x; i < sizeof(TileCfg) / 4; i += blockDim.x) ((uint32_t*)&stc)[i] = tsrc[i];
+    for (uint32_t i = threadIdx.x; i < sizeof(TileCfg) / 4; i += blockDim.x)
+      ((uint32_t*)&stc)[i] = i == offsetof(TileCfg, tag) / 4 ? tag : tsrc[i];
     __syncthreads();
     Work wr = w;
     wr.start = w.start + reps[r].space_off;
@@ -366,7 +461,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_bapply_tile(const BatchRep*
     wr.tracing = 0;
     // the ziggurat layers from the constant tables: the LDS they would take
     // is worth more as region entries here (more regions per CU)
-    apply_tile_run<D>(sg, sts + r, B, C, wr, stc, gt - toff[r], &w.acc_slots[r], kZigX, kZigF);
+    apply_tile_run<D, 1>(sg, sts + r, B, C, wr, stc, gt - toff[r], &w.acc_slots[r], kZigX, kZigF);
     __syncthreads();  // sg and stc are rewritten for the next round
   }
 }
@@ -376,6 +471,6 @@ template __global__ void k_apply_tile<2>(Geometry g, ApplyState* st, Bodies B, C
 template __global__ void k_apply_tile<3>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
 template __global__ void k_bapply_tile<3>(const BatchRep*, const TileCfg*, const uint32_t*, const uint32_t*,
                                           ApplyState*, const uint32_t*, const uint32_t*, uint32_t, uint32_t, uint32_t,
-                                          uint32_t, Bodies, Cells, Work);
+                                          uint32_t, uint32_t, Bodies, Cells, Work);
 
 }  // namespace hmc

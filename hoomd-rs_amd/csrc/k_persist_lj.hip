@@ -191,84 +191,6 @@ __device__ __forceinline__ bool lj_decide64(Sfc64& rng, const Lj64& s, double kT
   return lj_metropolis(rng, dH, delta, kT, amb) != 0;
 }
 
-// The halo reload of region_reload with the entries, not the cells, shared
-// out over the workgroup (an isotropic region's cells hold ~15 sites each):
-// wave 0 lists the halo cells of `colour` and the prefix of their entry
-// counts (at most kLjHalo cells, (T + 1)^D), then every thread reloads
-// entries tid, tid + NT, ... from the FP64 sites with device-scope loads, all
-// in flight together.  Ends with a barrier.
-constexpr uint32_t kLjHalo = 128;
-template <int D>
-__device__ __forceinline__ void region_reload_flat(const Geometry& g, const TileCfg& tc, const Region& rg,
-                                                   const Bodies& B, const RegionLds& l, uint32_t colour,
-                                                   uint32_t* hlo, uint32_t* hpre) {
-  constexpr int AL = D - 1;
-  const uint32_t CW = tc.E[AL] + 1;
-  const uint32_t tid = threadIdx.x, NT = blockDim.x;
-  if (tid < 64) {
-    uint32_t nc = 1, cnt[3] = {1, 1, 1};
-    for (int a = 0; a < D; ++a) {
-      cnt[a] = tc.T[a] + 1;
-      nc *= cnt[a];
-    }
-    uint32_t base = 0;
-    for (uint32_t c0 = 0; c0 < nc; c0 += 64) {
-      const uint32_t ci = c0 + tid;
-      uint32_t n = 0, ea = 0;
-      if (ci < nc) {
-        uint32_t r = ci, bc[3] = {0, 0, 0};
-        bool own = true;
-        for (int a = D - 1; a >= 0; --a) {
-          const uint32_t j = r % cnt[a];
-          r /= cnt[a];
-          bc[a] = 2 * j + (((colour >> (D - 1 - a)) & 1u) ? 0u : 1u);
-          const int32_t lc = (int32_t)bc[a] - 1;
-          if (lc < 0 || lc >= rg.rl[a]) own = false;
-        }
-        const uint32_t row = D == 3 ? bc[0] * tc.E[1] + bc[1] : bc[0];
-        ea = l.coff[row * CW + bc[AL]];
-        n = own ? 0u : l.coff[row * CW + bc[AL] + 1] - ea;
-      }
-      const uint32_t incl = wave_incl_scan(n);
-      if (ci < nc) {
-        hlo[ci] = ea;
-        hpre[ci] = base + incl - n;
-      }
-      base += __shfl(incl, 63, 64);
-    }
-    if (tid == 0) hpre[nc] = base;
-  }
-  __syncthreads();
-  uint32_t nc = 1;
-  for (int a = 0; a < D; ++a) nc *= tc.T[a] + 1;
-  const uint32_t total = hpre[nc];
-  for (uint32_t e0 = 0; e0 < total; e0 += 2 * NT) {
-    uint32_t dst[2] = {0, 0}, bd[2] = {0, 0};
-    double4 v[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t e = e0 + (uint32_t)h * NT + tid;
-      if (e < total) {
-        uint32_t lo = 0, hi = nc;  // the cell: the last k with hpre[k] <= e
-        while (hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (hpre[mid] <= e)
-            lo = mid;
-          else
-            hi = mid;
-        }
-        dst[h] = hlo[lo] + (e - hpre[lo]);
-        bd[h] = (uint32_t)__float_as_int(l.lb[dst[h]].w);
-        v[h] = ld_dev_d4(&B.spos[bd[h]]);
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      if (e0 + (uint32_t)h * NT + tid < total) l.lb[dst[h]] = stage_entry64<D>(g, rg.c64, v[h], bd[h]);
-  }
-  __syncthreads();
-}
-
 template <int D>
 __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, ApplyState* st, Bodies B, Cells C, Work w,
                                                              TileCfg tc) {
@@ -289,11 +211,10 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
   float4* lb = l.lb;
   __shared__ double zx[257], zf[257];
   __shared__ unsigned blk_acc;
-  __shared__ uint32_t hlo[kLjHalo], hpre[kLjHalo + 1];
+  __shared__ uint32_t hcnt[kHaloLists];
   __shared__ LjProp prop[kLjMaxTrials];
   __shared__ float shr[2][kLjRegionThreads / 32][11];  // shared trials: per half-wave partial sums, two buffers
   const uint32_t tid = threadIdx.x;
-  const uint32_t wid = tid >> 6, lane = tid & 63u;
   const uint32_t hw = tid >> 5, hl = tid & 31u, G = blockDim.x >> 5;  // trials hw, hw + G, ...
   const uint32_t cycles = st->cycles, substep0 = st->substep0;
   const uint64_t step = st->step;
@@ -306,13 +227,12 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
   const float sig2 = (float)(g.lj_sigma * g.lj_sigma), eps4 = (float)g.lj_eps4, shift = (float)g.lj_shift;
   const float blo = tc.band_lo, bhi = tc.band_hi, r2_open = tc.r2_open;
   const uint32_t ntr = tc.trials;
-  const uint32_t nnb = D == 3 ? 26u : 8u;
-  const uint32_t nbt = wid == 0 && lane < nnb ? region_neighbour<D>(tc, rg, lane) : tile;
 
   if (D == 3) stage_zig(zx, zf);
   if (tid == 0) blk_acc = 0;
-  const bool overflow = region_stage<D>(g, tc, rg, B, C, w, l);
-  if (tid == 0) w.mbox[tile * kMailboxStride + 3] = 1u;  // progress: staged
+  if (tid < (uint32_t)kHaloLists) hcnt[tid] = 0;
+  __shared__ uint32_t odd;  // (sites without images are found by their NaN entries)
+  const bool overflow = region_stage<D, 0>(g, tc, rg, B, C, w, l, &odd);
 
   unsigned retests = 0, ambiguous = 0;
   // The proposals of pass i, drawn while the neighbour regions finish pass
@@ -347,7 +267,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
       const uint32_t e0 = coff[crow * CW + cb[AL]];
       const uint32_t n = coff[crow * CW + cb[AL] + 1] - e0;
       if (n) {
-        Sfc64 rng = counter_rng(step, substep, seed, s);
+        Sfc64 rng = counter_rng<true>(step, substep, seed, s);
         const uint32_t self = e0 + choose_index(rng, n);
         const float4 se = lb[self];
         const uint32_t body = (uint32_t)__float_as_int(se.w);
@@ -356,14 +276,14 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
         ball_sample<D>(rng, max_move, zx, zf, v);
         double x[3] = {bp.x, bp.y, bp.z};
         for (int a = 0; a < D; ++a) x[a] += v[a];
-        for (int a = 0; a < D; ++a) x[a] = wrap1(x[a], g.L[a]);  // generate_trial_moves: wrap(propose(..))
+        for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a]);  // generate_trial_moves: wrap(propose(..))
         double t[3] = {0.0, 0.0, 0.0};
-        for (int a = 0; a < D; ++a) t[a] = wrap1(x[a], g.L[a]);  // wrap(x + 0) == wrap(x)
+        for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a]);  // wrap(x + 0) == wrap(x)
         // update_body_properties (microstate.rs:985-1034): site = wrap(body + 0)
         double nsp[3] = {0.0, 0.0, 0.0};
-        for (int a = 0; a < D; ++a) nsp[a] = wrap1(t[a] + 0.0, g.L[a]);
+        for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
         const double4 sp = pack_site(nsp, ghost_flags<D>(g, nsp));
-        const float4 te = stage_entry64<D>(g, rg.c64, make_double4(t[0], t[1], t[2], 0.0), 0u);
+        const float4 te = box_entry64<D>(g, rg.c64, t, 0u);
         pr.rng = rng;
         for (int a = 0; a < 3; ++a) pr.t[a] = t[a];
         pr.sp = sp;
@@ -515,6 +435,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
 
   const uint32_t npass = cycles * NCOL;
   if (npass && tid < ntr) propose(0, tid);
+  region_halo_lists<D>(tc, rg, l, hcnt);
   __syncthreads();
   unsigned nacc = 0;  // accepted trials (lane 0 of each half-wave)
   for (uint32_t i = 0; i < npass; ++i) {
@@ -546,12 +467,12 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
           ball_sample<D>(rng, max_move, zx, zf, v);
           const double4 bp = B.bpos[body];
           double x[3] = {bp.x, bp.y, bp.z};
-          for (int a = 0; a < D; ++a) x[a] = wrap1(x[a] + v[a], g.L[a]);
+          for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a] + v[a]);
           traced = true;
           tbody = body;
           if (space_of<D>(g, origin, x) == s) {
             double t[3] = {0.0, 0.0, 0.0};
-            for (int a = 0; a < D; ++a) t[a] = wrap1(x[a], g.L[a]);
+            for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a]);
             const double4 sp = ld_dev_d4(&B.spos[body]);
             const double xi[3] = {sp.x, sp.y, sp.z};
             // candidates: the slots of the 3^D neighbour spaces in order, their
@@ -595,7 +516,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
             ambiguous += (amb && hl == 0) ? 1u : 0u;
             if (accepted && hl == 0) {
               double nsp[3] = {0.0, 0.0, 0.0};
-              for (int a = 0; a < D; ++a) nsp[a] = wrap1(t[a] + 0.0, g.L[a]);
+              for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
               B.bpos[body] = make_double4(t[0], t[1], t[2], stamp);
               st_dev_d4(&B.spos[body], pack_site(nsp, ghost_flags<D>(g, nsp)));
             }
@@ -691,15 +612,16 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
       }
     }
     if (i + 1 == npass) break;  // no later pass reads the halo
-    region_publish(w.mbox, nbt, nnb, i & 1u);
-    if (tid == 0) w.mbox[tile * kMailboxStride + 4] = i + 1;  // progress: passes published
+    region_publish(w.mbox, tile, tc.tag, i + 1);
     if (tid < ntr) propose(i + 1, tid);
-    region_wait(st, w.mbox, tile, nnb, i);
-    if (tid == 0) w.mbox[tile * kMailboxStride + 5] = i + 1;  // progress: waits passed
-    if (!overflow)
-      region_reload_flat<D>(g, tc, rg, B, l, colour, hlo, hpre);
-    else
-      __syncthreads();
+    region_wait<D>(st, w.mbox, tc, rg, tile, i + 1);
+    // (cells of about 15 entries: 16 lanes each)
+    if (!overflow) {
+      RegionReload<D, 16, 2, 2> reload(g, tc, rg, B, l, hcnt, i + 1);
+      reload.issue();
+      reload.commit(&odd);
+    }
+    __syncthreads();
   }
   lane_add(&st->band_retests, retests);
   lane_add(&st->ambiguous, ambiguous);

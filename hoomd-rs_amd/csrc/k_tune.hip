@@ -107,9 +107,9 @@ __global__ void __launch_bounds__(kEnergyBlock) k_tune_eval(Geometry g, const Ap
   double x[3] = {bp.x, bp.y, D == 3 ? bp.z : 0.0};
   double v[3] = {0.0, 0.0, 0.0};
   ball_sample<D>(r, max_move, zx, zf, v);
-  for (int a = 0; a < D; ++a) x[a] = wrap1(x[a] + v[a], g.L[a]);  // wrap(propose(..))
+  for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a] + v[a]);  // wrap(propose(..))
   double t[3] = {0.0, 0.0, 0.0};
-  for (int a = 0; a < D; ++a) t[a] = wrap1(x[a] + 0.0, g.L[a]);  // the trial's site
+  for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, x[a] + 0.0);  // the trial's site
   bool outside = false;
   double bf = 0.0, bi = 0.0;
   const double ef = site_energy_excl<D>(g, st, B, w, t, body, &bf, &outside);

@@ -12,10 +12,10 @@ namespace hmc {
 // b owns a region of 2 T spaces per axis (the last region along an axis may
 // be shorter) and keeps the region plus a one-space halo -- every cell its
 // trials can read -- in LDS for the whole apply: staged once, its own cells
-// updated in place by its accepted moves, and after the pass of colour c the
-// halo cells of colour c (the only ones other workgroups have changed)
-// reloaded from the FP64 sites.  Consecutive passes are separated by a
-// neighbour synchronisation (below), not by a grid barrier.
+// updated in place by its accepted moves, and before a pass the halo cells
+// that neighbours have changed and this pass is the first to read reloaded
+// from the FP64 sites.  Consecutive passes are separated by a neighbour
+// synchronisation (below), not by a grid barrier.
 //
 // An LDS entry holds the site relative to the box centre in FP32 (NaN for a
 // site without images, as in the per-colour kernel) with the body index in w.
@@ -25,72 +25,164 @@ namespace hmc {
 // (rows x (E_last + 1) LDS offsets of the cell boundaries, 16-bit: a box
 // holds at most kTileLds / 16 entries), then the site entries.
 
-// Neighbour synchronisation of the persistent apply, through mailboxes: two
-// counters per region (one per pass parity), kMailboxStride words apart.
-// After pass i a region adds 1 to the counter i mod 2 of each of its 3^D - 1
-// neighbours (with multiplicity where the region grid wraps onto itself; the
-// relation is symmetric, so every region receives exactly 3^D - 1 per pass)
-// and then waits until its own counter reaches 3^D - 1, which it resets.  A
-// region reads only its own and its neighbours' cells, so once all of them
-// have finished pass i none can be a pass behind or ahead while it runs pass
-// i + 1: nothing it reads is being written.  A neighbour can therefore never
-// finish pass i + 2 (the next use of the same counter) before this region has
-// consumed pass i, and every counter is 0 again when an apply ends.  The
-// FP64 sites that neighbours read are written with device-scope stores, and
-// every wave waits for its stores to complete before the increments are sent
-// (no cache writeback or invalidation: those, issued by the regions that
-// finish first, stalled the ones still working); the neighbours read them
-// with device-scope loads.  One lane per region polls, on a counter of its
-// own.  The launch is cooperative, so every
-// region is resident.  The wait is bounded: past the bound the state's error
-// word is set and the wait returns, so every wave still ends.
-__device__ __forceinline__ void region_publish(uint32_t* mbox, uint32_t nbt, uint32_t nnb, uint32_t parity) {
+// Neighbour synchronisation of the persistent apply.  Every region has one
+// 64-bit progress word (kMailboxStride words apart): the launch's tag and the
+// passes the region has finished in it.
+//
+// What a region waits for before pass j.  Its box's halo holds cells of the
+// neighbour regions; a cell that lies in the halo along the axes A (a
+// non-empty subset) has the space parity its side fixes: odd on the lower
+// side (-1 along the axis), even on the upper one (region lengths are even).
+// The trials of colour j mod 2^D sit on even cells along the axes where j's
+// colour bit is 0 and read only the lower side there, on odd cells where it is
+// 1 and read only the upper side.  So of the 3^D - 1 neighbours only the
+// 2^D - 1 on j's sides are read, one per A, and of their cells only those of
+// colours k whose bits differ from j's on every axis of A.  The region
+// therefore waits, per A, until that neighbour has finished the last such
+// pass k < j (k = j - 1 for one to 2^D - 1 of the subsets: three of seven on
+// average in 3D), and the others may run ahead or behind.
+//
+// Why nothing it reads is being written.  The neighbour Y writes the cells of
+// colour k in this region X's halo along A in passes of k's bits on A, which
+// are exactly the passes whose sides make Y wait for X over A: before writing
+// them again in pass k + 2^D (or for the first time in pass k) Y has waited
+// for X's last pass with the other bits on A, which is or follows every pass of
+// X that reads the values of Y's pass before.  That covers the halo copies,
+// the FP64 sites that re-tests read in place, and regions staged late.
+//
+// The FP64 sites that neighbours read are written with device-scope stores;
+// every wave waits for its stores to complete before the progress word is
+// stored, and neighbours read the sites with device-scope loads (no cache
+// writeback or invalidation).  The launch is cooperative, so every region is
+// resident, and the region whose pass is lowest never waits for one ahead of
+// it, so all of them finish.  Waits are bounded: past the bound the state's
+// error word is set and the wait returns, so every wave still ends.
+//
+// Measured on C2's hard spheres (500 regions, 16 passes): see k_apply_tile.
+// The counters that all 26 neighbours incremented every pass, which this
+// replaces, made every pass last as long as the slowest of 27 regions.
+__device__ __forceinline__ void region_publish(uint32_t* mbox, uint32_t tile, uint32_t tag, uint32_t done) {
   __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have completed
   __syncthreads();
-  if (threadIdx.x < 64) {
-    if (threadIdx.x < nnb)
-      __hip_atomic_fetch_add(&mbox[nbt * kMailboxStride + parity], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-}
-__device__ __forceinline__ void region_wait(ApplyState* st, uint32_t* mbox, uint32_t tile, uint32_t nnb,
-                                            uint32_t pass) {
-  const uint32_t parity = pass & 1u;
-  if (threadIdx.x < 64) {
-    if (threadIdx.x == 0) {
-      uint32_t* box = &mbox[tile * kMailboxStride + parity];
-      uint32_t spins = 0;
-      while (__hip_atomic_load(box, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nnb) {
-        __builtin_amdgcn_s_sleep(1);
-        if (++spins > kBarrierSpins) {
-          atomicOr(&st->error, kErrBarrier);
-          atomicCAS(&st->wait_at, 0u, (tile << 12) | ((pass & 0xfffu) + 1u));
-          break;
-        }
-      }
-      __hip_atomic_store(box, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store((unsigned long long*)&mbox[tile * kMailboxStride], ((unsigned long long)tag << 32) | done,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// LDS entry of the persistent apply from a site's FP64 copy: the image
-// nearest the box centre c, relative to c, computed in FP64 and rounded once
-// to FP32 (NaN for a site without images), body index in w.
+// Box-relative FP32 position: the image of x nearest the box centre c, relative
+// to c, computed in FP64 and rounded once to FP32, w = body.
 template <int D>
-__device__ __forceinline__ float4 stage_entry64(const Geometry& g, const double* c, double4 sp, uint32_t body) {
-  const double x[3] = {sp.x, sp.y, sp.z};
+__device__ __forceinline__ float4 box_entry64(const Geometry& g, const double* c, const double* x, uint32_t body) {
   float r[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int a = 0; a < D; ++a) {
-    double u = x[a] - c[a];
-    if (u >= g.half[a])
-      u -= g.L[a];
-    else if (u < -g.half[a])
-      u += g.L[a];
-    r[a] = (float)u;
+    // (selects, not branches: this is inlined where a pass's latency counts)
+    const double u = x[a] - c[a], back = u >= g.half[a] ? g.L[a] : 0.0;
+    r[a] = (float)(u - (u < -g.half[a] ? -g.L[a] : back));
   }
-  if ((uint32_t)__double_as_longlong(sp.w) & kNoImages) r[0] = __int_as_float(0x7fc00000);
   return make_float4(r[0], r[1], r[2], __int_as_float((int)body));
+}
+// LDS entry of a site: as above, NaN for a site without images (one outside
+// [-L/2, L/2) on some axis, as in ghost_flags), body index in w.
+template <int D>
+__device__ __forceinline__ float4 stage_entry64(const Geometry& g, const double* c, const double* x, uint32_t body) {
+  float4 e = box_entry64<D>(g, c, x, body);
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+    if (x[a] < -g.half[a] || x[a] >= g.half[a]) e.x = __int_as_float(0x7fc00000);
+  return e;
+}
+template <int D>
+__device__ __forceinline__ float4 stage_entry64(const Geometry& g, const double* c, double4 sp, uint32_t body) {
+  const double x[3] = {sp.x, sp.y, sp.z};
+  return stage_entry64<D>(g, c, x, body);
+}
+
+// The system's constants read through the scalar cache where they are used:
+// held in registers across the passes they would not fit (spilled scalars cost
+// a lane read at every use).  Opaque, so that the loads stay in the loop.
+typedef const __attribute__((address_space(4))) Geometry* GeoPtr;
+__device__ __forceinline__ GeoPtr geo_ptr(const Geometry* self) {
+  // (uniform, also where it was read from LDS)
+  const uintptr_t u = (uintptr_t)self;
+  uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  asm volatile("" : "+s"(lo), "+s"(hi));
+  return (GeoPtr)(((uintptr_t)hi << 32) | lo);
+}
+
+// What a proposal x = body + displacement makes of a trial (translate moves):
+// x = wrap(x) (generate_trial_moves: wrap(propose(..))), in: x lies in the
+// trial's own space (multi-index own, as space_of forms it), t = wrap(x) the
+// trial body and site, n = wrap(t + 0) the site update_body_properties stores
+// (microstate.rs:985-1034), flags its ghost images.
+//
+// One lane's latency counts here, so it is all selects: a divergent branch
+// costs a wavefront 40 cycles, an FP64 operation 6.  Quotients by the box
+// edges and space widths are div_const_fast's; a numerator below its range, or
+// constants it does not cover, take trial_site_general (a coordinate of exactly
+// 0 does; other sums and differences of coordinates are far above 2^-900).
+template <int D>
+struct TrialSite {
+  double t[3], n[3];
+  uint32_t flags;
+  bool in;
+};
+__device__ __forceinline__ double wrap_lambda(double lambda, double L) {
+  lambda = lambda - round(lambda);
+  return (lambda == 0.5 ? -0.5 : lambda) * L;
+}
+template <int D>
+__device__ __noinline__ TrialSite<D> trial_site_general(const Geometry* gp, const ApplyState* st, double x0, double x1,
+                                                        double x2, uint32_t s) {
+  const Geometry& g = *gp;
+  TrialSite<D> o;
+  double x[3] = {x0, x1, x2};
+  for (int a = 0; a < D; ++a) x[a] = wrap1(g, a, x[a]);
+  o.in = space_of<D>(g, st->origin, x) == s;
+  for (int a = 0; a < 3; ++a) o.t[a] = o.n[a] = 0.0;
+  for (int a = 0; a < D; ++a) o.t[a] = wrap1(g, a, x[a]);
+  for (int a = 0; a < D; ++a) o.n[a] = wrap1(g, a, o.t[a] + 0.0);
+  o.flags = ghost_flags<D>(g, o.n);
+  return o;
+}
+template <int D>
+__device__ __forceinline__ TrialSite<D> trial_site(GeoPtr g, const ApplyState* st, const double* origin,
+                                                   const double* x0, const uint32_t* own, uint32_t s) {
+  TrialSite<D> o;
+  o.in = true;
+  o.flags = 0;
+  o.t[2] = o.n[2] = 0.0;
+  double least = 1.0;  // of the numerators' magnitudes
+  bool images = true;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const double L = g->L[a], y = g->inv_L[a], wd = g->width[a], yw = g->inv_width[a];
+    const double x = wrap_lambda(div_const_fast(x0[a], L, y), L);
+    const double p = x - origin[a];
+    double q = floor(div_const_fast(p, wd, yw));
+    q = q == (double)g->shape[a] ? 0.0 : q;
+    o.in = o.in & (q == (double)own[a]);
+    const double t = wrap_lambda(div_const_fast(x, L, y), L);
+    const double n = wrap_lambda(div_const_fast(t + 0.0, L, y), L);
+    least = fmin(fmin(least, fabs(x0[a])), fmin(fmin(fabs(x), fabs(p)), fabs(t)));
+    least = fmin(least, fmin(y, yw));
+    o.t[a] = t;
+    o.n[a] = n;
+    images = images & (n >= -g->half[a]) & (n < g->half[a]);
+    o.flags |= (n > g->ghost_hi[a] ? 2u : n < g->ghost_lo[a] ? 1u : 0u) << (2 * a);
+  }
+  o.flags = images ? o.flags : kNoImages;
+  if (!(least >= 0x1p-900)) o = trial_site_general<D>((const Geometry*)(uintptr_t)g, st, x0[0], x0[1], D == 3 ? x0[2] : 0.0, s);
+  return o;
+}
+// box_entry64 with the system's constants through the scalar cache
+template <int D>
+__device__ __forceinline__ void box_relative64(GeoPtr g, const double* c, const double* x, float* r) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const double L = g->L[a], half = g->half[a], u = x[a] - c[a];
+    r[a] = (float)(u - (u >= half ? L : u < -half ? -L : 0.0));
+  }
 }
 
 // Residency probe (tc.probe): the persistent launch relies on every region
@@ -160,189 +252,187 @@ __device__ __forceinline__ Region region_of(const Geometry& g, const TileCfg& tc
   return rg;
 }
 
-// The region that lane l < 3^D - 1 of wave 0 notifies after each pass: its
-// l-th neighbour (with the periodic wrap of the region grid: duplicates, and
-// the region itself, where the grid has fewer than three regions on an axis).
-template <int D>
-__device__ __forceinline__ uint32_t region_neighbour(const TileCfg& tc, const Region& rg, uint32_t lane) {
-  constexpr uint32_t nnb = D == 3 ? 26u : 8u;
-  uint32_t q = lane < nnb / 2 ? lane : lane + 1;  // skip the centre
-  uint32_t nd[3] = {0, 0, 0};
-  for (int a = D - 1; a >= 0; --a) {
-    nd[a] = q % 3u;
-    q /= 3u;
-  }
-  uint32_t nbt = 0;
-  for (int a = 0; a < D; ++a) nbt = nbt * tc.nt[a] + (rg.tcd[a] + tc.nt[a] + nd[a] - 1u) % tc.nt[a];
-  return nbt;
+// Passes back from pass j to the last one whose colour differs from j's on
+// every axis of `axes` (colour-bit mask, non-zero): 1 .. 2^D - 1.
+__host__ __device__ __forceinline__ uint32_t pass_distance(uint32_t j, uint32_t axes) {
+  uint32_t d = 1;
+  while ((((j - d) ^ j) & axes) != axes) ++d;
+  return d;
 }
 
-// LDS of a region's box: ri, coff, then the site entries.
+// Waits before pass j for the neighbours on j's sides (lane A - 1 of the
+// wavefront: the axes A).  Every wavefront polls for itself, so that each goes
+// on to its halo loads without a barrier.
+template <int D>
+__device__ __forceinline__ void region_wait(ApplyState* st, uint32_t* mbox, const TileCfg& tc, const Region& rg,
+                                            uint32_t tile, uint32_t j) {
+  constexpr uint32_t NS = (1u << D) - 1u;
+  const uint32_t lane = __lane_id();
+  if (lane < NS) {
+    const uint32_t axes = lane + 1u, d = pass_distance(j, axes);
+    uint32_t nb = 0;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const uint32_t bit = 1u << (D - 1 - a), n = tc.nt[a];
+      uint32_t t = rg.tcd[a];
+      if (axes & bit) t = (j & bit) ? (t + 1u == n ? 0u : t + 1u) : (t == 0u ? n - 1u : t - 1u);
+      nb = nb * n + t;
+    }
+    if (j >= d && nb != tile) {
+      const uint32_t need = j - d + 1u;
+      const unsigned long long* word = (const unsigned long long*)&mbox[nb * kMailboxStride];
+      uint32_t spins = 0;
+      for (;;) {
+        const unsigned long long v = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)(v >> 32) == tc.tag && (uint32_t)v >= need) break;
+        __builtin_amdgcn_s_sleep(1);
+        if (++spins > kBarrierSpins) {
+          atomicOr(&st->error, kErrBarrier);
+          atomicCAS(&st->wait_at, 0u, (tile << 12) | ((j & 0xfffu) + 1u));
+          break;
+        }
+      }
+    }
+  }
+  // (no later load of this wavefront moves above the polls)
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// LDS of a region's box: ri (staging only), whose space the halo cell lists
+// take over afterwards, coff, then the site entries.
 struct RegionLds {
   uint4* ri;
+  uint16_t* halo;
   uint16_t* coff;
   float4* lb;
 };
+// bytes of ri / the halo lists
+__host__ __device__ inline uint32_t region_head_bytes(uint32_t rows, uint32_t halo_cells) {
+  const uint32_t a = 16u * (rows + 1), b = (2u * halo_cells + 15u) & ~15u;
+  return a > b ? a : b;
+}
 template <int D>
 __device__ __forceinline__ RegionLds region_lds(unsigned char* smem, const TileCfg& tc) {
   const uint32_t R = tc.rows, CW = tc.E[D - 1] + 1;
+  const uint32_t head = region_head_bytes(R, tc.hoff[kHaloLists]);
   RegionLds l;
   l.ri = (uint4*)smem;
-  l.coff = (uint16_t*)(smem + 16u * (R + 1));
-  l.lb = (float4*)(smem + ((16u * (R + 1) + 2u * R * CW + 15u) & ~15u));
+  l.halo = (uint16_t*)smem;
+  l.coff = (uint16_t*)(smem + head);
+  l.lb = (float4*)(smem + ((head + 2u * R * CW + 15u) & ~15u));
   return l;
 }
 
 // Stages the region's box into LDS once per apply: every row's runs and cell
 // starts, then the sites (their FP64 copies as box-relative FP32 entries with
-// the body index).  Wave 0 loads the runs and scans the row lengths; every
-// thread loads cell starts with coalesced loads; a half-wave per row copies
-// its runs.  Ends with a barrier; returns true (uniform over the workgroup)
-// when the box holds more sites than the LDS capacity tc.maxb, in which case
-// no entries were written.
-template <int D>
+// the body index).  A thread per row loads its runs, wave 0 scans the row
+// lengths, and a half-wave per row copies its cell starts and its runs,
+// kStageRows rows in flight together.  Ends with a barrier; returns true
+// (uniform over the workgroup) when the box holds more sites than the LDS
+// capacity tc.maxb, in which case no entries were written.  PAD entries out of
+// reach follow the box's.  *odd (zeroed before) is set when a staged site has
+// no images, i.e. its entry is NaN.
+//
+// Written for few instructions: every launch fetches its code anew, a cache
+// line at a time, and straight-line code that runs once costs more in fetches
+// than in execution.  (With the cell starts taken 16 to a thread in unrolled
+// loops and the image selection in branches, the part of the kernel before
+// the first trial took 50 us of C2's 280 us apply.)
+template <int D, int PAD>
 __device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& tc, const Region& rg, const Bodies& B,
-                                             const Cells& C, const Work& w, const RegionLds& l) {
+                                             const Cells& C, const Work& w, const RegionLds& l, uint32_t* odd) {
   constexpr int AL = D - 1;
   const uint32_t R = tc.rows, EL = tc.E[AL], CW = EL + 1;
   const uint32_t tid = threadIdx.x, NT = blockDim.x;
-  const uint32_t wid = tid >> 6, lane = tid & 63u;
   const uint32_t p = rg.p, m0 = rg.m0;
-  const int32_t* mlo = rg.mlo;
   uint4* ri = l.ri;
   uint16_t* coff = l.coff;
   float4* lb = l.lb;
-  const uint32_t rpl = (R + 63) / 64;
-  uint32_t rq[kRowsPerLane][4];
-  if (wid == 0) {
+  // per row: its runs' lengths, first slots and the space it starts at (a run
+  // past 16 bits is no box that fits)
+  const uint32_t e1m = D == 3 ? (65536u + tc.E[1] - 1u) / tc.E[1] : 0u;  // row / E1 (rows <= 256)
+  for (uint32_t r = tid; r < R; r += NT) {
+    const uint32_t e0 = D == 3 ? (r * e1m) >> 16 : r;
+    const uint32_t e[2] = {e0, D == 3 ? r - e0 * tc.E[1] : 0u};
+    uint32_t sb = 0;
 #pragma unroll
-    for (int u = 0; u < kRowsPerLane; ++u) {
-      const uint32_t r = min(lane * rpl + (uint32_t)u, R - 1);
-      uint32_t sb = 0, q = r;
-      for (int a = AL - 1; a >= 0; --a) {
-        const uint32_t e = a > 0 ? q % tc.E[a] : q;
-        q = a > 0 ? q / tc.E[a] : 0u;
-        const int32_t sh = g.shape[a];
-        int32_t mm = mlo[a] + (int32_t)e;
-        mm = mm < 0 ? mm + sh : (mm >= sh ? mm - sh : mm);
-        sb += (uint32_t)mm * g.stride[a];
-      }
-      rq[u][0] = w.start[sb + m0];
-      rq[u][1] = w.start[sb + m0 + p];
-      rq[u][2] = w.start[sb];
-      rq[u][3] = w.start[sb + (EL - p)];
+    for (int a = 0; a < AL; ++a) {
+      const int32_t sh = g.shape[a], mm = rg.mlo[a] + (int32_t)e[a];
+      sb += (uint32_t)(mm < 0 ? mm + sh : (mm >= sh ? mm - sh : mm)) * g.stride[a];
     }
+    const uint32_t a0 = w.start[sb + m0], a1 = w.start[sb + m0 + p], b0 = w.start[sb], b1 = w.start[sb + (EL - p)];
+    ri[r] = make_uint4(min(a1 - a0, 0xffffu) | (min(b1 - b0, 0xffffu) << 16), a0, b0, sb);
   }
-  const uint32_t nvals = (R * (EL + 2) + NT - 1) / NT;
-  uint32_t raw[kValsPerThread], key[kValsPerThread];
-  {
-    uint32_t d[3] = {0, 0, 0};
-    uint32_t r = tid;
-    for (int a = AL; a > 0; --a) {
-      const uint32_t rad = a == AL ? EL + 2 : tc.E[a];
-      d[a] = r % rad;
-      r /= rad;
-    }
-    d[0] = r;
-#pragma unroll
-    for (int i = 0; i < kValsPerThread; ++i) {
-      raw[i] = 0u;
-      key[i] = 0xffffffffu;
-      if ((uint32_t)i < nvals) {
-        if (d[0] < tc.E[0]) {
-          uint32_t sb = 0, row = 0;
-          for (int a = 0; a < AL; ++a) {
-            const int32_t sh = g.shape[a];
-            int32_t mm = mlo[a] + (int32_t)d[a];
-            mm = mm < 0 ? mm + sh : (mm >= sh ? mm - sh : mm);
-            sb += (uint32_t)mm * g.stride[a];
-            row = row * tc.E[a] + d[a];
-          }
-          const uint32_t j = d[AL];
-          raw[i] = w.start[j <= p ? sb + m0 + j : sb + (j - p - 1)];
-          key[i] = (row << 8) | j;
-        }
-        uint32_t carry = 0;
-        for (int a = AL; a >= 0; --a) {
-          d[a] += tc.step[a] + carry;
-          carry = 0;
-          const uint32_t rad = a == AL ? EL + 2 : tc.E[a];
-          if (a > 0 && d[a] >= rad) {
-            d[a] -= rad;
-            carry = 1;
-          }
-        }
-      }
-    }
-  }
-  if (wid == 0) {
-    uint32_t len[kRowsPerLane], sum = 0;
-#pragma unroll
-    for (int u = 0; u < kRowsPerLane; ++u) {
-      const uint32_t r = lane * rpl + (uint32_t)u;
-      len[u] = (uint32_t)u < rpl && r < R ? (rq[u][1] - rq[u][0]) + (rq[u][3] - rq[u][2]) : 0u;
-      sum += len[u];
-    }
+  __syncthreads();
+  if (tid < 64) {
+    const uint32_t rpl = (R + 63) / 64, r0 = tid * rpl, r1 = min(r0 + rpl, R);
+    uint32_t sum = 0;
+    for (uint32_t r = r0; r < r1; ++r) sum += (ri[r].x & 0xffffu) + (ri[r].x >> 16);
     const uint32_t incl = wave_incl_scan(sum);
     uint32_t off = incl - sum;
-#pragma unroll
-    for (int u = 0; u < kRowsPerLane; ++u) {
-      const uint32_t r = lane * rpl + (uint32_t)u;
-      if ((uint32_t)u < rpl && r < R) ri[r] = make_uint4(off, rq[u][0], rq[u][1] - rq[u][0], rq[u][2]);
-      off += len[u];
+    for (uint32_t r = r0; r < r1; ++r) {
+      const uint32_t x = ri[r].x;
+      ri[r].x = (off & 0xffffu) | (x << 16);  // LDS offset, first run's length
+      off += (x & 0xffffu) + (x >> 16);
     }
-    if (lane == 63) ri[R] = make_uint4(incl, 0u, 0u, 0u);
+    if (tid == 63) ri[R].x = incl;
   }
   __syncthreads();
   const uint32_t total = ri[R].x;
-  const bool overflow = total > tc.maxb;  // uniform over the workgroup
+  const bool overflow = total > tc.maxb;  // uniform over the workgroup; else every offset fits 16 bits
   if (!overflow) {
+    if (tid < (uint32_t)PAD) lb[total + tid] = make_float4(kTileFar, 0.0f, 0.0f, 0.0f);
     const uint32_t hw = tid >> 5, hl = tid & 31u, NH = NT >> 5;
+    // boundary j of a row (j <= p) is the start of space m0 + j, the next ones
+    // that of j - p - 1 after the wrap; its LDS offset is written at j or j - 1
+    auto boundary = [&](const uint4& q, uint32_t r, uint32_t j, uint32_t start) {
+      const uint32_t o = q.x & 0xffffu;
+      coff[r * CW + (j <= p ? j : j - 1)] = (uint16_t)(j <= p ? o + (start - q.y) : o + (q.x >> 16) + (start - q.z));
+    };
+    auto slot_of = [&](const uint4& q, uint32_t e) {
+      return e < (q.x >> 16) ? q.y + e : q.z + (e - (q.x >> 16));
+    };
+    auto put = [&](uint32_t dst, const double4& sp, uint32_t body) {
+      const float4 en = stage_entry64<D>(g, rg.c64, sp, body);
+      lb[dst] = en;
+      if (!(en.x == en.x)) *odd = 1;
+    };
+#pragma unroll 1
     for (uint32_t r0 = hw; r0 < R; r0 += NH * kStageRows) {
-      uint32_t dst[kStageRows], src[kStageRows], bod[kStageRows];
+      uint4 q[kStageRows];
+      uint32_t len[kStageRows], bod[kStageRows], raw[kStageRows];
 #pragma unroll
       for (int u = 0; u < kStageRows; ++u) {
-        const uint32_t r = r0 + (uint32_t)u * NH;
-        dst[u] = 0xffffffffu;
-        src[u] = 0u;
-        if (r < R) {
-          const uint4 q = ri[r];
-          const uint32_t len = ri[r + 1].x - q.x;
-          if (hl < len) {
-            src[u] = hl < q.z ? q.y + hl : q.w + (hl - q.z);
-            dst[u] = q.x + hl;
-          }
-        }
-        if (dst[u] != 0xffffffffu) bod[u] = C.body[src[u]];
+        const uint32_t r = min(r0 + (uint32_t)u * NH, R - 1);
+        q[u] = ri[r];
+        len[u] = (ri[r + 1].x & 0xffffu) - (q[u].x & 0xffffu);
+        if (r0 + (uint32_t)u * NH >= R) len[u] = 0;
+        if (hl < len[u]) bod[u] = C.body[slot_of(q[u], hl)];
+        if (hl < EL + 2) raw[u] = w.start[q[u].w + (hl <= p ? m0 + hl : hl - p - 1)];
       }
       double4 tmp[kStageRows];
 #pragma unroll
       for (int u = 0; u < kStageRows; ++u)
-        if (dst[u] != 0xffffffffu) tmp[u] = B.spos[bod[u]];
+        if (hl < len[u]) tmp[u] = B.spos[bod[u]];
 #pragma unroll
-      for (int u = 0; u < kStageRows; ++u)
-        if (dst[u] != 0xffffffffu) lb[dst[u]] = stage_entry64<D>(g, rg.c64, tmp[u], bod[u]);
-      // entries past the first 32 of a row (rare)
+      for (int u = 0; u < kStageRows; ++u) {
+        const uint32_t r = min(r0 + (uint32_t)u * NH, R - 1);  // (the last row again: the same values)
+        if (hl < EL + 2) boundary(q[u], r, hl, raw[u]);
+        if (hl < len[u]) put((q[u].x & 0xffffu) + hl, tmp[u], bod[u]);
+      }
+      // entries and boundaries past the first 32 of a row
 #pragma unroll 1
       for (int u = 0; u < kStageRows; ++u) {
-        const uint32_t r = r0 + (uint32_t)u * NH;
-        if (r >= R) continue;
-        const uint4 q = ri[r];
-        const uint32_t len = ri[r + 1].x - q.x;
-        for (uint32_t e = 32u + hl; e < len; e += 32u) {
-          const uint32_t sl = e < q.z ? q.y + e : q.w + (e - q.z);
-          const uint32_t bd = C.body[sl];
-          lb[q.x + e] = stage_entry64<D>(g, rg.c64, B.spos[bd], bd);
+        const uint32_t r = min(r0 + (uint32_t)u * NH, R - 1);
+        const uint4 qr = ri[r];
+        const uint32_t o = qr.x & 0xffffu, n = (ri[r + 1].x & 0xffffu) - o;
+        for (uint32_t e = 32u + hl; e < max(n, EL + 2); e += 32u) {
+          if (e < EL + 2) boundary(qr, r, e, w.start[qr.w + (e <= p ? m0 + e : e - p - 1)]);
+          if (e < n) {
+            const uint32_t bd = C.body[slot_of(qr, e)];
+            put(o + e, B.spos[bd], bd);
+          }
         }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kValsPerThread; ++i) {
-      if (key[i] != 0xffffffffu) {
-        const uint32_t r = key[i] >> 8, j = key[i] & 0xffu;
-        const uint4 q = ri[r];
-        coff[r * CW + (j <= p ? j : j - 1)] =
-            (uint16_t)(j <= p ? q.x + (raw[i] - q.y) : q.x + q.z + (raw[i] - q.w));
       }
     }
   }
@@ -350,63 +440,127 @@ __device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& t
   return overflow;
 }
 
-// After the wait that follows the pass of `colour`: reloads the halo cells of
-// that colour -- box cells b with b = 1 - off (mod 2) per axis whose space
-// lies outside the region, the only ones other regions changed -- from the
-// FP64 sites, with device-scope loads (the first kRefreshHeld entries of a
-// thread are loaded together).  Ends with a barrier.
+// The halo cells of the box by the pass class (pass mod 2^D) that first reads
+// them after they change: list q holds, at halo[hoff[q]], the hcnt[q] cells
+// (index of their first boundary in coff) to reload before the passes j = q
+// (mod 2^D).  A cell of colour k in the halo along A is first read in the next
+// pass whose bits differ from k's on A.  Geometry alone decides, so the lists'
+// places are those of a full region (hoff, filled by the host); a shorter
+// region at the end of an axis has no more cells in any of them.  hcnt must be
+// zero, and a barrier must separate the staging from this and this from the
+// first reload.  (Listing by cell, not by entry: no capacity to overflow, and
+// built while the first proposals are drawn.)
 template <int D>
-__device__ __forceinline__ void region_reload(const Geometry& g, const TileCfg& tc, const Region& rg, const Bodies& B,
-                                              const RegionLds& l, uint32_t colour) {
+__host__ __device__ __forceinline__ uint32_t halo_list(const int32_t* lc, const int32_t* rl) {
+  uint32_t axes = 0, k = 0;
+  for (int a = 0; a < D; ++a) {
+    const uint32_t bit = 1u << (D - 1 - a);
+    if (lc[a] > rl[a]) return UINT32_MAX;  // past the halo of a short region
+    if (lc[a] < 0 || lc[a] == rl[a]) axes |= bit;
+    if (lc[a] & 1) k |= bit;  // (-1 is odd)
+  }
+  if (!axes) return UINT32_MAX;
+  uint32_t d = 1;
+  while (((k ^ (k + d)) & axes) != axes) ++d;
+  return (k + d) & ((1u << D) - 1u);
+}
+template <int D>
+__device__ __forceinline__ void region_halo_lists(const TileCfg& tc, const Region& rg, const RegionLds& l,
+                                                  uint32_t* hcnt) {
   constexpr int AL = D - 1;
-  const uint32_t CW = tc.E[AL] + 1;
-  const uint32_t tid = threadIdx.x, NT = blockDim.x;
-  const int32_t* rl = rg.rl;
-  const uint16_t* coff = l.coff;
-  float4* lb = l.lb;
-  uint32_t hdst[kRefreshHeld];
-  double4 hval[kRefreshHeld];
-  uint32_t nheld = 0;
-  {
-    uint32_t nc = 1, cnt[3] = {1, 1, 1};
-    for (int a = 0; a < D; ++a) {
-      cnt[a] = tc.T[a] + 1;
-      nc *= cnt[a];
-    }
-    for (uint32_t ci = tid; ci < nc; ci += NT) {
-      uint32_t r = ci, bc[3] = {0, 0, 0};
-      bool own = true;
-      for (int a = D - 1; a >= 0; --a) {
-        const uint32_t j = r % cnt[a];
-        r /= cnt[a];
-        bc[a] = 2 * j + (((colour >> (D - 1 - a)) & 1u) ? 0u : 1u);
-        const int32_t lc = (int32_t)bc[a] - 1;
-        if (lc < 0 || lc >= rl[a]) own = false;
-      }
-      if (own) continue;
-      const uint32_t row = D == 3 ? bc[0] * tc.E[1] + bc[1] : bc[0];
-      const uint32_t ea = coff[row * CW + bc[AL]], eb = coff[row * CW + bc[AL] + 1];
-      for (uint32_t e = ea; e < eb; ++e) {
-        const uint32_t bd = (uint32_t)__float_as_int(lb[e].w);
-        const double4 v = ld_dev_d4(&B.spos[bd]);
-        if (nheld < (uint32_t)kRefreshHeld) {
+  const uint32_t EL = tc.E[AL], E1 = D == 3 ? tc.E[1] : 1u;
+  const uint32_t elm = 0xffffffffu / EL + 1u, e1m = (65536u + E1 - 1u) / E1;  // / EL, / E1
+#pragma unroll 1
+  for (uint32_t ci = threadIdx.x; ci < tc.ncell; ci += blockDim.x) {
+    const uint32_t row = __umulhi(ci, elm), j = ci - row * EL, e0 = D == 3 ? (row * e1m) >> 16 : row;
+    const int32_t lc[3] = {(int32_t)e0 - 1, D == 3 ? (int32_t)(row - e0 * E1) - 1 : (int32_t)j - 1, (int32_t)j - 1};
+    const uint32_t q = halo_list<D>(lc, rg.rl);
+    if (q != UINT32_MAX) l.halo[tc.hoff[q] + atomicAdd(&hcnt[q], 1u)] = (uint16_t)(row * (EL + 1) + j);
+  }
+}
+
+// After the wait before pass j: reloads the halo cells whose new values pass j
+// is the first to read, from the FP64 sites with device-scope loads.  LPC lanes
+// per cell (lane `sub` takes entries sub, sub + LPC, ...).  issue() puts HELD
+// entries of CELLS cells per lane in flight together; commit() writes
+// their LDS entries and takes whatever is left (cells of more than HELD LPC
+// entries, lists of more than CELLS NT / LPC cells), one memory latency
+// per round.  *odd is set where an entry is NaN (a site without images).  No
+// barrier: one must follow before other wavefronts read the entries.
+template <int D, int LPC, int CELLS, int HELD>
+struct RegionReload {
+  const Geometry& g;
+  const Region& rg;
+  const Bodies& B;
+  const RegionLds& l;
+  const uint16_t* list;
+  uint32_t n, step, c0;
+  uint32_t e[CELLS], eb[CELLS];
+  double v[CELLS][HELD][3];
+
+  __device__ __forceinline__ RegionReload(const Geometry& g_, const TileCfg& tc, const Region& rg_, const Bodies& B_,
+                                          const RegionLds& l_, const uint32_t* hcnt, uint32_t j)
+      : g(g_), rg(rg_), B(B_), l(l_) {
+    const uint32_t q = j & ((1u << D) - 1u);
+    n = hcnt[q];
+    list = l.halo + tc.hoff[q];
+    step = blockDim.x / LPC;
+    c0 = threadIdx.x / LPC;
+  }
+  __device__ __forceinline__ void issue() {
+    const uint32_t sub = threadIdx.x % LPC;
 #pragma unroll
-          for (int h = 0; h < kRefreshHeld; ++h)
-            if ((uint32_t)h == nheld) {
-              hdst[h] = e;
-              hval[h] = v;
-            }
-          ++nheld;
-        } else {
-          lb[e] = stage_entry64<D>(g, rg.c64, v, bd);
-        }
+    for (int u = 0; u < CELLS; ++u) {
+      const uint32_t c = c0 + (uint32_t)u * step;
+      e[u] = eb[u] = 0;
+      if (c < n) {
+        const uint32_t cell = list[c];
+        e[u] = l.coff[cell] + sub;
+        eb[u] = l.coff[cell + 1];
+      }
+    }
+    uint32_t bd[CELLS][HELD];
+#pragma unroll
+    for (int u = 0; u < CELLS; ++u)
+#pragma unroll
+      for (int h = 0; h < HELD; ++h)
+        if (e[u] + (uint32_t)(h * LPC) < eb[u]) bd[u][h] = (uint32_t)__float_as_int(l.lb[e[u] + (uint32_t)(h * LPC)].w);
+#pragma unroll
+    for (int u = 0; u < CELLS; ++u)
+#pragma unroll
+      for (int h = 0; h < HELD; ++h)
+        if (e[u] + (uint32_t)(h * LPC) < eb[u]) fetch(bd[u][h], v[u][h]);
+  }
+  __device__ __forceinline__ void fetch(uint32_t body, double* sp) const {
+    const double* q = (const double*)&B.spos[body];
+#pragma unroll
+    for (int a = 0; a < D; ++a) sp[a] = __longlong_as_double((long long)ld_dev(q + a));
+  }
+  __device__ __forceinline__ void put(uint32_t x, const double* sp, uint32_t* odd) const {
+    const float4 en = stage_entry64<D>(g, rg.c64, sp, (uint32_t)__float_as_int(l.lb[x].w));
+    l.lb[x] = en;
+    if (!(en.x == en.x)) *odd = 1;
+  }
+  __device__ __forceinline__ void commit(uint32_t* odd) {
+#pragma unroll
+    for (int u = 0; u < CELLS; ++u)
+#pragma unroll
+      for (int h = 0; h < HELD; ++h)
+        if (e[u] + (uint32_t)(h * LPC) < eb[u]) put(e[u] + (uint32_t)(h * LPC), v[u][h], odd);
+    // what is left: entries past HELD of the cells in hand, then further cells
+    uint32_t c = c0, held = (uint32_t)(HELD * LPC);
+#pragma unroll 1
+    for (; c < n; c += step) {
+      if (c >= c0 + CELLS * step) held = 0;
+      const uint32_t cell = list[c];
+#pragma unroll 1
+      for (uint32_t x = l.coff[cell] + threadIdx.x % LPC + held; x < l.coff[cell + 1]; x += LPC) {
+        double sp[3];
+        fetch((uint32_t)__float_as_int(l.lb[x].w), sp);
+        put(x, sp, odd);
       }
     }
   }
-#pragma unroll
-  for (int h = 0; h < kRefreshHeld; ++h)
-    if ((uint32_t)h < nheld) lb[hdst[h]] = stage_entry64<D>(g, rg.c64, hval[h], (uint32_t)__float_as_int(lb[hdst[h]].w));
-  __syncthreads();
-}
+};
 
 }  // namespace hmc

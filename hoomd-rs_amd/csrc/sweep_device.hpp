@@ -80,6 +80,8 @@ struct Geometry {
   // pointer instead of the address of a kernel argument, which would make
   // every lane copy the whole struct to scratch memory at kernel entry.
   const Geometry* self;
+  // correctly rounded 1 / L and 1 / width for div_const_fast (0: divide)
+  double inv_L[3], inv_width[3];
 };
 
 // Mixed-precision hard convex polyhedra: the polytope's separating axes in
@@ -167,7 +169,7 @@ struct Work {
   hmc_trace_record* trace;
   uint64_t trace_cap;
   int tracing;
-  uint32_t* mbox;  // persistent apply: per region two pass counters (by parity), kMailboxStride words apart
+  uint32_t* mbox;  // persistent apply: per region its progress word (64 bits), kMailboxStride words apart
   unsigned long long* scan_status;  // single-pass scan: per block its tagged aggregate or inclusive prefix
 };
 
@@ -179,11 +181,11 @@ __device__ __forceinline__ double move_stamp(uint32_t epoch) { return __longlong
 __device__ __forceinline__ uint32_t stamp_of(double w) { return (uint32_t)__double_as_longlong(w); }
 
 // Periodic<Hypercuboid>::wrap (hoomd-microstate/src/boundary/periodic/cuboid.rs:90-103)
-__device__ __forceinline__ double wrap1(double x, double L) {
-  double lambda = x / L;
+__device__ __forceinline__ double wrap1(const Geometry& g, int a, double x) {
+  double lambda = x / g.L[a];
   lambda = lambda - round(lambda);
   if (lambda == 0.5) lambda = -0.5;
-  return lambda * L;
+  return lambda * g.L[a];
 }
 
 // Ghost image flags of a site (cuboid.rs:108-161): 2 bits per axis,
@@ -515,7 +517,13 @@ struct TileCfg {
   float r2_open;           // isotropic persistent apply: pairs with FP32 r2 below it are left to FP64
   uint32_t probe;          // persistent apply: 1 = only check that every region is resident (region_probe)
   uint32_t step[3];        // the workgroup size in the mixed radix (E0, .., E[D-2], E[D-1] + 2) of the row starts
+  uint32_t tag;            // persistent apply: tells this launch's progress words from older ones
+  uint32_t hoff[9];        // persistent apply: first cell of each halo list of a full region, then their total
 };
+constexpr int kTilePad = 16;           // out-of-reach entries after a hard-shape box's sites (tile_overlaps)
+constexpr float kTileFar = 1e15f;      // their x coordinate
+constexpr uint32_t kMaxRegionRows = 256;  // rows of a region's box (region_stage divides them by 16-bit reciprocals)
+constexpr int kHaloLists = 8;  // halo lists (pass classes) of a region: 2^D of them are used
 
 constexpr int kTileThreads = 256;       // upper bound of the workgroup size
 constexpr int kValsPerThread = 16;      // row starts per thread: rows (E + 2) <= 16 x threads
@@ -578,7 +586,6 @@ __device__ __forceinline__ typename CellCopy<PREC>::type stage_entry(const Geome
 
 // Persistent apply: words between region mailboxes (256 B: separate channels)
 constexpr uint32_t kMailboxStride = 64;       // words between region mailboxes (256 B: separate channels)
-constexpr int kRefreshHeld = 2;               // halo entries per thread loaded together in a refresh
 constexpr int kStageRows = 4;                 // rows per half-wave staged together by the persistent apply
 
 // Device-scope (agent) accesses to the FP64 sites, the only data one region

@@ -403,15 +403,16 @@ int hmc_profile_read(hmc_ctx* ctx, double* pass_ms_total, uint64_t* pass_launche
                      uint64_t* builds);
 
 /* Test hook: the mailbox words of every region of the persistent apply, six
- * per region (the two pass-parity counters, the residency probe's counter in
- * region 0, then the isotropic apply's progress: staged, passes published,
- * waits passed). No reference counterpart. */
+ * per region (the passes finished in the last launch, that launch's tag, the
+ * residency probe's counter in region 0, three unused words). No reference
+ * counterpart. */
 int hmc_debug_regions(hmc_ctx* ctx, uint32_t* out, uint64_t cap, uint64_t* n);
 
 /* Evaluate the library's device math on n inputs: kind 0 cbrt, 1 log,
  * 2 exp, 5 the sine and 6 the cosine of one sincos call (the device's
  * restatements of the glibc functions Rust's std calls on Linux), 3 sqrt,
- * 4 division in[2i]/in[2i+1].  Test hook for bit-exactness checks of the
+ * 4 division in[2i]/in[2i+1], 7 the same through the division by a constant
+ * where it applies.  Test hook for bit-exactness checks of the
  * device arithmetic against the host C library. */
 int hmc_debug_math(int device, int kind, const double* in, double* out, uint64_t n);
 

@@ -45,21 +45,36 @@ Geometry sdf_geometry(const Geometry& g, double xmax) {
   return s;
 }
 
+// Lanes per neighbour query (k_energy, k_insert_energy): half a wavefront where
+// a space holds four bodies or more or there are too few queries to fill the
+// device with eight lanes each.
+static int query_lanes(const Geometry& g, uint64_t queries) {
+  return (uint64_t)g.n_bodies >= 4ull * g.n_spaces || queries < (1u << 16) ? 32 : 8;
+}
+// Sites a group of lanes takes in turn, so that the partials of all blocks fit
+// the scratch's kNoAllocBlocks, and those blocks.
+static uint32_t energy_per(const Geometry& g) {
+  return std::max(1u, grid_for(g.n_bodies, (uint32_t)(kEnergyBlock / query_lanes(g, g.n_bodies)) * kNoAllocBlocks));
+}
+static uint32_t energy_blocks(const Geometry& g) {
+  return grid_for(g.n_bodies, (uint32_t)(kEnergyBlock / query_lanes(g, g.n_bodies)) * energy_per(g));
+}
+
 // PairwiseCutoff::total_energy of the current state with the block partials
-// in part (4 nblk + 4 doubles, nblk = ceil(N / kEnergyBlock)): the cells of
+// in part (4 nblk + 4 doubles, nblk = energy_blocks(g)): the cells of
 // the current counter's checkerboard, k_energy per block, k_energy_final in
 // a fixed order.  Allocates nothing; reads back only the result and the
 // state's error word.
-int total_energy_into(hmc_ctx* c, double* part, double* energy, double* bound) {
+int total_energy_into(hmc_ctx* c, double* part, double* total, double* bound) {
   const Geometry& g = c->g;
   const uint32_t N = g.n_bodies;
   if (N == 0) {
-    *energy = 0.0;
+    *total = 0.0;
     if (bound) *bound = 0.0;
     return HMC_OK;
   }
   hipStream_t s = c->stream;
-  const uint32_t nblk = grid_for(N, kEnergyBlock);
+  const uint32_t nblk = energy_blocks(g), per = energy_per(g);
   // cells for the neighbour search: the checkerboard of the current counter
   k_setup<<<1, 64, 0, s>>>(g, c->st, 0, 0, 0, 1.0, 1.0, 0, 0, 0u, 0);
   if (g.dim == 2)
@@ -70,10 +85,9 @@ int total_energy_into(hmc_ctx* c, double* part, double* energy, double* bound) {
   k_scan_top<<<1, 1024, 0, s>>>(g, c->st, c->w.block_sums, c->w.block_ne, c->n_scan_blocks, c->w.start, 0);
   k_scan_add<<<grid_for(g.n_spaces, 256), 256, 0, s>>>(c->w.start, c->w.block_sums, c->w.cnt, g.n_spaces);
   k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
-  if (g.dim == 2)
-    k_energy<2><<<nblk, kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, part);
-  else
-    k_energy<3><<<nblk, kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, part);
+  const bool wide = query_lanes(g, N) == 32;
+  const auto energy = g.dim == 2 ? (wide ? k_energy<2, 32> : k_energy<2, 8>) : (wide ? k_energy<3, 32> : k_energy<3, 8>);
+  energy<<<nblk, kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, per, part);
   k_energy_final<<<1, kEnergyFinal, 0, s>>>(part, nblk, part + 4 * (size_t)nblk);
   double out[4] = {0, 0, 0, 0};
   uint32_t err = 0;
@@ -88,7 +102,7 @@ int total_energy_into(hmc_ctx* c, double* part, double* energy, double* bound) {
   // any two summation orders of n terms differ by at most 2 gamma_{n-1} sum|terms|
   const double n = std::max(out[2], 1.0);
   const double gam = n * 0x1p-53 / (1.0 - n * 0x1p-53);
-  *energy = out[3] != 0.0 ? std::numeric_limits<double>::infinity() : out[0];
+  *total = out[3] != 0.0 ? std::numeric_limits<double>::infinity() : out[0];
   if (bound) *bound = out[3] != 0.0 ? 0.0 : 2.0 * gam * out[1];
   return HMC_OK;
 }
@@ -228,12 +242,11 @@ int hmc_delta_energy_insert(hmc_ctx* c, const double* body_pos, uint64_t n, doub
   if (e == hipSuccess) e = hipMemsetAsync(flag, 0, sizeof(uint32_t), s);
   if (e == hipSuccess) {
     launch_cell_lists(c);  // cells of the current state, as for the total energy
-    if (D == 2)
-      k_insert_energy<2><<<grid_for(n, kEnergyBlock), kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, dc,
-                                                                           (uint32_t)n, dout, flag);
-    else
-      k_insert_energy<3><<<grid_for(n, kEnergyBlock), kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, dc,
-                                                                           (uint32_t)n, dout, flag);
+    const int lanes = query_lanes(g, n);
+    const auto insert = D == 2 ? (lanes == 32 ? k_insert_energy<2, 32> : k_insert_energy<2, 8>)
+                               : (lanes == 32 ? k_insert_energy<3, 32> : k_insert_energy<3, 8>);
+    insert<<<grid_for(n, (uint32_t)(kEnergyBlock / lanes)), kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, dc,
+                                                                                 (uint32_t)n, dout, flag);
     e = hipGetLastError();
   }
   std::vector<double> hout(2 * (size_t)n);
@@ -261,7 +274,7 @@ int hmc_total_energy(hmc_ctx* c, double* energy, double* bound) {
   if (!c->have_state) return fail(c, HMC_ERR_STATE, "hmc_set_state was not called");
   HIPCHK(c, hipSetDevice(c->device));
   if (c->g.n_bodies == 0) return total_energy_into(c, nullptr, energy, bound);
-  const uint32_t nblk = grid_for(c->g.n_bodies, kEnergyBlock);
+  const uint32_t nblk = energy_blocks(c->g);
   double* part = nullptr;
   HIPCHK(c, hipMallocAsync((void**)&part, (4 * (size_t)nblk + 4) * sizeof(double), c->stream));
   const int rc = total_energy_into(c, part, energy, bound);

@@ -4,106 +4,134 @@
 
 namespace hmc {
 
+// ------------------------------------------------ lanes sharing one query --
+// A site's neighbour query on G lanes: lane gl takes the neighbour spaces gl,
+// gl + G, ... of the 3^D (5^D) around the site's space, each space once.  One
+// lane per site ran all its candidates in a chain of dependent loads on few
+// wavefronts (864 LJ bodies: 4 workgroups, 317 us; on half-waves 22 us).
+// G = 32 where spaces hold several bodies, 8 where they hold about one (the
+// setup every lane of a group repeats then costs more than the candidates):
+// query_lanes on the host.
+struct Neighbours {
+  uint32_t n[3], first[3];  // spaces visited along each axis, the first of them
+};
+template <int D>
+__device__ __forceinline__ Neighbours neighbours_of(const Geometry& g, uint32_t s) {
+  Neighbours q;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) q.n[a] = 1, q.first[a] = 0;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const uint32_t sh = (uint32_t)g.shape[a], r = (uint32_t)g.reach[a], m = (s / g.stride[a]) % sh;
+    const bool all = 2u * r + 1u >= sh;  // the whole axis
+    q.n[a] = all ? sh : 2u * r + 1u;
+    q.first[a] = all ? 0u : (m >= r ? m - r : m + sh - r);
+  }
+  return q;
+}
+template <int D>
+__device__ __forceinline__ uint32_t neighbour_space(const Geometry& g, const Neighbours& q, uint32_t j) {
+  uint32_t s = 0;
+#pragma unroll
+  for (int a = D - 1; a >= 0; --a) {
+    const uint32_t d = j % q.n[a], sh = (uint32_t)g.shape[a];
+    j /= q.n[a];
+    const uint32_t m = q.first[a] + d;
+    s += (m >= sh ? m - sh : m) * g.stride[a];
+  }
+  return s;
+}
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+#pragma unroll
+  for (int d = G / 2; d >= 1; d >>= 1) v += __shfl_xor(v, d, G);
+  return v;
+}
+
 // ------------------------------------------------------------- total energy --
 // PairwiseCutoff::total_energy (pairwise_cutoff.rs:720-745): the sum over
 // sites i and neighbours j with site_tag_i < site_tag_j (body index = site
 // tag for single-site bodies) of the pair energy, infinite on any hard
-// overlap.  Per block: the partial sum, the sum of |terms|, the number of
-// non-zero terms and an overlap flag, reduced in a fixed order.
-
-template <int D>
+// overlap.  Per block of `per` consecutive sites to each group of G lanes: the
+// partial sum, the sum of |terms|, the number of non-zero terms and an overlap
+// flag, reduced in a fixed order.
+template <int D, int G>
 __global__ void __launch_bounds__(kEnergyBlock) k_energy(Geometry g, const ApplyState* st, Bodies B, Work w,
-                                                         double* part) {
+                                                         uint32_t per, double* part) {
   __shared__ double vx[3 * kMaxVertices];
-  __shared__ double re[kEnergyBlock], ra[kEnergyBlock], rn[kEnergyBlock];
+  constexpr int kGroups = kEnergyBlock / G;
+  __shared__ double red[kGroups][3];
   __shared__ int any_inf;
   if (threadIdx.x == 0) any_inf = 0;
   if (g.model == HMC_CONVEX_POLYHEDRON) stage_verts(g, vx);
   __syncthreads();
-  const uint32_t i = blockIdx.x * kEnergyBlock + threadIdx.x;
+  const uint32_t gr = threadIdx.x / G, gl = threadIdx.x % G;
+  const uint32_t i0 = (blockIdx.x * kGroups + gr) * per;
   double e = 0.0, a = 0.0, cnt = 0.0;
   bool inf = false;
-  if (i < g.n_bodies) {
+  for (uint32_t i = i0; i < min(i0 + per, g.n_bodies); ++i) {
     const double4 si = B.spos[i];
     const double t[3] = {si.x, si.y, si.z};
     const double4 bp = B.bpos[i];
     const double x[3] = {bp.x, bp.y, bp.z};
     uint32_t s = space_of<D>(g, st->origin, x);
     if (s == UINT32_MAX) s = 0;  // outside the checkerboard: reported as an error by the host
-    int32_t m[3] = {0, 0, 0};
-    for (int ax = 0; ax < D; ++ax) m[ax] = (int32_t)((s / g.stride[ax]) % (uint32_t)g.shape[ax]);
-    uint32_t nb[3][5];
-    int nn[3] = {1, 1, 1};
-    for (int ax = 0; ax < D; ++ax) {
-      const int32_t sh = g.shape[ax], r = g.reach[ax];
-      int k = 0;
-      for (int off = -r; off <= r; ++off) {
-        const int32_t mm = ((m[ax] + off) % sh + sh) % sh;
-        bool seen = false;
-        for (int j = 0; j < k; ++j) seen |= nb[ax][j] == (uint32_t)mm * g.stride[ax];
-        if (!seen) nb[ax][k++] = (uint32_t)mm * g.stride[ax];
-      }
-      nn[ax] = k;
-    }
+    const Neighbours nq = neighbours_of<D>(g, s);
+    const uint32_t NS = nq.n[0] * nq.n[1] * nq.n[2];
     quat qi = {1.0, {0.0, 0.0, 0.0}};
     if (g.model == HMC_CONVEX_POLYHEDRON) {
       const double4 q4 = B.squat[i];
       qi = {q4.x, {q4.y, q4.z, q4.w}};
     }
-    for (int i0 = 0; i0 < nn[0] && !inf; ++i0)
-      for (int i1 = 0; i1 < nn[1] && !inf; ++i1)
-        for (int i2 = 0; i2 < (D == 3 ? nn[2] : 1) && !inf; ++i2) {
-          const uint32_t ns = nb[0][i0] + nb[1][i1] + (D == 3 ? nb[2][i2] : 0u);
-          const uint32_t q0 = w.start[ns], q1 = w.start[ns + 1];
-          for (uint32_t q = q0; q < q1 && !inf; ++q) {
-            const uint32_t j = w.tmp_body[q];
-            if (j <= i) continue;
-            const double4 sj = B.spos[j];
-            if (g.model == HMC_HARD_SPHERE) {
-              inf = overlap64<D>(g, t, sj);
-            } else if (g.model == HMC_CONVEX_POLYHEDRON) {
-              v3 rj;
-              const double d2 = convex_image(g, t, sj, &rj);
-              if (d2 < g.cv_rcut2) {
-                const double4 q4 = B.squat[j];
-                inf = convex_overlap(vx, g.nverts, g.cv_rcut2, d2, v3{t[0], t[1], t[2]}, qi, rj,
-                                     quat{q4.x, {q4.y, q4.z, q4.w}});
-              }
-            } else {
-              const double r2 = lj_r2<D>(g, t, sj);
-              if (r2 < g.lj_rc2) {
-                const double one = lj_energy(g, r2);
-                if (one == INFINITY) {  // pairwise_cutoff.rs:720-745 returns at once
-                  inf = true;
-                  break;
-                }
-                e += one;
-                a += fabs(one);
-                cnt += 1.0;
-              }
+    for (uint32_t k = gl; k < NS; k += G) {
+      const uint32_t ns = neighbour_space<D>(g, nq, k);
+      const uint32_t q1 = w.start[ns + 1];
+      for (uint32_t q = w.start[ns]; q < q1 && !inf; ++q) {
+        const uint32_t j = w.tmp_body[q];
+        if (j <= i) continue;
+        const double4 sj = B.spos[j];
+        if (g.model == HMC_HARD_SPHERE) {
+          inf = overlap64<D>(g, t, sj);
+        } else if (g.model == HMC_CONVEX_POLYHEDRON) {
+          v3 rj;
+          const double d2 = convex_image(g, t, sj, &rj);
+          if (d2 < g.cv_rcut2) {
+            const double4 q4 = B.squat[j];
+            inf = convex_overlap(vx, g.nverts, g.cv_rcut2, d2, v3{t[0], t[1], t[2]}, qi, rj,
+                                 quat{q4.x, {q4.y, q4.z, q4.w}});
+          }
+        } else {
+          const double r2 = lj_r2<D>(g, t, sj);
+          if (r2 < g.lj_rc2) {
+            const double one = lj_energy(g, r2);
+            if (one == INFINITY) {  // pairwise_cutoff.rs:720-745 returns at once
+              inf = true;
+              break;
             }
+            e += one;
+            a += fabs(one);
+            cnt += 1.0;
           }
         }
+      }
+    }
   }
   if (inf) any_inf = 1;
-  re[threadIdx.x] = e;
-  ra[threadIdx.x] = a;
-  rn[threadIdx.x] = cnt;
+  e = group_sum<G>(e);
+  a = group_sum<G>(a);
+  cnt = group_sum<G>(cnt);
+  if (gl == 0) {
+    red[gr][0] = e;
+    red[gr][1] = a;
+    red[gr][2] = cnt;
+  }
   __syncthreads();
-  for (int h = kEnergyBlock / 2; h >= 1; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      re[threadIdx.x] += re[threadIdx.x + h];
-      ra[threadIdx.x] += ra[threadIdx.x + h];
-      rn[threadIdx.x] += rn[threadIdx.x + h];
-    }
-    __syncthreads();
+  if (threadIdx.x < 3) {
+    double v = 0.0;
+    for (int h = 0; h < kGroups; ++h) v += red[h][threadIdx.x];
+    part[4 * blockIdx.x + threadIdx.x] = v;
   }
-  if (threadIdx.x == 0) {
-    part[4 * blockIdx.x] = re[0];
-    part[4 * blockIdx.x + 1] = ra[0];
-    part[4 * blockIdx.x + 2] = rn[0];
-    part[4 * blockIdx.x + 3] = any_inf ? 1.0 : 0.0;
-  }
+  if (threadIdx.x == 3) part[4 * blockIdx.x + 3] = any_inf ? 1.0 : 0.0;
 }
 
 // Sum of the block partials by one workgroup of kEnergyFinal threads: thread t
@@ -143,66 +171,58 @@ __global__ void __launch_bounds__(kEnergyFinal) k_energy_final(const double* par
 // PairwiseCutoff::delta_energy_insert (pairwise_cutoff.rs:1017-1025 with
 // :420-488): the energy of a new body's site wrap(body + 0) with every site of
 // the microstate (the new body has no tag yet, so nothing is filtered),
-// infinite on a hard overlap or an infinite pair term.  One thread per
+// infinite on a hard overlap or an infinite pair term.  G lanes per
 // candidate over the 3^D (or 5^D) neighbour spaces of the current cells;
 // out[2 k] is the energy, out[2 k + 1] the bound 2 gamma_n sum |terms| on its
 // difference from the reference's summation order.
-template <int D>
+template <int D, int G>
 __global__ void __launch_bounds__(kEnergyBlock) k_insert_energy(Geometry g, const ApplyState* st, Bodies B, Work w,
                                                                 const double* __restrict__ cand, uint32_t n,
                                                                 double* __restrict__ out, uint32_t* outside) {
-  const uint32_t k = blockIdx.x * kEnergyBlock + threadIdx.x;
-  if (k >= n) return;
+  const uint32_t k = blockIdx.x * (kEnergyBlock / G) + threadIdx.x / G, gl = threadIdx.x % G;
+  if (k >= n) return;  // (a whole group)
   double t[3] = {0.0, 0.0, 0.0};
   for (int a = 0; a < D; ++a) t[a] = wrap1(g, a, cand[(size_t)k * D + a] + 0.0);
   const uint32_t s = space_of<D>(g, st->origin, t);
   if (s == UINT32_MAX) {  // outside the checkerboard: reported as an error by the host
-    atomicOr(outside, 1u);
-    out[2 * (size_t)k] = 0.0;
-    out[2 * (size_t)k + 1] = 0.0;
+    if (gl == 0) {
+      atomicOr(outside, 1u);
+      out[2 * (size_t)k] = 0.0;
+      out[2 * (size_t)k + 1] = 0.0;
+    }
     return;
   }
-  int32_t m[3] = {0, 0, 0};
-  for (int ax = 0; ax < D; ++ax) m[ax] = (int32_t)((s / g.stride[ax]) % (uint32_t)g.shape[ax]);
-  uint32_t nb[3][5];
-  int nn[3] = {1, 1, 1};
-  for (int ax = 0; ax < D; ++ax) {
-    const int32_t sh = g.shape[ax], r = g.reach[ax];
-    int kk = 0;
-    for (int off = -r; off <= r; ++off) {
-      const int32_t mm = ((m[ax] + off) % sh + sh) % sh;
-      bool seen = false;
-      for (int j = 0; j < kk; ++j) seen |= nb[ax][j] == (uint32_t)mm * g.stride[ax];
-      if (!seen) nb[ax][kk++] = (uint32_t)mm * g.stride[ax];
-    }
-    nn[ax] = kk;
-  }
+  const Neighbours nq = neighbours_of<D>(g, s);
+  const uint32_t NS = nq.n[0] * nq.n[1] * nq.n[2];
   double e = 0.0, a = 0.0, cnt = 0.0;
   bool inf = false;
-  for (int i0 = 0; i0 < nn[0] && !inf; ++i0)
-    for (int i1 = 0; i1 < nn[1] && !inf; ++i1)
-      for (int i2 = 0; i2 < (D == 3 ? nn[2] : 1) && !inf; ++i2) {
-        const uint32_t ns = nb[0][i0] + nb[1][i1] + (D == 3 ? nb[2][i2] : 0u);
-        const uint32_t q0 = w.start[ns], q1 = w.start[ns + 1];
-        for (uint32_t q = q0; q < q1 && !inf; ++q) {
-          const double4 sj = B.spos[w.tmp_body[q]];
-          if (g.model == HMC_HARD_SPHERE) {
-            inf = overlap64<D>(g, t, sj);
-          } else {
-            const double r2 = lj_r2<D>(g, t, sj);
-            if (r2 < g.lj_rc2) {
-              const double one = lj_energy(g, r2);
-              if (one == INFINITY) {
-                inf = true;
-                break;
-              }
-              e += one;
-              a += fabs(one);
-              cnt += 1.0;
-            }
+  for (uint32_t j = gl; j < NS; j += G) {
+    const uint32_t ns = neighbour_space<D>(g, nq, j);
+    const uint32_t q1 = w.start[ns + 1];
+    for (uint32_t q = w.start[ns]; q < q1 && !inf; ++q) {
+      const double4 sj = B.spos[w.tmp_body[q]];
+      if (g.model == HMC_HARD_SPHERE) {
+        inf = overlap64<D>(g, t, sj);
+      } else {
+        const double r2 = lj_r2<D>(g, t, sj);
+        if (r2 < g.lj_rc2) {
+          const double one = lj_energy(g, r2);
+          if (one == INFINITY) {
+            inf = true;
+            break;
           }
+          e += one;
+          a += fabs(one);
+          cnt += 1.0;
         }
       }
+    }
+  }
+  e = group_sum<G>(e);
+  a = group_sum<G>(a);
+  cnt = group_sum<G>(cnt);
+  inf = group_sum<G>(inf ? 1.0 : 0.0) > 0.0;
+  if (gl != 0) return;
   const double nt = fmax(cnt, 1.0);
   const double gam = nt * 0x1p-53 / (1.0 - nt * 0x1p-53);
   out[2 * (size_t)k] = inf ? INFINITY : e;
@@ -316,10 +336,14 @@ __global__ void __launch_bounds__(kBlock) k_sdf(const BatchRep* reps, const uint
 }
 
 // explicit instantiations (launched from the host translation units)
-template __global__ void k_energy<2>(Geometry g, const ApplyState* st, Bodies B, Work w, double* part);
-template __global__ void k_energy<3>(Geometry g, const ApplyState* st, Bodies B, Work w, double* part);
-template __global__ void k_insert_energy<2>(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
-template __global__ void k_insert_energy<3>(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
+template __global__ void k_energy<2, 8>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_energy<2, 32>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_energy<3, 8>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_energy<3, 32>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_insert_energy<2, 8>(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
+template __global__ void k_insert_energy<2, 32>(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
+template __global__ void k_insert_energy<3, 8>(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
+template __global__ void k_insert_energy<3, 32>(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
 template __global__ void k_sdf<2>(const BatchRep* reps, const uint32_t* boff, uint32_t R, uint32_t n_total, Bodies B, Work w, double xmax, double dx, uint32_t nbins, uint32_t* hist, uint32_t* ovl);
 template __global__ void k_sdf<3>(const BatchRep* reps, const uint32_t* boff, uint32_t R, uint32_t n_total, Bodies B, Work w, double xmax, double dx, uint32_t nbins, uint32_t* hist, uint32_t* ovl);
 

@@ -48,10 +48,10 @@ template <int D, int PREC>
 __global__ void k_bpass_tile(const BatchRep* reps, const TileCfg* tcs, const uint32_t* toff, const uint32_t* trep, ApplyState* sts, uint32_t ntiles, uint32_t xcd_chunk, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle);
 template <int D, int PREC>
 __global__ void k_bguard(const BatchRep* reps, ApplyState* sts, Bodies B, Cells C, Work w, uint32_t first_cycle);
-template <int D>
-__global__ void k_energy(Geometry g, const ApplyState* st, Bodies B, Work w, double* part);
+template <int D, int G>
+__global__ void k_energy(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
 __global__ void k_energy_final(const double* part, uint32_t nblocks, double* out);
-template <int D>
+template <int D, int G>
 __global__ void k_insert_energy(Geometry g, const ApplyState* st, Bodies B, Work w, const double* __restrict__ cand, uint32_t n, double* __restrict__ out, uint32_t* outside);
 template <int D>
 __global__ void k_tune_eval(Geometry g, const ApplyState* st, Bodies B, Work w, const uint64_t* __restrict__ xs, uint32_t M, double max_move, double kT, uint32_t* __restrict__ next, uint8_t* __restrict__ flags);

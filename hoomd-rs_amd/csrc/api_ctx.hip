@@ -16,6 +16,15 @@ hipEvent_t take_event(hmc_ctx* c) {
   return e;
 }
 
+// The persistent apply's kernel for a context.
+static const void* persist_kernel(const hmc_ctx* c) {
+  const bool d2 = c->g.dim == 2;
+  if (is_isotropic(c->g.model)) return d2 ? (const void*)k_apply_lj<2> : (const void*)k_apply_lj<3>;
+  if (c->cfg.precision == HMC_MIXED)
+    return d2 ? (const void*)k_apply_tile<2, float> : (const void*)k_apply_tile<3, float>;
+  return d2 ? (const void*)k_apply_tile<2, double> : (const void*)k_apply_tile<3, double>;
+}
+
 template <int D, int PREC>
 int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t substep, uint32_t seed, double kT,
                  double max_move, uint32_t move) {
@@ -64,9 +73,8 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
     ApplyState* stp = c->st;
     c->pc.tag += 1;
     void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&c->pc};
-    const void* fn = is_isotropic(g.model) ? (const void*)k_apply_lj<D> : (const void*)k_apply_tile<D>;
     const hipError_t le =
-        hipLaunchCooperativeKernel(fn, dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, s);
+        hipLaunchCooperativeKernel(persist_kernel(c), dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, s);
     if (le != hipSuccess) return fail(c, HMC_ERR_DEVICE, std::string("cooperative launch: ") + hipGetErrorString(le));
     if (prof) {
       p1 = take_event(c);
@@ -190,6 +198,17 @@ int read_state(hmc_ctx* c, ApplyState* out, bool check_errors) {
   return HMC_OK;
 }
 
+// The same in FP64, for the persistent apply's FP64 box-relative test (E the
+// bound on its displacement, three fused roundings of d^2 and the reference's).
+bool contact_band64(double E, double sigma, double sigma2, double edge2, int D, double* lo, double* hi) {
+  const double dref = 1.01 * sigma;
+  const double Bd = (2.0 * E * std::sqrt((double)D) * dref + D * E * E + 12.0 * 0x1p-53 * dref * dref) * 1.1;
+  if (!(Bd < 0.01 * sigma2)) return false;
+  *lo = edge2 - Bd;
+  *hi = sigma2 + Bd;
+  return true;
+}
+
 // FP32 thresholds around contact for a per-axis error bound E on the FP32
 // displacement: d2 < lo overlaps (and lies below the edge region), d2 >= hi
 // does not.  The bound on d^2 near sigma^2 is 2 E sqrt(D) d + D E^2 +
@@ -284,7 +303,9 @@ bool choose_tiles(const Geometry& g, int D, double occ, size_t vt, int cus, Tile
 
 // Region shape of the persistent apply (k_apply_tile).  A region is 2 T
 // spaces per axis; its box (the region and a one-space halo, 2 T + 2 spaces)
-// must span at most shape - 2 spaces.  Every region must be resident at once,
+// must span at most shape - 2 spaces.  entry: bytes of a staged site (in FP64
+// about 600,000 spheres fit the device; larger systems take the per-colour
+// passes).  Every region must be resident at once,
 // so a shape qualifies only if all its workgroups fit on the device (LDS: the
 // box's offsets and a site capacity of 1.1x its expected count plus 64).
 // Among those the fewest lanes per workgroup win -- a colour pass lasts as
@@ -307,7 +328,7 @@ void fill_halo_lists(TileCfg* tc, int D) {
   for (int q = 0; q < kHaloLists; ++q) tc->hoff[q + 1] = tc->hoff[q] + cnt[q];
 }
 
-bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out) {
+bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus, TileCfg* out) {
   uint32_t lim[3] = {1, 1, 1};
   const uint32_t cap[3] = {16, 16, 32};
   for (int a = 0; a < D; ++a) {
@@ -337,7 +358,7 @@ bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out)
         if (rows > kMaxRegionRows) continue;
         const uint32_t maxb = (uint32_t)std::ceil(1.1 * occ * ncell) + 64;
         const size_t lds = ((region_head_bytes(rows, ncell - own) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
-                           (size_t)(maxb + kTilePad) * sizeof(float4);
+                           (size_t)(maxb + kTilePad) * entry;
         if (lds > kTileLds) continue;
         const uint32_t per_cu = std::min<uint32_t>((uint32_t)(cu_lds / (lds + static_lds)), cu_waves / (threads / 64));
         const uint32_t grid = ((ntiles + 7) / 8) * 8;
@@ -375,12 +396,9 @@ bool persist_probe(hmc_ctx* c) {
   Geometry g = c->g;
   ApplyState* stp = c->st;
   void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&pc};
-  const int D = g.dim;
-  const void* fn = is_isotropic(g.model) ? (D == 2 ? (const void*)k_apply_lj<2> : (const void*)k_apply_lj<3>)
-                                         : (D == 2 ? (const void*)k_apply_tile<2> : (const void*)k_apply_tile<3>);
   const size_t fbytes = (size_t)c->pc.ntiles * kMailboxStride * sizeof(uint32_t);
   uint32_t err = 0;
-  bool ok = hipLaunchCooperativeKernel(fn, dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, c->stream) ==
+  bool ok = hipLaunchCooperativeKernel(persist_kernel(c), dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, c->stream) ==
                 hipSuccess &&
             hipMemcpyAsync(&err, &c->st->error, sizeof err, hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
             hipStreamSynchronize(c->stream) == hipSuccess;
@@ -817,10 +835,11 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     }
     int coop = 0;
     // (the FP32 error report runs the per-colour passes)
-    if (c->tiled && cfg->precision == HMC_MIXED && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) &&
+    const bool mixed = cfg->precision == HMC_MIXED;
+    if (c->tiled && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) &&
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop) {
       TileCfg pc{};
-      if (choose_regions(g, D, (double)cfg->n_bodies / (double)spaces, cus, &pc)) {
+      if (choose_regions(g, D, (double)cfg->n_bodies / (double)spaces, mixed ? sizeof(float4) : sizeof(double4), cus, &pc)) {
         fill_halo_lists(&pc, D);
         // Band of the persistent layout, whose LDS entries are the FP64
         // box-relative positions rounded once to FP32.  Per axis: that
@@ -832,7 +851,11 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         double R = 0.0;
         for (int a = 0; a < D; ++a) R = std::max(R, 0.5 * pc.E[a] * g.width[a] + g.width[a]);
         const double Et = (0x1p-24 * (2.0 * R + 2.0 * sigma) + 0x1p-53 * (4.0 * lmax + 2.0 * sigma)) * 1.01;
-        const void* fn = D == 2 ? (const void*)k_apply_tile<2> : (const void*)k_apply_tile<3>;
+        // In FP64 the same with 2^-53 for every rounding: x - c, the image
+        // shift and the rounding of the difference on both sides, and the
+        // reference's own displacement.
+        const double E64 = 0x1p-53 * (6.0 * lmax + 4.0 * R + 4.0 * sigma) * 1.01;
+        const void* fn = persist_kernel(c);
         // one lane per trial, and where the regions leave compute units to
         // spare, wavefronts that only stage and reload (a small system's box of
         // 1000 cells staged by one wavefront took 40 us of a 200 us apply)
@@ -840,6 +863,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         if (pc.xcd_chunk * 8u <= (uint32_t)cus) threads = kTileThreads;
         int per_cu = 0;
         if (contact_band(Et, sigma, g.sigma2, g.edge2, D, &pc.band_lo, &pc.band_hi) &&
+            contact_band64(E64, sigma, g.sigma2, g.edge2, D, &pc.band64_lo, &pc.band64_hi) &&
             hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pc.lds_bytes) == hipSuccess &&
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, (int)threads, pc.lds_bytes) == hipSuccess &&
             (uint64_t)per_cu * (uint64_t)cus >= (uint64_t)pc.xcd_chunk * 8u) {
@@ -1462,7 +1486,8 @@ int hmc_get_stats(hmc_ctx* c, hmc_stats* out) {
   out->ambiguous = s.ambiguous;
   std::memcpy(&out->fp32_error_max, &s.fp32_err_max, sizeof(double));
   std::memcpy(&out->fp32_error_bound, &s.fp32_err_ratio, sizeof(double));
-  out->tiled = c->persist ? 2u : (c->tiled ? 1u : 0u);
+  // (an FP64 hard-shape apply reports LDS tiles in either layout; regions tells)
+  out->tiled = c->persist && (is_isotropic(c->g.model) || c->cfg.precision == HMC_MIXED) ? 2u : (c->tiled ? 1u : 0u);
   for (int a = 0; a < 3; ++a) out->tile_shape[a] = c->persist ? c->pc.T[a] : (c->tiled ? c->tc.T[a] : 0u);
   out->regions = c->persist ? c->pc.ntiles : 0u;
   out->region_threads = c->persist ? c->pthreads : 0u;

@@ -137,7 +137,7 @@ bool contact_band(double E, double sigma, double sigma2, double edge2, int D, fl
 bool choose_tiles(const Geometry& g, int D, double occ, size_t vt, int cus, TileCfg* out);
 // The places of the halo lists (TileCfg::hoff) of a full region of shape T.
 void fill_halo_lists(TileCfg* tc, int D);
-bool choose_regions(const Geometry& g, int D, double occ, int cus, TileCfg* out);
+bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus, TileCfg* out);
 bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* out);
 int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_out, double* lmax_out);
 const char* sdf_check(const Geometry& g, double xmax, double dx, uint32_t nbins);

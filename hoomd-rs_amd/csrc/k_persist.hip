@@ -1,4 +1,4 @@
-// The persistent apply (mixed precision, hard spheres and disks): one
+// The persistent apply of hard spheres and disks (mixed precision and FP64): one
 // cooperative launch runs every cycle and colour of an apply.
 #include "persist.hpp"
 
@@ -85,16 +85,24 @@ __device__ __noinline__ TrialOut trial_global_dev(const Geometry* gp, ApplyState
   return o;
 }
 
-// FP32 squared distance of a staged site from the trial site (fused: three
-// roundings, within the band's 4 u relative term).
-template <int D>
-__device__ __forceinline__ float tile_dist2(const float4& q, const float* tr) {
-  const float dx = q.x - tr[0], dy = q.y - tr[1];
+// Squared distance of a staged site from the trial site in the region's scalar
+// (fused: three roundings, within the band's relative term).
+template <int D, class S>
+__device__ __forceinline__ S tile_dist2(const Ent<S>& q, const S* tr) {
+  const S dx = q.x - tr[0], dy = q.y - tr[1];
   if (D == 3) {
-    const float dz = q.z - tr[2];
-    return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    const S dz = q.z - tr[2];
+    return fma(dx, dx, fma(dy, dy, dz * dz));
   }
-  return fmaf(dx, dx, dy * dy);
+  return fma(dx, dx, dy * dy);
+}
+template <class S>
+__device__ __forceinline__ S band_lo(const TileCfg& tc) {
+  return std::is_same<S, float>::value ? (S)tc.band_lo : (S)tc.band64_lo;
+}
+template <class S>
+__device__ __forceinline__ S band_hi(const TileCfg& tc) {
+  return std::is_same<S, float>::value ? (S)tc.band_hi : (S)tc.band64_hi;
 }
 
 // The rows of a trial: the 3^D cells around the trial's own are 3^(D-1) rows
@@ -111,17 +119,17 @@ __device__ __forceinline__ float tile_dist2(const float4& q, const float* tr) {
 // Sorted by length so that the walk below runs as many slots as the
 // wavefront's fullest lanes have sites: on C2 32 for 27 candidates a lane,
 // where rounds over all rows in place took 71.
-template <int D>
+template <int D, class S>
 __device__ __forceinline__ void tile_rows(GeoPtr g, const TileCfg& tc, const uint16_t* coff,
-                                          const uint32_t* cb, const float* tr, uint32_t* key) {
+                                          const uint32_t* cb, const S* tr, uint32_t* key) {
   constexpr int AL = D - 1, NR = D == 3 ? 9 : 3;
-  const float cut = tc.band_hi * (1.0f + 1e-4f);
+  const float cut = (float)band_hi<S>(tc) * (1.0f + 1e-4f);
   // squared distance from the trial site to the lower and upper face of its cell
   float flo[3] = {0.0f, 0.0f, 0.0f}, fhi[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int a = 0; a < D; ++a) {
     const float wd = (float)g->width[a];
-    const float u = tr[a] - ((float)cb[a] - 0.5f * (float)tc.E[a]) * wd;
+    const float u = (float)tr[a] - ((float)cb[a] - 0.5f * (float)tc.E[a]) * wd;
     const float dl = fmaxf(u, 0.0f), dh = fmaxf(wd - u, 0.0f);
     flo[a] = dl * dl;
     fhi[a] = dh * dh;
@@ -157,40 +165,40 @@ __device__ __forceinline__ void tile_rows(GeoPtr g, const TileCfg& tc, const uin
   }
 }
 
-// Does the trial site (FP64 t, box-relative FP32 tr) overlap a staged site of
+// Does the trial site (FP64 t, box-relative tr) overlap a staged site of
 // its rows other than its own, entry `self` (value old) of lb?
 //
 // Three rows at a time, one site of each per round, while any lane has a site
 // left in the longest of them.  A lane past the end of its row reads on into
 // the sites that follow: they are sites of the box too, either in the trial's
-// neighbourhood or a space's width or more away (a site's FP32 coordinates
-// never leave its space by more than rounding, also while another trial moves
-// it), and at the end of the box kTilePad entries out of reach.  So no slot
+// neighbourhood or a space's width or more away (a site's coordinates never
+// leave its space by more than rounding, also while another trial moves it),
+// and at the end of the box kTilePad entries out of reach.  So no slot
 // needs a validity test; the own entry is moved out of reach for the walk.
-// (The 12-byte LDS reads at scattered entries bound the walk.)
+// (The LDS reads of 12 or 24 bytes at scattered entries bound the walk.)
 //
 // Pairs inside the band are re-tested in FP64 after the walk when no certain
 // overlap was found.  `odd`: the box holds a site without images, whose entry
 // is NaN and which is always re-tested; such a box, and a row longer than
 // kTilePad, is walked one site at a time.  lb[self] holds `old` again on
 // return.
-template <int D>
-__device__ __forceinline__ bool tile_overlaps(const Geometry& g, const TileCfg& tc, float4* lb, const double4* spos,
-                                              const double* t, const float* tr, uint32_t* key, uint32_t self,
-                                              float4 old, bool odd, unsigned* retests) {
+template <int D, class S>
+__device__ __forceinline__ bool tile_overlaps(const Geometry& g, const TileCfg& tc, Ent<S>* lb, const double4* spos,
+                                              const double* t, const S* tr, uint32_t* key, uint32_t self,
+                                              const Ent<S>& old, bool odd, unsigned* retests) {
   constexpr int NR = D == 3 ? 9 : 3;
-  const float lo = tc.band_lo, hi = tc.band_hi;
-  lb[self] = make_float4(kTileFar, 0.0f, 0.0f, 0.0f);
+  const S lo = band_lo<S>(tc), hi = band_hi<S>(tc);
+  lb[self].x = (S)kTileFar;
   bool hit = false, walk = __any(odd || (key[0] >> 16) > (uint32_t)kTilePad);
   if (!walk) {  // uniform
-    const float4* p[NR];
+    const Ent<S>* p[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) p[r] = lb + (key[r] & 0xffffu);
-    float near2 = kTileFar;
+    S near2 = (S)kTileFar;
     auto slots = [&](int r0, uint32_t k) {
-      const float4 a = p[r0][k], b = p[r0 + 1][k], c = p[r0 + 2][k];
-      near2 = fminf(near2, tile_dist2<D>(a, tr));
-      near2 = fminf(near2, fminf(tile_dist2<D>(b, tr), tile_dist2<D>(c, tr)));
+      const Ent<S> a = p[r0][k], b = p[r0 + 1][k], c = p[r0 + 2][k];
+      near2 = fmin(near2, tile_dist2<D, S>(a, tr));
+      near2 = fmin(near2, fmin(tile_dist2<D, S>(b, tr), tile_dist2<D, S>(c, tr)));
     };
     for (uint32_t k = 0; __any(!(near2 < lo) && (key[0] >> 16) > k); ++k) {
       slots(0, k);
@@ -212,12 +220,12 @@ __device__ __forceinline__ bool tile_overlaps(const Geometry& g, const TileCfg& 
       for (int i = 0; i + 1 < NR; ++i) key[i] = key[i + 1];
 #pragma unroll 1
       for (uint32_t k = 0; k < n && !hit; ++k) {
-        const float4 q = lb[b + k];
-        const float d2 = tile_dist2<D>(q, tr);
+        const Ent<S> q = lb[b + k];
+        const S d2 = tile_dist2<D, S>(q, tr);
         if (d2 < lo) hit = true;
         if (d2 < lo || d2 >= hi) continue;
         ++*retests;
-        hit = retest64_body<D>(g.self, spos, (uint32_t)__float_as_int(q.w), t[0], t[1], t[2]);
+        hit = retest64_body<D>(g.self, spos, Staged<S>::body(q), t[0], t[1], t[2]);
       }
     }
   }
@@ -241,17 +249,17 @@ __device__ __forceinline__ bool tile_overlaps(const Geometry& g, const TileCfg& 
 //   the halo entries into LDS, a barrier, the trials.
 // None of the proposal reads what pass i or a neighbour changed: a trial's
 // body belongs to its own colour's cell, and cells' offsets are static.
-template <int D, int CELLS>
+template <int D, class S, int CELLS>
 __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st, const Bodies& B, const Cells& C,
                                                const Work& w, const TileCfg& tc, uint32_t tile,
                                                unsigned long long* acc, const double* zx, const double* zf) {
   constexpr int AL = D - 1;  // the row axis (stride 1)
   constexpr uint32_t NCOL = 1u << D;
   extern __shared__ __align__(16) unsigned char smem[];
-  const RegionLds l = region_lds<D>(smem, tc);
+  const RegionLds<S> l = region_lds<D, S>(smem, tc);
   const uint32_t CW = tc.E[AL] + 1;
   const uint16_t* coff = l.coff;
-  float4* lb = l.lb;
+  Ent<S>* lb = l.lb;
   __shared__ unsigned blk_acc;
   __shared__ uint32_t hcnt[kHaloLists];
   __shared__ uint32_t odd;  // the box holds (or held) a site without images
@@ -280,7 +288,7 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
 
   if (tid == 0) blk_acc = odd = 0;
   if (tid < (uint32_t)kHaloLists) hcnt[tid] = 0;
-  const bool overflow = region_stage<D, kTilePad>(g, tc, rg, B, C, w, l, &odd);
+  const bool overflow = region_stage<D, S, kTilePad>(g, tc, rg, B, C, w, l, &odd);
 
   unsigned retests = 0;
   // the proposal of this thread's trial
@@ -288,9 +296,9 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
   uint32_t ps = 0, self = 0, body = 0;
   uint32_t pcb[3] = {0, 0, 0}, key[9];
   double v[3] = {0.0, 0.0, 0.0}, pt[3] = {0.0, 0.0, 0.0};
-  float ptr[3] = {0.0f, 0.0f, 0.0f};
+  S ptr[3] = {0, 0, 0};
   double4 bp = make_double4(0.0, 0.0, 0.0, 0.0), psp = bp;
-  float4 pent = make_float4(0.0f, 0.0f, 0.0f, 0.0f), pold = pent;
+  Ent<S> pent{}, pold{};
   for (int r = 0; r < 9; ++r) key[r] = 0;
   // the draws of pass i (cycle i / 2^D, colour i mod 2^D)
   auto draw = [&](uint32_t i) {
@@ -315,7 +323,7 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
     Sfc64 rng = counter_rng<true>(step, substep, seed, s);
     self = e0 + choose_index(rng, n);
     pold = lb[self];
-    body = (uint32_t)__float_as_int(pold.w);
+    body = Staged<S>::body(pold);
     bp = B.bpos[body];
     ball_sample<D>(rng, max_move, zx, zf, v);
   };
@@ -330,11 +338,12 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
     pin = ts.in;
     for (int a = 0; a < D; ++a) pt[a] = ts.t[a];
     psp = pack_site(ts.n, ts.flags);
-    box_relative64<D>(gp, c64, ts.t, ptr);
-    float e[3] = {0.0f, 0.0f, 0.0f};
-    box_relative64<D>(gp, c64, ts.n, e);
-    pent = make_float4(ts.flags == kNoImages ? __int_as_float(0x7fc00000) : e[0], e[1], e[2], __int_as_float((int)body));
-    tile_rows<D>(gp, tc, coff, pcb, ptr, key);
+    box_relative64<D>(*gp, c64, ts.t, ptr);
+    S e[3] = {0, 0, 0};
+    box_relative64<D>(*gp, c64, ts.n, e);
+    e[0] = ts.flags == kNoImages ? (S)__builtin_nanf("") : e[0];
+    pent = Staged<S>::make(e, body);
+    tile_rows<D, S>(gp, tc, coff, pcb, ptr, key);
   };
 
   const uint32_t npass = cycles * NCOL;
@@ -347,11 +356,11 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
     // the body's position is here before the halo loads are issued: the
     // compiler cannot count those, and would wait for them all to use it
     asm volatile("" : "+v"(bp.x), "+v"(bp.y), "+v"(bp.z));
-    RegionReload<D, 1, CELLS, 3> reload(g, tc, rg, B, l, hcnt, i);
+    RegionReload<D, S, 1, CELLS, 3> reload(g, tc, rg, B, l, hcnt, i);
     if (i && !overflow) reload.issue();
     finish();
     if (i && !overflow) reload.commit(&odd);
-    if (i == 0) region_halo_lists<D>(tc, rg, l, hcnt);  // (read after the next barrier)
+    if (i == 0) region_halo_lists<D, S>(tc, rg, l, hcnt);  // (read after the next barrier)
     if (i) __syncthreads();
     unsigned accepted = 0;
     if (has_trial && overflow) {
@@ -372,7 +381,7 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
       }
     } else if (pgo) {
       // ---- the trial of this pass from LDS
-      if (pin && !tile_overlaps<D>(g, tc, lb, B.spos, pt, ptr, key, self, pold, odd != 0, &retests)) {
+      if (pin && !tile_overlaps<D, S>(g, tc, lb, B.spos, pt, ptr, key, self, pold, odd != 0, &retests)) {
         // update_body_properties (microstate.rs:985-1034), formed with the proposal
         B.bpos[body] = make_double4(pt[0], pt[1], pt[2], stamp);
         st_dev_d4(&B.spos[body], psp);
@@ -403,7 +412,7 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
   if (tid == 0 && blk_acc) atomicAdd(acc, (unsigned long long)blk_acc);
 }
 
-template <int D>
+template <int D, class S>
 __global__ void __launch_bounds__(kTileThreads, 2) k_apply_tile(Geometry g, ApplyState* st, Bodies B, Cells C, Work w,
                                                              TileCfg tc) {
   const uint32_t b = blockIdx.x;
@@ -415,7 +424,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_apply_tile(Geometry g, Appl
   }
   __shared__ double zx[257], zf[257];
   if (D == 3) stage_zig(zx, zf);  // (read after region_stage's barriers)
-  apply_tile_run<D, 2>(g, st, B, C, w, tc, tile, &w.acc_slots[b & (kAccSlots - 1)], zx, zf);
+  apply_tile_run<D, S, 2>(g, st, B, C, w, tc, tile, &w.acc_slots[b & (kAccSlots - 1)], zx, zf);
 }
 
 // The persistent applies of every replica of a batch in one cooperative
@@ -461,14 +470,16 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_bapply_tile(const BatchRep*
     wr.tracing = 0;
     // the ziggurat layers from the constant tables: the LDS they would take
     // is worth more as region entries here (more regions per CU)
-    apply_tile_run<D, 1>(sg, sts + r, B, C, wr, stc, gt - toff[r], &w.acc_slots[r], kZigX, kZigF);
+    apply_tile_run<D, float, 1>(sg, sts + r, B, C, wr, stc, gt - toff[r], &w.acc_slots[r], kZigX, kZigF);
     __syncthreads();  // sg and stc are rewritten for the next round
   }
 }
 
 // explicit instantiations (launched from the host translation units)
-template __global__ void k_apply_tile<2>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
-template __global__ void k_apply_tile<3>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
+template __global__ void k_apply_tile<2, float>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
+template __global__ void k_apply_tile<2, double>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
+template __global__ void k_apply_tile<3, float>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
+template __global__ void k_apply_tile<3, double>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
 template __global__ void k_bapply_tile<3>(const BatchRep*, const TileCfg*, const uint32_t*, const uint32_t*,
                                           ApplyState*, const uint32_t*, const uint32_t*, uint32_t, uint32_t, uint32_t,
                                           uint32_t, uint32_t, Bodies, Cells, Work);

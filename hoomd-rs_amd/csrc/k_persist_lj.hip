@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
     return;
   }
   extern __shared__ __align__(16) unsigned char smem[];
-  const RegionLds l = region_lds<D>(smem, tc);
+  const RegionLds<float> l = region_lds<D, float>(smem, tc);
   const uint32_t CW = tc.E[AL] + 1;
   const uint16_t* coff = l.coff;
   float4* lb = l.lb;
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
   if (tid == 0) blk_acc = 0;
   if (tid < (uint32_t)kHaloLists) hcnt[tid] = 0;
   __shared__ uint32_t odd;  // (sites without images are found by their NaN entries)
-  const bool overflow = region_stage<D, 0>(g, tc, rg, B, C, w, l, &odd);
+  const bool overflow = region_stage<D, float, 0>(g, tc, rg, B, C, w, l, &odd);
 
   unsigned retests = 0, ambiguous = 0;
   // The proposals of pass i, drawn while the neighbour regions finish pass
@@ -283,14 +283,15 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
         double nsp[3] = {0.0, 0.0, 0.0};
         for (int a = 0; a < D; ++a) nsp[a] = wrap1(g, a, t[a] + 0.0);
         const double4 sp = pack_site(nsp, ghost_flags<D>(g, nsp));
-        const float4 te = box_entry64<D>(g, rg.c64, t, 0u);
+        float te[3] = {0.0f, 0.0f, 0.0f};
+        box_relative64<D>(g, rg.c64, t, te);
         pr.rng = rng;
         for (int a = 0; a < 3; ++a) pr.t[a] = t[a];
         pr.sp = sp;
-        pr.ent = stage_entry64<D>(g, rg.c64, sp, body);
-        pr.tr[0] = te.x;
-        pr.tr[1] = te.y;
-        pr.tr[2] = te.z;
+        pr.ent = stage_entry64<D, float>(g, rg.c64, nsp, body);
+        pr.tr[0] = te[0];
+        pr.tr[1] = te[1];
+        pr.tr[2] = te[2];
         pr.xr[0] = se.x;
         pr.xr[1] = se.y;
         pr.xr[2] = se.z;
@@ -435,7 +436,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
 
   const uint32_t npass = cycles * NCOL;
   if (npass && tid < ntr) propose(0, tid);
-  region_halo_lists<D>(tc, rg, l, hcnt);
+  region_halo_lists<D, float>(tc, rg, l, hcnt);
   __syncthreads();
   unsigned nacc = 0;  // accepted trials (lane 0 of each half-wave)
   for (uint32_t i = 0; i < npass; ++i) {
@@ -617,7 +618,7 @@ __global__ void __launch_bounds__(kLjRegionThreads, 2) k_apply_lj(Geometry g, Ap
     region_wait<D>(st, w.mbox, tc, rg, tile, i + 1);
     // (cells of about 15 entries: 16 lanes each)
     if (!overflow) {
-      RegionReload<D, 16, 2, 2> reload(g, tc, rg, B, l, hcnt, i + 1);
+      RegionReload<D, float, 16, 2, 2> reload(g, tc, rg, B, l, hcnt, i + 1);
       reload.issue();
       reload.commit(&odd);
     }

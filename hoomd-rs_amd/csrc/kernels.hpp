@@ -20,7 +20,7 @@ template <int D, int PREC, bool FAST>
 __global__ void k_pass(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
 template <int D, int PREC, bool FP32_ERROR = false>
 __global__ void k_pass_tile(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, TileCfg tc);
-template <int D>
+template <int D, class S>
 __global__ void k_apply_tile(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
 template <int D>
 __global__ void k_bapply_tile(const BatchRep* reps, const TileCfg* tcs, const uint32_t* toff, const uint32_t* trep, ApplyState* sts, const uint32_t* rt0, const uint32_t* rn, uint32_t nrounds, uint32_t nwg, uint32_t xcd_chunk, uint32_t probe, uint32_t tag, Bodies B, Cells C, Work w);

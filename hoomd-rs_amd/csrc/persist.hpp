@@ -17,8 +17,8 @@ namespace hmc {
 // from the FP64 sites.  Consecutive passes are separated by a neighbour
 // synchronisation (below), not by a grid barrier.
 //
-// An LDS entry holds the site relative to the box centre in FP32 (NaN for a
-// site without images, as in the per-colour kernel) with the body index in w.
+// An LDS entry holds the site relative to the box centre, in FP32 (mixed
+// precision) or FP64, NaN for a site without images, with the body index in w.
 
 // A region's box is staged as in k_pass_tile: ri (rows + 1 uint4: LDS offset
 // of the row, first run start, first run length, second run start), coff
@@ -69,33 +69,50 @@ __device__ __forceinline__ void region_publish(uint32_t* mbox, uint32_t tile, ui
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Box-relative FP32 position: the image of x nearest the box centre c, relative
-// to c, computed in FP64 and rounded once to FP32, w = body.
-template <int D>
-__device__ __forceinline__ float4 box_entry64(const Geometry& g, const double* c, const double* x, uint32_t body) {
-  float r[3] = {0.0f, 0.0f, 0.0f};
+// The staged sites of a box in the region's scalar S: x, y, z and the body
+// index in w (S = float: a mixed-precision region; double: an FP64 one).
+template <class S>
+struct Staged;
+template <>
+struct Staged<float> {
+  using type = float4;
+  __device__ __forceinline__ static float4 make(const float* r, uint32_t body) {
+    return make_float4(r[0], r[1], r[2], __int_as_float((int)body));
+  }
+  __device__ __forceinline__ static uint32_t body(const float4& e) { return (uint32_t)__float_as_int(e.w); }
+};
+template <>
+struct Staged<double> {
+  using type = double4;
+  __device__ __forceinline__ static double4 make(const double* r, uint32_t body) {
+    return make_double4(r[0], r[1], r[2], __longlong_as_double((long long)body));
+  }
+  __device__ __forceinline__ static uint32_t body(const double4& e) { return (uint32_t)__double_as_longlong(e.w); }
+};
+template <class S>
+using Ent = typename Staged<S>::type;
+
+// Box-relative position: the image of x nearest the box centre c, relative to
+// c, computed in FP64 and rounded once to S.  (Selects, not branches: this is
+// inlined where a pass's latency counts.)
+template <int D, class S, class G>
+__device__ __forceinline__ void box_relative64(const G& g, const double* c, const double* x, S* r) {
 #pragma unroll
   for (int a = 0; a < D; ++a) {
-    // (selects, not branches: this is inlined where a pass's latency counts)
-    const double u = x[a] - c[a], back = u >= g.half[a] ? g.L[a] : 0.0;
-    r[a] = (float)(u - (u < -g.half[a] ? -g.L[a] : back));
+    const double L = g.L[a], half = g.half[a], u = x[a] - c[a];
+    r[a] = (S)(u - (u >= half ? L : u < -half ? -L : 0.0));
   }
-  return make_float4(r[0], r[1], r[2], __int_as_float((int)body));
 }
 // LDS entry of a site: as above, NaN for a site without images (one outside
 // [-L/2, L/2) on some axis, as in ghost_flags), body index in w.
-template <int D>
-__device__ __forceinline__ float4 stage_entry64(const Geometry& g, const double* c, const double* x, uint32_t body) {
-  float4 e = box_entry64<D>(g, c, x, body);
+template <int D, class S>
+__device__ __forceinline__ Ent<S> stage_entry64(const Geometry& g, const double* c, const double* x, uint32_t body) {
+  S r[3] = {0, 0, 0};
+  box_relative64<D>(g, c, x, r);
 #pragma unroll
   for (int a = 0; a < D; ++a)
-    if (x[a] < -g.half[a] || x[a] >= g.half[a]) e.x = __int_as_float(0x7fc00000);
-  return e;
-}
-template <int D>
-__device__ __forceinline__ float4 stage_entry64(const Geometry& g, const double* c, double4 sp, uint32_t body) {
-  const double x[3] = {sp.x, sp.y, sp.z};
-  return stage_entry64<D>(g, c, x, body);
+    if (x[a] < -g.half[a] || x[a] >= g.half[a]) r[0] = (S)__builtin_nanf("");
+  return Staged<S>::make(r, body);
 }
 
 // The system's constants read through the scalar cache where they are used:
@@ -175,16 +192,6 @@ __device__ __forceinline__ TrialSite<D> trial_site(GeoPtr g, const ApplyState* s
   if (!(least >= 0x1p-900)) o = trial_site_general<D>((const Geometry*)(uintptr_t)g, st, x0[0], x0[1], D == 3 ? x0[2] : 0.0, s);
   return o;
 }
-// box_entry64 with the system's constants through the scalar cache
-template <int D>
-__device__ __forceinline__ void box_relative64(GeoPtr g, const double* c, const double* x, float* r) {
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    const double L = g->L[a], half = g->half[a], u = x[a] - c[a];
-    r[a] = (float)(u - (u >= half ? L : u < -half ? -L : 0.0));
-  }
-}
-
 // Residency probe (tc.probe): the persistent launch relies on every region
 // being resident at once, which the host checks with the occupancy API; the
 // probe checks it on the device with the kernel's own resources.  Thread 0 of
@@ -300,26 +307,27 @@ __device__ __forceinline__ void region_wait(ApplyState* st, uint32_t* mbox, cons
 
 // LDS of a region's box: ri (staging only), whose space the halo cell lists
 // take over afterwards, coff, then the site entries.
+template <class S>
 struct RegionLds {
   uint4* ri;
   uint16_t* halo;
   uint16_t* coff;
-  float4* lb;
+  Ent<S>* lb;
 };
 // bytes of ri / the halo lists
 __host__ __device__ inline uint32_t region_head_bytes(uint32_t rows, uint32_t halo_cells) {
   const uint32_t a = 16u * (rows + 1), b = (2u * halo_cells + 15u) & ~15u;
   return a > b ? a : b;
 }
-template <int D>
-__device__ __forceinline__ RegionLds region_lds(unsigned char* smem, const TileCfg& tc) {
+template <int D, class S>
+__device__ __forceinline__ RegionLds<S> region_lds(unsigned char* smem, const TileCfg& tc) {
   const uint32_t R = tc.rows, CW = tc.E[D - 1] + 1;
   const uint32_t head = region_head_bytes(R, tc.hoff[kHaloLists]);
-  RegionLds l;
+  RegionLds<S> l;
   l.ri = (uint4*)smem;
   l.halo = (uint16_t*)smem;
   l.coff = (uint16_t*)(smem + head);
-  l.lb = (float4*)(smem + ((head + 2u * R * CW + 15u) & ~15u));
+  l.lb = (Ent<S>*)(smem + ((head + 2u * R * CW + 15u) & ~15u));
   return l;
 }
 
@@ -338,16 +346,16 @@ __device__ __forceinline__ RegionLds region_lds(unsigned char* smem, const TileC
 // than in execution.  (With the cell starts taken 16 to a thread in unrolled
 // loops and the image selection in branches, the part of the kernel before
 // the first trial took 50 us of C2's 280 us apply.)
-template <int D, int PAD>
+template <int D, class S, int PAD>
 __device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& tc, const Region& rg, const Bodies& B,
-                                             const Cells& C, const Work& w, const RegionLds& l, uint32_t* odd) {
+                                             const Cells& C, const Work& w, const RegionLds<S>& l, uint32_t* odd) {
   constexpr int AL = D - 1;
   const uint32_t R = tc.rows, EL = tc.E[AL], CW = EL + 1;
   const uint32_t tid = threadIdx.x, NT = blockDim.x;
   const uint32_t p = rg.p, m0 = rg.m0;
   uint4* ri = l.ri;
   uint16_t* coff = l.coff;
-  float4* lb = l.lb;
+  Ent<S>* lb = l.lb;
   // per row: its runs' lengths, first slots and the space it starts at (a run
   // past 16 bits is no box that fits)
   const uint32_t e1m = D == 3 ? (65536u + tc.E[1] - 1u) / tc.E[1] : 0u;  // row / E1 (rows <= 256)
@@ -381,7 +389,7 @@ __device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& t
   const uint32_t total = ri[R].x;
   const bool overflow = total > tc.maxb;  // uniform over the workgroup; else every offset fits 16 bits
   if (!overflow) {
-    if (tid < (uint32_t)PAD) lb[total + tid] = make_float4(kTileFar, 0.0f, 0.0f, 0.0f);
+    if (tid < (uint32_t)PAD) lb[total + tid] = Ent<S>{(S)kTileFar, 0, 0, 0};
     const uint32_t hw = tid >> 5, hl = tid & 31u, NH = NT >> 5;
     // boundary j of a row (j <= p) is the start of space m0 + j, the next ones
     // that of j - p - 1 after the wrap; its LDS offset is written at j or j - 1
@@ -393,7 +401,8 @@ __device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& t
       return e < (q.x >> 16) ? q.y + e : q.z + (e - (q.x >> 16));
     };
     auto put = [&](uint32_t dst, const double4& sp, uint32_t body) {
-      const float4 en = stage_entry64<D>(g, rg.c64, sp, body);
+      const double x[3] = {sp.x, sp.y, sp.z};
+      const Ent<S> en = stage_entry64<D, S>(g, rg.c64, x, body);
       lb[dst] = en;
       if (!(en.x == en.x)) *odd = 1;
     };
@@ -464,8 +473,8 @@ __host__ __device__ __forceinline__ uint32_t halo_list(const int32_t* lc, const 
   while (((k ^ (k + d)) & axes) != axes) ++d;
   return (k + d) & ((1u << D) - 1u);
 }
-template <int D>
-__device__ __forceinline__ void region_halo_lists(const TileCfg& tc, const Region& rg, const RegionLds& l,
+template <int D, class S>
+__device__ __forceinline__ void region_halo_lists(const TileCfg& tc, const Region& rg, const RegionLds<S>& l,
                                                   uint32_t* hcnt) {
   constexpr int AL = D - 1;
   const uint32_t EL = tc.E[AL], E1 = D == 3 ? tc.E[1] : 1u;
@@ -487,19 +496,19 @@ __device__ __forceinline__ void region_halo_lists(const TileCfg& tc, const Regio
 // entries, lists of more than CELLS NT / LPC cells), one memory latency
 // per round.  *odd is set where an entry is NaN (a site without images).  No
 // barrier: one must follow before other wavefronts read the entries.
-template <int D, int LPC, int CELLS, int HELD>
+template <int D, class S, int LPC, int CELLS, int HELD>
 struct RegionReload {
   const Geometry& g;
   const Region& rg;
   const Bodies& B;
-  const RegionLds& l;
+  const RegionLds<S>& l;
   const uint16_t* list;
   uint32_t n, step, c0;
   uint32_t e[CELLS], eb[CELLS];
   double v[CELLS][HELD][3];
 
   __device__ __forceinline__ RegionReload(const Geometry& g_, const TileCfg& tc, const Region& rg_, const Bodies& B_,
-                                          const RegionLds& l_, const uint32_t* hcnt, uint32_t j)
+                                          const RegionLds<S>& l_, const uint32_t* hcnt, uint32_t j)
       : g(g_), rg(rg_), B(B_), l(l_) {
     const uint32_t q = j & ((1u << D) - 1u);
     n = hcnt[q];
@@ -524,7 +533,7 @@ struct RegionReload {
     for (int u = 0; u < CELLS; ++u)
 #pragma unroll
       for (int h = 0; h < HELD; ++h)
-        if (e[u] + (uint32_t)(h * LPC) < eb[u]) bd[u][h] = (uint32_t)__float_as_int(l.lb[e[u] + (uint32_t)(h * LPC)].w);
+        if (e[u] + (uint32_t)(h * LPC) < eb[u]) bd[u][h] = Staged<S>::body(l.lb[e[u] + (uint32_t)(h * LPC)]);
 #pragma unroll
     for (int u = 0; u < CELLS; ++u)
 #pragma unroll
@@ -537,7 +546,7 @@ struct RegionReload {
     for (int a = 0; a < D; ++a) sp[a] = __longlong_as_double((long long)ld_dev(q + a));
   }
   __device__ __forceinline__ void put(uint32_t x, const double* sp, uint32_t* odd) const {
-    const float4 en = stage_entry64<D>(g, rg.c64, sp, (uint32_t)__float_as_int(l.lb[x].w));
+    const Ent<S> en = stage_entry64<D, S>(g, rg.c64, sp, Staged<S>::body(l.lb[x]));
     l.lb[x] = en;
     if (!(en.x == en.x)) *odd = 1;
   }
@@ -556,7 +565,7 @@ struct RegionReload {
 #pragma unroll 1
       for (uint32_t x = l.coff[cell] + threadIdx.x % LPC + held; x < l.coff[cell + 1]; x += LPC) {
         double sp[3];
-        fetch((uint32_t)__float_as_int(l.lb[x].w), sp);
+        fetch(Staged<S>::body(l.lb[x]), sp);
         put(x, sp, odd);
       }
     }

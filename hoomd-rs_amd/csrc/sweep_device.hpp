@@ -517,6 +517,7 @@ struct TileCfg {
   float r2_open;           // isotropic persistent apply: pairs with FP32 r2 below it are left to FP64
   uint32_t probe;          // persistent apply: 1 = only check that every region is resident (region_probe)
   uint32_t step[3];        // the workgroup size in the mixed radix (E0, .., E[D-2], E[D-1] + 2) of the row starts
+  double band64_lo, band64_hi;  // FP64 persistent apply: band of the FP64 box-relative test
   uint32_t tag;            // persistent apply: tells this launch's progress words from older ones
   uint32_t hoff[9];        // persistent apply: first cell of each halo list of a full region, then their total
 };

@@ -134,7 +134,9 @@ typedef struct {
   uint32_t tiled;           /* 1: one launch per colour pass, staging each
                                workgroup's neighbourhood box in LDS; 2: one
                                persistent launch per apply, each workgroup
-                               keeping its region and halo in LDS; 0: no LDS */
+                               keeping its region and halo in LDS (mixed
+                               precision; in FP64 reported as 1 with
+                               regions > 0); 0: no LDS */
   uint32_t tile_shape[3];   /* colour spaces per workgroup along each axis */
   uint64_t ambiguous;       /* LJ: Metropolis decisions that the bound on the
                                summation-order difference could not settle

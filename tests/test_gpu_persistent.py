@@ -105,3 +105,13 @@ def test_coordinates_of_exactly_zero(hmc, wl):
     st = _replay(hmc, L, pos, 1e-300, 3, "mixed")
     assert st["tiled"] == 2
     _replay(hmc, L, pos, 0.1, 6, "mixed")
+
+
+@pytest.mark.parametrize("cells,phi,d", [((4, 4, 4), 0.50, 0.08), ((5, 9, 13), 0.42, 0.15), ((29, 23, 31), 0.45, 0.1),
+                                         ((8, 8, 8), 0.05, 0.9)])
+def test_fp64_regions(hmc, wl, cells, phi, d):
+    # FP64 box-relative entries with the exact re-test inside the band
+    L, pos = wl.fcc_spheres(cells, packing_fraction=phi)
+    st = _replay(hmc, L, pos, d, 6, "fp64")
+    assert st["tiled"] == 1 and st["regions"] > 0
+    log(f"{cells} phi {phi}: {st['regions']} regions of {st['tile_shape']}, {st['band_retests']} re-tests")

@@ -51,8 +51,8 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
   }
   if (N) {
     k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
-    // the persistent apply stages its sites from the FP64 copies
-    if (c->persist)
+    // (these applies stage their sites from the FP64 copies)
+    if (c->persist || c->small_wpt)
       k_place<PREC, false><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
     else
       k_place<PREC><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
@@ -81,6 +81,24 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
       (void)hipEventRecord(p1, s);
       c->pass_events.push_back({p0, p1});
     }
+    c->applies += 1;
+    return HMC_OK;
+  }
+  if (c->small_wpt) {
+    hipEvent_t p0 = nullptr, p1 = nullptr;
+    if (prof) {
+      p0 = take_event(c);
+      (void)hipEventRecord(p0, s);
+    }
+    k_apply_small<D><<<1, kSmallThreads, SmallLds::of(g).total, s>>>(g, c->st, c->bodies, c->cells, c->w,
+                                                                                 c->small_wpt);
+    if (prof) {
+      p1 = take_event(c);
+      (void)hipEventRecord(p1, s);
+      c->pass_events.push_back({p0, p1});
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(c, HMC_ERR_DEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
     c->applies += 1;
     return HMC_OK;
   }
@@ -942,6 +960,21 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         }
       }
     }
+  }
+  // A small system with isotropic pair energies in FP64: whole applies by one
+  // workgroup, where the system fits its LDS (about 1,400 bodies).  The
+  // per-colour passes cost a launch (15 us) per pass whatever the size.
+  // Measured us per step, they and this: 108 LJ bodies at density 0.8 1230 and
+  // 284, 864 1790 and 649, 1,372 3211 and 1242; 1,372 at 0.1 (64 trials a pass
+  // of two candidates) 351 and 342; 864 overlap-penalty bodies (125 trials a
+  // pass) 231 and 224, where the line is.
+  if (lj && !lj_mixed && g.n_bodies && g.n_bodies < 5000 && g.per_colour <= 128 && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS))) {
+    const SmallLds l = SmallLds::of(g);
+    const void* fn = D == 2 ? (const void*)k_apply_small<2> : (const void*)k_apply_small<3>;
+    hipFuncAttributes at{};
+    if (hipFuncGetAttributes(&at, fn) == hipSuccess && at.sharedSizeBytes + l.total <= 160 * 1024 &&
+        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.total) == hipSuccess)
+      c->small_wpt = g.per_colour <= 4 ? 4u : (g.per_colour <= 8 ? 2u : 1u);
   }
   const uint32_t N = g.n_bodies;
   c->n_scan_blocks = grid_for(g.n_spaces, kScanBlock);

@@ -26,6 +26,7 @@ struct hmc_ctx {
   TileCfg tc{};
   bool persist = false;  // one cooperative launch per apply (k_apply_tile)
   TileCfg pc{};
+  uint32_t small_wpt = 0;  // a small isotropic system: k_apply_small with this many wavefronts per trial (0: not)
   uint32_t pgrid = 0, pthreads = 0, pper_cu = 0;
   double* verts = nullptr;  // convex polyhedron vertices (device)
   SatShape sat{};           // convex, mixed precision: the FP32 separating axes (else use = 0)

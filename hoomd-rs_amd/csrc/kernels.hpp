@@ -26,6 +26,8 @@ template <int D>
 __global__ void k_bapply_tile(const BatchRep* reps, const TileCfg* tcs, const uint32_t* toff, const uint32_t* trep, ApplyState* sts, const uint32_t* rt0, const uint32_t* rn, uint32_t nrounds, uint32_t nwg, uint32_t xcd_chunk, uint32_t probe, uint32_t tag, Bodies B, Cells C, Work w);
 template <int D>
 __global__ void k_apply_lj(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
+template <int D>
+__global__ void k_apply_small(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t wpt);
 template <int D, int PREC>
 __global__ void k_guard(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t first_cycle);
 template <int D, int PREC>

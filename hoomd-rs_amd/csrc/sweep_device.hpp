@@ -728,6 +728,16 @@ __device__ __forceinline__ int lj_metropolis(Sfc64& rng, double dH, double delta
   *ambiguous = false;
   if (hi <= 0.0) return 1;
   const double u = uniform01(rng);
+  // The hardware's FP32 exp2 of FP32 quotients first, where they are moderate:
+  // q = -dH / kT to 2^-21 of |q| < 80, so exp(q) to 4e-5 and the hardware's ulp,
+  // decided with a margin of 2^-14 = 6.1e-5.  (Division and exp in FP64 are
+  // most of a decision otherwise.)
+  const float ik = __builtin_amdgcn_rcpf((float)kT) * 1.44269504f;
+  const float eh = -(float)hi * ik, el = -(float)lo * ik;
+  if (eh > -115.0f) {
+    if (u < (double)__builtin_amdgcn_exp2f(eh) * (1.0 - 0x1p-14)) return 1;
+    if (lo > 0.0 && u >= (double)__builtin_amdgcn_exp2f(el) * (1.0 + 0x1p-14)) return 0;
+  }
   // exp(q) for q within the interval, with the roundings of -dH / kT and of
   // exp itself covered by a relative margin of 2^-45 (1 + |q|)
   const double qa = -hi / kT;
@@ -752,6 +762,37 @@ struct LjOut {
 
 constexpr uint32_t kLjBatch = 4;  // candidate rounds of an LJ trial with their loads in flight together
 constexpr uint32_t kLjTab = 1024;  // candidate slots of an LJ trial laid out in LDS (else searched)
+
+// ------------------------------------------------------- small systems --
+constexpr int kSmallThreads = 1024;  // k_apply_small: 16 wavefronts
+constexpr int kSmallList = 256;      // squared distances a wavefront lists before evaluating them
+// Byte offsets of k_apply_small's dynamic LDS: the sites (32 bytes), their ghost
+// images (24) and the bodies (24) in slot order, a proposal per space, the neighbour rows of every space
+// (8 bytes each), the spaces' first slots and the spaces by colour (16 bits).
+struct SmallLds {
+  static constexpr uint32_t kPropBytes = 88;
+  uint32_t site, rows, prop, body, ghost, start, order, total;
+  __host__ __device__ static SmallLds of(uint32_t n, uint32_t spaces, uint32_t nrows) {
+    SmallLds l;
+    l.site = 0;
+    l.rows = 32u * n;
+    l.prop = l.rows + 8u * nrows * spaces;
+    l.body = l.prop + kPropBytes * spaces;
+    l.ghost = l.body + 24u * n;
+    l.start = l.ghost + 24u * n;
+    l.order = l.start + 2u * (spaces + 1u);
+    l.total = (l.order + 2u * spaces + 15u) & ~15u;
+    return l;
+  }
+  __host__ __device__ static SmallLds of(const Geometry& g) {
+    uint32_t n[3] = {1, 1, 1};
+    for (int a = 0; a < g.dim; ++a) {
+      const uint32_t w = 2u * (uint32_t)g.reach[a] + 1u, sh = (uint32_t)g.shape[a];
+      n[a] = w < sh ? w : sh;
+    }
+    return of(g.n_bodies, g.n_spaces, g.dim == 3 ? n[0] * n[1] : n[0]);
+  }
+};
 
 // ------------------------------------------------------ convex polyhedra --
 // Image of site sj nearest q per axis (the one the reference's neighbour

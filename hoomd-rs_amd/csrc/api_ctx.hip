@@ -19,6 +19,8 @@ hipEvent_t take_event(hmc_ctx* c) {
 // The persistent apply's kernel for a context.
 static const void* persist_kernel(const hmc_ctx* c) {
   const bool d2 = c->g.dim == 2;
+  if (c->g.model == HMC_CONVEX_POLYHEDRON)
+    return c->g.cv_mixed ? (const void*)k_apply_convex<true> : (const void*)k_apply_convex<false>;
   if (is_isotropic(c->g.model)) return d2 ? (const void*)k_apply_lj<2> : (const void*)k_apply_lj<3>;
   if (c->cfg.precision == HMC_MIXED)
     return d2 ? (const void*)k_apply_tile<2, float> : (const void*)k_apply_tile<3, float>;
@@ -52,7 +54,7 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
   if (N) {
     k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
     // (these applies stage their sites from the FP64 copies)
-    if (c->persist || c->small_wpt)
+    if ((c->persist && g.model != HMC_CONVEX_POLYHEDRON) || c->small_wpt)
       k_place<PREC, false><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
     else
       k_place<PREC><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
@@ -72,7 +74,8 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
     }
     ApplyState* stp = c->st;
     c->pc.tag += 1;
-    void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&c->pc};
+    void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&c->pc,
+                    (void*)&c->sat};  // (the last for convex polyhedra)
     const hipError_t le =
         hipLaunchCooperativeKernel(persist_kernel(c), dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, s);
     if (le != hipSuccess) return fail(c, HMC_ERR_DEVICE, std::string("cooperative launch: ") + hipGetErrorString(le));
@@ -413,7 +416,8 @@ bool persist_probe(hmc_ctx* c) {
   pc.probe = 1;
   Geometry g = c->g;
   ApplyState* stp = c->st;
-  void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&pc};
+  void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&pc,
+                  (void*)&c->sat};
   const size_t fbytes = (size_t)c->pc.ntiles * kMailboxStride * sizeof(uint32_t);
   uint32_t err = 0;
   bool ok = hipLaunchCooperativeKernel(persist_kernel(c), dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, c->stream) ==
@@ -495,6 +499,38 @@ bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* o
           out->xcd_chunk = (ntiles + 7) / 8;
           out->lds_bytes = (uint32_t)lds;
         }
+      }
+  return found;
+}
+
+// Region shape of the persistent convex apply (k_apply_convex), whose sites
+// stay in global memory: at most kCvTrials spaces of a colour, with all regions
+// resident together; the fewest regions, then the smallest surface (1 x 2 x 2
+// where the shape divides evenly).  False where more trials per region would be
+// needed: with two rounds of them 262,144 cubes took 1737, 2583 and 2077 us per
+// step at packing fractions 0.3, 0.4 and 0.5, with one launch per colour 1519,
+// 2021 and 1528; with one round (125,000 cubes) 941, 1115 and 1140 against 1219,
+// 1469 and 1522 with one launch per colour.
+static bool choose_regions_convex(const Geometry& g, uint32_t resident, TileCfg* out) {
+  bool found = false;
+  uint32_t best_face = 0;
+  for (uint32_t t0 = 1; t0 <= std::min<uint32_t>(g.half_shape[0], kCvTrials); ++t0)
+    for (uint32_t t1 = 1; t1 <= std::min<uint32_t>(g.half_shape[1], kCvTrials); ++t1)
+      for (uint32_t t2 = 1; t2 <= std::min<uint32_t>(g.half_shape[2], kCvTrials); ++t2) {
+        const uint32_t T[3] = {t0, t1, t2}, face = t0 * t1 + t1 * t2 + t2 * t0;
+        uint64_t n = 1;
+        for (int a = 0; a < 3; ++a) n *= (g.half_shape[a] + T[a] - 1) / T[a];
+        if (t0 * t1 * t2 > kCvTrials || (n + 7) / 8 * 8 > resident) continue;
+        if (found && (n > out->ntiles || (n == out->ntiles && face >= best_face))) continue;
+        found = true;
+        best_face = face;
+        for (int a = 0; a < 3; ++a) {
+          out->T[a] = T[a];
+          out->nt[a] = (g.half_shape[a] + T[a] - 1) / T[a];
+        }
+        out->trials = t0 * t1 * t2;
+        out->ntiles = (uint32_t)n;
+        out->xcd_chunk = (out->ntiles + 7) / 8;
       }
   return found;
 }
@@ -958,6 +994,29 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
           delete c;
           return HMC_ERR_DEVICE;
         }
+      }
+    }
+  }
+  // Convex polyhedra: one persistent launch per apply (k_apply_convex) where
+  // the neighbour scan reaches one space out and a wavefront per kCvTrials
+  // spaces of a colour is resident.
+  if (convex && g.reach[0] == 1 && g.reach[1] == 1 && g.reach[2] == 1 &&
+      !(cfg_in->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS))) {
+    int cus = 0, coop = 0, per_cu = 0;
+    TileCfg pc{};
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, persist_kernel(c), kCvApply, 0) == hipSuccess &&
+        choose_regions_convex(g, (uint32_t)per_cu * (uint32_t)cus, &pc)) {
+      c->persist = true;
+      c->pc = pc;
+      c->pgrid = pc.xcd_chunk * 8u;
+      c->pthreads = kCvApply;
+      c->pper_cu = (uint32_t)per_cu;
+      const size_t fbytes = (size_t)pc.ntiles * kMailboxStride * sizeof(uint32_t);
+      if (hipMalloc((void**)&c->w.mbox, fbytes) != hipSuccess || hipMemset(c->w.mbox, 0, fbytes) != hipSuccess) {
+        delete c;
+        return HMC_ERR_DEVICE;
       }
     }
   }

@@ -1,5 +1,5 @@
 // Hard convex polyhedra: translate and rotate trials with XenoCollide.
-#include "sweep_device.hpp"
+#include "persist.hpp"
 
 namespace hmc {
 
@@ -270,29 +270,43 @@ __device__ __forceinline__ uint32_t sat_dispatch(const SatShape& S, bool act, co
 }
 
 // Convex pass layout: kCvTrials trials per wavefront, one per group of
-// kCvLanes lanes (the group draws its trial's proposal and lists its
+// kCvLanes lanes (the group draws its trial's proposal and lists its rows of
 // neighbour spaces); the candidate sites of all the wavefront's trials are
 // tested against the circumsphere cutoff 64 at a time (kCvBatch rounds with
 // their loads in flight together), the pairs within it are gathered in a
 // per-wavefront list, and XenoCollide runs over that list 64 pairs at a time.
 // Any overlap rejects a hard-shape trial, so the order of the pair tests does
 // not change a decision (parallel_sweep.rs:267-273).
-constexpr uint32_t kCvSegs = 128;  // neighbour spaces of one trial: at most 5^3
-constexpr uint32_t kCvBatch = 4;
-constexpr uint32_t kCvPairs = 384;  // listed pairs; tested once more than kCvPairs - 64 kCvBatch are pending
+constexpr uint32_t kCvRows = 25;    // rows of neighbour spaces of one trial: at most 5^2
+constexpr uint32_t kCvBatch = 6;    // rounds of 64 candidates with their loads in flight together
+constexpr uint32_t kCvPairs = 512;  // listed pairs; tested once more than kCvPairs - 64 kCvBatch are pending
 struct CvWave {
-  uint32_t pre[kCvTrials][kCvSegs];  // index of the first candidate of each neighbour space, per trial
-  uint32_t lo[kCvTrials][kCvSegs];   // its first slot
+  // per trial and row: its candidates are `la` slots from ra, then the slots from
+  // rb; x = ra, y = la, z = rb - la, w = the index of its first candidate
+  uint4 row[kCvTrials][kCvRows];
   uint32_t qs[kCvPairs];             // the listed pair's neighbour slot
   uint32_t tk[kCvPairs];             // and trial
   double t[kCvTrials][3];            // trial site position
   double qt[kCvTrials][4];           // trial site orientation
+  // what an acceptance stores besides: the body's orientation, the site and its
+  // ghost flags (kept here, not in registers, while the pairs are tested)
+  double qb[kCvTrials][4];
+  double ns[kCvTrials][3];
+  uint32_t flags[kCvTrials];
 };
 
 // XenoCollide over the np listed pairs; returns the trials (bits) that
 // found an overlap, skipping pairs of trials already in `hits`.  NV: the
 // vertex count when it is one of the specialised ones, else 0.
-template <int NV>
+//
+// DEV: the sites are read with device-scope loads (the persistent apply, where
+// other regions write them during the launch).
+template <bool DEV>
+__device__ __forceinline__ double4 cv_load(const double4* p) {
+  if constexpr (DEV) return ld_dev_d4(p);
+  return *p;
+}
+template <int NV, bool DEV>
 __device__ __forceinline__ uint32_t cv_pair_tests(const Geometry& g, const Cells& C, const CvWave& W,
                                                   const double* vx, uint32_t np, uint32_t hits) {
   const uint32_t lane = __lane_id();
@@ -304,8 +318,8 @@ __device__ __forceinline__ uint32_t cv_pair_tests(const Geometry& g, const Cells
       kp = W.tk[p];
       if (!((hits >> kp) & 1u)) {
         const uint32_t qs = W.qs[p];
-        const double4 sj = C.pos64[qs];
-        const double4 qj4 = C.quat64[qs];
+        const double4 sj = cv_load<DEV>(&C.pos64[qs]);
+        const double4 qj4 = cv_load<DEV>(&C.quat64[qs]);
         const double tq[3] = {W.t[kp][0], W.t[kp][1], W.t[kp][2]};
         v3 rj;
         (void)convex_image(g, tq, sj, &rj);  // the image found when the pair was listed
@@ -326,6 +340,7 @@ __device__ __forceinline__ uint32_t cv_pair_tests(const Geometry& g, const Cells
 // Certain overlaps set their trial's bit in *hits; the undecided pairs are
 // moved to the front of the list (in order) for XenoCollide in FP64, and
 // their number is returned.
+template <bool DEV>
 __device__ __forceinline__ uint32_t cv_sat_filter(const Geometry& g, const Cells& C, CvWave& W, const SatShape& S,
                                                   uint32_t np, uint32_t* hits) {
   const uint32_t lane = __lane_id();
@@ -340,8 +355,8 @@ __device__ __forceinline__ uint32_t cv_sat_filter(const Geometry& g, const Cells
       if (!((*hits >> kp) & 1u)) {
         act = true;
         qs = W.qs[p];
-        const double4 sj = C.pos64[qs];
-        const double4 qj4 = C.quat64[qs];
+        const double4 sj = cv_load<DEV>(&C.pos64[qs]);
+        const double4 qj4 = cv_load<DEV>(&C.quat64[qs]);
         const double tq[3] = {W.t[kp][0], W.t[kp][1], W.t[kp][2]};
         v3 rj;
         (void)convex_image(g, tq, sj, &rj);  // the image found when the pair was listed
@@ -364,90 +379,87 @@ __device__ __forceinline__ uint32_t cv_sat_filter(const Geometry& g, const Cells
   return nb;
 }
 
-// One colour of one cycle for convex polyhedra: kCvTrials spaces per
-// wavefront.  Each trial is the one of trial_convex (parallel_sweep.rs:234-277
-// with Translate or Rotate<Versor>).
+// Trials of convex polyhedra: kCvTrials spaces per wavefront.  Each trial is the
+// one of trial_convex (parallel_sweep.rs:234-277 with Translate or
+// Rotate<Versor>).
 // (three wavefronts per SIMD: 22% faster on C3 than the two its free
-// register use allows)
+// register use allows; with rows listed by compares instead of 27 spaces by
+// remainders, rows and row ends beyond the cutoff left out, and what an
+// acceptance stores kept in LDS, 262,144 cubes at packing fractions 0.3, 0.4
+// and 0.5 went from 1819, 2432 and 1815 us per step to 1519, 2021 and 1528)
 // MIXED: the listed pairs go through the FP32 separating-axis tests first
 // (cv_sat_filter); only the undecided ones run XenoCollide in FP64.
-template <bool MIXED>
-__global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyState* st, Bodies B, Cells C, Work w,
-                                                        uint32_t colour, uint32_t cycle, uint32_t xcd_chunk,
-                                                        SatShape sat) {
-  if (cycle >= st->cycles) return;  // uniform over the grid
-  __shared__ unsigned blk_acc;
-  __shared__ double zx[257], zf[257];
-  __shared__ double vx[3 * kMaxVertices];
-  __shared__ CvWave cw[kBlock / 64];
-  if (threadIdx.x == 0) blk_acc = 0;
-  stage_zig(zx, zf);
-  stage_verts(g, vx);
-  __syncthreads();
-  const uint32_t b = blockIdx.x;
-  const uint32_t lb = (b & 7u) * xcd_chunk + (b >> 3);
+// The trials of one wavefront: lane group k's in space s (multi-index m) where
+// `have` holds (all lanes of a group alike).  ready(): called by the whole
+// wavefront before it reads any neighbour's site; what precedes it -- the
+// neighbour listing and the proposal -- reads only static cell data and the
+// trial's own body.
+template <bool MIXED, bool DEV, class Ready>
+__device__ __forceinline__ void cv_trials(const Geometry& g, ApplyState* st, const Bodies& B, const Cells& C,
+                                          const Work& w, CvWave& W, const double* vx, const double* zx,
+                                          const double* zf, const SatShape& sat, bool have, uint32_t s,
+                                          const int32_t* m, uint32_t colour, uint32_t substep, unsigned* blk_acc,
+                                          Ready ready) {
   const uint32_t lane = __lane_id(), k = lane / kCvLanes, kl = lane % kCvLanes;
-  CvWave& W = cw[threadIdx.x >> 6];
-  const uint32_t tix = (lb * (kBlock / 64) + (threadIdx.x >> 6)) * kCvTrials + k;
-  const uint32_t substep = st->substep0 + cycle;
-  // the trial of lane group k (all its lanes draw the same proposal)
-  bool tried = false, active = false;
-  uint32_t s = 0, slot = 0xFFFFFFFFu, body = 0;
-  int32_t m[3] = {0, 0, 0};
-  double x[3] = {0.0, 0.0, 0.0};
-  quat q = {1.0, {0.0, 0.0, 0.0}};
+  const GeoPtr gp = geo_ptr(g.self);
+  bool tried = false;
+  uint32_t slot = 0xFFFFFFFFu, body = 0;
   Sfc64 rng = {0, 0, 0, 0};
-  if (tix < g.per_colour) {
-    s = colour_space<3>(g, colour, tix, m);
+  // The rows of neighbour spaces along the last axis (each space once, as the
+  // reference's cell list visits them), a lane per row: the first slots of the
+  // row's lower, own and upper space (lo, mid, hi; the next space's where that is
+  // contiguous), loaded before the proposal is drawn.  Where the scan reaches
+  // two spaces or an axis has two, the row is one run (lo .. hi) or two.
+  uint32_t nn[3], first[3];
+  bool plain = true;  // three distinct spaces along every axis
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const uint32_t sh = (uint32_t)g.shape[a], r = (uint32_t)g.reach[a], x = (uint32_t)m[a];
+    const bool all = 2u * r + 1u >= sh;
+    nn[a] = all ? sh : 2u * r + 1u;
+    first[a] = all ? 0u : (x >= r ? x - r : x + sh - r);
+    plain = plain && r == 1u && sh >= 3u;
+  }
+  if (plain) {  // (of three spaces, too, the lower one comes first)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) first[a] = m[a] ? (uint32_t)m[a] - 1u : (uint32_t)g.shape[a] - 1u;
+  }
+  const uint32_t nrow = nn[0] * nn[1], inv1 = (256u + nn[1] - 1u) / nn[1];
+  uint32_t st0[2] = {0, 0}, st1[2] = {0, 0}, st2[2] = {0, 0}, st3[2] = {0, 0}, st4[2] = {0, 0}, st5[2] = {0, 0};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t j = kl + (uint32_t)h * kCvLanes;
+    if (!have || j >= nrow) continue;
+    const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn[1];
+    uint32_t y0 = first[0] + i0, y1 = first[1] + i1;
+    y0 = y0 >= (uint32_t)g.shape[0] ? y0 - (uint32_t)g.shape[0] : y0;
+    y1 = y1 >= (uint32_t)g.shape[1] ? y1 - (uint32_t)g.shape[1] : y1;
+    const uint32_t sb = y0 * g.stride[0] + y1 * g.stride[1], sh = (uint32_t)g.shape[2];
+    if (plain) {
+      const uint32_t mid = sb + (uint32_t)m[2], hi = sb + ((uint32_t)m[2] + 1u == sh ? 0u : (uint32_t)m[2] + 1u);
+      st0[h] = w.start[sb + first[2]];
+      st1[h] = w.start[sb + first[2] + 1u];
+      st2[h] = w.start[mid];
+      st3[h] = w.start[mid + 1u];
+      st4[h] = w.start[hi];
+      st5[h] = w.start[hi + 1u];
+    } else {
+      const uint32_t end = first[2] + nn[2];
+      st2[h] = w.start[sb + first[2]];
+      st3[h] = w.start[sb + min(end, sh)];
+      st4[h] = w.start[sb];
+      st5[h] = end > sh ? w.start[sb + end - sh] : st4[h];
+    }
+  }
+  if (have) {
     const uint32_t s0 = w.start[s];
     const uint32_t n = w.start[s + 1] - s0;
     if (n) {
       tried = true;
-      rng = counter_rng(st->step, substep, st->seed, s);
+      rng = counter_rng<DEV>(st->step, substep, st->seed, s);
       slot = s0 + choose_index(rng, n);
       body = C.body[slot];
     }
-  }
-  // the trial's neighbour spaces (distinct ones, as the reference's cell
-  // list visits each once) and the first candidate index of each; listed
-  // before the proposal is drawn so that their loads overlap the body's
-  uint32_t nb[3][5];
-  uint32_t nn[3] = {0, 0, 0};
-  if (tried) {
-    for (int a = 0; a < 3; ++a) {
-      const int32_t sh = g.shape[a], r = g.reach[a];
-      uint32_t c = 0;
-      for (int off = -r; off <= r; ++off) {
-        const int32_t mm = ((m[a] + off) % sh + sh) % sh;
-        bool seen = false;
-        for (uint32_t j = 0; j < c; ++j) seen |= nb[a][j] == (uint32_t)mm * g.stride[a];
-        if (!seen) nb[a][c++] = (uint32_t)mm * g.stride[a];
-      }
-      nn[a] = c;
-    }
-  }
-  const uint32_t NS = nn[0] * nn[1] * nn[2];  // at most 125
-  uint32_t tot = 0;
-  for (uint32_t j0 = 0; __ballot(j0 < NS) != 0ull; j0 += kCvLanes) {
-    const uint32_t j = j0 + kl;
-    uint32_t cnt = 0, lo = 0;
-    if (j < NS) {
-      const uint32_t i2 = j % nn[2], i1 = (j / nn[2]) % nn[1], i0 = j / (nn[2] * nn[1]);
-      const uint32_t ns = nb[0][i0] + nb[1][i1] + nb[2][i2];
-      lo = w.start[ns];
-      cnt = w.start[ns + 1] - lo;
-    }
-    uint32_t incl = cnt;
-#pragma unroll
-    for (uint32_t d = 1; d < kCvLanes; d <<= 1) {
-      const uint32_t u = __shfl_up(incl, d, kCvLanes);
-      if (kl >= d) incl += u;
-    }
-    if (j < NS) {
-      W.pre[k][j] = tot + incl - cnt;
-      W.lo[k][j] = lo;
-    }
-    tot += __shfl(incl, (int)(lane | (kCvLanes - 1)), 64);
   }
   // the proposal (the random draws overlap the loads of the body)
   double4 bp = make_double4(0.0, 0.0, 0.0, 0.0), bq = make_double4(1.0, 0.0, 0.0, 0.0);
@@ -457,38 +469,86 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
   }
   double v[3] = {0.0, 0.0, 0.0};
   quat dq = {1.0, {0.0, 0.0, 0.0}};
+  const bool translate = st->move == 0;
   if (tried) {
-    if (st->move == 0)
+    if (translate)
       ball_sample<3>(rng, st->max_move, zx, zf, v);
     else
       dq = versor_displacement(rng, st->max_move, zx, zf);
   }
-  if (tried) {
-    x[0] = bp.x;
-    x[1] = bp.y;
-    x[2] = bp.z;
-    q = {bq.x, {bq.y, bq.z, bq.w}};
-    if (st->move == 0) {
-      for (int a = 0; a < 3; ++a) x[a] += v[a];
-    } else {
-      q = qmul(dq, q);
-    }
-    for (int a = 0; a < 3; ++a) x[a] = wrap1(g, a, x[a]);  // wrap(propose(..))
-    active = space_of<3>(g, st->origin, x) == s;
-  }
-  if (!active) tot = 0;  // a trial outside its space is rejected without pair tests
-  // the trial site: wrap(x + rotate(q, 0)) with orientation q * identity
-  // (property/oriented_point.rs:107-113)
+  quat q = {bq.x, {bq.y, bq.z, bq.w}};
+  if (!translate) q = qmul(dq, q);
+  // The trial body wrap(propose(..)), its site wrap(x + rotate(q, 0)) with
+  // orientation q * identity (property/oriented_point.rs:107-113) and the site
+  // an acceptance stores: rotate(q, 0) is zero, so they are those of a point
+  // body (a NaN orientation makes the position NaN, as in the reference).
   const v3 r0 = qrotate(q, v3{0.0, 0.0, 0.0});
   const quat qt = qmul(q, quat{1.0, {0.0, 0.0, 0.0}});
+  const double origin[3] = {st->origin[0], st->origin[1], st->origin[2]};
+  const double x0[3] = {bp.x + v[0] + r0.x, bp.y + v[1] + r0.y, bp.z + v[2] + r0.z};
+  const uint32_t own[3] = {(uint32_t)m[0], (uint32_t)m[1], (uint32_t)m[2]};
+  TrialSite<3> ts{};
+  if (tried) ts = trial_site<3>(gp, st, origin, x0, own, s);
+  const bool active = tried && ts.in;
   if (active && kl == 0) {
-    W.t[k][0] = wrap1(g, 0, x[0] + r0.x);
-    W.t[k][1] = wrap1(g, 1, x[1] + r0.y);
-    W.t[k][2] = wrap1(g, 2, x[2] + r0.z);
+    W.t[k][0] = ts.t[0];
+    W.t[k][1] = ts.t[1];
+    W.t[k][2] = ts.t[2];
     W.qt[k][0] = qt.s;
     W.qt[k][1] = qt.v.x;
     W.qt[k][2] = qt.v.y;
     W.qt[k][3] = qt.v.z;
+    W.qb[k][0] = q.s;
+    W.qb[k][1] = q.v.x;
+    W.qb[k][2] = q.v.y;
+    W.qb[k][3] = q.v.z;
+    W.ns[k][0] = ts.n[0];
+    W.ns[k][1] = ts.n[1];
+    W.ns[k][2] = ts.n[2];
+    W.flags[k] = ts.flags;
+  }
+  // Rows and row ends whose nearest point is the circumsphere cutoff away hold no
+  // pair (27 spaces become 20 on average): cut by the distance from the trial
+  // site to the faces of its space, with a margin of 10^-4 for the roundings.
+  // (A trial outside its space is rejected without pair tests.)
+  const float cut = (float)g.cv_rcut2 * (1.0f + 1e-4f);
+  float flo[3], fhi[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    double u = ts.t[a] - origin[a];
+    u = u >= gp->L[a] ? u - gp->L[a] : u;
+    u -= (double)own[a] * gp->width[a];
+    const float wd = (float)gp->width[a], uf = (float)u, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
+    flo[a] = dl * dl;
+    fhi[a] = dh * dh;
+  }
+  uint32_t tot = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t j = kl + (uint32_t)h * kCvLanes;
+    const bool mine = active && j < nrow;
+    uint32_t ra = st2[h], ea = st3[h], rb = st4[h], eb = plain ? st4[h] : st5[h];
+    if (plain) {
+      const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn[1];
+      const float d = (i0 == 0 ? flo[0] : i0 == 2 ? fhi[0] : 0.0f) + (i1 == 0 ? flo[1] : i1 == 2 ? fhi[1] : 0.0f);
+      const bool lo = d + flo[2] < cut, hi = d + fhi[2] < cut;
+      const bool wlo = m[2] == 0, whi = m[2] + 1 == g.shape[2];  // the lower / upper space lies across the face
+      ra = lo && !wlo ? st0[h] : ra;
+      ea = hi && !whi ? st5[h] : ea;
+      rb = wlo ? st0[h] : st4[h];
+      eb = wlo ? (lo ? st1[h] : rb) : (whi && hi ? st5[h] : rb);
+      if (!(d < cut)) ea = ra, eb = rb;
+    }
+    const uint32_t la = ea - ra, cnt = mine ? la + (eb - rb) : 0u;
+    uint32_t incl = cnt;
+#pragma unroll
+    for (uint32_t dd = 1; dd < kCvLanes; dd <<= 1) {
+      const uint32_t u = __shfl_up(incl, dd, kCvLanes);
+      if (kl >= dd) incl += u;
+    }
+    if (mine) W.row[k][j] = make_uint4(ra, la, rb - la, tot + incl - cnt);
+    tot += __shfl(incl, (int)(lane | (kCvLanes - 1)), 64);
+    if (h == 0 && !__any(nrow > kCvLanes)) break;
   }
   uint32_t base[kCvTrials + 1];
   base[0] = 0;
@@ -496,6 +556,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
   for (uint32_t i = 0; i < kCvTrials; ++i) base[i + 1] = base[i] + __shfl(tot, (int)(i * kCvLanes), 64);
   const uint32_t total = base[kCvTrials];
   wave_lds_order();
+  ready();
   uint32_t hits = 0;  // trials with an overlap (uniform over the wavefront)
   uint32_t np = 0;    // listed pairs (uniform)
   uint32_t nband = 0; // MIXED: pairs left to FP64 XenoCollide (uniform)
@@ -512,20 +573,21 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
           kc = i;
           bk = base[i];
         }
-      const uint32_t nsk = __shfl(NS, (int)(kc * kCvLanes), 64);
       const uint32_t slk = __shfl(slot, (int)(kc * kCvLanes), 64);
       ok[r] = c < total && !((hits >> kc) & 1u);
       uint32_t qs = 0;
       if (ok[r]) {
-        // neighbour space of candidate c: last one whose first index is <= c
+        // row of candidate c: the last one whose first index is <= c (nrow is
+        // the same for every trial)
         const uint32_t cl = c - bk;
         uint32_t jlo = 0;
-#pragma unroll
-        for (uint32_t sw = kCvSegs / 2; sw >= 1; sw >>= 1) {
+        for (uint32_t sw = nrow > 16u ? 16u : 8u; sw >= 1; sw >>= 1) {
           const uint32_t mid = jlo + sw;
-          if (mid < nsk && W.pre[kc][mid] <= cl) jlo = mid;
+          if (mid < nrow && W.row[kc][mid].w <= cl) jlo = mid;
         }
-        qs = W.lo[kc][jlo] + (cl - W.pre[kc][jlo]);
+        const uint4 q4 = W.row[kc][jlo];
+        const uint32_t e = cl - q4.w;
+        qs = (e < q4.y ? q4.x : q4.z) + e;
         ok[r] = qs != slk;
       }
       qsv[r] = qs;
@@ -533,7 +595,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
     }
     double4 sj[kCvBatch];
 #pragma unroll
-    for (uint32_t r = 0; r < kCvBatch; ++r) sj[r] = ok[r] ? C.pos64[qsv[r]] : make_double4(0.0, 0.0, 0.0, 0.0);
+    for (uint32_t r = 0; r < kCvBatch; ++r) sj[r] = ok[r] ? cv_load<DEV>(&C.pos64[qsv[r]]) : make_double4(0.0, 0.0, 0.0, 0.0);
 #pragma unroll
     for (uint32_t r = 0; r < kCvBatch; ++r) {
       bool inr = false;
@@ -553,7 +615,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
     if (np + 64 * kCvBatch > kCvPairs || c0 + 64 * kCvBatch >= total) {  // uniform
       wave_lds_order();
       if (MIXED && sat.use) {
-        np = cv_sat_filter(g, C, W, sat, np, &hits);
+        np = cv_sat_filter<DEV>(g, C, W, sat, np, &hits);
         nband += np;
         wave_lds_order();
       }
@@ -562,13 +624,13 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
       // made those wavefronts slower)
       if (np == 0) {
       } else if (g.nverts == 8)
-        hits = cv_pair_tests<8>(g, C, W, vx, np, hits);
+        hits = cv_pair_tests<8, DEV>(g, C, W, vx, np, hits);
       else if (g.nverts == 6)
-        hits = cv_pair_tests<6>(g, C, W, vx, np, hits);
+        hits = cv_pair_tests<6, DEV>(g, C, W, vx, np, hits);
       else if (g.nverts == 4)
-        hits = cv_pair_tests<4>(g, C, W, vx, np, hits);
+        hits = cv_pair_tests<4, DEV>(g, C, W, vx, np, hits);
       else
-        hits = cv_pair_tests<0>(g, C, W, vx, np, hits);
+        hits = cv_pair_tests<0, DEV>(g, C, W, vx, np, hits);
       np = 0;
       wave_lds_order();
     }
@@ -579,20 +641,20 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
     if (accept) {
       // update_body_properties (microstate.rs:985-1034): body = wrap(props),
       // site = wrap(body.transform(site))
-      double nb3[3], ns3[3];
-      for (int a = 0; a < 3; ++a) nb3[a] = wrap1(g, a, x[a]);
-      const double r0a[3] = {r0.x, r0.y, r0.z};
-      for (int a = 0; a < 3; ++a) ns3[a] = wrap1(g, a, nb3[a] + r0a[a]);
-      const uint32_t fl = ghost_flags<3>(g, ns3);
-      B.bpos[body] = make_double4(nb3[0], nb3[1], nb3[2], move_stamp(st->epoch));
-      B.bquat[body] = make_double4(q.s, q.v.x, q.v.y, q.v.z);
-      const double4 sp = pack_site(ns3, fl);
-      const double4 sq = make_double4(qt.s, qt.v.x, qt.v.y, qt.v.z);
+      B.bpos[body] = make_double4(W.t[k][0], W.t[k][1], W.t[k][2], move_stamp(st->epoch));
+      B.bquat[body] = make_double4(W.qb[k][0], W.qb[k][1], W.qb[k][2], W.qb[k][3]);
+      const double4 sp = pack_site(W.ns[k], W.flags[k]);
+      const double4 sq = make_double4(W.qt[k][0], W.qt[k][1], W.qt[k][2], W.qt[k][3]);
       B.spos[body] = sp;
       B.squat[body] = sq;
-      C.pos64[slot] = sp;
-      C.quat64[slot] = sq;
-      atomicAdd(&blk_acc, 1u);
+      if constexpr (DEV) {
+        st_dev_d4(&C.pos64[slot], sp);
+        st_dev_d4(&C.quat64[slot], sq);
+      } else {
+        C.pos64[slot] = sp;
+        C.quat64[slot] = sq;
+      }
+      atomicAdd(blk_acc, 1u);
     }
     if (w.tracing) {
       unsigned long long ti = atomicAdd((unsigned long long*)&st->trace_n, 1ull);
@@ -607,6 +669,94 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
         w.trace[ti] = rec;
       }
     }
+  }
+}
+
+template <bool MIXED>
+__global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyState* st, Bodies B, Cells C, Work w,
+                                                        uint32_t colour, uint32_t cycle, uint32_t xcd_chunk,
+                                                        SatShape sat) {
+  if (cycle >= st->cycles) return;  // uniform over the grid
+  __shared__ unsigned blk_acc;
+  __shared__ double zx[257], zf[257];
+  __shared__ double vx[3 * kMaxVertices];
+  __shared__ CvWave cw[kBlock / 64];
+  if (threadIdx.x == 0) blk_acc = 0;
+  stage_zig(zx, zf);
+  stage_verts(g, vx);
+  __syncthreads();
+  const uint32_t b = blockIdx.x;
+  const uint32_t lb = (b & 7u) * xcd_chunk + (b >> 3);
+  const uint32_t tix = (lb * (kBlock / 64) + (threadIdx.x >> 6)) * kCvTrials + __lane_id() / kCvLanes;
+  int32_t m[3] = {0, 0, 0};
+  uint32_t s = 0;
+  const bool have = tix < g.per_colour;
+  if (have) s = colour_space<3>(g, colour, tix, m);
+  cv_trials<MIXED, false>(g, st, B, C, w, cw[threadIdx.x >> 6], vx, zx, zf, sat, have, s, m, colour,
+                          st->substep0 + cycle, &blk_acc, [] {});
+  __syncthreads();
+  if (threadIdx.x == 0 && blk_acc) atomicAdd(&w.acc_slots[b & (kAccSlots - 1)], (unsigned long long)blk_acc);
+}
+
+// Every cycle and colour of an apply in one cooperative launch: wavefront b
+// owns a region of 2 T spaces per axis with at most kCvTrials of each colour
+// and runs them as a pass of cv_trials.  The sites stay in global memory
+// (stores and loads of device scope), and a region waits only for the
+// neighbours its next trials read (region_wait), after their proposals.
+// One launch per pass spent most of its time on the launch, on fetching the
+// code anew (55 KB) and on the slowest wavefront of the whole device: 262,144
+// cubes at packing fraction 0.55 (10,648 trials per pass) took 2421 us per step
+// and take 1821, 2,744 cubes 1321 and 923.  Regions of four wavefronts took
+// 1949 (a pass of a region is as long as its slowest wavefront), of two 1911.
+// Bound by the chain of a pass: proposal 8, XenoCollide of the slowest pair 15,
+// candidates 9, waits 20 thousand cycles of 60.
+template <bool MIXED>
+__global__ void __launch_bounds__(kCvApply, 3) k_apply_convex(Geometry g, ApplyState* st, Bodies B, Cells C, Work w,
+                                                         TileCfg tc, SatShape sat) {
+  const uint32_t b = blockIdx.x;
+  const uint32_t tile = (b & 7u) * tc.xcd_chunk + (b >> 3);  // XCD-aware region order
+  if (tile >= tc.ntiles) return;  // padding workgroups (grid rounded up to 8) take part in nothing
+  if (tc.probe) {
+    region_probe(st, w.mbox, tc.ntiles);
+    return;
+  }
+  __shared__ unsigned blk_acc;
+  __shared__ double zx[257], zf[257];
+  __shared__ double vx[3 * kMaxVertices];
+  __shared__ CvWave cw;
+  if (threadIdx.x == 0) blk_acc = 0;
+  stage_zig(zx, zf);
+  stage_verts(g, vx);
+  Region rg{};
+  {
+    uint32_t r = tile;
+    for (int a = 2; a >= 0; --a) {
+      rg.tcd[a] = r % tc.nt[a];
+      r /= tc.nt[a];
+      rg.org[a] = (int32_t)(2 * rg.tcd[a] * tc.T[a]);
+      rg.rl[a] = min((int32_t)(2 * tc.T[a]), g.shape[a] - rg.org[a]);
+    }
+  }
+  const uint32_t cycles = st->cycles, substep0 = st->substep0;
+  __syncthreads();
+  for (uint32_t i = 0; i < 8 * cycles; ++i) {
+    const uint32_t colour = i & 7u;
+    if (i) region_publish(w.mbox, tile, tc.tag, i);
+    uint32_t t = __lane_id() / kCvLanes;
+    bool have = t < tc.trials;
+    int32_t m[3] = {0, 0, 0};
+    uint32_t s = 0;
+    for (int a = 2; a >= 0; --a) {
+      const int32_t l = (int32_t)(2 * (t % tc.T[a]) + ((colour >> (2 - a)) & 1u));
+      t /= tc.T[a];
+      have = have && l < rg.rl[a];
+      m[a] = rg.org[a] + l;
+      s += (uint32_t)m[a] * g.stride[a];
+    }
+    if (!have) s = 0;
+    cv_trials<MIXED, true>(g, st, B, C, w, cw, vx, zx, zf, sat, have, s, m, colour, substep0 + (i >> 3), &blk_acc, [&] {
+      if (i) region_wait<3>(st, w.mbox, tc, rg, tile, i);
+    });
   }
   __syncthreads();
   if (threadIdx.x == 0 && blk_acc) atomicAdd(&w.acc_slots[b & (kAccSlots - 1)], (unsigned long long)blk_acc);
@@ -776,6 +926,8 @@ __global__ void k_debug_convex(int kind, const double* vx, uint32_t nv, double r
 }
 
 // explicit instantiations (launched from the host translation units)
+template __global__ void k_apply_convex<false>(Geometry, ApplyState*, Bodies, Cells, Work, TileCfg, SatShape);
+template __global__ void k_apply_convex<true>(Geometry, ApplyState*, Bodies, Cells, Work, TileCfg, SatShape);
 template __global__ void k_pass_convex<false>(Geometry, ApplyState*, Bodies, Cells, Work, uint32_t, uint32_t, uint32_t,
                                               SatShape);
 template __global__ void k_pass_convex<true>(Geometry, ApplyState*, Bodies, Cells, Work, uint32_t, uint32_t, uint32_t,

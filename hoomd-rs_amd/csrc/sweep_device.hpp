@@ -893,6 +893,7 @@ __device__ __forceinline__ uint32_t find_replica(const uint32_t* off, uint32_t R
 
 constexpr uint32_t kCvTrials = 4;  // convex pass: trials per wavefront
 constexpr uint32_t kCvLanes = 64 / kCvTrials;
+constexpr uint32_t kCvApply = 64;  // threads of a region of the persistent convex apply
 
 constexpr int kEnergyBlock = 256;
 constexpr int kEnergyFinal = 256;

@@ -101,9 +101,9 @@ enum {
   HMC_FLAG_NO_GRAPH = 2,    /* hmc_run_translate launches every apply directly
                                instead of replaying a captured hipGraph
                                (same results) */
-  HMC_FLAG_PER_COLOUR = 4,  /* MIXED hard shapes: one launch per colour pass
-                               instead of the default single persistent launch
-                               per apply (same results) */
+  HMC_FLAG_PER_COLOUR = 4,  /* hard shapes, convex polyhedra and MIXED LJ: one
+                               launch per colour pass instead of the default
+                               single persistent launch per apply (same results) */
   HMC_FLAG_FP32_ERROR = 8   /* MIXED: also measure in FP64 and record the
                                largest FP32 error and its ratio to the error
                                bound (hmc_stats; same decisions, slower).
@@ -136,7 +136,9 @@ typedef struct {
                                persistent launch per apply, each workgroup
                                keeping its region and halo in LDS (mixed
                                precision; in FP64 reported as 1 with
-                               regions > 0); 0: no LDS */
+                               regions > 0); 0: no staged sites (regions > 0:
+                               a persistent launch with its sites in global
+                               memory, convex polyhedra) */
   uint32_t tile_shape[3];   /* colour spaces per workgroup along each axis */
   uint64_t ambiguous;       /* LJ: Metropolis decisions that the bound on the
                                summation-order difference could not settle

@@ -17,10 +17,20 @@ hipEvent_t take_event(hmc_ctx* c) {
 }
 
 // The persistent apply's kernel for a context.
+static const void* iso_apply_kernel(uint32_t lanes, int dim) {
+  if (dim == 2)
+    return lanes == 64   ? (const void*)k_apply_iso<2, 64>
+           : lanes == 16 ? (const void*)k_apply_iso<2, 16>
+                         : (const void*)k_apply_iso<2, 8>;
+  return lanes == 64   ? (const void*)k_apply_iso<3, 64>
+         : lanes == 16 ? (const void*)k_apply_iso<3, 16>
+                       : (const void*)k_apply_iso<3, 8>;
+}
 static const void* persist_kernel(const hmc_ctx* c) {
   const bool d2 = c->g.dim == 2;
   if (c->g.model == HMC_CONVEX_POLYHEDRON)
     return c->g.cv_mixed ? (const void*)k_apply_convex<true> : (const void*)k_apply_convex<false>;
+  if (c->iso_lanes) return iso_apply_kernel(c->iso_lanes, c->g.dim);
   if (is_isotropic(c->g.model)) return d2 ? (const void*)k_apply_lj<2> : (const void*)k_apply_lj<3>;
   if (c->cfg.precision == HMC_MIXED)
     return d2 ? (const void*)k_apply_tile<2, float> : (const void*)k_apply_tile<3, float>;
@@ -54,7 +64,7 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
   if (N) {
     k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
     // (these applies stage their sites from the FP64 copies)
-    if ((c->persist && g.model != HMC_CONVEX_POLYHEDRON) || c->small_wpt)
+    if ((c->persist && g.model != HMC_CONVEX_POLYHEDRON && !c->iso_lanes) || c->small_wpt)
       k_place<PREC, false><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
     else
       k_place<PREC><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
@@ -116,6 +126,7 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
   const uint32_t launched = c->cycles_guess + (lj ? 1u : 0u);
   const uint32_t lj_blocks = grid_for(g.per_colour, kBlock / 64);
   const uint32_t lj_chunk = (lj_blocks + 7) / 8;
+  const uint32_t iso_chunk = (grid_for(g.per_colour, kBlock / 8) + 7) / 8;
   const uint32_t cv_chunk = (grid_for(g.per_colour, (kBlock / 64) * kCvTrials) + 7) / 8;
   for (uint32_t k = 0; k < launched; ++k) {
     for (int col = 0; col < (1 << D); ++col) {
@@ -129,9 +140,12 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
         if (g.lj_mixed)
           k_pass_lj<D, HMC_MIXED><<<lj_chunk * 8, kBlock, 0, s>>>(g, c->st, c->bodies, c->cells, c->w, (uint32_t)col,
                                                                   k, lj_chunk);
+        else if (c->iso_lanes == 64)
+          k_pass_iso<D, 64><<<lj_chunk * 8, kBlock, 0, s>>>(g, c->st, c->bodies, c->cells, c->w, (uint32_t)col, k,
+                                                            lj_chunk);
         else
-          k_pass_lj<D, HMC_FP64><<<lj_chunk * 8, kBlock, 0, s>>>(g, c->st, c->bodies, c->cells, c->w, (uint32_t)col,
-                                                                 k, lj_chunk);
+          k_pass_iso<D, 8><<<iso_chunk * 8, kBlock, 0, s>>>(g, c->st, c->bodies, c->cells, c->w, (uint32_t)col, k,
+                                                            iso_chunk);
       }
       else if (convex && g.cv_mixed)
         k_pass_convex<true><<<cv_chunk * 8, kBlock, 0, s>>>(g, c->st, c->bodies, c->cells, c->w, (uint32_t)col, k,
@@ -511,22 +525,22 @@ bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* o
 // step at packing fractions 0.3, 0.4 and 0.5, with one launch per colour 1519,
 // 2021 and 1528; with one round (125,000 cubes) 941, 1115 and 1140 against 1219,
 // 1469 and 1522 with one launch per colour.
-static bool choose_regions_convex(const Geometry& g, uint32_t resident, TileCfg* out) {
+static bool choose_regions_wave(const Geometry& g, uint32_t trials, uint32_t resident, TileCfg* out) {
   bool found = false;
   uint32_t best_face = 0;
-  for (uint32_t t0 = 1; t0 <= std::min<uint32_t>(g.half_shape[0], kCvTrials); ++t0)
-    for (uint32_t t1 = 1; t1 <= std::min<uint32_t>(g.half_shape[1], kCvTrials); ++t1)
-      for (uint32_t t2 = 1; t2 <= std::min<uint32_t>(g.half_shape[2], kCvTrials); ++t2) {
+  for (uint32_t t0 = 1; t0 <= std::min<uint32_t>(g.half_shape[0], trials); ++t0)
+    for (uint32_t t1 = 1; t1 <= std::min<uint32_t>(g.half_shape[1], trials); ++t1)
+      for (uint32_t t2 = 1; t2 <= (g.dim == 3 ? std::min<uint32_t>(g.half_shape[2], trials) : 1u); ++t2) {
         const uint32_t T[3] = {t0, t1, t2}, face = t0 * t1 + t1 * t2 + t2 * t0;
         uint64_t n = 1;
-        for (int a = 0; a < 3; ++a) n *= (g.half_shape[a] + T[a] - 1) / T[a];
-        if (t0 * t1 * t2 > kCvTrials || (n + 7) / 8 * 8 > resident) continue;
+        for (int a = 0; a < g.dim; ++a) n *= (g.half_shape[a] + T[a] - 1) / T[a];
+        if (t0 * t1 * t2 > trials || (n + 7) / 8 * 8 > resident) continue;
         if (found && (n > out->ntiles || (n == out->ntiles && face >= best_face))) continue;
         found = true;
         best_face = face;
         for (int a = 0; a < 3; ++a) {
           out->T[a] = T[a];
-          out->nt[a] = (g.half_shape[a] + T[a] - 1) / T[a];
+          out->nt[a] = a < g.dim ? (g.half_shape[a] + T[a] - 1) / T[a] : 1;
         }
         out->trials = t0 * t1 * t2;
         out->ntiles = (uint32_t)n;
@@ -1007,7 +1021,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, persist_kernel(c), kCvApply, 0) == hipSuccess &&
-        choose_regions_convex(g, (uint32_t)per_cu * (uint32_t)cus, &pc)) {
+        choose_regions_wave(g, kCvTrials, (uint32_t)per_cu * (uint32_t)cus, &pc)) {
       c->persist = true;
       c->pc = pc;
       c->pgrid = pc.xcd_chunk * 8u;
@@ -1021,19 +1035,64 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     }
   }
   // A small system with isotropic pair energies in FP64: whole applies by one
-  // workgroup, where the system fits its LDS (about 1,400 bodies).  The
-  // per-colour passes cost a launch (15 us) per pass whatever the size.
-  // Measured us per step, they and this: 108 LJ bodies at density 0.8 1230 and
-  // 284, 864 1790 and 649, 1,372 3211 and 1242; 1,372 at 0.1 (64 trials a pass
-  // of two candidates) 351 and 342; 864 overlap-penalty bodies (125 trials a
-  // pass) 231 and 224, where the line is.
-  if (lj && !lj_mixed && g.n_bodies && g.n_bodies < 5000 && g.per_colour <= 128 && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS))) {
+  // workgroup, where the system fits its LDS (about 1,400 bodies) and a colour
+  // has at most 32 spaces.  Measured us per step, this and a persistent launch of
+  // a wavefront per trial (k_apply_iso): 108 LJ bodies at density 0.8 292 and
+  // 727, 864 648 and 1133, 1,372 1251 and 1900; 400 LJ disks (16 trials a pass) 131
+  // and 199, 256 overlap-penalty bodies (27 trials) 118 and 155; beyond the line
+  // 900 LJ disks (49 trials) 203 and 153, 500 overlap-penalty bodies (64) 194 and
+  // 153.
+  if (lj && !lj_mixed && g.n_bodies && g.n_bodies < 5000 && g.per_colour <= 32 && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS))) {
     const SmallLds l = SmallLds::of(g);
     const void* fn = D == 2 ? (const void*)k_apply_small<2> : (const void*)k_apply_small<3>;
     hipFuncAttributes at{};
     if (hipFuncGetAttributes(&at, fn) == hipSuccess && at.sharedSizeBytes + l.total <= 160 * 1024 &&
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.total) == hipSuccess)
       c->small_wpt = g.per_colour <= 4 ? 4u : (g.per_colour <= 8 ? 2u : 1u);
+  }
+  // Other isotropic pair energies in FP64: lanes per trial, and one persistent
+  // launch per apply (k_apply_iso) where the neighbour scan reaches one space out
+  // and a wavefront per 64 / lanes spaces of a colour is resident.  With more
+  // than 64 candidates per trial 64 lanes share them (442,368 LJ bodies at
+  // density 0.8: 2261 us per step; with 16 lanes 3053, with 8 5553).  With fewer,
+  // 64 lanes while that is at most four wavefronts per compute unit, 16 while
+  // the regions are resident, else 8: overlap penalty, us per step with 64, 16 and
+  // 8 lanes, 6,912 bodies 171, 187, 214; 16,384 206, 195, 221; 55,296 418 (not
+  // resident), 229, 234; 131,072 765, 302 (neither resident), 290.
+  if (lj && !lj_mixed && !c->small_wpt && g.n_bodies) {
+    double cand = (double)g.n_bodies / (double)g.n_spaces;
+    bool one = true;
+    for (int a = 0; a < D; ++a) {
+      cand *= 3.0;
+      one = one && g.reach[a] == 1;
+    }
+    const bool many = cand > 64.0;
+    int cus = 0, coop = 0;
+    if (one && !(cfg_in->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS)) &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop) {
+      for (uint32_t lanes : {64u, 16u, 8u}) {
+        int per_cu = 0;
+        TileCfg pc{};
+        if (c->persist || (many && lanes != 64) ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, iso_apply_kernel(lanes, D), 64, 0) != hipSuccess)
+          continue;
+        const uint32_t resident = (uint32_t)(lanes == 64 && !many ? std::min(per_cu, 4) : per_cu) * (uint32_t)cus;
+        if (!choose_regions_wave(g, 64u / lanes, resident, &pc)) continue;
+        c->persist = true;
+        c->iso_lanes = lanes;
+        c->pc = pc;
+        c->pgrid = pc.xcd_chunk * 8u;
+        c->pthreads = 64;
+        c->pper_cu = (uint32_t)per_cu;
+        const size_t fbytes = (size_t)pc.ntiles * kMailboxStride * sizeof(uint32_t);
+        if (hipMalloc((void**)&c->w.mbox, fbytes) != hipSuccess || hipMemset(c->w.mbox, 0, fbytes) != hipSuccess) {
+          delete c;
+          return HMC_ERR_DEVICE;
+        }
+      }
+    }
+    if (!c->persist) c->iso_lanes = many ? 64u : 8u;
   }
   const uint32_t N = g.n_bodies;
   c->n_scan_blocks = grid_for(g.n_spaces, kScanBlock);
@@ -1084,6 +1143,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     return HMC_ERR_DEVICE;
   }
   if (c->persist && !persist_probe(c)) c->persist = false;  // the per-colour passes instead
+  if (c->iso_lanes == 16 && !c->persist) c->iso_lanes = 8;  // (passes have no 16)
   *out = c;
   return HMC_OK;
 }
@@ -1579,7 +1639,7 @@ int hmc_get_stats(hmc_ctx* c, hmc_stats* out) {
   std::memcpy(&out->fp32_error_max, &s.fp32_err_max, sizeof(double));
   std::memcpy(&out->fp32_error_bound, &s.fp32_err_ratio, sizeof(double));
   // (an FP64 hard-shape apply reports LDS tiles in either layout; regions tells)
-  out->tiled = c->persist && (is_isotropic(c->g.model) || c->cfg.precision == HMC_MIXED) ? 2u : (c->tiled ? 1u : 0u);
+  out->tiled = c->persist && !c->iso_lanes && (is_isotropic(c->g.model) || c->cfg.precision == HMC_MIXED) ? 2u : (c->tiled ? 1u : 0u);
   for (int a = 0; a < 3; ++a) out->tile_shape[a] = c->persist ? c->pc.T[a] : (c->tiled ? c->tc.T[a] : 0u);
   out->regions = c->persist ? c->pc.ntiles : 0u;
   out->region_threads = c->persist ? c->pthreads : 0u;

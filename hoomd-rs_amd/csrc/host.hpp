@@ -29,6 +29,7 @@ struct hmc_ctx {
   uint32_t small_wpt = 0;  // a small isotropic system: k_apply_small with this many wavefronts per trial (0: not)
   uint32_t pgrid = 0, pthreads = 0, pper_cu = 0;
   double* verts = nullptr;  // convex polyhedron vertices (device)
+  uint32_t iso_lanes = 0;   // isotropic FP64 beyond small_wpt: lanes per trial (k_pass_iso, k_apply_iso)
   SatShape sat{};           // convex, mixed precision: the FP32 separating axes (else use = 0)
   Geometry* gdev = nullptr;  // device copy of g (g.self)
   uint32_t n_scan_blocks = 0;

@@ -277,13 +277,10 @@ __device__ __forceinline__ uint32_t sat_dispatch(const SatShape& S, bool act, co
 // per-wavefront list, and XenoCollide runs over that list 64 pairs at a time.
 // Any overlap rejects a hard-shape trial, so the order of the pair tests does
 // not change a decision (parallel_sweep.rs:267-273).
-constexpr uint32_t kCvRows = 25;    // rows of neighbour spaces of one trial: at most 5^2
 constexpr uint32_t kCvBatch = 6;    // rounds of 64 candidates with their loads in flight together
 constexpr uint32_t kCvPairs = 512;  // listed pairs; tested once more than kCvPairs - 64 kCvBatch are pending
 struct CvWave {
-  // per trial and row: its candidates are `la` slots from ra, then the slots from
-  // rb; x = ra, y = la, z = rb - la, w = the index of its first candidate
-  uint4 row[kCvTrials][kCvRows];
+  uint4 row[kCvTrials][NeighbourRows<3, kCvLanes>::kRows];
   uint32_t qs[kCvPairs];             // the listed pair's neighbour slot
   uint32_t tk[kCvPairs];             // and trial
   double t[kCvTrials][3];            // trial site position
@@ -405,52 +402,8 @@ __device__ __forceinline__ void cv_trials(const Geometry& g, ApplyState* st, con
   bool tried = false;
   uint32_t slot = 0xFFFFFFFFu, body = 0;
   Sfc64 rng = {0, 0, 0, 0};
-  // The rows of neighbour spaces along the last axis (each space once, as the
-  // reference's cell list visits them), a lane per row: the first slots of the
-  // row's lower, own and upper space (lo, mid, hi; the next space's where that is
-  // contiguous), loaded before the proposal is drawn.  Where the scan reaches
-  // two spaces or an axis has two, the row is one run (lo .. hi) or two.
-  uint32_t nn[3], first[3];
-  bool plain = true;  // three distinct spaces along every axis
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const uint32_t sh = (uint32_t)g.shape[a], r = (uint32_t)g.reach[a], x = (uint32_t)m[a];
-    const bool all = 2u * r + 1u >= sh;
-    nn[a] = all ? sh : 2u * r + 1u;
-    first[a] = all ? 0u : (x >= r ? x - r : x + sh - r);
-    plain = plain && r == 1u && sh >= 3u;
-  }
-  if (plain) {  // (of three spaces, too, the lower one comes first)
-#pragma unroll
-    for (int a = 0; a < 3; ++a) first[a] = m[a] ? (uint32_t)m[a] - 1u : (uint32_t)g.shape[a] - 1u;
-  }
-  const uint32_t nrow = nn[0] * nn[1], inv1 = (256u + nn[1] - 1u) / nn[1];
-  uint32_t st0[2] = {0, 0}, st1[2] = {0, 0}, st2[2] = {0, 0}, st3[2] = {0, 0}, st4[2] = {0, 0}, st5[2] = {0, 0};
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint32_t j = kl + (uint32_t)h * kCvLanes;
-    if (!have || j >= nrow) continue;
-    const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn[1];
-    uint32_t y0 = first[0] + i0, y1 = first[1] + i1;
-    y0 = y0 >= (uint32_t)g.shape[0] ? y0 - (uint32_t)g.shape[0] : y0;
-    y1 = y1 >= (uint32_t)g.shape[1] ? y1 - (uint32_t)g.shape[1] : y1;
-    const uint32_t sb = y0 * g.stride[0] + y1 * g.stride[1], sh = (uint32_t)g.shape[2];
-    if (plain) {
-      const uint32_t mid = sb + (uint32_t)m[2], hi = sb + ((uint32_t)m[2] + 1u == sh ? 0u : (uint32_t)m[2] + 1u);
-      st0[h] = w.start[sb + first[2]];
-      st1[h] = w.start[sb + first[2] + 1u];
-      st2[h] = w.start[mid];
-      st3[h] = w.start[mid + 1u];
-      st4[h] = w.start[hi];
-      st5[h] = w.start[hi + 1u];
-    } else {
-      const uint32_t end = first[2] + nn[2];
-      st2[h] = w.start[sb + first[2]];
-      st3[h] = w.start[sb + min(end, sh)];
-      st4[h] = w.start[sb];
-      st5[h] = end > sh ? w.start[sb + end - sh] : st4[h];
-    }
-  }
+  NeighbourRows<3, kCvLanes> nbr;
+  nbr.issue(g, w.start, m, have, kl);
   if (have) {
     const uint32_t s0 = w.start[s];
     const uint32_t n = w.start[s + 1] - s0;
@@ -507,49 +460,10 @@ __device__ __forceinline__ void cv_trials(const Geometry& g, ApplyState* st, con
     W.ns[k][2] = ts.n[2];
     W.flags[k] = ts.flags;
   }
-  // Rows and row ends whose nearest point is the circumsphere cutoff away hold no
-  // pair (27 spaces become 20 on average): cut by the distance from the trial
-  // site to the faces of its space, with a margin of 10^-4 for the roundings.
-  // (A trial outside its space is rejected without pair tests.)
-  const float cut = (float)g.cv_rcut2 * (1.0f + 1e-4f);
+  // (a trial outside its space is rejected without pair tests)
   float flo[3], fhi[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    double u = ts.t[a] - origin[a];
-    u = u >= gp->L[a] ? u - gp->L[a] : u;
-    u -= (double)own[a] * gp->width[a];
-    const float wd = (float)gp->width[a], uf = (float)u, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
-    flo[a] = dl * dl;
-    fhi[a] = dh * dh;
-  }
-  uint32_t tot = 0;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint32_t j = kl + (uint32_t)h * kCvLanes;
-    const bool mine = active && j < nrow;
-    uint32_t ra = st2[h], ea = st3[h], rb = st4[h], eb = plain ? st4[h] : st5[h];
-    if (plain) {
-      const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn[1];
-      const float d = (i0 == 0 ? flo[0] : i0 == 2 ? fhi[0] : 0.0f) + (i1 == 0 ? flo[1] : i1 == 2 ? fhi[1] : 0.0f);
-      const bool lo = d + flo[2] < cut, hi = d + fhi[2] < cut;
-      const bool wlo = m[2] == 0, whi = m[2] + 1 == g.shape[2];  // the lower / upper space lies across the face
-      ra = lo && !wlo ? st0[h] : ra;
-      ea = hi && !whi ? st5[h] : ea;
-      rb = wlo ? st0[h] : st4[h];
-      eb = wlo ? (lo ? st1[h] : rb) : (whi && hi ? st5[h] : rb);
-      if (!(d < cut)) ea = ra, eb = rb;
-    }
-    const uint32_t la = ea - ra, cnt = mine ? la + (eb - rb) : 0u;
-    uint32_t incl = cnt;
-#pragma unroll
-    for (uint32_t dd = 1; dd < kCvLanes; dd <<= 1) {
-      const uint32_t u = __shfl_up(incl, dd, kCvLanes);
-      if (kl >= dd) incl += u;
-    }
-    if (mine) W.row[k][j] = make_uint4(ra, la, rb - la, tot + incl - cnt);
-    tot += __shfl(incl, (int)(lane | (kCvLanes - 1)), 64);
-    if (h == 0 && !__any(nrow > kCvLanes)) break;
-  }
+  face_gaps2<3>(gp, origin, own, ts.t, flo, fhi);
+  const uint32_t tot = nbr.list(g, m, kl, active, (float)g.cv_rcut2 * (1.0f + 1e-4f), flo, fhi, W.row[k]);
   uint32_t base[kCvTrials + 1];
   base[0] = 0;
 #pragma unroll
@@ -577,17 +491,7 @@ __device__ __forceinline__ void cv_trials(const Geometry& g, ApplyState* st, con
       ok[r] = c < total && !((hits >> kc) & 1u);
       uint32_t qs = 0;
       if (ok[r]) {
-        // row of candidate c: the last one whose first index is <= c (nrow is
-        // the same for every trial)
-        const uint32_t cl = c - bk;
-        uint32_t jlo = 0;
-        for (uint32_t sw = nrow > 16u ? 16u : 8u; sw >= 1; sw >>= 1) {
-          const uint32_t mid = jlo + sw;
-          if (mid < nrow && W.row[kc][mid].w <= cl) jlo = mid;
-        }
-        const uint4 q4 = W.row[kc][jlo];
-        const uint32_t e = cl - q4.w;
-        qs = (e < q4.y ? q4.x : q4.z) + e;
+        qs = nbr.slot_of(W.row[kc], c - bk);  // (the rows' number is the same for every trial)
         ok[r] = qs != slk;
       }
       qsv[r] = qs;
@@ -727,33 +631,15 @@ __global__ void __launch_bounds__(kCvApply, 3) k_apply_convex(Geometry g, ApplyS
   if (threadIdx.x == 0) blk_acc = 0;
   stage_zig(zx, zf);
   stage_verts(g, vx);
-  Region rg{};
-  {
-    uint32_t r = tile;
-    for (int a = 2; a >= 0; --a) {
-      rg.tcd[a] = r % tc.nt[a];
-      r /= tc.nt[a];
-      rg.org[a] = (int32_t)(2 * rg.tcd[a] * tc.T[a]);
-      rg.rl[a] = min((int32_t)(2 * tc.T[a]), g.shape[a] - rg.org[a]);
-    }
-  }
+  const Region rg = wave_region<3>(g, tc, tile);
   const uint32_t cycles = st->cycles, substep0 = st->substep0;
   __syncthreads();
   for (uint32_t i = 0; i < 8 * cycles; ++i) {
     const uint32_t colour = i & 7u;
     if (i) region_publish(w.mbox, tile, tc.tag, i);
-    uint32_t t = __lane_id() / kCvLanes;
-    bool have = t < tc.trials;
-    int32_t m[3] = {0, 0, 0};
-    uint32_t s = 0;
-    for (int a = 2; a >= 0; --a) {
-      const int32_t l = (int32_t)(2 * (t % tc.T[a]) + ((colour >> (2 - a)) & 1u));
-      t /= tc.T[a];
-      have = have && l < rg.rl[a];
-      m[a] = rg.org[a] + l;
-      s += (uint32_t)m[a] * g.stride[a];
-    }
-    if (!have) s = 0;
+    int32_t m[3];
+    uint32_t s;
+    const bool have = wave_region_space<3>(g, tc, rg, colour, __lane_id() / kCvLanes, &s, m);
     cv_trials<MIXED, true>(g, st, B, C, w, cw, vx, zx, zf, sat, have, s, m, colour, substep0 + (i >> 3), &blk_acc, [&] {
       if (i) region_wait<3>(st, w.mbox, tc, rg, tile, i);
     });

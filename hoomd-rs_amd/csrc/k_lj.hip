@@ -1,5 +1,5 @@
-// Isotropic pair energies (LJ, shifted LJ, the overlap penalty): one
-// wavefront per trial with a Metropolis decision on dH.
+// Isotropic pair energies: one wavefront per trial with a Metropolis decision on
+// dH (the mixed mode's passes, and the guard of every mode).
 #include "sweep_device.hpp"
 
 namespace hmc {
@@ -312,9 +312,7 @@ __global__ void __launch_bounds__(kGuardThreads) k_guard_lj(Geometry g, ApplySta
 
 // explicit instantiations (launched from the host translation units)
 template __global__ void k_pass_lj<2, HMC_MIXED>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
-template __global__ void k_pass_lj<2, HMC_FP64>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
 template __global__ void k_pass_lj<3, HMC_MIXED>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
-template __global__ void k_pass_lj<3, HMC_FP64>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
 template __global__ void k_guard_lj<2>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t first_cycle);
 template __global__ void k_guard_lj<3>(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t first_cycle);
 

@@ -32,6 +32,10 @@ template <int D, int PREC>
 __global__ void k_guard(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t first_cycle);
 template <int D, int PREC>
 __global__ void k_pass_lj(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
+template <int D, int G>
+__global__ void k_pass_iso(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t colour, uint32_t cycle, uint32_t xcd_chunk);
+template <int D, int G>
+__global__ void k_apply_iso(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, TileCfg tc);
 template <int D>
 __global__ void k_guard_lj(Geometry g, ApplyState* st, Bodies B, Cells C, Work w, uint32_t first_cycle);
 template <bool MIXED>

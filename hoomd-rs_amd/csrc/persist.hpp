@@ -192,6 +192,136 @@ __device__ __forceinline__ TrialSite<D> trial_site(GeoPtr g, const ApplyState* s
   if (!(least >= 0x1p-900)) o = trial_site_general<D>((const Geometry*)(uintptr_t)g, st, x0[0], x0[1], D == 3 ? x0[2] : 0.0, s);
   return o;
 }
+// Squared distances from a site in space `own` to the space's lower and upper
+// faces (0 where it lies beyond one by rounding).
+template <int D>
+__device__ __forceinline__ void face_gaps2(GeoPtr g, const double* origin, const uint32_t* own, const double* x,
+                                           float* lo, float* hi) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    double u = x[a] - origin[a];
+    u = u >= g->L[a] ? u - g->L[a] : u;
+    u -= (double)own[a] * g->width[a];
+    const float wd = (float)g->width[a], uf = (float)u, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
+    lo[a] = dl * dl;
+    hi[a] = dh * dh;
+  }
+}
+
+// The neighbour spaces of a trial (each once, as the reference's cell list
+// visits them) as rows along the last axis, listed by a group of G lanes, a lane
+// per row.  issue() loads each row's slots, before the proposal is drawn; list()
+// writes its runs to LDS and returns the number of candidates.
+//
+// With three or more spaces along every axis and a scan of one space (`plain`), a row
+// is a lower, an own and an upper space, and rows and row ends whose nearest
+// point is the cutoff away are left out: 27 spaces become 20 on average.
+// (face_gaps2 to the faces; cut2 holds a margin for its roundings.)  Otherwise a
+// row is one run of slots, or two across the periodic face.
+template <int D, int G>
+struct NeighbourRows {
+  static constexpr uint32_t kRows = D == 3 ? 25 : 5, H = (kRows + G - 1) / G;  // at most 5^(D - 1) rows
+  uint32_t nrow, nn1, inv1;
+  bool plain;
+  uint32_t e[H][6];  // plain: first and last slots of the lower, own and upper space; else of the two runs
+  __device__ __forceinline__ void issue(const Geometry& g, const uint32_t* start, const int32_t* m, bool have,
+                                        uint32_t kl) {
+    constexpr int AL = D - 1;
+    uint32_t nn[3] = {1, 1, 1}, first[3] = {0, 0, 0};
+    plain = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) plain = plain && g.reach[a] == 1 && g.shape[a] >= 3;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const uint32_t sh = (uint32_t)g.shape[a], r = (uint32_t)g.reach[a], x = (uint32_t)m[a];
+      const bool all = 2u * r + 1u >= sh && !plain;  // (of three spaces, too, the lower one comes first)
+      nn[a] = min(2u * r + 1u, sh);
+      first[a] = all ? 0u : (x >= r ? x - r : x + sh - r);
+    }
+    nn1 = D == 3 ? nn[1] : 1u;
+    nrow = D == 3 ? nn[0] * nn[1] : nn[0];
+    inv1 = (256u + nn1 - 1u) / nn1;
+    const uint32_t sh = (uint32_t)g.shape[AL], ml = (uint32_t)m[AL];
+#pragma unroll
+    for (uint32_t h = 0; h < H; ++h) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) e[h][q] = 0;
+      const uint32_t j = kl + h * G;
+      if (!have || j >= nrow) continue;
+      const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn1;
+      uint32_t y0 = first[0] + i0;
+      y0 = y0 >= (uint32_t)g.shape[0] ? y0 - (uint32_t)g.shape[0] : y0;
+      uint32_t sb = y0 * g.stride[0];
+      if constexpr (D == 3) {
+        const uint32_t y1 = first[1] + i1;
+        sb += (y1 >= (uint32_t)g.shape[1] ? y1 - (uint32_t)g.shape[1] : y1) * g.stride[1];
+      }
+      if (plain) {
+        const uint32_t lo = sb + first[AL], mid = sb + ml, hi = sb + (ml + 1u == sh ? 0u : ml + 1u);
+        e[h][0] = start[lo];
+        e[h][1] = start[lo + 1u];
+        e[h][2] = start[mid];
+        e[h][3] = start[mid + 1u];
+        e[h][4] = start[hi];
+        e[h][5] = start[hi + 1u];
+      } else {
+        const uint32_t end = first[AL] + nn[AL];
+        e[h][2] = start[sb + first[AL]];
+        e[h][3] = start[sb + min(end, sh)];
+        e[h][4] = start[sb];
+        e[h][5] = end > sh ? start[sb + end - sh] : e[h][4];
+      }
+    }
+  }
+  // rows[j] = {first slot of the first run, its length, second run's first slot
+  // less that length, index of the row's first candidate}
+  __device__ __forceinline__ uint32_t list(const Geometry& g, const int32_t* m, uint32_t kl, bool active, float cut2,
+                                           const float* flo, const float* fhi, uint4* rows) const {
+    constexpr int AL = D - 1;
+    const bool wlo = m[AL] == 0, whi = m[AL] + 1 == g.shape[AL];  // the lower / upper space lies across the face
+    uint32_t tot = 0;
+#pragma unroll
+    for (uint32_t h = 0; h < H; ++h) {
+      if (h && h * G >= nrow) break;  // uniform
+      const uint32_t j = kl + h * G;
+      const bool mine = active && j < nrow;
+      uint32_t ra = e[h][2], ea = e[h][3], rb = e[h][4], eb = e[h][5];
+      if (plain) {
+        const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn1;
+        float d = i0 == 0 ? flo[0] : i0 == 2 ? fhi[0] : 0.0f;
+        if constexpr (D == 3) d += i1 == 0 ? flo[1] : i1 == 2 ? fhi[1] : 0.0f;
+        const bool lo = d + flo[AL] < cut2, hi = d + fhi[AL] < cut2;
+        ra = lo && !wlo ? e[h][0] : ra;
+        ea = hi && !whi ? e[h][5] : ea;
+        rb = wlo ? e[h][0] : e[h][4];
+        eb = wlo ? (lo ? e[h][1] : rb) : (whi && hi ? e[h][5] : rb);
+        if (!(d < cut2)) ea = ra, eb = rb;
+      }
+      const uint32_t la = ea - ra, cnt = mine ? la + (eb - rb) : 0u;
+      uint32_t incl = cnt;
+#pragma unroll
+      for (uint32_t dd = 1; dd < G; dd <<= 1) {
+        const uint32_t u = __shfl_up(incl, dd, G);
+        if (kl >= dd) incl += u;
+      }
+      if (mine) rows[j] = make_uint4(ra, la, rb - la, tot + incl - cnt);
+      tot += __shfl(incl, (int)(__lane_id() | (G - 1)), 64);
+    }
+    return tot;
+  }
+  // slot of candidate c: in the last row whose first candidate is <= c
+  __device__ __forceinline__ uint32_t slot_of(const uint4* rows, uint32_t c) const {
+    uint32_t j = 0;
+    for (uint32_t sw = nrow > 16u ? 16u : 8u; sw >= 1; sw >>= 1) {
+      const uint32_t mid = j + sw;
+      if (mid < nrow && rows[mid].w <= c) j = mid;
+    }
+    const uint4 q = rows[j];
+    const uint32_t i = c - q.w;
+    return (i < q.y ? q.x : q.z) + i;
+  }
+};
+
 // Residency probe (tc.probe): the persistent launch relies on every region
 // being resident at once, which the host checks with the occupancy API; the
 // probe checks it on the device with the kernel's own resources.  Thread 0 of
@@ -226,6 +356,37 @@ struct Region {
   uint32_t p, m0;
   double c64[3];
 };
+
+// Position of a region whose sites are not staged, and its space for trial t of
+// a colour (false: none there).
+template <int D>
+__device__ __forceinline__ Region wave_region(const Geometry& g, const TileCfg& tc, uint32_t tile) {
+  Region rg{};
+  for (int a = D - 1; a >= 0; --a) {
+    rg.tcd[a] = tile % tc.nt[a];
+    tile /= tc.nt[a];
+    rg.org[a] = (int32_t)(2 * rg.tcd[a] * tc.T[a]);
+    rg.rl[a] = min((int32_t)(2 * tc.T[a]), g.shape[a] - rg.org[a]);
+  }
+  return rg;
+}
+template <int D>
+__device__ __forceinline__ bool wave_region_space(const Geometry& g, const TileCfg& tc, const Region& rg,
+                                                  uint32_t colour, uint32_t t, uint32_t* s, int32_t* m) {
+  bool have = t < tc.trials;
+  uint32_t sp = 0;
+  m[0] = m[1] = m[2] = 0;
+#pragma unroll
+  for (int a = D - 1; a >= 0; --a) {
+    const int32_t l = (int32_t)(2 * (t % tc.T[a]) + ((colour >> (D - 1 - a)) & 1u));
+    t /= tc.T[a];
+    have = have && l < rg.rl[a];
+    m[a] = rg.org[a] + l;
+    sp += (uint32_t)m[a] * g.stride[a];
+  }
+  *s = have ? sp : 0u;
+  return have;
+}
 
 template <int D>
 __device__ __forceinline__ Region region_of(const Geometry& g, const TileCfg& tc, const double* origin,

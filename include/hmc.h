@@ -101,8 +101,7 @@ enum {
   HMC_FLAG_NO_GRAPH = 2,    /* hmc_run_translate launches every apply directly
                                instead of replaying a captured hipGraph
                                (same results) */
-  HMC_FLAG_PER_COLOUR = 4,  /* hard shapes, convex polyhedra and MIXED LJ: one
-                               launch per colour pass instead of the default
+  HMC_FLAG_PER_COLOUR = 4,  /* one launch per colour pass instead of the default
                                single persistent launch per apply (same results) */
   HMC_FLAG_FP32_ERROR = 8   /* MIXED: also measure in FP64 and record the
                                largest FP32 error and its ratio to the error
@@ -138,7 +137,7 @@ typedef struct {
                                precision; in FP64 reported as 1 with
                                regions > 0); 0: no staged sites (regions > 0:
                                a persistent launch with its sites in global
-                               memory, convex polyhedra) */
+                               memory: convex polyhedra, FP64 pair energies) */
   uint32_t tile_shape[3];   /* colour spaces per workgroup along each axis */
   uint64_t ambiguous;       /* LJ: Metropolis decisions that the bound on the
                                summation-order difference could not settle

@@ -87,10 +87,10 @@ void batch_step(hmc_batch* b, int from_args, int advance, uint32_t launched) {
 int batch_read(hmc_batch* b, std::vector<ApplyState>& st, std::vector<unsigned long long>& acc) {
   st.resize(b->R);
   acc.resize(b->R);
-  BHIPCHK(b, hipMemcpyAsync(st.data(), b->sts, b->R * sizeof(ApplyState), hipMemcpyDeviceToHost, b->stream));
-  BHIPCHK(b, hipMemcpyAsync(acc.data(), b->w.acc_slots, b->R * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                            b->stream));
-  BHIPCHK(b, hipStreamSynchronize(b->stream));
+  // (whole rows: the width is the stride)
+  constexpr uint32_t words = sizeof(ApplyState) / 8;
+  BHIPCHK(b, b->rb.read(b->sts, nullptr, words, words, b->R, st.data(), nullptr, b->stream));
+  BHIPCHK(b, b->rb.read(b->w.acc_slots, nullptr, 1, 1, b->R, acc.data(), nullptr, b->stream));
   for (uint32_t r = 0; r < b->R; ++r) {
     if (st[r].error & kErrBarrier)
       return bfail(b, HMC_ERR_DEVICE, "a neighbour wait of the persistent apply timed out (replica " +
@@ -510,7 +510,8 @@ int hmc_batch_create(uint32_t n_replicas, const hmc_config* cfgs, hmc_batch** ou
   ok = ok && dalloc(&b->w.cnt, b->s_total) == hipSuccess && dalloc(&b->w.start, b->s_total + 1) == hipSuccess &&
        dalloc(&b->w.elem_space, N) == hipSuccess && dalloc(&b->w.elem_rank, N) == hipSuccess &&
        dalloc(&b->w.tmp_body, N) == hipSuccess && dalloc(&b->w.block_sums, b->n_scan_blocks) == hipSuccess &&
-       dalloc(&b->w.block_ne, b->n_scan_blocks) == hipSuccess && dalloc(&b->w.acc_slots, kAccSlots) == hipSuccess;
+       dalloc(&b->w.block_ne, b->n_scan_blocks) == hipSuccess && dalloc(&b->w.acc_slots, kAccSlots) == hipSuccess &&
+       b->rb.init(std::max<uint64_t>(2 * (uint64_t)N * (uint32_t)b->dim, R * (sizeof(ApplyState) / 8))) == hipSuccess;
   if (ok)
     for (uint32_t r = 0; r < R; ++r) b->hreps[r].g.self = &b->reps[r].g;
   ok = ok && hipMemcpy(b->reps, b->hreps.data(), R * sizeof(BatchRep), hipMemcpyHostToDevice) == hipSuccess &&
@@ -590,21 +591,8 @@ int hmc_batch_set_state(hmc_batch* b, uint32_t replica, const double* body_pos, 
 int hmc_batch_get_state(hmc_batch* b, uint32_t replica, double* body_pos, double* site_pos) {
   if (!b || replica >= b->R) return HMC_ERR_INVALID;
   const uint32_t N = b->hreps[replica].g.n_bodies, off = b->boff[replica];
-  const int D = b->dim;
-  std::vector<double4> hb(N), hs(N);
   BHIPCHK(b, hipSetDevice(b->device));
-  if (N) {
-    BHIPCHK(b, hipMemcpyAsync(hb.data(), b->bodies.bpos + off, N * sizeof(double4), hipMemcpyDeviceToHost, b->stream));
-    BHIPCHK(b, hipMemcpyAsync(hs.data(), b->bodies.spos + off, N * sizeof(double4), hipMemcpyDeviceToHost, b->stream));
-  }
-  BHIPCHK(b, hipStreamSynchronize(b->stream));
-  for (uint32_t i = 0; i < N; ++i) {
-    const double bv[3] = {hb[i].x, hb[i].y, hb[i].z}, sv[3] = {hs[i].x, hs[i].y, hs[i].z};
-    for (int a = 0; a < D; ++a) {
-      if (body_pos) body_pos[(size_t)i * D + a] = bv[a];
-      if (site_pos) site_pos[(size_t)i * D + a] = sv[a];
-    }
-  }
+  BHIPCHK(b, b->rb.read(b->bodies.bpos + off, b->bodies.spos + off, 4, (uint32_t)b->dim, N, body_pos, site_pos, b->stream));
   return HMC_OK;
 }
 

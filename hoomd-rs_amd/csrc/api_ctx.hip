@@ -216,13 +216,7 @@ void collect_events(hmc_ctx* c, std::vector<std::pair<hipEvent_t, hipEvent_t>>& 
 }
 
 int read_state(hmc_ctx* c, ApplyState* out, bool check_errors) {
-  std::vector<unsigned long long> slots(kAccSlots);
-  HIPCHK(c, hipMemcpyAsync(out, c->st, sizeof(ApplyState), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(slots.data(), c->w.acc_slots, kAccSlots * sizeof(unsigned long long),
-                           hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  out->accepted_total = 0;
-  for (unsigned long long v : slots) out->accepted_total += v;
+  HIPCHK(c, c->rb.state(c->st, c->w.acc_slots, out, c->stream));
   if (c->profiling) {
     collect_events(c, c->pass_events, c->pass_ms, c->pass_n);
     collect_events(c, c->build_events, c->build_ms, c->build_n);
@@ -1107,7 +1101,8 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
        dalloc(&c->w.elem_space, N) == hipSuccess && dalloc(&c->w.elem_rank, N) == hipSuccess &&
        dalloc(&c->w.tmp_body, N) == hipSuccess && dalloc(&c->w.block_sums, c->n_scan_blocks) == hipSuccess &&
        dalloc(&c->w.block_ne, c->n_scan_blocks) == hipSuccess && dalloc(&c->st, 1) == hipSuccess &&
-       dalloc(&c->w.acc_slots, kAccSlots) == hipSuccess && dalloc(&c->w.scan_status, c->n_scan_blocks) == hipSuccess;
+       dalloc(&c->w.acc_slots, kAccSlots) == hipSuccess && dalloc(&c->w.scan_status, c->n_scan_blocks) == hipSuccess &&
+       c->rb.init(2 * (uint64_t)N * (convex ? 4u : (uint32_t)D)) == hipSuccess;
   if (ok && convex) {
     // orientations start at the identity; vertices live on the device
     ok = dalloc(&c->bodies.bquat, N) == hipSuccess && dalloc(&c->bodies.squat, N) == hipSuccess &&
@@ -1208,28 +1203,8 @@ int hmc_get_orientations(hmc_ctx* c, double* body_quat, double* site_quat) {
   if (!c) return HMC_ERR_INVALID;
   if (c->g.model != HMC_CONVEX_POLYHEDRON) return fail(c, HMC_ERR_UNSUPPORTED, "bodies have no orientation");
   const uint32_t N = c->g.n_bodies;
-  std::vector<double4> hb(N), hs(N);
   HIPCHK(c, hipSetDevice(c->device));
-  if (N) {
-    HIPCHK(c, hipMemcpyAsync(hb.data(), c->bodies.bquat, N * sizeof(double4), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(hs.data(), c->bodies.squat, N * sizeof(double4), hipMemcpyDeviceToHost, c->stream));
-  }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (uint32_t i = 0; i < N; ++i) {
-    const double4 b = hb[i], q = hs[i];
-    if (body_quat) {
-      body_quat[4 * (size_t)i] = b.x;
-      body_quat[4 * (size_t)i + 1] = b.y;
-      body_quat[4 * (size_t)i + 2] = b.z;
-      body_quat[4 * (size_t)i + 3] = b.w;
-    }
-    if (site_quat) {
-      site_quat[4 * (size_t)i] = q.x;
-      site_quat[4 * (size_t)i + 1] = q.y;
-      site_quat[4 * (size_t)i + 2] = q.z;
-      site_quat[4 * (size_t)i + 3] = q.w;
-    }
-  }
+  HIPCHK(c, c->rb.read(c->bodies.bquat, c->bodies.squat, 4, 4, N, body_quat, site_quat, c->stream));
   return HMC_OK;
 }
 
@@ -1350,22 +1325,8 @@ int hmc_get_state(hmc_ctx* c, double* body_pos, double* site_pos) {
   if (!c) return HMC_ERR_INVALID;
   if (!c->have_state) return fail(c, HMC_ERR_STATE, "no state");
   const uint32_t N = c->g.n_bodies;
-  const int D = c->g.dim;
-  std::vector<double4> hb(N), hs(N);
   HIPCHK(c, hipSetDevice(c->device));
-  if (N) {
-    HIPCHK(c, hipMemcpyAsync(hb.data(), c->bodies.bpos, N * sizeof(double4), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(hs.data(), c->bodies.spos, N * sizeof(double4), hipMemcpyDeviceToHost, c->stream));
-  }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (uint32_t i = 0; i < N; ++i) {
-    double v[3] = {hb[i].x, hb[i].y, hb[i].z};
-    double u[3] = {hs[i].x, hs[i].y, hs[i].z};
-    for (int a = 0; a < D; ++a) {
-      if (body_pos) body_pos[(size_t)i * D + a] = v[a];
-      if (site_pos) site_pos[(size_t)i * D + a] = u[a];
-    }
-  }
+  HIPCHK(c, c->rb.read(c->bodies.bpos, c->bodies.spos, 4, (uint32_t)c->g.dim, N, body_pos, site_pos, c->stream));
   return HMC_OK;
 }
 

@@ -6,6 +6,31 @@
 
 #include "kernels.hpp"
 
+namespace hmc {
+
+// Pinned memory through which a context's state is read (readback.hip): two
+// halves of at most 1 MiB, its owner's for its lifetime.  One read at a time.
+class Readback {
+ public:
+  ~Readback();
+  hipError_t init(uint64_t largest);  // words of the largest read
+  // the apply state and the sum of the accepted moves' counters
+  hipError_t state(const ApplyState* st, const unsigned long long* acc_slots, ApplyState* out, hipStream_t s);
+  // `rows` rows of `width` words (of `stride` in the source) of a and of b; an
+  // output may be null.  Waits for the stream.
+  hipError_t read(const void* a, const void* b, uint32_t stride, uint32_t width, uint64_t rows, void* out_a, void* out_b,
+                  hipStream_t s);
+
+ private:
+  static constexpr uint64_t kChunkWords = 1u << 17;
+  std::mutex use;
+  uint64_t chunk = 0;
+  unsigned long long *host = nullptr, *dev = nullptr;
+  hipEvent_t done[2] = {nullptr, nullptr};
+};
+
+}  // namespace hmc
+
 using namespace hmc;
 
 struct hmc_ctx {
@@ -19,6 +44,7 @@ struct hmc_ctx {
   Cells cells{};
   Work w{};
   ApplyState* st = nullptr;
+  Readback rb;
   bool have_state = false;
   uint32_t cycles_guess = 1;
   bool fast = false;  // every axis: >= 3 spaces and reach 1
@@ -71,6 +97,7 @@ struct hmc_batch {
   Cells cells{};
   Work w{};
   hipStream_t stream = nullptr;
+  Readback rb;
   uint32_t n_scan_blocks = 0;
   uint32_t cycles_guess = 1;
   hipGraph_t graph = nullptr;

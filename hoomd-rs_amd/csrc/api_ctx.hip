@@ -459,9 +459,9 @@ bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* o
     if (g.shape[a] < 6 || g.reach[a] != 1) return false;
     lim[a] = std::min<uint32_t>(std::min<uint32_t>(g.half_shape[a], 8u), (uint32_t)(g.shape[a] - 4) / 2);
   }
-  // ziggurat tables, 12 proposals of 160 bytes, the shared trials' partial
-  // sums (2 x 8 x 11 floats), the halo lists' counts
-  const size_t static_lds = 2 * 257 * sizeof(double) + 12 * 160 + 2 * 8 * 11 * 4 + kHaloLists * 4 + 64;
+  // ziggurat tables, 2 x 12 proposals of 160 bytes, the quads' sums (64 x 48
+  // bytes), the halo lists' counts
+  const size_t static_lds = 2 * 257 * sizeof(double) + 2 * 12 * 160 + 64 * 48 + kHaloLists * 4 + 64;
   const size_t cu_lds = 160 * 1024;
   const uint32_t cu_waves = 8;
   bool found = false;

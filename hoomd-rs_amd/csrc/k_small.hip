@@ -35,25 +35,6 @@ struct SmallProp {
 };
 static_assert(sizeof(SmallProp) == SmallLds::kPropBytes, "proposal size counted in the host's LDS budget");
 
-// A DPP move of an FP64 value's halves (rows outside ROW_MASK read 0).
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROW_MASK, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-// Sum over the wavefront, in every lane, without LDS round trips.
-__device__ __forceinline__ double wave_sum_dpp(double v) {
-  v += dpp_f64<0xb1, 0xf>(v);   // quad_perm [1, 0, 3, 2]
-  v += dpp_f64<0x4e, 0xf>(v);   // quad_perm [2, 3, 0, 1]
-  v += dpp_f64<0x141, 0xf>(v);  // row_half_mirror
-  v += dpp_f64<0x140, 0xf>(v);  // row_mirror
-  v += dpp_f64<0x142, 0xa>(v);  // row_bcast15: rows 1 and 3
-  v += dpp_f64<0x143, 0xc>(v);  // row_bcast31: rows 2 and 3
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
-                          __builtin_amdgcn_readlane(__double2loint(v), 63));
-}
-
 // lj_r2 from a site and its ghost image per axis (the site again where there is
 // none): the smaller displacement by selects.  Nearly every site of a small box
 // has ghosts, and the shared image's sum x + T is formed once per move.

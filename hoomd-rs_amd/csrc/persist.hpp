@@ -61,12 +61,17 @@ namespace hmc {
 // Measured on C2's hard spheres (500 regions, 16 passes): see k_apply_tile.
 // The counters that all 26 neighbours incremented every pass, which this
 // replaces, made every pass last as long as the slowest of 27 regions.
+// wave_publish: by the wavefront that made all of the pass's stores.
+__device__ __forceinline__ void wave_publish(uint32_t* mbox, uint32_t tile, uint32_t tag, uint32_t done) {
+  __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have completed
+  if (__lane_id() == 0)
+    __hip_atomic_store((unsigned long long*)&mbox[tile * kMailboxStride], ((unsigned long long)tag << 32) | done,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void region_publish(uint32_t* mbox, uint32_t tile, uint32_t tag, uint32_t done) {
   __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have completed
   __syncthreads();
-  if (threadIdx.x == 0)
-    __hip_atomic_store((unsigned long long*)&mbox[tile * kMailboxStride], ((unsigned long long)tag << 32) | done,
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x < 64u) wave_publish(mbox, tile, tag, done);
 }
 
 // The staged sites of a box in the region's scalar S: x, y, z and the body
@@ -669,12 +674,13 @@ struct RegionReload {
   double v[CELLS][HELD][3];
 
   __device__ __forceinline__ RegionReload(const Geometry& g_, const TileCfg& tc, const Region& rg_, const Bodies& B_,
-                                          const RegionLds<S>& l_, const uint32_t* hcnt, uint32_t j)
+                                          const RegionLds<S>& l_, const uint32_t* hcnt, uint32_t j,
+                                          uint32_t threads = blockDim.x)
       : g(g_), rg(rg_), B(B_), l(l_) {
     const uint32_t q = j & ((1u << D) - 1u);
-    n = hcnt[q];
+    n = threadIdx.x < threads ? hcnt[q] : 0u;
     list = l.halo + tc.hoff[q];
-    step = blockDim.x / LPC;
+    step = threads / LPC;
     c0 = threadIdx.x / LPC;
   }
   __device__ __forceinline__ void issue() {

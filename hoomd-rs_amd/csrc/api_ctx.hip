@@ -49,25 +49,31 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
     e0 = take_event(c);
     (void)hipEventRecord(e0, s);
   }
-  k_setup<<<1, 64, 0, s>>>(g, c->st, step, substep, seed, kT, max_move, from_args, advance, move, 1);
-  // (the per-space counts are zero: cleared at creation and by k_scan_add)
-  if (N) k_bin<D><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->st, c->bodies, c->w);
-  if (N < (1u << kLookbackBits) && g.n_spaces < (1u << kLookbackBits)) {
-    k_scan_lookback<<<c->n_scan_blocks, 256, 0, s>>>(g, c->st, c->w.cnt, c->w.start, c->w.scan_status, g.n_spaces,
-                                                     c->n_scan_blocks);
+  if (c->persist && c->w.bucket) {
+    const ApplyArgs a = {step, kT, max_move, substep, seed, from_args, advance, move};
+    if (N) k_bin_bucket<D><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->st, c->bodies, c->w, a);
+    k_scan_place<<<c->n_scan_blocks, 256, 0, s>>>(g, c->st, c->w, c->cells.body, a, g.n_spaces, c->n_scan_blocks);
   } else {
-    k_scan_blocks<<<c->n_scan_blocks, 256, 0, s>>>(c->w.cnt, c->w.start, c->w.block_sums, c->w.block_ne,
-                                                   g.n_spaces);
-    k_scan_top<<<1, 1024, 0, s>>>(g, c->st, c->w.block_sums, c->w.block_ne, c->n_scan_blocks, c->w.start, 1);
-    k_scan_add<<<grid_for(g.n_spaces, 256), 256, 0, s>>>(c->w.start, c->w.block_sums, c->w.cnt, g.n_spaces);
-  }
-  if (N) {
-    k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
-    // (these applies stage their sites from the FP64 copies)
-    if ((c->persist && g.model != HMC_CONVEX_POLYHEDRON && !c->iso_lanes) || c->small_wpt)
-      k_place<PREC, false><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
-    else
-      k_place<PREC><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
+    k_setup<<<1, 64, 0, s>>>(g, c->st, step, substep, seed, kT, max_move, from_args, advance, move, 1);
+    // (the per-space counts are zero: cleared at creation and by k_scan_add)
+    if (N) k_bin<D><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->st, c->bodies, c->w);
+    if (N < (1u << kLookbackBits) && g.n_spaces < (1u << kLookbackBits)) {
+      k_scan_lookback<<<c->n_scan_blocks, 256, 0, s>>>(g, c->st, c->w.cnt, c->w.start, c->w.scan_status, g.n_spaces,
+                                                       c->n_scan_blocks);
+    } else {
+      k_scan_blocks<<<c->n_scan_blocks, 256, 0, s>>>(c->w.cnt, c->w.start, c->w.block_sums, c->w.block_ne,
+                                                     g.n_spaces);
+      k_scan_top<<<1, 1024, 0, s>>>(g, c->st, c->w.block_sums, c->w.block_ne, c->n_scan_blocks, c->w.start, 1);
+      k_scan_add<<<grid_for(g.n_spaces, 256), 256, 0, s>>>(c->w.start, c->w.block_sums, c->w.cnt, g.n_spaces);
+    }
+    if (N) {
+      k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
+      // (these applies stage their sites from the FP64 copies)
+      if ((c->persist && g.model != HMC_CONVEX_POLYHEDRON && !c->iso_lanes) || c->small_wpt)
+        k_place<PREC, false><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
+      else
+        k_place<PREC><<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->bodies, c->cells, c->w);
+    }
   }
   if (prof) {
     e1 = take_event(c);
@@ -1103,6 +1109,9 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
        dalloc(&c->w.block_ne, c->n_scan_blocks) == hipSuccess && dalloc(&c->st, 1) == hipSuccess &&
        dalloc(&c->w.acc_slots, kAccSlots) == hipSuccess && dalloc(&c->w.scan_status, c->n_scan_blocks) == hipSuccess &&
        c->rb.init(2 * (uint64_t)N * (convex ? 4u : (uint32_t)D)) == hipSuccess;
+  // persistent hard shapes: the two-kernel build
+  if (ok && c->persist && !lj && !convex && N < (1u << kLookbackBits) && g.n_spaces < (1u << kLookbackBits))
+    ok = dalloc(&c->w.bucket, (size_t)g.n_spaces * kBucket) == hipSuccess;
   if (ok && convex) {
     // orientations start at the identity; vertices live on the device
     ok = dalloc(&c->bodies.bquat, N) == hipSuccess && dalloc(&c->bodies.squat, N) == hipSuccess &&
@@ -1693,7 +1702,7 @@ void hmc_destroy(hmc_ctx* c) {
                   (void*)c->cells.body, (void*)c->cells.pos32, (void*)c->cells.quat64, (void*)c->verts,
                   (void*)c->gdev,
                   (void*)c->cells.pos64, (void*)c->w.cnt, (void*)c->w.start, (void*)c->w.elem_space,
-                  (void*)c->w.elem_rank, (void*)c->w.tmp_body, (void*)c->w.block_sums, (void*)c->w.block_ne,
+                  (void*)c->w.elem_rank, (void*)c->w.bucket, (void*)c->w.tmp_body, (void*)c->w.block_sums, (void*)c->w.block_ne,
                   (void*)c->w.acc_slots, (void*)c->w.trace, (void*)c->w.mbox, (void*)c->w.scan_status,
                   (void*)c->st})
     if (p) (void)hipFree(p);

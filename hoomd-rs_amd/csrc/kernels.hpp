@@ -12,6 +12,9 @@ __global__ void k_bin(Geometry g, ApplyState* st, Bodies B, Work w);
 __global__ void k_scan_blocks(const uint32_t* cnt, uint32_t* start, uint32_t* block_sums, uint32_t* block_ne, uint32_t n);
 __global__ void k_scan_top(Geometry g, ApplyState* st, uint32_t* block_sums, const uint32_t* block_ne, uint32_t nblocks, uint32_t* start, int count);
 __global__ void k_scan_lookback(Geometry g, ApplyState* st, uint32_t* cnt, uint32_t* start, unsigned long long* status, uint32_t n, uint32_t nblocks);
+template <int D>
+__global__ void k_bin_bucket(Geometry g, ApplyState* st, Bodies B, Work w, ApplyArgs a);
+__global__ void k_scan_place(Geometry g, ApplyState* st, Work w, uint32_t* body, ApplyArgs a, uint32_t n, uint32_t nblocks);
 __global__ void k_scan_add(uint32_t* start, const uint32_t* block_sums, uint32_t* cnt, uint32_t n);
 __global__ void k_scatter(Geometry g, Work w);
 template <int PREC, bool COPY = true>

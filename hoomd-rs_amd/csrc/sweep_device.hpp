@@ -143,6 +143,15 @@ struct ApplyState {
   uint32_t pad2;
 };
 
+// What an apply is asked for (k_setup's arguments).
+struct ApplyArgs {
+  uint64_t step;
+  double kT, max_move;
+  uint32_t substep, seed;
+  int from_args, advance;
+  uint32_t move;
+};
+
 struct Bodies {
   double4* bpos;
   double4* spos;
@@ -162,6 +171,7 @@ struct Work {
   uint32_t* start;
   uint32_t* elem_space;
   uint32_t* elem_rank;
+  uint32_t* bucket;  // k_bin_bucket: kBucket words per space (else null)
   uint32_t* tmp_body;
   uint32_t* block_sums;
   uint32_t* block_ne;
@@ -275,6 +285,7 @@ __device__ __forceinline__ void lane_add(unsigned long long* dst, unsigned v) {
   if (v) atomicAdd(dst, (unsigned long long)v);
 }
 
+constexpr uint32_t kBucket = 8;         // bodies of a space kept in its bucket
 constexpr uint32_t kLookbackBits = 27;  // count bits of the look-back scan's status words
 
 // Ball::sample (hoomd-vector/src/distribution.rs:39-70): the displacement of

@@ -561,8 +561,8 @@ class GpuBatch:
         lds_tiles=False runs every pass a lane per space from global memory
         instead of on LDS tiles (same decisions).  persistent=False keeps a
         mixed-precision 3D batch on one launch per colour pass instead of
-        persistent applies (one cooperative launch per group of replicas per
-        step, not graph-captured; same decisions)."""
+        persistent applies (one launch per step, not graph-captured; same
+        decisions)."""
         self.R = len(systems)
         cfgs = (Config * self.R)()
         self.dims = []

@@ -37,15 +37,15 @@ void launch_batch_step(hmc_batch* b, int from_args, int advance, uint32_t launch
   if constexpr (D == 3 && PREC == HMC_MIXED) {
     if (b->persist) {
       // the persistent applies stage their sites from the FP64 copies: one
-      // cooperative launch runs every cycle of every replica, round by round
+      // launch runs every cycle of every replica, round by round
       k_place<PREC, false><<<grid_for(b->n_total, kBlock), kBlock, 0, s>>>(b->gtot, b->bodies, b->cells, b->w);
       uint32_t nrounds = (uint32_t)b->grp_tile0.size(), nwg = b->nwg, chunk = (nwg + 7) / 8, probe = 0,
                tag = ++b->sync_tag;
       void* args[] = {(void*)&b->reps, (void*)&b->dptcs, (void*)&b->dptoff, (void*)&b->dptrep, (void*)&b->sts,
                       (void*)&b->drt0, (void*)&b->drn,   (void*)&nrounds,   (void*)&nwg,       (void*)&chunk,
                       (void*)&probe,   (void*)&tag,      (void*)&b->bodies, (void*)&b->cells, (void*)&b->w};
-      const hipError_t e = hipLaunchCooperativeKernel((const void*)k_bapply_tile<3>, dim3(chunk * 8),
-                                                      dim3(b->pthreads), args, b->plds, s);
+      const hipError_t e =
+          launch_resident(b->device, (const void*)k_bapply_tile<3>, chunk * 8, b->pthreads, args, b->plds, s);
       if (e != hipSuccess && b->launch_err == hipSuccess) b->launch_err = e;
       return;
     }
@@ -379,8 +379,7 @@ bool batch_regions(hmc_batch* b, int cus) {
     void* args[] = {(void*)&b->reps, (void*)&b->dptcs, (void*)&b->dptoff, (void*)&b->dptrep, (void*)&b->sts,
                     (void*)&b->drt0, (void*)&b->drn,   (void*)&nrounds,   (void*)&nwg,       (void*)&chunk,
                     (void*)&probe,   (void*)&tag,      (void*)&b->bodies, (void*)&b->cells, (void*)&b->w};
-    if (hipLaunchCooperativeKernel(fn, dim3(chunk * 8), dim3(best_threads), args, best_lds, b->stream) !=
-            hipSuccess ||
+    if (launch_resident(b->device, fn, chunk * 8, best_threads, args, best_lds, b->stream) != hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)
       return false;
   }
@@ -537,8 +536,7 @@ int hmc_batch_create(uint32_t n_replicas, const hmc_config* cfgs, hmc_batch** ou
       hmc_batch_destroy(b);
       return HMC_ERR_DEVICE;
     }
-    // mixed precision in 3D: persistent applies, one cooperative launch per
-    // group of replicas per step (HMC_FLAG_PER_COLOUR keeps the per-colour
+    // mixed precision in 3D: persistent applies, one launch per step (HMC_FLAG_PER_COLOUR keeps the per-colour
     // tile passes)
     int cus = 0, coop = 0;
     if (b->tiled && b->dim == 3 && b->precision == HMC_MIXED && !(cfgs[0].flags & HMC_FLAG_PER_COLOUR) &&
@@ -612,7 +610,7 @@ int hmc_batch_run_translate(hmc_batch* b, const uint64_t* step0, const uint32_t*
   if (rc) return rc;
   const uint32_t launched = b->cycles_guess;
   for (uint32_t i = 0; i < n_steps; ++i) {
-    // (cooperative launches are not captured: persistent steps launch directly)
+    // (persistent launches carry their own tag: not captured, launched directly)
     if (i == 0 || !use_graph || b->persist) {
       batch_step(b, i == 0 ? 1 : 0, i == 0 ? 0 : 1, launched);
       continue;
@@ -634,7 +632,7 @@ int hmc_batch_run_translate(hmc_batch* b, const uint64_t* step0, const uint32_t*
   if (b->launch_err != hipSuccess) {
     const hipError_t e = b->launch_err;
     b->launch_err = hipSuccess;
-    return bfail(b, HMC_ERR_DEVICE, std::string("cooperative launch: ") + hipGetErrorString(e));
+    return bfail(b, HMC_ERR_DEVICE, std::string("persistent launch: ") + hipGetErrorString(e));
   }
   rc = batch_read(b, st1, a1);
   if (rc) return rc;
@@ -828,7 +826,10 @@ void hmc_batch_destroy(hmc_batch* b) {
                   (void*)b->dptcs, (void*)b->dptoff, (void*)b->dptrep, (void*)b->w.mbox, (void*)b->drt0,
                   (void*)b->drn})
     if (p) (void)hipFree(p);
-  if (b->stream) (void)hipStreamDestroy(b->stream);
+  if (b->stream) {
+    forget_resident(b->device, b->stream);
+    (void)hipStreamDestroy(b->stream);
+  }
   delete b;
 }
 

@@ -92,9 +92,8 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
     c->pc.tag += 1;
     void* args[] = {(void*)&g, (void*)&stp, (void*)&c->bodies, (void*)&c->cells, (void*)&c->w, (void*)&c->pc,
                     (void*)&c->sat};  // (the last for convex polyhedra)
-    const hipError_t le =
-        hipLaunchCooperativeKernel(persist_kernel(c), dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, s);
-    if (le != hipSuccess) return fail(c, HMC_ERR_DEVICE, std::string("cooperative launch: ") + hipGetErrorString(le));
+    const hipError_t le = launch_resident(c->device, persist_kernel(c), c->pgrid, c->pthreads, args, c->pc.lds_bytes, s);
+    if (le != hipSuccess) return fail(c, HMC_ERR_DEVICE, std::string("persistent launch: ") + hipGetErrorString(le));
     if (prof) {
       p1 = take_event(c);
       (void)hipEventRecord(p1, s);
@@ -434,7 +433,7 @@ bool persist_probe(hmc_ctx* c) {
                   (void*)&c->sat};
   const size_t fbytes = (size_t)c->pc.ntiles * kMailboxStride * sizeof(uint32_t);
   uint32_t err = 0;
-  bool ok = hipLaunchCooperativeKernel(persist_kernel(c), dim3(c->pgrid), dim3(c->pthreads), args, c->pc.lds_bytes, c->stream) ==
+  bool ok = launch_resident(c->device, persist_kernel(c), c->pgrid, c->pthreads, args, c->pc.lds_bytes, c->stream) ==
                 hipSuccess &&
             hipMemcpyAsync(&err, &c->st->error, sizeof err, hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
             hipStreamSynchronize(c->stream) == hipSuccess;
@@ -1404,7 +1403,7 @@ int hmc_run(hmc_ctx* c, uint64_t step0, uint32_t seed, double kT, const hmc_move
   const bool tally = n_moves > 1;
   if (tally) k_tally<<<1, kAccSlots, 0, c->stream>>>(c->st, c->w.acc_slots, (uint32_t)kMaxMoves);
   const bool lj = is_isotropic(c->g.model);
-  // (a cooperative launch is not captured: the persistent apply launches directly)
+  // (a persistent launch carries its own tag: not captured, launched directly)
   const bool graphs = !(c->cfg.flags & HMC_FLAG_NO_GRAPH) && !c->persist;
   // one step: apply each move in order (the step's substeps follow on), then
   // Microstate::increment_step before the next step
@@ -1709,7 +1708,10 @@ void hmc_destroy(hmc_ctx* c) {
   collect_events(c, c->pass_events, c->pass_ms, c->pass_n);
   collect_events(c, c->build_events, c->build_ms, c->build_n);
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
-  if (c->stream) (void)hipStreamDestroy(c->stream);
+  if (c->stream) {
+    forget_resident(c->device, c->stream);
+    (void)hipStreamDestroy(c->stream);
+  }
   delete c;
 }
 

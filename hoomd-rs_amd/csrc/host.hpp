@@ -50,7 +50,7 @@ struct hmc_ctx {
   bool fast = false;  // every axis: >= 3 spaces and reach 1
   bool tiled = false;  // LDS-staged pass (requires fast)
   TileCfg tc{};
-  bool persist = false;  // one cooperative launch per apply (k_apply_tile)
+  bool persist = false;  // one persistent launch per apply (k_apply_tile, k_apply_lj, k_apply_convex, k_apply_iso)
   TileCfg pc{};
   uint32_t small_wpt = 0;  // a small isotropic system: k_apply_small with this many wavefronts per trial (0: not)
   uint32_t pgrid = 0, pthreads = 0, pper_cu = 0;
@@ -155,6 +155,11 @@ hipError_t dalloc(T** p, size_t n) {
 
 inline uint32_t grid_for(uint64_t n, uint32_t block) { return (uint32_t)((n + block - 1) / block); }
 
+// A persistent apply's launch (resident.hip), and what precedes the end of a stream
+// that such launches used, its work complete.
+hipError_t launch_resident(int device, const void* fn, uint32_t blocks, uint32_t threads, void** args, size_t lds,
+                           hipStream_t s);
+void forget_resident(int device, hipStream_t s);
 hipEvent_t take_event(hmc_ctx* c);
 int dispatch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t substep, uint32_t seed,
                    double kT, double max_move, uint32_t move);

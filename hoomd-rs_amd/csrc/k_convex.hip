@@ -602,7 +602,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
   if (threadIdx.x == 0 && blk_acc) atomicAdd(&w.acc_slots[b & (kAccSlots - 1)], (unsigned long long)blk_acc);
 }
 
-// Every cycle and colour of an apply in one cooperative launch: wavefront b
+// Every cycle and colour of an apply in one launch: wavefront b
 // owns a region of 2 T spaces per axis with at most kCvTrials of each colour
 // and runs them as a pass of cv_trials.  The sites stay in global memory
 // (stores and loads of device scope), and a region waits only for the

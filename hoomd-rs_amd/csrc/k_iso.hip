@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_pass_iso(Geometry g, ApplyState* 
   if (threadIdx.x == 0 && blk_acc) atomicAdd(&w.acc_slots[b & (kAccSlots - 1)], (unsigned long long)blk_acc);
 }
 
-// Every cycle and colour of an apply in one cooperative launch, a wavefront per
+// Every cycle and colour of an apply in one launch, a wavefront per
 // region with at most 64 / G trials of a colour (as k_apply_convex).  Against one
 // launch per colour: 131,072 LJ bodies 1467 and 1956 us per step, 16,384
 // overlap-penalty bodies with 8 lanes 221 and 236.

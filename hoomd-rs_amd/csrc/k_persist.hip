@@ -1,5 +1,5 @@
 // The persistent apply of hard spheres and disks (mixed precision and FP64): one
-// cooperative launch runs every cycle and colour of an apply.
+// launch runs every cycle and colour of an apply.
 #include "persist.hpp"
 
 namespace hmc {
@@ -427,8 +427,7 @@ __global__ void __launch_bounds__(kTileThreads, 2) k_apply_tile(Geometry g, Appl
   apply_tile_run<D, S, 2>(g, st, B, C, w, tc, tile, &w.acc_slots[b & (kAccSlots - 1)], zx, zf);
 }
 
-// The persistent applies of every replica of a batch in one cooperative
-// launch.  The batch's regions are packed, whole replicas at a time, into
+// The persistent applies of every replica of a batch in one launch.  The batch's regions are packed, whole replicas at a time, into
 // rounds of at most one region per workgroup (round k: regions rt0[k] ..
 // rt0[k] + rn[k] - 1 of the batch; trep: a region's replica, toff: the
 // replicas' first regions).  Workgroup b runs its region of round 0 through

@@ -1,5 +1,5 @@
 // The persistent apply for isotropic pair energies (LJ and shifted LJ, mixed
-// precision): one cooperative launch runs every cycle and colour of an apply,
+// precision): one launch runs every cycle and colour of an apply,
 // as k_apply_tile does for hard shapes.  A region's 4 to 12 trials of a pass share
 // out all lanes of the workgroup, whole quads to each; quads' sums are combined in
 // LDS and decided together by wavefront 0, four lanes to a trial, which stores

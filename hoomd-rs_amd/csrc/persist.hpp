@@ -8,7 +8,7 @@
 namespace hmc {
 
 // ------------------------------------------------ persistent apply (mixed) --
-// One cooperative launch runs every cycle and colour of an apply.  Workgroup
+// One launch runs every cycle and colour of an apply.  Workgroup
 // b owns a region of 2 T spaces per axis (the last region along an axis may
 // be shorter) and keeps the region plus a one-space halo -- every cell its
 // trials can read -- in LDS for the whole apply: staged once, its own cells
@@ -53,8 +53,7 @@ namespace hmc {
 // The FP64 sites that neighbours read are written with device-scope stores;
 // every wave waits for its stores to complete before the progress word is
 // stored, and neighbours read the sites with device-scope loads (no cache
-// writeback or invalidation).  The launch is cooperative, so every region is
-// resident, and the region whose pass is lowest never waits for one ahead of
+// writeback or invalidation).  Every region is resident (launch_resident), and the region whose pass is lowest never waits for one ahead of
 // it, so all of them finish.  Waits are bounded: past the bound the state's
 // error word is set and the wait returns, so every wave still ends.
 //

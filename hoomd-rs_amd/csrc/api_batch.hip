@@ -689,12 +689,10 @@ int hmc_batch_sdf(hmc_batch* b, double xmax, double dx, uint32_t nbins, uint64_t
     k_scan_top<<<1, 1024, 0, s>>>(gt, b->sts + b->R, b->w.block_sums, b->w.block_ne, nsb, b->w.start, 0);
     k_scan_add<<<grid_for(stot, 256), 256, 0, s>>>(b->w.start, b->w.block_sums, nullptr, stot);
     k_scatter<<<grid_for(b->n_total, kBlock), kBlock, 0, s>>>(b->gtot, b->w);
-    if (b->dim == 2)
-      k_sdf<2><<<grid_for(b->n_total, kBlock), kBlock, 0, s>>>(dreps, b->dboff, b->R, b->n_total, b->bodies, b->w,
-                                                               xmax, dx, nbins, dh, dh + (size_t)b->R * nbins);
-    else
-      k_sdf<3><<<grid_for(b->n_total, kBlock), kBlock, 0, s>>>(dreps, b->dboff, b->R, b->n_total, b->bodies, b->w,
-                                                               xmax, dx, nbins, dh, dh + (size_t)b->R * nbins);
+    const SdfGrid q = sdf_grid(b->n_total);
+    (b->dim == 2 ? k_sdf<2> : k_sdf<3>)<<<q.chunk * 8, kSdfThreads, 0, s>>>(
+        dreps, b->sts, b->dboff, b->R, b->n_total, q.chunk, q.per, 0, b->bodies, b->w, xmax, dx, nbins, dh,
+        dh + (size_t)b->R * nbins);
   }
   std::vector<uint32_t> h(cells, 0u);
   if (e == hipSuccess) e = hipGetLastError();

@@ -172,12 +172,10 @@ int hmc_sdf(hmc_ctx* c, double xmax, double dx, uint32_t nbins, uint64_t* hist, 
       k_scan_top<<<1, 1024, 0, s>>>(g, c->st, c->w.block_sums, c->w.block_ne, nsb, c->w.start, 0);
       k_scan_add<<<grid_for(g.n_spaces, 256), 256, 0, s>>>(c->w.start, c->w.block_sums, c->w.cnt, g.n_spaces);
       k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
-      if (g.dim == 2)
-        k_sdf<2><<<grid_for(N, kBlock), kBlock, 0, s>>>(drep, dboff, 1u, N, c->bodies, c->w, xmax, dx, nbins, dh,
-                                                        dh + nbins);
-      else
-        k_sdf<3><<<grid_for(N, kBlock), kBlock, 0, s>>>(drep, dboff, 1u, N, c->bodies, c->w, xmax, dx, nbins, dh,
-                                                        dh + nbins);
+      const SdfGrid q = sdf_grid(N);
+      const bool lds = nbins <= kSdfLdsBins;
+      (g.dim == 2 ? k_sdf<2> : k_sdf<3>)<<<q.chunk * 8, kSdfThreads, lds ? (nbins + 1) * sizeof(uint32_t) : 0, s>>>(
+          drep, c->st, dboff, 1u, N, q.chunk, q.per, lds ? 1 : 0, c->bodies, c->w, xmax, dx, nbins, dh, dh + nbins);
     }
     e = hipGetLastError();
   }

@@ -153,6 +153,17 @@ hipError_t dalloc(T** p, size_t n) {
   return hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T));
 }
 
+// k_sdf's grid over n slots: blocks per XCD, slots per block.
+struct SdfGrid {
+  uint32_t chunk, per;
+};
+inline SdfGrid sdf_grid(uint32_t n) {
+  const uint32_t need = (uint32_t)(((uint64_t)n + kSdfThreads - 1) / kSdfThreads);
+  const uint32_t chunk = (std::min(std::max(need, 1u), kSdfBlocks) + 7) / 8;
+  const uint64_t per = ((uint64_t)n + chunk * 8 - 1) / (chunk * 8);
+  return {chunk, (uint32_t)((per + kSdfThreads - 1) / kSdfThreads * kSdfThreads)};
+}
+
 inline uint32_t grid_for(uint64_t n, uint32_t block) { return (uint32_t)((n + block - 1) / block); }
 
 // A persistent apply's launch (resident.hip), and what precedes the end of a stream

@@ -69,7 +69,7 @@ __global__ void k_tune_eval(Geometry g, const ApplyState* st, Bodies B, Work w, 
 template <int D>
 __global__ void k_remove_energy(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t body, double* out);
 template <int D>
-__global__ void k_sdf(const BatchRep* reps, const uint32_t* boff, uint32_t R, uint32_t n_total, Bodies B, Work w, double xmax, double dx, uint32_t nbins, uint32_t* hist, uint32_t* ovl);
+__global__ void k_sdf(const BatchRep* reps, const ApplyState* sts, const uint32_t* boff, uint32_t R, uint32_t n_total, uint32_t xcd_chunk, uint32_t per, int lds, Bodies B, Work w, double xmax, double dx, uint32_t nbins, uint32_t* hist, uint32_t* ovl);
 template <int D>
 __global__ void k_init_sites(Geometry g, Bodies B, int have_sites);
 template <int D>

@@ -925,6 +925,9 @@ constexpr uint32_t kCvTrials = 4;  // convex pass: trials per wavefront
 constexpr uint32_t kCvLanes = 64 / kCvTrials;
 constexpr uint32_t kCvApply = 64;  // threads of a region of the persistent convex apply
 
+constexpr uint32_t kSdfThreads = 512;
+constexpr uint32_t kSdfBlocks = 768;      // of the SDF at most: three per CU
+constexpr uint32_t kSdfLdsBins = 8192;    // bins summed in LDS at most
 constexpr int kEnergyBlock = 256;
 constexpr int kEnergyFinal = 256;
 

@@ -362,6 +362,14 @@ void fill_halo_lists(TileCfg* tc, int D) {
   for (int q = 0; q < kHaloLists; ++q) tc->hoff[q + 1] = tc->hoff[q] + cnt[q];
 }
 
+// Region shape of a persistent hard-shape apply: the fewest threads, then the
+// least staging over all regions.  Where one region per compute unit suffices
+// (with 64 lanes' trials each), about as many regions as that gives, at least
+// three quarters: their boxes are smaller, and staging and reloading a box is
+// much of a small system's apply.  Measured us per apply, least staging alone and
+// so: 400 disks 49.7 (4 regions) and 45.3 (100), 1,024 48.3 (4) and 42.9 (256),
+// 4,000 spheres 143 (8) and 119 (256), 13,500 146 (27) and 129 (216), 70,304 143
+// (147) and 141 (196); with the most regions 83,000 in FP64 took 149 instead of 145.
 bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus, TileCfg* out) {
   uint32_t lim[3] = {1, 1, 1};
   const uint32_t cap[3] = {16, 16, 32};
@@ -374,48 +382,58 @@ bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus,
   const uint32_t cu_waves = 8;  // two waves per SIMD at the kernel's register use
   uint32_t best_threads = 0;
   double best_work = 0.0;
-  bool found = false;
-  for (uint32_t t0 = 1; t0 <= lim[0]; ++t0)
-    for (uint32_t t1 = 1; t1 <= lim[1]; ++t1)
-      for (uint32_t t2 = 1; t2 <= lim[2]; ++t2) {
-        const uint32_t T[3] = {t0, t1, t2};
-        const uint32_t trials = T[0] * T[1] * T[2];
-        if (trials > (uint32_t)kTileThreads) continue;
-        const uint32_t threads = ((trials + 63) / 64) * 64;
-        uint32_t ncell = 1, ntiles = 1, own = 1;
-        for (int a = 0; a < D; ++a) {
-          ncell *= 2 * T[a] + 2;
-          own *= 2 * T[a];
-          ntiles *= (g.half_shape[a] + T[a] - 1) / T[a];
-        }
-        const uint32_t EL = 2 * T[D - 1] + 2, rows = ncell / EL;
-        if (rows > kMaxRegionRows) continue;
-        const uint32_t maxb = (uint32_t)std::ceil(1.1 * occ * ncell) + 64;
-        const size_t lds = ((region_head_bytes(rows, ncell - own) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
-                           (size_t)(maxb + kTilePad) * entry;
-        if (lds > kTileLds) continue;
-        const uint32_t per_cu = std::min<uint32_t>((uint32_t)(cu_lds / (lds + static_lds)), cu_waves / (threads / 64));
-        const uint32_t grid = ((ntiles + 7) / 8) * 8;
-        if (per_cu == 0 || grid > per_cu * (uint32_t)cus) continue;
-        const double work = (double)ntiles * ncell;
-        if (!found || threads < best_threads || (threads == best_threads && work < best_work)) {
-          found = true;
-          best_threads = threads;
-          best_work = work;
-          for (int a = 0; a < 3; ++a) {
-            out->T[a] = a < D ? T[a] : 1;
-            out->nt[a] = a < D ? (g.half_shape[a] + T[a] - 1) / T[a] : 1;
-            out->E[a] = a < D ? 2 * T[a] + 2 : 1;
+  bool found = false, best_spread = false;
+  uint32_t most = 0;  // regions of a shape with at most one per compute unit
+  for (int pass = 0; pass < 2; ++pass)
+    for (uint32_t t0 = 1; t0 <= lim[0]; ++t0)
+      for (uint32_t t1 = 1; t1 <= lim[1]; ++t1)
+        for (uint32_t t2 = 1; t2 <= lim[2]; ++t2) {
+          const uint32_t T[3] = {t0, t1, t2};
+          const uint32_t trials = T[0] * T[1] * T[2];
+          if (trials > (uint32_t)kTileThreads) continue;
+          const uint32_t threads = ((trials + 63) / 64) * 64;
+          uint32_t ncell = 1, ntiles = 1, own = 1;
+          for (int a = 0; a < D; ++a) {
+            ncell *= 2 * T[a] + 2;
+            own *= 2 * T[a];
+            ntiles *= (g.half_shape[a] + T[a] - 1) / T[a];
           }
-          out->trials = trials;
-          out->ncell = ncell;
-          out->rows = rows;
-          out->maxb = maxb;
-          out->ntiles = ntiles;
-          out->xcd_chunk = (ntiles + 7) / 8;
-          out->lds_bytes = (uint32_t)lds;
+          const uint32_t EL = 2 * T[D - 1] + 2, rows = ncell / EL;
+          if (rows > kMaxRegionRows) continue;
+          const uint32_t maxb = (uint32_t)std::ceil(1.1 * occ * ncell) + 64;
+          const size_t lds = ((region_head_bytes(rows, ncell - own) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
+                             (size_t)(maxb + kTilePad) * entry;
+          if (lds > kTileLds) continue;
+          const uint32_t per_cu = std::min<uint32_t>((uint32_t)(cu_lds / (lds + static_lds)), cu_waves / (threads / 64));
+          const uint32_t grid = ((ntiles + 7) / 8) * 8;
+          if (per_cu == 0 || grid > per_cu * (uint32_t)cus) continue;
+          const double work = (double)ntiles * ncell;
+          bool spread = threads == 64 && grid <= (uint32_t)cus;
+          if (pass == 0) {
+            if (spread) most = std::max(most, ntiles);
+            continue;
+          }
+          spread = spread && 4 * ntiles >= 3 * most;
+          if (!found || threads < best_threads || (threads == best_threads && spread && !best_spread) ||
+              (threads == best_threads && spread == best_spread && work < best_work)) {
+            found = true;
+            best_spread = spread;
+            best_threads = threads;
+            best_work = work;
+            for (int a = 0; a < 3; ++a) {
+              out->T[a] = a < D ? T[a] : 1;
+              out->nt[a] = a < D ? (g.half_shape[a] + T[a] - 1) / T[a] : 1;
+              out->E[a] = a < D ? 2 * T[a] + 2 : 1;
+            }
+            out->trials = trials;
+            out->ncell = ncell;
+            out->rows = rows;
+            out->maxb = maxb;
+            out->ntiles = ntiles;
+            out->xcd_chunk = (ntiles + 7) / 8;
+            out->lds_bytes = (uint32_t)lds;
+          }
         }
-      }
   return found;
 }
 

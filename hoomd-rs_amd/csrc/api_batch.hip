@@ -690,8 +690,9 @@ int hmc_batch_sdf(hmc_batch* b, double xmax, double dx, uint32_t nbins, uint64_t
     k_scan_add<<<grid_for(stot, 256), 256, 0, s>>>(b->w.start, b->w.block_sums, nullptr, stot);
     k_scatter<<<grid_for(b->n_total, kBlock), kBlock, 0, s>>>(b->gtot, b->w);
     const SdfGrid q = sdf_grid(b->n_total);
-    (b->dim == 2 ? k_sdf<2> : k_sdf<3>)<<<q.chunk * 8, kSdfThreads, 0, s>>>(
-        dreps, b->sts, b->dboff, b->R, b->n_total, q.chunk, q.per, 0, b->bodies, b->w, xmax, dx, nbins, dh,
+    const bool lds = nbins <= kSdfLdsBins;
+    (b->dim == 2 ? k_sdf<2> : k_sdf<3>)<<<q.chunk * 8, kSdfThreads, lds ? (nbins + 1) * sizeof(uint32_t) : 0, s>>>(
+        dreps, b->sts, b->dboff, b->R, b->n_total, q.chunk, q.per, lds ? 1 : 0, b->bodies, b->w, xmax, dx, nbins, dh,
         dh + (size_t)b->R * nbins);
   }
   std::vector<uint32_t> h(cells, 0u);

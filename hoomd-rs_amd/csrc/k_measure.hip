@@ -363,9 +363,9 @@ __device__ __forceinline__ uint32_t sdf_bin(const Geometry& g, const double* ori
 }
 
 // Blocks of kSdfThreads take runs of `per` slots; the blocks of an XCD take a
-// slab.  One system's counts are summed in LDS first (`lds`: nbins + 1 words
-// of it): with an atomic operation per body on a few hundred counters the kernel
-// took 611 us.
+// slab.  The counts of the run's first system (most runs lie in one) are summed in
+// LDS first (`lds`: nbins + 1 words of it): with an atomic operation per body on a
+// few hundred counters the kernel took 611 us.
 template <int D>
 __global__ void __launch_bounds__(kSdfThreads) k_sdf(const BatchRep* reps, const ApplyState* sts,
                                                      const uint32_t* boff, uint32_t R, uint32_t n_total,
@@ -374,17 +374,26 @@ __global__ void __launch_bounds__(kSdfThreads) k_sdf(const BatchRep* reps, const
                                                      uint32_t* ovl) {
   extern __shared__ uint32_t lh[];
   const uint32_t lb = (blockIdx.x & 7u) * xcd_chunk + (blockIdx.x >> 3);
+  const uint64_t begin = (uint64_t)lb * per, end = min(begin + per, (uint64_t)n_total);
+  if (begin >= end) return;  // uniform
   if (lds) {
     for (uint32_t i = threadIdx.x; i <= nbins; i += kSdfThreads) lh[i] = 0;
     __syncthreads();
   }
-  const uint64_t end = min((uint64_t)(lb + 1u) * per, (uint64_t)n_total);
-  for (uint64_t q = (uint64_t)lb * per + threadIdx.x; q < end; q += kSdfThreads) {
+  const uint32_t r0 = R > 1 ? find_replica(boff, R, (uint32_t)begin) : 0u;
+  uint32_t r = r0;
+  for (uint64_t q = begin + threadIdx.x; q < end; q += kSdfThreads) {
     const uint32_t p = (uint32_t)q, b = w.tmp_body[p];
-    const uint32_t r = R > 1 ? find_replica(boff, R, b) : 0u;
-    const uint32_t k = sdf_bin<D>(reps[r].g, sts[r].origin, reps[r].space_off, p, b, B, w, xmax, dx, nbins);
+    while (r + 1u < R && p >= boff[r + 1u]) ++r;
+    uint32_t k = UINT32_MAX;
+    for (bool done = false; !done;) {  // one system of the wavefront at a time: its constants are scalars
+      const uint32_t ru = __builtin_amdgcn_readfirstlane(r);
+      if (r != ru) continue;
+      k = sdf_bin<D>(reps[ru].g, sts[ru].origin, reps[ru].space_off, p, b, B, w, xmax, dx, nbins);
+      done = true;
+    }
     if (k == UINT32_MAX) continue;
-    if (lds)
+    if (lds && r == r0)
       atomicAdd(&lh[k], 1u);
     else
       atomicAdd(k < nbins ? &hist[(size_t)r * nbins + k] : &ovl[r], 1u);
@@ -395,7 +404,7 @@ __global__ void __launch_bounds__(kSdfThreads) k_sdf(const BatchRep* reps, const
   const uint32_t n = nbins + 1u, first = (lb * 37u) % n;
   for (uint32_t i = threadIdx.x; i < n; i += kSdfThreads) {
     const uint32_t k = i + first < n ? i + first : i + first - n;
-    if (lh[k]) atomicAdd(k < nbins ? &hist[k] : &ovl[0], lh[k]);
+    if (lh[k]) atomicAdd(k < nbins ? &hist[(size_t)r0 * nbins + k] : &ovl[r0], lh[k]);
   }
 }
 

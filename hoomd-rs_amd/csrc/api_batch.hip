@@ -222,6 +222,12 @@ bool batch_regions(hmc_batch* b, int cus) {
     }
   constexpr int D = 3;
   const void* fn = (const void*)k_bapply_tile<3>;
+  // the places of the halo lists of a region of T^3 colour spaces
+  std::array<TileCfg, 7> lists{};
+  for (uint32_t T = 2; T <= 6; ++T) {
+    for (int a = 0; a < D; ++a) lists[T].T[a] = T;
+    fill_halo_lists(&lists[T], D);
+  }
   // the region shape T of replica r for a workgroup of `threads` and an LDS
   // budget `cap`: the fewest regions (then the least LDS); false if none fits
   auto shape_for = [&](uint32_t r, uint32_t threads, uint32_t cap, TileCfg& out) {
@@ -258,7 +264,7 @@ bool batch_regions(hmc_batch* b, int cus) {
                       : (uint32_t)std::ceil(1.1 * occ * ncell) + 64;
       tc.ntiles = ntiles;
       tc.xcd_chunk = (ntiles + 7) / 8;
-      fill_halo_lists(&tc, D);
+      std::memcpy(tc.hoff, lists[T].hoff, sizeof tc.hoff);
       const size_t lr = ((region_head_bytes(rows, tc.hoff[kHaloLists]) + 2 * (size_t)rows * (EL + 1) + 15) & ~(size_t)15) +
                         (size_t)(tc.maxb + kTilePad) * sizeof(float4);
       if (lr > cap || lr > kTileLds) ok = false;
@@ -318,7 +324,10 @@ bool batch_regions(hmc_batch* b, int cus) {
         round_of[r] = (uint32_t)k;
       }
       if (!ok) continue;
-      if (best.empty() || load.size() < best_groups || (load.size() == best_groups && threads < best_threads)) {
+      // the fewest rounds, then the most threads: lanes beyond the trials stage and
+      // reload.  (64 replicas of 864 to 32,000 bodies, us per step: 247 with 128
+      // threads, 970 with 64 and the same 64 trials per region.)
+      if (best.empty() || load.size() < best_groups || (load.size() == best_groups && threads > best_threads)) {
         std::vector<uint32_t> t0(load.size(), 0);
         for (size_t k = 1; k < load.size(); ++k) t0[k] = t0[k - 1] + load[k - 1];
         best = tcs;
@@ -536,8 +545,8 @@ int hmc_batch_create(uint32_t n_replicas, const hmc_config* cfgs, hmc_batch** ou
       hmc_batch_destroy(b);
       return HMC_ERR_DEVICE;
     }
-    // mixed precision in 3D: persistent applies, one launch per step (HMC_FLAG_PER_COLOUR keeps the per-colour
-    // tile passes)
+    // mixed precision in 3D: persistent applies, one launch per step
+    // (HMC_FLAG_PER_COLOUR keeps the per-colour tile passes)
     int cus = 0, coop = 0;
     if (b->tiled && b->dim == 3 && b->precision == HMC_MIXED && !(cfgs[0].flags & HMC_FLAG_PER_COLOUR) &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) == hipSuccess && cus > 0 &&

@@ -292,14 +292,9 @@ __device__ __forceinline__ uint32_t sdf_bin(const Geometry& g, const double* ori
     const float cut = (float)(rmax * rmax) * (1.0f + 1e-4f);
     float flo[3], fhi[3];
 #pragma unroll
-    for (int a = 0; a < D; ++a) {
-      double u = t[a] - origin[a];
-      u = u >= g.L[a] ? u - g.L[a] : u;
-      u -= (double)m[a] * g.width[a];
-      const float wd = (float)g.width[a], uf = (float)u, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
-      flo[a] = dl * dl;
-      fhi[a] = dh * dh;
-    }
+    for (int a = 0; a < D; ++a)
+      face_gap2(space_offset(t[a] - origin[a], (double)m[a], g.width[a], g.L[a], g.half[a]), g.width[a], &flo[a],
+                &fhi[a]);
     const int32_t sh = g.shape[AL], ml = m[AL];
     const bool wlo = ml == 0, whi = ml + 1 == sh;  // the lower / upper space lies across the face
     constexpr int NR = D == 3 ? 9 : 3;

@@ -202,14 +202,9 @@ template <int D>
 __device__ __forceinline__ void face_gaps2(GeoPtr g, const double* origin, const uint32_t* own, const double* x,
                                            float* lo, float* hi) {
 #pragma unroll
-  for (int a = 0; a < D; ++a) {
-    double u = x[a] - origin[a];
-    u = u >= g->L[a] ? u - g->L[a] : u;
-    u -= (double)own[a] * g->width[a];
-    const float wd = (float)g->width[a], uf = (float)u, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
-    lo[a] = dl * dl;
-    hi[a] = dh * dh;
-  }
+  for (int a = 0; a < D; ++a)
+    face_gap2(space_offset(x[a] - origin[a], (double)own[a], g->width[a], g->L[a], g->half[a]), g->width[a], &lo[a],
+              &hi[a]);
 }
 
 // The neighbour spaces of a trial (each once, as the reference's cell list

@@ -233,6 +233,21 @@ __device__ __forceinline__ uint32_t space_of(const Geometry& g, const double* or
   return index;
 }
 
+// Offset of a site (u from the origin of the checkerboard) from the lower face of
+// its space, the m-th along an axis of three spaces or more.  Folded by the
+// offset: space_of counts u / width == shape as space 0 and rounds, so that a
+// site of space 0 may have u an ulp below L, and one of the last space u = L.
+__device__ __forceinline__ double space_offset(double u, double m, double width, double L, double half) {
+  const double v = u - m * width;
+  return v > half ? v - L : v < -half ? v + L : v;
+}
+// The squared distances of such an offset to the space's faces.
+__device__ __forceinline__ void face_gap2(double v, double width, float* lo, float* hi) {
+  const float wd = (float)width, uf = (float)v, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
+  *lo = dl * dl;
+  *hi = dh * dh;
+}
+
 // The t-th space of colour c, in the order of
 // HypercuboidCheckerboard::construct_space_indices_by_color (hypercuboid.rs:231-255):
 // multi-index 2h + offset(c), h running over the half grid, last axis fastest.

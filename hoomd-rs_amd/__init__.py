@@ -40,6 +40,7 @@ EXPORTS = ["hmc_create", "hmc_set_state", "hmc_get_state", "hmc_clone_with_bound
            "hmc_apply_rotate",
            "hmc_set_orientations", "hmc_get_orientations", "hmc_run_translate", "hmc_total_energy",
            "hmc_total_energy_noalloc", "hmc_run", "hmc_moved_since", "hmc_get_bodies", "hmc_debug_regions",
+           "hmc_debug_form",
            "hmc_trace_enable", "hmc_trace_read", "hmc_get_stats", "hmc_profile_enable", "hmc_profile_read",
            "hmc_debug_math", "hmc_debug_normals", "hmc_debug_convex", "hmc_debug_convex_axes", "hmc_last_error",
            "hmc_destroy",
@@ -164,6 +165,7 @@ def lib():
                                       C.POINTER(C.c_uint64)]
         L.hmc_get_bodies.argtypes = [vp, C.POINTER(C.c_uint32), C.c_uint64, D_P, D_P, D_P, D_P]
         L.hmc_debug_regions.argtypes = [vp, C.POINTER(C.c_uint32), C.c_uint64, C.POINTER(C.c_uint64)]
+        L.hmc_debug_form.argtypes = [vp, C.POINTER(C.c_uint32)]
         u64p = C.POINTER(C.c_uint64)
         L.hmc_sdf.argtypes = [vp, C.c_double, C.c_double, C.c_uint32, u64p, u64p]
         L.hmc_batch_sdf.argtypes = [vp, C.c_double, C.c_double, C.c_uint32, u64p, u64p]
@@ -431,6 +433,12 @@ class GpuParallelSweep:
         n = C.c_uint64()
         self._check(lib().hmc_debug_regions(self.h, out.ctypes.data_as(C.POINTER(C.c_uint32)), cap, C.byref(n)))
         return out[: 6 * n.value].reshape(-1, 6)
+
+    def debug_form(self):
+        """The form of the next apply (hmc_debug_form)."""
+        out = (C.c_uint32 * 4)()
+        self._check(lib().hmc_debug_form(self.h, out))
+        return dict(zip(("persistent", "iso_lanes", "small_waves", "bucket_build"), out))
 
     def moved_since(self, since):
         """(indices of the bodies moved by applies after epoch `since`, the

@@ -411,6 +411,12 @@ int hmc_profile_read(hmc_ctx* ctx, double* pass_ms_total, uint64_t* pass_launche
  * counterpart. */
 int hmc_debug_regions(hmc_ctx* ctx, uint32_t* out, uint64_t cap, uint64_t* n);
 
+/* Test hook: the form that the next apply takes, four words: 1 for a persistent
+ * launch; the lanes per trial of FP64 pair energies (else 0); the wavefronts per
+ * trial of a system that one workgroup runs (else 0); 1 for the two-kernel build
+ * of persistent hard shapes. */
+int hmc_debug_form(const hmc_ctx* ctx, uint32_t* out);
+
 /* Evaluate the library's device math on n inputs: kind 0 cbrt, 1 log,
  * 2 exp, 5 the sine and 6 the cosine of one sincos call (the device's
  * restatements of the glibc functions Rust's std calls on Linux), 3 sqrt,

@@ -1076,6 +1076,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
   // the regions are resident, else 8: overlap penalty, us per step with 64, 16 and
   // 8 lanes, 6,912 bodies 171, 187, 214; 16,384 206, 195, 221; 55,296 418 (not
   // resident), 229, 234; 131,072 765, 302 (neither resident), 290.
+  uint32_t pass_lanes = 8;
   if (lj && !lj_mixed && !c->small_wpt && g.n_bodies) {
     double cand = (double)g.n_bodies / (double)g.n_spaces;
     bool one = true;
@@ -1109,7 +1110,14 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         }
       }
     }
-    if (!c->persist) c->iso_lanes = many ? 64u : 8u;
+    // One launch per colour: 64 lanes too for more than 16 candidates while a
+    // colour's trials are at most twelve wavefronts per compute unit.  us per step
+    // with 64 and 8 lanes: LJ disks at density 0.7 (40 candidates), 10,000 bodies
+    // (1,296 trials a colour) 174 and 254, 40,000 (2,209) 216 and 255, 100,000 (5,625)
+    // 331 and 264, at density 0.16 (9), 10,000 (2,500) 101 and 94; overlap penalty (30),
+    // 9,000 bodies (1,000) 183 and 230, 30,000 (4,096) 266 and 224.
+    pass_lanes = many || (cand > 16.0 && g.per_colour <= 12u * 256u) ? 64u : 8u;
+    if (!c->persist) c->iso_lanes = pass_lanes;
   }
   const uint32_t N = g.n_bodies;
   c->n_scan_blocks = grid_for(g.n_spaces, kScanBlock);
@@ -1174,7 +1182,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     return HMC_ERR_DEVICE;
   }
   if (c->persist && !persist_probe(c)) c->persist = false;  // the per-colour passes instead
-  if (c->iso_lanes == 16 && !c->persist) c->iso_lanes = 8;  // (passes have no 16)
+  if (c->iso_lanes && !c->persist) c->iso_lanes = pass_lanes;
   *out = c;
   return HMC_OK;
 }

@@ -43,3 +43,25 @@ def test_build_of_wide_spaces(hmc, L, n, width, bucket, precision):
         out.append((counts, np.concatenate([x.ravel() for x in sim.positions()]).view(np.uint64)))
         sim.close()
     assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("L,n,model,form", [
+    ((120.0, 121.0), 10000, "lj_shifted", dict(persistent=0, iso_lanes=64)),  # a scan of two, 576 trials a colour
+    ((375.0, 376.0), 100000, "lj_shifted", dict(persistent=0, iso_lanes=8)),  # 5,625
+    ((250.0, 251.0), 10000, "lj_shifted", dict(persistent=0, iso_lanes=8)),  # 2,500, nine candidates
+    ((20.0, 21.3, 22.3), 9000, "overlap_penalty", dict(persistent=0, iso_lanes=64)),  # 1,100
+    ((32.0, 33.3, 34.3), 33000, "overlap_penalty", dict(persistent=0, iso_lanes=8)),  # 4,352
+    ((60.3, 72.1), 2400, "lj_shifted", dict(persistent=1, iso_lanes=64)),
+    ((25.3, 27.2, 26.1), 15000, "overlap_penalty", dict(persistent=1, iso_lanes=16)),
+    ((51.3, 50.2, 49.1), 110000, "overlap_penalty", dict(persistent=1, iso_lanes=8)),
+    ((36.2, 31.1, 35.3), 30000, "lj_shifted", dict(persistent=1, iso_lanes=64)),
+    ((9.3, 12.2, 10.1), 1100, "overlap_penalty", dict(persistent=1, iso_lanes=64, small_waves=0)),
+    ((15.5, 15.4, 15.3), 1100, "lj_shifted", dict(persistent=0, iso_lanes=0, small_waves=1)),
+    ((10.1, 10.2, 10.3), 700, "lj_shifted", dict(persistent=0, iso_lanes=0, small_waves=2)),
+    ((5.3, 5.2, 5.4), 60, "lj_shifted", dict(persistent=0, iso_lanes=0, small_waves=4)),
+])
+def test_lanes_of_pair_energies(hmc, L, n, model, form):
+    sim = hmc.GpuParallelSweep(np.array(L), _lattice(L, n), model=model)
+    got = sim.debug_form()
+    sim.close()
+    assert {k: got[k] for k in form} == form

@@ -45,19 +45,34 @@ Geometry sdf_geometry(const Geometry& g, double xmax) {
   return s;
 }
 
-// Lanes per neighbour query (k_energy, k_insert_energy): half a wavefront where
-// a space holds four bodies or more or there are too few queries to fill the
-// device with eight lanes each.
-static int query_lanes(const Geometry& g, uint64_t queries) {
-  return (uint64_t)g.n_bodies >= 4ull * g.n_spaces || queries < (1u << 16) ? 32 : 8;
+// Lanes per site of the total energy (k_energy): as many as it takes to fill the
+// device, since every lane of a site repeats its setup.  More than 64 candidates
+// per site are worth half a wavefront up to 65,536 sites.  Measured us per call with 32,
+// 8, 2 and 1 lanes: LJ at density 0.8 (340 candidates), 20,000 bodies 178, 168, 319 and
+// 551, 160,000 787, 527, 462 and 557, 600,000 2359, 1539, 1117 and 1239; hard spheres,
+// 20,000 102, 83, 101 and 99, 60,000 132, 100, 108 and 107, 160,000 227, 141, 129 and 112,
+// 600,000 434, 310, 222 and 204.
+static int energy_lanes(const Geometry& g) {
+  double cand = (double)g.n_bodies / (double)g.n_spaces;
+  for (int a = 0; a < g.dim; ++a) cand *= std::min(2.0 * g.reach[a] + 1.0, (double)g.shape[a]);
+  const uint32_t n = g.n_bodies;
+  if (n <= (cand > 64.0 ? 1u << 16 : 1u << 14)) return 32;
+  if (n <= 3u << 15) return 8;
+  return cand > 64.0 ? 2 : 1;
 }
+// Lanes per insertion energy (k_insert_energy).  us per call with 32, 8 and 1 lanes:
+// LJ at density 0.8, 4,096 bodies into 160,000 190, 244 and 820, 20,000 274, 298 and
+// 820, 65,536 570, 606 and 940, 200,000 1366, 1429 and 1752; into 200, whose few spaces every
+// lane finds in its cache, 20,000 541, 496 and 586, 65,536 506, 364 and 436, 200,000 1202, 794
+// and 874.
+static int insert_lanes(uint64_t queries) { return queries <= 1u << 15 ? 32 : 8; }
 // Sites a group of lanes takes in turn, so that the partials of all blocks fit
 // the scratch's kNoAllocBlocks, and those blocks.
 static uint32_t energy_per(const Geometry& g) {
-  return std::max(1u, grid_for(g.n_bodies, (uint32_t)(kEnergyBlock / query_lanes(g, g.n_bodies)) * kNoAllocBlocks));
+  return std::max(1u, grid_for(g.n_bodies, (uint32_t)(kEnergyBlock / energy_lanes(g)) * kNoAllocBlocks));
 }
 static uint32_t energy_blocks(const Geometry& g) {
-  return grid_for(g.n_bodies, (uint32_t)(kEnergyBlock / query_lanes(g, g.n_bodies)) * energy_per(g));
+  return grid_for(g.n_bodies, (uint32_t)(kEnergyBlock / energy_lanes(g)) * energy_per(g));
 }
 
 // PairwiseCutoff::total_energy of the current state with the block partials
@@ -85,8 +100,9 @@ int total_energy_into(hmc_ctx* c, double* part, double* total, double* bound) {
   k_scan_top<<<1, 1024, 0, s>>>(g, c->st, c->w.block_sums, c->w.block_ne, c->n_scan_blocks, c->w.start, 0);
   k_scan_add<<<grid_for(g.n_spaces, 256), 256, 0, s>>>(c->w.start, c->w.block_sums, c->w.cnt, g.n_spaces);
   k_scatter<<<grid_for(N, kBlock), kBlock, 0, s>>>(g, c->w);
-  const bool wide = query_lanes(g, N) == 32;
-  const auto energy = g.dim == 2 ? (wide ? k_energy<2, 32> : k_energy<2, 8>) : (wide ? k_energy<3, 32> : k_energy<3, 8>);
+  const int lanes = energy_lanes(g);
+  const auto energy = g.dim == 2 ? (lanes == 32 ? k_energy<2, 32> : lanes == 8 ? k_energy<2, 8> : lanes == 2 ? k_energy<2, 2> : k_energy<2, 1>)
+                                 : (lanes == 32 ? k_energy<3, 32> : lanes == 8 ? k_energy<3, 8> : lanes == 2 ? k_energy<3, 2> : k_energy<3, 1>);
   energy<<<nblk, kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, per, part);
   k_energy_final<<<1, kEnergyFinal, 0, s>>>(part, nblk, part + 4 * (size_t)nblk);
   double out[4] = {0, 0, 0, 0};
@@ -240,7 +256,7 @@ int hmc_delta_energy_insert(hmc_ctx* c, const double* body_pos, uint64_t n, doub
   if (e == hipSuccess) e = hipMemsetAsync(flag, 0, sizeof(uint32_t), s);
   if (e == hipSuccess) {
     launch_cell_lists(c);  // cells of the current state, as for the total energy
-    const int lanes = query_lanes(g, n);
+    const int lanes = insert_lanes(n);
     const auto insert = D == 2 ? (lanes == 32 ? k_insert_energy<2, 32> : k_insert_energy<2, 8>)
                                : (lanes == 32 ? k_insert_energy<3, 32> : k_insert_energy<3, 8>);
     insert<<<grid_for(n, (uint32_t)(kEnergyBlock / lanes)), kEnergyBlock, 0, s>>>(g, c->st, c->bodies, c->w, dc,

@@ -9,9 +9,8 @@ namespace hmc {
 // gl + G, ... of the 3^D (5^D) around the site's space, each space once.  One
 // lane per site ran all its candidates in a chain of dependent loads on few
 // wavefronts (864 LJ bodies: 4 workgroups, 317 us; on half-waves 22 us).
-// G = 32 where spaces hold several bodies, 8 where they hold about one (the
-// setup every lane of a group repeats then costs more than the candidates):
-// query_lanes on the host.
+// The setup every lane of a group repeats costs more than it gives once one lane
+// per query fills the device: energy_lanes and insert_lanes on the host.
 struct Neighbours {
   uint32_t n[3], first[3];  // spaces visited along each axis, the first of them
 };
@@ -404,6 +403,10 @@ __global__ void __launch_bounds__(kSdfThreads) k_sdf(const BatchRep* reps, const
 }
 
 // explicit instantiations (launched from the host translation units)
+template __global__ void k_energy<2, 1>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_energy<2, 2>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_energy<3, 1>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
+template __global__ void k_energy<3, 2>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
 template __global__ void k_energy<2, 8>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
 template __global__ void k_energy<2, 32>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);
 template __global__ void k_energy<3, 8>(Geometry g, const ApplyState* st, Bodies B, Work w, uint32_t per, double* part);

@@ -292,8 +292,7 @@ __device__ __forceinline__ uint32_t sdf_bin(const Geometry& g, const double* ori
     float flo[3], fhi[3];
 #pragma unroll
     for (int a = 0; a < D; ++a)
-      face_gap2(space_offset(t[a] - origin[a], (double)m[a], g.width[a], g.L[a], g.half[a]), g.width[a], &flo[a],
-                &fhi[a]);
+      face_gap2(t[a] - origin[a], (double)m[a], g.width[a], g.L[a], &flo[a], &fhi[a]);
     const int32_t sh = g.shape[AL], ml = m[AL];
     const bool wlo = ml == 0, whi = ml + 1 == sh;  // the lower / upper space lies across the face
     constexpr int NR = D == 3 ? 9 : 3;

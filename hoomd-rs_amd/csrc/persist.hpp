@@ -203,8 +203,7 @@ __device__ __forceinline__ void face_gaps2(GeoPtr g, const double* origin, const
                                            float* lo, float* hi) {
 #pragma unroll
   for (int a = 0; a < D; ++a)
-    face_gap2(space_offset(x[a] - origin[a], (double)own[a], g->width[a], g->L[a], g->half[a]), g->width[a], &lo[a],
-              &hi[a]);
+    face_gap2(x[a] - origin[a], (double)own[a], g->width[a], g->L[a], &lo[a], &hi[a]);
 }
 
 // The neighbour spaces of a trial (each once, as the reference's cell list

@@ -233,17 +233,14 @@ __device__ __forceinline__ uint32_t space_of(const Geometry& g, const double* or
   return index;
 }
 
-// Offset of a site (u from the origin of the checkerboard) from the lower face of
-// its space, the m-th along an axis of three spaces or more.  Folded by the
-// offset: space_of counts u / width == shape as space 0 and rounds, so that a
-// site of space 0 may have u an ulp below L, and one of the last space u = L.
-__device__ __forceinline__ double space_offset(double u, double m, double width, double L, double half) {
-  const double v = u - m * width;
-  return v > half ? v - L : v < -half ? v + L : v;
-}
-// The squared distances of such an offset to the space's faces.
-__device__ __forceinline__ void face_gap2(double v, double width, float* lo, float* hi) {
-  const float wd = (float)width, uf = (float)v, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
+// Squared distances of a site to the lower and upper face of its space, the m-th
+// along an axis of three spaces or more; u: the site from the checkerboard's
+// origin, up to L and a width.  space_of rounds u / width before it takes shape as 0: a
+// site of space 0 may have u an ulp below L (it lies on the lower face), one of the
+// last space u = L (on its upper face).
+__device__ __forceinline__ void face_gap2(double u, double m, double width, double L, float* lo, float* hi) {
+  const float wd = (float)width, v = (float)((u >= L ? u - L : u) - m * width);
+  const float uf = v > 2.0f * wd ? 0.0f : v < -wd ? wd : v, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
   *lo = dl * dl;
   *hi = dh * dh;
 }

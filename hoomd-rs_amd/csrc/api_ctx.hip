@@ -836,6 +836,177 @@ int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_
   return HMC_OK;
 }
 
+// One persistent launch per apply for hard shapes (k_apply_tile), its regions for
+// occ bodies per space.  False where there is none.
+static bool plan_hard(const hmc_ctx* c, double occ, RegionPlan* out) {
+  const Geometry& g = c->g;
+  const int D = g.dim;
+  int cus = 0, coop = 0;
+  // (the FP32 error report runs the per-colour passes)
+  if (!c->tiled || (c->cfg.flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0 ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop)
+    return false;
+  TileCfg pc{};
+  const size_t entry = c->cfg.precision == HMC_MIXED ? sizeof(float4) : sizeof(double4);
+  if (!choose_regions(g, D, occ, entry, cus, &pc)) return false;
+  fill_halo_lists(&pc, D);
+  // Band of the persistent layout, whose LDS entries are the FP64
+  // box-relative positions rounded once to FP32.  Per axis: that
+  // rounding for the site and for the trial site (2^-24 R each, R the
+  // largest box-relative coordinate), the rounding of their FP32
+  // difference (2^-24 |d|), and the FP64 roundings of x - c and of the
+  // image shift on both sides as well as of the reference's own
+  // displacement (2^-53 (4 L + 2 |d|)).
+  const double sigma = g.sigma;
+  double R = 0.0, lmax = 0.0;
+  for (int a = 0; a < D; ++a) {
+    R = std::max(R, 0.5 * pc.E[a] * g.width[a] + g.width[a]);
+    lmax = std::max(lmax, g.L[a]);
+  }
+  const double Et = (0x1p-24 * (2.0 * R + 2.0 * sigma) + 0x1p-53 * (4.0 * lmax + 2.0 * sigma)) * 1.01;
+  // In FP64 the same with 2^-53 for every rounding: x - c, the image
+  // shift and the rounding of the difference on both sides, and the
+  // reference's own displacement.
+  const double E64 = 0x1p-53 * (6.0 * lmax + 4.0 * R + 4.0 * sigma) * 1.01;
+  const void* fn = persist_kernel(c);
+  // one lane per trial, and where the regions leave compute units to
+  // spare, wavefronts that only stage and reload (a small system's box of
+  // 1000 cells staged by one wavefront took 40 us of a 200 us apply)
+  uint32_t threads = ((pc.trials + 63) / 64) * 64;
+  if (pc.xcd_chunk * 8u <= (uint32_t)cus) threads = kTileThreads;
+  int per_cu = 0;
+  if (!contact_band(Et, sigma, g.sigma2, g.edge2, D, &pc.band_lo, &pc.band_hi) ||
+      !contact_band64(E64, sigma, g.sigma2, g.edge2, D, &pc.band64_lo, &pc.band64_hi) ||
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pc.lds_bytes) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, (int)threads, pc.lds_bytes) != hipSuccess ||
+      (uint64_t)per_cu * (uint64_t)cus < (uint64_t)pc.xcd_chunk * 8u)
+    return false;
+  *out = {pc, threads, (uint32_t)per_cu, 0u};
+  return true;
+}
+
+// Candidates of a trial (the bodies of the 3^D spaces around it) where the bodies
+// fill `spaces` spaces.
+static double candidates(const Geometry& g, uint32_t spaces) {
+  double n = (double)g.n_bodies / (double)std::max<uint32_t>(spaces, 1);
+  for (int a = 0; a < g.dim; ++a) n *= 3.0;
+  return n;
+}
+
+// FP64 pair energies beyond k_apply_small, one launch per colour: lanes per trial.
+// 64 for more than 64 candidates (cand), and for more than 16 while a
+// colour's trials are at most twelve wavefronts per compute unit.  us per step
+// with 64 and 8 lanes: LJ disks at density 0.7 (40 candidates), 10,000 bodies
+// (1,296 trials a colour) 174 and 254, 40,000 (2,209) 216 and 255, 100,000 (5,625)
+// 331 and 264, at density 0.16 (9), 10,000 (2,500) 101 and 94; overlap penalty (30),
+// 9,000 bodies (1,000) 183 and 230, 30,000 (4,096) 266 and 224.
+static uint32_t pass_lanes(const Geometry& g, double cand) {
+  return cand > 64.0 || (cand > 16.0 && g.per_colour <= 12u * 256u) ? 64u : 8u;
+}
+
+// The same in one persistent launch per apply (k_apply_iso) where the neighbour
+// scan reaches one space out and a wavefront per 64 / lanes spaces of a colour is
+// resident.  With more than 64 candidates per trial 64 lanes share them (442,368
+// LJ bodies at density 0.8: 2261 us per step; with 16 lanes 3053, with 8 5553).
+// With fewer, 64 lanes while that is at most four wavefronts per compute unit, 16
+// while the regions are resident, else 8: overlap penalty, us per step with 64, 16
+// and 8 lanes, 6,912 bodies 171, 187, 214; 16,384 206, 195, 221; 55,296 418 (not
+// resident), 229, 234; 131,072 765, 302 (neither resident), 290.
+static bool plan_iso(const hmc_ctx* c, double cand, RegionPlan* out) {
+  const Geometry& g = c->g;
+  int cus = 0, coop = 0;
+  for (int a = 0; a < g.dim; ++a)
+    if (g.reach[a] != 1) return false;
+  if ((c->cfg.flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS)) ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0 ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop)
+    return false;
+  const bool many = cand > 64.0;
+  for (uint32_t lanes : {64u, 16u, 8u}) {
+    int per_cu = 0;
+    TileCfg pc{};
+    if ((many && lanes != 64) || hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                                     &per_cu, iso_apply_kernel(lanes, g.dim), 64, 0) != hipSuccess)
+      continue;
+    const uint32_t resident = (uint32_t)(lanes == 64 && !many ? std::min(per_cu, 4) : per_cu) * (uint32_t)cus;
+    if (!choose_regions_wave(g, 64u / lanes, resident, &pc)) continue;
+    *out = {pc, 64u, (uint32_t)per_cu, lanes};
+    return true;
+  }
+  return false;
+}
+
+static bool hard_shape(int model) { return model == HMC_HARD_SPHERE; }
+
+// Makes a plan the context's (its stream idle, if it has one).  False: no memory
+// for the mailboxes; the plan before stays.
+static bool adopt(hmc_ctx* c, const RegionPlan& plan) {
+  const size_t fbytes = (size_t)plan.pc.ntiles * kMailboxStride * sizeof(uint32_t);
+  uint32_t* mbox = nullptr;
+  if (hipMalloc((void**)&mbox, fbytes) != hipSuccess || hipMemset(mbox, 0, fbytes) != hipSuccess) {
+    (void)hipFree(mbox);
+    return false;
+  }
+  (void)hipFree(c->w.mbox);
+  c->w.mbox = mbox;
+  const uint32_t tag = c->pc.tag;
+  c->pc = plan.pc;
+  c->pc.tag = tag;
+  c->persist = true;
+  c->iso_lanes = plan.lanes;
+  c->pgrid = plan.pc.xcd_chunk * 8u;
+  c->pthreads = plan.threads;
+  c->pper_cu = plan.per_cu;
+  return true;
+}
+
+// One launch per colour from the next apply on (the stream idle).
+static void leave_persistent(hmc_ctx* c) {
+  c->persist = false;
+  forget_resident(c->device, c->stream);
+}
+
+// Plans made at creation take the bodies to fill the box.  Where a state says
+// otherwise -- a drop or a slab beside vapour or nothing -- its applies take the
+// plan that fits it, from the state s that the last apply left (the stream idle):
+//  - hard shapes: boxes beyond their LDS capacity run their trials from global
+//    memory, and every region comes to wait for such a one.  More than one per
+//    four applies: regions for the most sites a box held; without such regions
+//    FP64 takes one launch per colour;
+//  - FP64 pair energies: the candidates of a trial among the spaces that hold any.
+// us per apply with the plan of the mean density, one launch per colour, and so: in a
+// box of eight times their volume 20,000 spheres in FP64 with spaces of 1.0 diameters 509,
+// 485 and 180, of 1.3 1314, 876 and 191; 50,000 LJ bodies at density 0.8 2370, 1440 and 1440
+// (no regions with 64 lanes), 8,000 in 64 times 1915, 1157 and 1157.  A state set
+// later keeps the plan until an apply on it says otherwise; FP64 hard shapes that
+// took one launch per colour keep that.
+static void replan(hmc_ctx* c, const ApplyState& s) {
+  const Geometry& g = c->g;
+  RegionPlan plan;
+  if (c->persist && hard_shape(g.model)) {
+    const uint64_t over = s.tile_overflows - c->over_seen, applies = c->applies - c->applies_seen;
+    c->over_seen = s.tile_overflows;
+    c->applies_seen = c->applies;
+    if (4 * over <= applies) return;
+    const double occ = std::max((double)s.box_most / c->pc.ncell, (double)g.n_bodies / std::max<uint32_t>(s.nonempty, 1));
+    if (occ <= c->occ_tried) return;  // (planned for as much, or no such regions)
+    c->occ_tried = 1.05 * occ;
+    const bool fits = plan_hard(c, occ, &plan) && adopt(c, plan);
+    if (fits ? !persist_probe(c) : c->cfg.precision == HMC_FP64) leave_persistent(c);
+    (void)hipMemsetAsync(&c->st->box_most, 0, sizeof(uint32_t), c->stream);
+  } else if (c->iso_lanes) {
+    // (a wide margin, so that a fluctuation does not plan anew)
+    const double cand = candidates(g, s.nonempty);
+    if (c->iso_cand > 64.0 ? cand > 51.0 : cand < 80.0) return;
+    c->iso_cand = cand;
+    drop_graph(c);
+    if (plan_iso(c, cand, &plan) && adopt(c, plan) && persist_probe(c)) return;
+    if (c->persist) leave_persistent(c);
+    c->iso_lanes = pass_lanes(g, cand);
+  }
+}
+
 }  // namespace hmc
 
 extern "C" {
@@ -918,52 +1089,10 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         return HMC_ERR_DEVICE;
       }
     }
-    int coop = 0;
-    // (the FP32 error report runs the per-colour passes)
-    const bool mixed = cfg->precision == HMC_MIXED;
-    if (c->tiled && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) &&
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop) {
-      TileCfg pc{};
-      if (choose_regions(g, D, (double)cfg->n_bodies / (double)spaces, mixed ? sizeof(float4) : sizeof(double4), cus, &pc)) {
-        fill_halo_lists(&pc, D);
-        // Band of the persistent layout, whose LDS entries are the FP64
-        // box-relative positions rounded once to FP32.  Per axis: that
-        // rounding for the site and for the trial site (2^-24 R each, R the
-        // largest box-relative coordinate), the rounding of their FP32
-        // difference (2^-24 |d|), and the FP64 roundings of x - c and of the
-        // image shift on both sides as well as of the reference's own
-        // displacement (2^-53 (4 L + 2 |d|)).
-        double R = 0.0;
-        for (int a = 0; a < D; ++a) R = std::max(R, 0.5 * pc.E[a] * g.width[a] + g.width[a]);
-        const double Et = (0x1p-24 * (2.0 * R + 2.0 * sigma) + 0x1p-53 * (4.0 * lmax + 2.0 * sigma)) * 1.01;
-        // In FP64 the same with 2^-53 for every rounding: x - c, the image
-        // shift and the rounding of the difference on both sides, and the
-        // reference's own displacement.
-        const double E64 = 0x1p-53 * (6.0 * lmax + 4.0 * R + 4.0 * sigma) * 1.01;
-        const void* fn = persist_kernel(c);
-        // one lane per trial, and where the regions leave compute units to
-        // spare, wavefronts that only stage and reload (a small system's box of
-        // 1000 cells staged by one wavefront took 40 us of a 200 us apply)
-        uint32_t threads = ((pc.trials + 63) / 64) * 64;
-        if (pc.xcd_chunk * 8u <= (uint32_t)cus) threads = kTileThreads;
-        int per_cu = 0;
-        if (contact_band(Et, sigma, g.sigma2, g.edge2, D, &pc.band_lo, &pc.band_hi) &&
-            contact_band64(E64, sigma, g.sigma2, g.edge2, D, &pc.band64_lo, &pc.band64_hi) &&
-            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pc.lds_bytes) == hipSuccess &&
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, (int)threads, pc.lds_bytes) == hipSuccess &&
-            (uint64_t)per_cu * (uint64_t)cus >= (uint64_t)pc.xcd_chunk * 8u) {
-          c->persist = true;
-          c->pc = pc;
-          c->pgrid = pc.xcd_chunk * 8u;
-          c->pthreads = threads;
-          c->pper_cu = (uint32_t)per_cu;
-          const size_t fbytes = (size_t)pc.ntiles * kMailboxStride * sizeof(uint32_t);
-          if (hipMalloc((void**)&c->w.mbox, fbytes) != hipSuccess || hipMemset(c->w.mbox, 0, fbytes) != hipSuccess) {
-            delete c;
-            return HMC_ERR_DEVICE;
-          }
-        }
-      }
+    RegionPlan plan;
+    if (plan_hard(c, (double)cfg->n_bodies / (double)spaces, &plan) && !adopt(c, plan)) {
+      delete c;
+      return HMC_ERR_DEVICE;
     }
   }
   // Isotropic pair energies in mixed precision: one persistent launch per
@@ -1015,13 +1144,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
           hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pc.lds_bytes) == hipSuccess &&
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, (int)threads, pc.lds_bytes) == hipSuccess &&
           (uint64_t)per_cu * (uint64_t)cus >= (uint64_t)pc.xcd_chunk * 8u) {
-        c->persist = true;
-        c->pc = pc;
-        c->pgrid = pc.xcd_chunk * 8u;
-        c->pthreads = threads;
-        c->pper_cu = (uint32_t)per_cu;
-        const size_t fbytes = (size_t)pc.ntiles * kMailboxStride * sizeof(uint32_t);
-        if (hipMalloc((void**)&c->w.mbox, fbytes) != hipSuccess || hipMemset(c->w.mbox, 0, fbytes) != hipSuccess) {
+        if (!adopt(c, {pc, threads, (uint32_t)per_cu, 0u})) {
           delete c;
           return HMC_ERR_DEVICE;
         }
@@ -1039,13 +1162,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, persist_kernel(c), kCvApply, 0) == hipSuccess &&
         choose_regions_wave(g, kCvTrials, (uint32_t)per_cu * (uint32_t)cus, &pc)) {
-      c->persist = true;
-      c->pc = pc;
-      c->pgrid = pc.xcd_chunk * 8u;
-      c->pthreads = kCvApply;
-      c->pper_cu = (uint32_t)per_cu;
-      const size_t fbytes = (size_t)pc.ntiles * kMailboxStride * sizeof(uint32_t);
-      if (hipMalloc((void**)&c->w.mbox, fbytes) != hipSuccess || hipMemset(c->w.mbox, 0, fbytes) != hipSuccess) {
+      if (!adopt(c, {pc, kCvApply, (uint32_t)per_cu, 0u})) {
         delete c;
         return HMC_ERR_DEVICE;
       }
@@ -1067,57 +1184,14 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
         hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.total) == hipSuccess)
       c->small_wpt = g.per_colour <= 4 ? 4u : (g.per_colour <= 8 ? 2u : 1u);
   }
-  // Other isotropic pair energies in FP64: lanes per trial, and one persistent
-  // launch per apply (k_apply_iso) where the neighbour scan reaches one space out
-  // and a wavefront per 64 / lanes spaces of a colour is resident.  With more
-  // than 64 candidates per trial 64 lanes share them (442,368 LJ bodies at
-  // density 0.8: 2261 us per step; with 16 lanes 3053, with 8 5553).  With fewer,
-  // 64 lanes while that is at most four wavefronts per compute unit, 16 while
-  // the regions are resident, else 8: overlap penalty, us per step with 64, 16 and
-  // 8 lanes, 6,912 bodies 171, 187, 214; 16,384 206, 195, 221; 55,296 418 (not
-  // resident), 229, 234; 131,072 765, 302 (neither resident), 290.
-  uint32_t pass_lanes = 8;
   if (lj && !lj_mixed && !c->small_wpt && g.n_bodies) {
-    double cand = (double)g.n_bodies / (double)g.n_spaces;
-    bool one = true;
-    for (int a = 0; a < D; ++a) {
-      cand *= 3.0;
-      one = one && g.reach[a] == 1;
+    c->iso_cand = candidates(g, g.n_spaces);
+    RegionPlan plan;
+    if (plan_iso(c, c->iso_cand, &plan) && !adopt(c, plan)) {
+      delete c;
+      return HMC_ERR_DEVICE;
     }
-    const bool many = cand > 64.0;
-    int cus = 0, coop = 0;
-    if (one && !(cfg_in->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS)) &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop) {
-      for (uint32_t lanes : {64u, 16u, 8u}) {
-        int per_cu = 0;
-        TileCfg pc{};
-        if (c->persist || (many && lanes != 64) ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, iso_apply_kernel(lanes, D), 64, 0) != hipSuccess)
-          continue;
-        const uint32_t resident = (uint32_t)(lanes == 64 && !many ? std::min(per_cu, 4) : per_cu) * (uint32_t)cus;
-        if (!choose_regions_wave(g, 64u / lanes, resident, &pc)) continue;
-        c->persist = true;
-        c->iso_lanes = lanes;
-        c->pc = pc;
-        c->pgrid = pc.xcd_chunk * 8u;
-        c->pthreads = 64;
-        c->pper_cu = (uint32_t)per_cu;
-        const size_t fbytes = (size_t)pc.ntiles * kMailboxStride * sizeof(uint32_t);
-        if (hipMalloc((void**)&c->w.mbox, fbytes) != hipSuccess || hipMemset(c->w.mbox, 0, fbytes) != hipSuccess) {
-          delete c;
-          return HMC_ERR_DEVICE;
-        }
-      }
-    }
-    // One launch per colour: 64 lanes too for more than 16 candidates while a
-    // colour's trials are at most twelve wavefronts per compute unit.  us per step
-    // with 64 and 8 lanes: LJ disks at density 0.7 (40 candidates), 10,000 bodies
-    // (1,296 trials a colour) 174 and 254, 40,000 (2,209) 216 and 255, 100,000 (5,625)
-    // 331 and 264, at density 0.16 (9), 10,000 (2,500) 101 and 94; overlap penalty (30),
-    // 9,000 bodies (1,000) 183 and 230, 30,000 (4,096) 266 and 224.
-    pass_lanes = many || (cand > 16.0 && g.per_colour <= 12u * 256u) ? 64u : 8u;
-    if (!c->persist) c->iso_lanes = pass_lanes;
+    if (!c->persist) c->iso_lanes = pass_lanes(g, c->iso_cand);
   }
   const uint32_t N = g.n_bodies;
   c->n_scan_blocks = grid_for(g.n_spaces, kScanBlock);
@@ -1182,7 +1256,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     return HMC_ERR_DEVICE;
   }
   if (c->persist && !persist_probe(c)) c->persist = false;  // the per-colour passes instead
-  if (c->iso_lanes && !c->persist) c->iso_lanes = pass_lanes;
+  if (c->iso_lanes && !c->persist) c->iso_lanes = pass_lanes(g, c->iso_cand);
   *out = c;
   return HMC_OK;
 }
@@ -1215,6 +1289,7 @@ int hmc_set_state(hmc_ctx* c, const double* body_pos, const double* site_pos) {
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->have_state = true;
+  c->fresh = true;
   return HMC_OK;
 }
 
@@ -1361,6 +1436,7 @@ int hmc_clone_with_boundary(hmc_ctx* c, const double* new_edges, hmc_ctx** out) 
     return fail(c, HMC_ERR_INVALID, "a body lies outside the boundary (map_point: PointOutsideShape)");
   }
   d->have_state = true;
+  d->fresh = true;
   *out = d;
   return HMC_OK;
 }
@@ -1391,6 +1467,8 @@ static int apply_one(hmc_ctx* c, uint64_t step, uint32_t substep, uint32_t seed,
   rc = read_state(c, &after);
   if (rc) return rc;
   c->cycles_guess = std::max<uint32_t>(after.cycles, 1);
+  c->fresh = false;
+  replan(c, after);
   uint64_t acc = after.accepted_total - before.accepted_total;
   uint64_t tri = after.trials_total - before.trials_total;
   if (out) {
@@ -1440,7 +1518,7 @@ int hmc_run(hmc_ctx* c, uint64_t step0, uint32_t seed, double kT, const hmc_move
   if (tally) k_tally<<<1, kAccSlots, 0, c->stream>>>(c->st, c->w.acc_slots, (uint32_t)kMaxMoves);
   const bool lj = is_isotropic(c->g.model);
   // (a persistent launch carries its own tag: not captured, launched directly)
-  const bool graphs = !(c->cfg.flags & HMC_FLAG_NO_GRAPH) && !c->persist;
+  bool graphs = !(c->cfg.flags & HMC_FLAG_NO_GRAPH) && !c->persist;
   // one step: apply each move in order (the step's substeps follow on), then
   // Microstate::increment_step before the next step
   auto step_launches = [&](bool first) -> int {
@@ -1458,6 +1536,15 @@ int hmc_run(hmc_ctx* c, uint64_t step0, uint32_t seed, double kT, const hmc_move
     if (i == 0 || !graphs || timed) {
       rc = step_launches(i == 0);
       if (rc) return rc;
+      if (c->fresh && ((c->persist && hard_shape(c->g.model)) || c->iso_lanes) && n_steps > 1) {
+        ApplyState first;  // (a new state's first apply says whether the plan fits it)
+        rc = read_state(c, &first);
+        if (rc) return rc;
+        c->cycles_guess = std::max<uint32_t>(first.cycles, 1);
+        replan(c, first);
+        graphs = !(c->cfg.flags & HMC_FLAG_NO_GRAPH) && !c->persist;
+      }
+      c->fresh = false;
       continue;
     }
     // later steps: replay one captured step
@@ -1486,7 +1573,10 @@ int hmc_run(hmc_ctx* c, uint64_t step0, uint32_t seed, double kT, const hmc_move
   ApplyState after;
   rc = read_state(c, &after);
   if (rc) return rc;
-  if (n_steps) c->cycles_guess = std::max<uint32_t>(after.cycles, 1);
+  if (n_steps) {
+    c->cycles_guess = std::max<uint32_t>(after.cycles, 1);
+    replan(c, after);
+  }
   if (out) {
     if (tally) {
       for (uint32_t m = 0; m < n_moves; ++m) {

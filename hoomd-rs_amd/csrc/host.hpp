@@ -33,6 +33,12 @@ class Readback {
 
 using namespace hmc;
 
+// The regions of a context's persistent apply and their launch.
+struct RegionPlan {
+  TileCfg pc{};
+  uint32_t threads = 0, per_cu = 0, lanes = 0;  // per region, resident regions per CU, lanes per trial (k_apply_iso)
+};
+
 struct hmc_ctx {
   hmc_config cfg;
   hmc_config cfg_user;              // as given to hmc_create (vertices -> verts_host)
@@ -56,6 +62,10 @@ struct hmc_ctx {
   uint32_t pgrid = 0, pthreads = 0, pper_cu = 0;
   double* verts = nullptr;  // convex polyhedron vertices (device)
   uint32_t iso_lanes = 0;   // isotropic FP64 beyond small_wpt: lanes per trial (k_pass_iso, k_apply_iso)
+  double iso_cand = 0.0;    // the candidates per trial that they are planned for
+  double occ_tried = 0.0;   // persistent hard shapes: bodies per space up to which regions were sought
+  bool fresh = true;        // no apply has run on this state
+  uint64_t over_seen = 0, applies_seen = 0;  // overflowing boxes and applies when last planned (replan)
   SatShape sat{};           // convex, mixed precision: the FP32 separating axes (else use = 0)
   Geometry* gdev = nullptr;  // device copy of g (g.self)
   uint32_t n_scan_blocks = 0;

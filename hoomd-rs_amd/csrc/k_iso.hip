@@ -62,6 +62,7 @@ __device__ __forceinline__ void iso_trials(const Geometry& g, ApplyState* st, co
       body = C.body[slot];
     }
   }
+  if (!DEV && G == 64 && !tried) return;  // (uniform; half of 50,000 LJ bodies' time where 63 of 64 spaces are empty)
   double4 bp = make_double4(0.0, 0.0, 0.0, 0.0), sp = bp;
   double v[3] = {0.0, 0.0, 0.0};
   TrialSite<D> ts{};

@@ -288,7 +288,9 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
 
   if (tid == 0) blk_acc = odd = 0;
   if (tid < (uint32_t)kHaloLists) hcnt[tid] = 0;
-  const bool overflow = region_stage<D, S, kTilePad>(g, tc, rg, B, C, w, l, &odd);
+  const uint32_t beyond = region_stage<D, S, kTilePad>(g, tc, rg, B, C, w, l, &odd);
+  const bool overflow = beyond != 0;
+  if (tid == 0 && overflow) atomicMax(&st->box_most, beyond);
 
   unsigned retests = 0;
   // the proposal of this thread's trial

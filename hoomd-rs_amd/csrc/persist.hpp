@@ -494,10 +494,10 @@ __device__ __forceinline__ RegionLds<S> region_lds(unsigned char* smem, const Ti
 // starts, then the sites (their FP64 copies as box-relative FP32 entries with
 // the body index).  A thread per row loads its runs, wave 0 scans the row
 // lengths, and a half-wave per row copies its cell starts and its runs,
-// kStageRows rows in flight together.  Ends with a barrier; returns true
-// (uniform over the workgroup) when the box holds more sites than the LDS
-// capacity tc.maxb, in which case no entries were written.  PAD entries out of
-// reach follow the box's.  *odd (zeroed before) is set when a staged site has
+// kStageRows rows in flight together.  Ends with a barrier; returns the number of
+// sites (uniform over the workgroup) when it exceeds the LDS capacity tc.maxb, in
+// which case no entries were written, else 0.  PAD entries out of reach follow the
+// box's.  *odd (zeroed before) is set when a staged site has
 // no images, i.e. its entry is NaN.
 //
 // Written for few instructions: every launch fetches its code anew, a cache
@@ -506,7 +506,7 @@ __device__ __forceinline__ RegionLds<S> region_lds(unsigned char* smem, const Ti
 // loops and the image selection in branches, the part of the kernel before
 // the first trial took 50 us of C2's 280 us apply.)
 template <int D, class S, int PAD>
-__device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& tc, const Region& rg, const Bodies& B,
+__device__ __forceinline__ uint32_t region_stage(const Geometry& g, const TileCfg& tc, const Region& rg, const Bodies& B,
                                              const Cells& C, const Work& w, const RegionLds<S>& l, uint32_t* odd) {
   constexpr int AL = D - 1;
   const uint32_t R = tc.rows, EL = tc.E[AL], CW = EL + 1;
@@ -605,7 +605,7 @@ __device__ __forceinline__ bool region_stage(const Geometry& g, const TileCfg& t
     }
   }
   __syncthreads();
-  return overflow;
+  return overflow ? total : 0u;
 }
 
 // The halo cells of the box by the pass class (pass mod 2^D) that first reads

@@ -140,7 +140,7 @@ struct ApplyState {
   unsigned long long move_trials[kMaxMoves];
   unsigned long long tally_acc, tally_trials;
   uint32_t wait_at;  // the first neighbour wait that timed out: (region << 12) | (pass + 1)
-  uint32_t pad2;
+  uint32_t box_most; // persistent hard shapes: the most sites a box beyond its LDS capacity held
 };
 
 // What an apply is asked for (k_setup's arguments).

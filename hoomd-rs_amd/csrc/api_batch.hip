@@ -458,6 +458,7 @@ int hmc_batch_create(uint32_t n_replicas, const hmc_config* cfgs, hmc_batch** ou
   b->precision = cfgs[0].precision;
   b->hreps.resize(n_replicas);
   b->boff.assign(n_replicas + 1, 0);
+  b->apart.assign(n_replicas, false);
   b->coff.assign(n_replicas + 1, 0);
   uint64_t nb = 0, ns = 0, npc = 0;
   for (uint32_t r = 0; r < n_replicas; ++r) {
@@ -587,10 +588,15 @@ int hmc_batch_set_state(hmc_batch* b, uint32_t replica, const double* body_pos, 
     BHIPCHK(b, hipGetLastError());
   }
   BHIPCHK(b, hipStreamSynchronize(b->stream));
-  if (b->persist) {
+  b->apart[replica] = site_pos && sites_apart(g, body_pos, site_pos, N);
+  if (b->persist || b->parked) {
     if (b->box_max.size() != b->R) b->box_max.assign(b->R, std::array<uint32_t, 7>{});
     b->box_max[replica] = box_counts(g, body_pos, N);
     b->regions_stale = true;
+    // (the persistent applies take sites to lie in their bodies' spaces)
+    b->parked = std::find(b->apart.begin(), b->apart.end(), true) != b->apart.end();
+    b->persist = !b->parked;
+    if (b->parked) forget_resident(b->device, b->stream);
   }
   return HMC_OK;
 }
@@ -669,7 +675,7 @@ int hmc_batch_sdf(hmc_batch* b, double xmax, double dx, uint32_t nbins, uint64_t
   uint32_t stot = 0;
   for (uint32_t r = 0; r < b->R; ++r) {
     hr[r] = b->hreps[r];
-    hr[r].g = sdf_geometry(b->hreps[r].g, xmax);
+    hr[r].g = sdf_geometry(b->hreps[r].g, xmax, b->apart[r]);
     hr[r].space_off = stot;
     stot += hr[r].g.n_spaces;
   }

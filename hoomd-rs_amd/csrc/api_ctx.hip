@@ -831,9 +831,22 @@ int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_
     return HMC_ERR_UNSUPPORTED;
   }
 
+  g.row_cut2 = row_cut2(sigma, false);
   *sigma_out = sigma;
   *lmax_out = lmax;
   return HMC_OK;
+}
+
+bool sites_apart(const Geometry& g, const double* body, const double* site, uint32_t n) {
+  for (uint32_t i = 0; i < n; ++i)
+    for (int a = 0; a < g.dim; ++a) {
+      const double tol = 0x1p-50 * g.L[a];
+      double d = site[(size_t)i * g.dim + a] - body[(size_t)i * g.dim + a];
+      if (std::fabs(d) <= tol) continue;
+      d -= g.L[a] * std::rint(d / g.L[a]);
+      if (!(std::fabs(d) <= tol)) return true;
+    }
+  return false;
 }
 
 // One persistent launch per apply for hard shapes (k_apply_tile), its regions for
@@ -967,6 +980,24 @@ static void leave_persistent(hmc_ctx* c) {
   forget_resident(c->device, c->stream);
 }
 
+// For a state whose sites lie away from their bodies: no neighbour row is left out
+// for its distance, and the applies that stage boxes of sites (k_apply_tile,
+// k_apply_lj), which take a site to lie in its body's space, give way to one
+// launch per colour.  (An accepted move puts a body's site back.)
+static void set_apart(hmc_ctx* c, bool apart) {
+  if (apart == c->apart) return;
+  c->apart = apart;
+  drop_graph(c);  // (it holds the geometry)
+  c->g.row_cut2 = row_cut2(c->range, apart);
+  if (apart && c->persist && !c->iso_lanes && c->g.model != HMC_CONVEX_POLYHEDRON) {
+    leave_persistent(c);
+    c->parked = true;
+  } else if (!apart && c->parked) {
+    c->persist = true;
+    c->parked = false;
+  }
+}
+
 // Plans made at creation take the bodies to fill the box.  Where a state says
 // otherwise -- a drop or a slab beside vapour or nothing -- its applies take the
 // plan that fits it, from the state s that the last apply left (the stream idle):
@@ -1043,6 +1074,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
   c->cfg_user.vertices = nullptr;
   c->device = cfg->device;
   c->g = g0;
+  c->range = sigma;
   c->g.lj_mixed = lj_mixed ? 1 : 0;
   c->g.cv_mixed = cv_mixed ? 1 : 0;
   if (cv_mixed) sat_build(cfg_in->vertices, cfg_in->n_vertices, &c->sat);
@@ -1290,6 +1322,7 @@ int hmc_set_state(hmc_ctx* c, const double* body_pos, const double* site_pos) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->have_state = true;
   c->fresh = true;
+  set_apart(c, site_pos && sites_apart(c->g, body_pos, site_pos, N));
   return HMC_OK;
 }
 

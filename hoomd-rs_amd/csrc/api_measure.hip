@@ -22,9 +22,10 @@ const char* sdf_check(const Geometry& g, double xmax, double dx, uint32_t nbins)
 // The SDF's own cells: the checkerboard with spaces at least r_max (1 + 2^-29)
 // wide (never more spaces than the sweep's, whose buffers it reuses), so
 // that one neighbour space on each side covers r_max.
-Geometry sdf_geometry(const Geometry& g, double xmax) {
+Geometry sdf_geometry(const Geometry& g, double xmax, bool apart) {
   Geometry s = g;
   const double rmax = g.sigma / (1.0 - xmax);
+  s.row_cut2 = row_cut2(rmax, apart);
   uint64_t spaces = 1;
   for (int a = 0; a < g.dim; ++a) {
     int64_t k = (int64_t)std::floor(g.L[a] / (rmax * (1.0 + 0x1p-29)));
@@ -158,7 +159,7 @@ int hmc_sdf(hmc_ctx* c, double xmax, double dx, uint32_t nbins, uint64_t* hist, 
   if (!c->have_state) return fail(c, HMC_ERR_STATE, "hmc_set_state was not called");
   if (const char* why = sdf_check(c->g, xmax, dx, nbins))
     return fail(c, c->g.model != HMC_HARD_SPHERE ? HMC_ERR_UNSUPPORTED : HMC_ERR_INVALID, why);
-  const Geometry g = sdf_geometry(c->g, xmax);
+  const Geometry g = sdf_geometry(c->g, xmax, c->apart);
   const uint32_t nsb = grid_for(g.n_spaces, kScanBlock);
   const uint32_t N = g.n_bodies;
   HIPCHK(c, hipSetDevice(c->device));

@@ -65,6 +65,9 @@ struct hmc_ctx {
   double iso_cand = 0.0;    // the candidates per trial that they are planned for
   double occ_tried = 0.0;   // persistent hard shapes: bodies per space up to which regions were sought
   bool fresh = true;        // no apply has run on this state
+  double range = 0.0;       // the interaction range
+  bool apart = false;       // sites_apart of the state
+  bool parked = false;      // a persistent plan waits for sites that lie in their bodies' spaces
   uint64_t over_seen = 0, applies_seen = 0;  // overflowing boxes and applies when last planned (replan)
   SatShape sat{};           // convex, mixed precision: the FP32 separating axes (else use = 0)
   Geometry* gdev = nullptr;  // device copy of g (g.self)
@@ -132,6 +135,8 @@ struct hmc_batch {
   uint32_t* drt0 = nullptr;                     // the rounds' first regions and sizes (device)
   uint32_t* drn = nullptr;
   uint32_t nwg = 0;                             // workgroups of the launch: the largest round
+  std::vector<bool> apart;                      // sites_apart of the replicas
+  bool parked = false;                          // persistent but for such replicas
   uint32_t sync_tag = 0;                        // persistent launches so far (their progress words' tag)
   uint32_t pper_cu = 0, pregions = 0;           // resident regions per CU; all regions
   std::vector<TileCfg> hptcs;                   // the replicas' region shapes (host copy)
@@ -195,8 +200,15 @@ void fill_halo_lists(TileCfg* tc, int D);
 bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus, TileCfg* out);
 bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* out);
 int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_out, double* lmax_out);
+// Whether some given site lies away from its body (by more than the roundings of a
+// wrap, over the periodic box), so that it may lie in another space.
+bool sites_apart(const Geometry& g, const double* body, const double* site, uint32_t n);
+// row_cut2 for a range r, or none.
+inline float row_cut2(double r, bool apart) {
+  return apart ? std::numeric_limits<float>::infinity() : (float)(r * r) * (1.0f + 1e-4f);
+}
 const char* sdf_check(const Geometry& g, double xmax, double dx, uint32_t nbins);
-Geometry sdf_geometry(const Geometry& g, double xmax);
+Geometry sdf_geometry(const Geometry& g, double xmax, bool apart);
 int total_energy_into(hmc_ctx* c, double* part, double* energy, double* bound);
 // Cell lists of the current state on c's stream (checkerboard spaces at
 // origin 0, bodies of each space in body order: w.start, w.tmp_body).

@@ -463,7 +463,7 @@ __device__ __forceinline__ void cv_trials(const Geometry& g, ApplyState* st, con
   // (a trial outside its space is rejected without pair tests)
   float flo[3], fhi[3];
   face_gaps2<3>(gp, origin, own, ts.t, flo, fhi);
-  const uint32_t tot = nbr.list(g, m, kl, active, (float)g.cv_rcut2 * (1.0f + 1e-4f), flo, fhi, W.row[k]);
+  const uint32_t tot = nbr.list(g, m, kl, active, g.row_cut2, flo, fhi, W.row[k]);
   uint32_t base[kCvTrials + 1];
   base[0] = 0;
 #pragma unroll

@@ -85,7 +85,7 @@ __device__ __forceinline__ void iso_trials(const Geometry& g, ApplyState* st, co
     flo[a] = fminf(flo[a], glo[a]);
     fhi[a] = fminf(fhi[a], ghi[a]);
   }
-  const uint32_t tot = nbr.list(g, m, kl, active, (float)g.lj_rc2 * (1.0f + 1e-4f), flo, fhi, W.row[k]);
+  const uint32_t tot = nbr.list(g, m, kl, active, g.row_cut2, flo, fhi, W.row[k]);
   wave_lds_order();
   ready();
   double ef = 0.0, ei = 0.0, mag = 0.0;

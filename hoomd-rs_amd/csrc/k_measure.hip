@@ -286,9 +286,8 @@ __device__ __forceinline__ uint32_t sdf_bin(const Geometry& g, const double* ori
     if (q != p) best = fmin(best, r2);
   };
   if (plain) {
-    // squared distances to the faces of the space; a margin of 10^-4 on the
-    // square of r_max covers their roundings
-    const float cut = (float)(rmax * rmax) * (1.0f + 1e-4f);
+    // squared distances to the faces of the space
+    const float cut = g.row_cut2;
     float flo[3], fhi[3];
 #pragma unroll
     for (int a = 0; a < D; ++a)

@@ -82,6 +82,10 @@ struct Geometry {
   const Geometry* self;
   // correctly rounded 1 / L and 1 / width for div_const_fast (0: divide)
   double inv_L[3], inv_width[3];
+  // squared cutoff (a margin of 10^-4 for the FP32 distances to a space's faces)
+  // beyond which neighbour rows are left out; infinite where a site need not lie in
+  // its body's space (sites_apart)
+  float row_cut2;
 };
 
 // Mixed-precision hard convex polyhedra: the polytope's separating axes in

@@ -162,7 +162,11 @@ int hmc_create(const hmc_config* cfg, hmc_ctx** out);
 /* Upload body positions (the microstate's wrapped body properties, body index
  * order).  site_pos may be NULL: sites are then wrap(body + 0) as
  * Microstate::add_body / update_body_properties set them
- * (hoomd-microstate/src/microstate.rs:777-835, 985-1034). */
+ * (hoomd-microstate/src/microstate.rs:777-835, 985-1034).  Given sites need not
+ * be those: a trial's neighbours are then the sites of the bodies in the spaces
+ * around its own, wherever the sites are, and until the next state is set no
+ * such space is left out for its distance and hard shapes and mixed-precision LJ
+ * take one launch per colour pass. */
 int hmc_set_state(hmc_ctx* ctx, const double* body_pos, const double* site_pos);
 
 /* Download body and site positions in body index order (site_pos may be NULL). */

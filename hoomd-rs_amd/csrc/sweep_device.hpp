@@ -777,10 +777,11 @@ __device__ __forceinline__ int lj_metropolis(Sfc64& rng, double dH, double delta
   // The hardware's FP32 exp2 of FP32 quotients first, where they are moderate:
   // q = -dH / kT to 2^-21 of |q| < 80, so exp(q) to 4e-5 and the hardware's ulp,
   // decided with a margin of 2^-14 = 6.1e-5.  (Division and exp in FP64 are
-  // most of a decision otherwise.)
+  // most of a decision otherwise.)  Not for a kT whose reciprocal leaves FP32's
+  // normal range (the hardware's is 0 there, and every trial would be accepted).
   const float ik = __builtin_amdgcn_rcpf((float)kT) * 1.44269504f;
   const float eh = -(float)hi * ik, el = -(float)lo * ik;
-  if (eh > -115.0f) {
+  if (eh > -115.0f && ik > 0x1p-120f) {
     if (u < (double)__builtin_amdgcn_exp2f(eh) * (1.0 - 0x1p-14)) return 1;
     if (lo > 0.0 && u >= (double)__builtin_amdgcn_exp2f(el) * (1.0 + 0x1p-14)) return 0;
   }

@@ -213,6 +213,8 @@ bool batch_regions(hmc_batch* b, int cus) {
   const uint32_t R = b->R;
   b->pcus = cus;
   b->regions_stale = false;
+  for (const BatchRep& r : b->hreps)
+    if (!fits_fp32(r.g.sigma)) return false;
   if (hipStreamSynchronize(b->stream) != hipSuccess) return false;
   for (void** p : {(void**)&b->dptcs, (void**)&b->dptoff, (void**)&b->dptrep, (void**)&b->w.mbox, (void**)&b->drt0,
                    (void**)&b->drn})

@@ -856,7 +856,7 @@ static bool plan_hard(const hmc_ctx* c, double occ, RegionPlan* out) {
   const int D = g.dim;
   int cus = 0, coop = 0;
   // (the FP32 error report runs the per-colour passes)
-  if (!c->tiled || (c->cfg.flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) ||
+  if (!c->tiled || !fits_fp32(g.sigma) || (c->cfg.flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0 ||
       hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop)
     return false;
@@ -1048,8 +1048,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
   // LJ in mixed precision keeps the FP64 data layout and passes; only its
   // pair energies run in FP32 (Geometry::lj_mixed)
   hmc_config cfg_local = *cfg_in;
-  const bool lj_mixed = (cfg_in->model == HMC_LJ || cfg_in->model == HMC_LJ_SHIFTED) &&
-                        cfg_in->precision == HMC_MIXED;
+  bool lj_mixed = (cfg_in->model == HMC_LJ || cfg_in->model == HMC_LJ_SHIFTED) && cfg_in->precision == HMC_MIXED;
   if (lj_mixed) cfg_local.precision = HMC_FP64;
   // so do convex polyhedra: their listed pairs go through FP32 separating
   // axes first (Geometry::cv_mixed)
@@ -1063,6 +1062,8 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     const int rc = make_geometry(cfg, g0, &fast0, &sigma, &lmax);
     if (rc) return rc;
   }
+  // (at scales that FP32 does not hold the FP64 forms decide the same)
+  if (!fits_fp32(sigma) && !(cfg_in->flags & HMC_FLAG_FP32_ERROR)) lj_mixed = false;
   const int D = (int)cfg->dim;
   const bool lj = is_isotropic(cfg->model);
   const bool convex = cfg->model == HMC_CONVEX_POLYHEDRON;

@@ -203,9 +203,12 @@ int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_
 // Whether some given site lies away from its body (by more than the roundings of a
 // wrap, over the periodic box), so that it may lie in another space.
 bool sites_apart(const Geometry& g, const double* body, const double* site, uint32_t n);
+// Ranges whose squares, and those of the distances in a region's box, FP32 holds
+// with room on both sides (in a box of 66 spaces and beside kTileFar).
+inline bool fits_fp32(double range) { return range >= 0x1p-40 && range <= 0x1p40; }
 // row_cut2 for a range r, or none.
 inline float row_cut2(double r, bool apart) {
-  return apart ? std::numeric_limits<float>::infinity() : (float)(r * r) * (1.0f + 1e-4f);
+  return apart || !fits_fp32(r) ? std::numeric_limits<float>::infinity() : (float)(r * r) * (1.0f + 1e-4f);
 }
 const char* sdf_check(const Geometry& g, double xmax, double dx, uint32_t nbins);
 Geometry sdf_geometry(const Geometry& g, double xmax, bool apart);

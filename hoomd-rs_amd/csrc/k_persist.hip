@@ -194,7 +194,7 @@ __device__ __forceinline__ bool tile_overlaps(const Geometry& g, const TileCfg& 
     const Ent<S>* p[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) p[r] = lb + (key[r] & 0xffffu);
-    S near2 = (S)kTileFar;
+    S near2 = (S)__builtin_inf();
     auto slots = [&](int r0, uint32_t k) {
       const Ent<S> a = p[r0][k], b = p[r0 + 1][k], c = p[r0 + 2][k];
       near2 = fmin(near2, tile_dist2<D, S>(a, tr));

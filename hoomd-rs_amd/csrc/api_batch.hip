@@ -615,7 +615,8 @@ int hmc_batch_run_translate(hmc_batch* b, const uint64_t* step0, const uint32_t*
                             const double* max_distance, uint32_t n_steps, int use_graph, hmc_count* out) {
   if (!b || !step0 || !seeds || !max_distance || !(kT > 0.0)) return HMC_ERR_INVALID;
   for (uint32_t r = 0; r < b->R; ++r)
-    if (!(max_distance[r] > 0.0)) return bfail(b, HMC_ERR_INVALID, "max_distance must be > 0");
+    if (!(max_distance[r] > 0.0) || !draws_end(b->dim, max_distance[r]))
+      return bfail(b, HMC_ERR_INVALID, "max_distance must be > 0 (in 2D its square too, and finite)");
   BHIPCHK(b, hipSetDevice(b->device));
   b->kT = kT;
   BHIPCHK(b, hipMemcpyAsync(b->dstep, step0, b->R * sizeof(uint64_t), hipMemcpyHostToDevice, b->stream));
@@ -732,7 +733,8 @@ int hmc_batch_autotune(hmc_batch* b, const uint64_t* step0, const uint32_t* seed
                        const double* max_distance, uint32_t n_steps, double* best_ms, uint32_t* best_policy) {
   if (!b || !step0 || !seeds || !max_distance || !(kT > 0.0) || n_steps == 0) return HMC_ERR_INVALID;
   for (uint32_t r = 0; r < b->R; ++r)
-    if (!(max_distance[r] > 0.0)) return bfail(b, HMC_ERR_INVALID, "max_distance must be > 0");
+    if (!(max_distance[r] > 0.0) || !draws_end(b->dim, max_distance[r]))
+      return bfail(b, HMC_ERR_INVALID, "max_distance must be > 0 (in 2D its square too, and finite)");
   if (!b->tiled) return bfail(b, HMC_ERR_UNSUPPORTED, "the batch does not run on LDS tiles");
   BHIPCHK(b, hipSetDevice(b->device));
   hipStream_t s = b->stream;

@@ -1489,6 +1489,7 @@ static int apply_one(hmc_ctx* c, uint64_t step, uint32_t substep, uint32_t seed,
   if (!c) return HMC_ERR_INVALID;
   if (!c->have_state) return fail(c, HMC_ERR_STATE, "hmc_set_state was not called");
   if (!(max_move > 0.0) || !(kT > 0.0)) return fail(c, HMC_ERR_INVALID, "the move size and kT must be > 0");
+  if (!draws_end(c->g.dim, max_move)) return fail(c, HMC_ERR_INVALID, "a disk's move size must have a positive, finite square");
   if (move == 1 && c->g.model != HMC_CONVEX_POLYHEDRON)
     return fail(c, HMC_ERR_UNSUPPORTED, "rotation moves need oriented bodies");
   HIPCHK(c, hipSetDevice(c->device));
@@ -1541,6 +1542,7 @@ int hmc_run(hmc_ctx* c, uint64_t step0, uint32_t seed, double kT, const hmc_move
     if (moves[m].move != HMC_MOVE_TRANSLATE && moves[m].move != HMC_MOVE_ROTATE)
       return fail(c, HMC_ERR_INVALID, "hmc_run: unknown move");
     if (!(moves[m].size > 0.0)) return fail(c, HMC_ERR_INVALID, "the move sizes must be > 0");
+    if (!draws_end(c->g.dim, moves[m].size)) return fail(c, HMC_ERR_INVALID, "a disk's move size must have a positive, finite square");
     if (moves[m].move == HMC_MOVE_ROTATE && c->g.model != HMC_CONVEX_POLYHEDRON)
       return fail(c, HMC_ERR_UNSUPPORTED, "rotation moves need oriented bodies");
   }

@@ -434,7 +434,8 @@ int hmc_tune_local(hmc_ctx* c, uint32_t move, uint64_t step, uint32_t substep, u
   uint64_t amb = 0;
   for (uint32_t t = 0; t < steps && !rc; ++t) {
     uint64_t acc = 0, rej = 0, a = 0, p = 0;
-    for (;;) {
+    if (!draws_end(D, *maximum_distance)) rc = fail(c, HMC_ERR_INVALID, "tune: a disk's move size must have a positive, finite square");
+    while (!rc) {
       if (M > 0x7fffffffull) {
         rc = fail(c, HMC_ERR_DEVICE, "tune: the sample chain outgrew its stream");
         break;

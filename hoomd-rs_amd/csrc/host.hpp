@@ -200,6 +200,9 @@ void fill_halo_lists(TileCfg* tc, int D);
 bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus, TileCfg* out);
 bool choose_regions_lj(const Geometry& g, int D, double occ, int cus, TileCfg* out);
 int make_geometry(const hmc_config* cfg, Geometry& g, bool* fast, double* sigma_out, double* lmax_out);
+// Whether the draws of a displacement within r end: a disk's are points of a square
+// until one lies within r^2 (ball_sample), which none does where that is 0 or infinite.
+inline bool draws_end(int dim, double r) { return dim != 2 || (r * r > 0.0 && std::isfinite(r * r)); }
 // Whether some given site lies away from its body (by more than the roundings of a
 // wrap, over the periodic box), so that it may lie in another space.
 bool sites_apart(const Geometry& g, const double* body, const double* site, uint32_t n);

@@ -7,6 +7,14 @@
 namespace {
 bool batch_regions(hmc_batch* b, int cus);
 
+// Regions of a persistent launch for the batch's states, or none: its steps are then
+// captured in graphs, and the device's order of persistent launches must not name
+// its stream (a probe's, or earlier steps').
+void choose_batch_regions(hmc_batch* b, int cus) {
+  b->persist = batch_regions(b, cus);
+  if (!b->persist) forget_resident(b->device, b->stream);
+}
+
 int bfail(hmc_batch* b, int code, const std::string& msg) {
   if (b) b->err = msg;
   return code;
@@ -73,7 +81,7 @@ void launch_batch_step(hmc_batch* b, int from_args, int advance, uint32_t launch
 void batch_step(hmc_batch* b, int from_args, int advance, uint32_t launched) {
   // regions sized for the states set since the last choice (never under
   // graph capture: persistent steps are not captured)
-  if (b->persist && b->regions_stale) b->persist = batch_regions(b, b->pcus);
+  if (b->persist && b->regions_stale) choose_batch_regions(b, b->pcus);
   if (b->dim == 2 && b->precision == HMC_FP64)
     launch_batch_step<2, HMC_FP64>(b, from_args, advance, launched);
   else if (b->dim == 2)
@@ -554,7 +562,7 @@ int hmc_batch_create(uint32_t n_replicas, const hmc_config* cfgs, hmc_batch** ou
     if (b->tiled && b->dim == 3 && b->precision == HMC_MIXED && !(cfgs[0].flags & HMC_FLAG_PER_COLOUR) &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) == hipSuccess && cus > 0 &&
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, b->device) == hipSuccess && coop)
-      b->persist = batch_regions(b, cus);
+      choose_batch_regions(b, cus);
   }
   *out = b;
   return HMC_OK;

@@ -974,7 +974,8 @@ static bool adopt(hmc_ctx* c, const RegionPlan& plan) {
   return true;
 }
 
-// One launch per colour from the next apply on (the stream idle).
+// One launch per colour from the next apply on (the stream idle, and out of the
+// device's order of persistent launches: its steps may be captured in graphs).
 static void leave_persistent(hmc_ctx* c) {
   c->persist = false;
   forget_resident(c->device, c->stream);
@@ -1288,7 +1289,7 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
     hmc_destroy(c);
     return HMC_ERR_DEVICE;
   }
-  if (c->persist && !persist_probe(c)) c->persist = false;  // the per-colour passes instead
+  if (c->persist && !persist_probe(c)) leave_persistent(c);  // the per-colour passes instead
   if (c->iso_lanes && !c->persist) c->iso_lanes = pass_lanes(g, c->iso_cand);
   *out = c;
   return HMC_OK;
@@ -1803,6 +1804,8 @@ int hmc_debug_form(const hmc_ctx* c, uint32_t* out) {
   out[3] = c->persist && c->w.bucket ? 1u : 0u;
   return HMC_OK;
 }
+
+int hmc_debug_order(int device) { return resident_order(device) ? 1 : 0; }
 
 int hmc_profile_enable(hmc_ctx* c, int on) {
   if (!c) return HMC_ERR_INVALID;

@@ -181,11 +181,13 @@ inline SdfGrid sdf_grid(uint32_t n) {
 
 inline uint32_t grid_for(uint64_t n, uint32_t block) { return (uint32_t)((n + block - 1) / block); }
 
-// A persistent apply's launch (resident.hip), and what precedes the end of a stream
-// that such launches used, its work complete.
+// A persistent apply's launch (resident.hip).  forget_resident: before a stream that
+// such launches used ends or captures, its work complete.  resident_order: whether
+// the device's order names a stream.
 hipError_t launch_resident(int device, const void* fn, uint32_t blocks, uint32_t threads, void** args, size_t lds,
                            hipStream_t s);
 void forget_resident(int device, hipStream_t s);
+bool resident_order(int device);
 hipEvent_t take_event(hmc_ctx* c);
 int dispatch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t substep, uint32_t seed,
                    double kT, double max_move, uint32_t move);

@@ -53,4 +53,10 @@ void forget_resident(int device, hipStream_t s) {
   gates().erase(it);
 }
 
+bool resident_order(int device) {
+  std::lock_guard<std::mutex> lock(gates_use);
+  auto it = gates().find(device);
+  return it != gates().end() && it->second.last;
+}
+
 }  // namespace hmc

@@ -421,6 +421,10 @@ int hmc_debug_regions(hmc_ctx* ctx, uint32_t* out, uint64_t cap, uint64_t* n);
  * of persistent hard shapes. */
 int hmc_debug_form(const hmc_ctx* ctx, uint32_t* out);
 
+/* Test hook: 1 when the device's order of persistent launches (each waits, on the
+ * device, for the work of the last one's stream) names a stream, else 0. */
+int hmc_debug_order(int device);
+
 /* Evaluate the library's device math on n inputs: kind 0 cbrt, 1 log,
  * 2 exp, 5 the sine and 6 the cosine of one sincos call (the device's
  * restatements of the glibc functions Rust's std calls on Linux), 3 sqrt,

@@ -213,7 +213,7 @@ bool sites_apart(const Geometry& g, const double* body, const double* site, uint
 inline bool fits_fp32(double range) { return range >= 0x1p-40 && range <= 0x1p40; }
 // row_cut2 for a range r, or none.
 inline float row_cut2(double r, bool apart) {
-  return apart || !fits_fp32(r) ? std::numeric_limits<float>::infinity() : (float)(r * r) * (1.0f + 1e-4f);
+  return apart || !fits_fp32(r) ? std::numeric_limits<float>::quiet_NaN() : (float)(r * r) * (1.0f + 1e-4f);
 }
 const char* sdf_check(const Geometry& g, double xmax, double dx, uint32_t nbins);
 Geometry sdf_geometry(const Geometry& g, double xmax, bool apart);

@@ -309,10 +309,10 @@ __device__ __forceinline__ uint32_t sdf_bin(const Geometry& g, const double* ori
         y1 = y1 < 0 ? y1 + g.shape[1] : y1 == g.shape[1] ? 0 : y1;
         sb += (uint32_t)y1 * g.stride[1];
       }
-      const bool lower = d + flo[AL] < cut, upper = d + fhi[AL] < cut;
+      const bool lower = !(d + flo[AL] >= cut), upper = !(d + fhi[AL] >= cut);
       const uint32_t ca = sb + (uint32_t)ml - (lower && !wlo ? 1u : 0u), cz = sb + (uint32_t)ml + (upper && !whi ? 2u : 1u);
       lo[k] = hi[k] = 0;
-      if (d < cut) {
+      if (!(d >= cut)) {
         lo[k] = w.start[ca];
         hi[k] = w.start[cz];
         if ((wlo && lower) || (whi && upper)) {  // across the face

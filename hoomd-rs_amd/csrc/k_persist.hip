@@ -290,7 +290,6 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
   if (tid < (uint32_t)kHaloLists) hcnt[tid] = 0;
   const uint32_t beyond = region_stage<D, S, kTilePad>(g, tc, rg, B, C, w, l, &odd);
   const bool overflow = beyond != 0;
-  if (tid == 0 && overflow) atomicMax(&st->box_most, beyond);
 
   unsigned retests = 0;
   // the proposal of this thread's trial
@@ -409,7 +408,10 @@ __device__ __forceinline__ void apply_tile_run(const Geometry& g, ApplyState* st
     if (__lane_id() == 0 && mk) atomicAdd(&blk_acc, (unsigned)__popcll(mk));
   }
   lane_add(&st->band_retests, retests);
-  if (tid == 0 && overflow) atomicAdd(&st->tile_overflows, 1ull);
+  if (tid == 0 && overflow) {
+    atomicAdd(&st->tile_overflows, 1ull);
+    atomicMax(&st->box_most, beyond);
+  }
   __syncthreads();
   if (tid == 0 && blk_acc) atomicAdd(acc, (unsigned long long)blk_acc);
 }

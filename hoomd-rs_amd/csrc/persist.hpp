@@ -288,12 +288,12 @@ struct NeighbourRows {
         const uint32_t i0 = (j * inv1) >> 8, i1 = j - i0 * nn1;
         float d = i0 == 0 ? flo[0] : i0 == 2 ? fhi[0] : 0.0f;
         if constexpr (D == 3) d += i1 == 0 ? flo[1] : i1 == 2 ? fhi[1] : 0.0f;
-        const bool lo = d + flo[AL] < cut2, hi = d + fhi[AL] < cut2;
+        const bool lo = !(d + flo[AL] >= cut2), hi = !(d + fhi[AL] >= cut2);
         ra = lo && !wlo ? e[h][0] : ra;
         ea = hi && !whi ? e[h][5] : ea;
         rb = wlo ? e[h][0] : e[h][4];
         eb = wlo ? (lo ? e[h][1] : rb) : (whi && hi ? e[h][5] : rb);
-        if (!(d < cut2)) ea = ra, eb = rb;
+        if (d >= cut2) ea = ra, eb = rb;
       }
       const uint32_t la = ea - ra, cnt = mine ? la + (eb - rb) : 0u;
       uint32_t incl = cnt;

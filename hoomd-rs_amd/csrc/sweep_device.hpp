@@ -82,9 +82,9 @@ struct Geometry {
   const Geometry* self;
   // correctly rounded 1 / L and 1 / width for div_const_fast (0: divide)
   double inv_L[3], inv_width[3];
-  // squared cutoff (a margin of 10^-4 for the FP32 distances to a space's faces)
-  // beyond which neighbour rows are left out; infinite where a site need not lie in
-  // its body's space (sites_apart), or where FP32 does not hold it (fits_fp32)
+  // squared cutoff (a margin of 10^-4 for the FP32 distances to a space's faces) from
+  // which neighbour rows are left out; NaN, which no distance reaches, where a site
+  // need not lie in its body's space (sites_apart) or FP32 does not hold it (fits_fp32)
   float row_cut2;
 };
 
@@ -241,12 +241,15 @@ __device__ __forceinline__ uint32_t space_of(const Geometry& g, const double* or
 // along an axis of three spaces or more; u: the site from the checkerboard's
 // origin, up to L and a width.  space_of rounds u / width before it takes shape as 0: a
 // site of space 0 may have u an ulp below L (it lies on the lower face), one of the
-// last space u = L (on its upper face).  (Finite, so below a row_cut2 that is not.)
+// last space u = L (on its upper face).  A distance of more than two widths comes
+// from that and is none.
 __device__ __forceinline__ void face_gap2(double u, double m, double width, double L, float* lo, float* hi) {
-  const float wd = (float)width, v = (float)((u >= L ? u - L : u) - m * width);
-  const float uf = v > 2.0f * wd ? 0.0f : v < -wd ? wd : v, dl = fmaxf(uf, 0.0f), dh = fmaxf(wd - uf, 0.0f);
-  *lo = fminf(dl * dl, 0x1p125f);
-  *hi = fminf(dh * dh, 0x1p125f);
+  const float wd = (float)width, v = (float)((u >= L ? u - L : u) - m * width), far = 2.0f * wd;
+  float dl = fmaxf(v, 0.0f), dh = fmaxf(wd - v, 0.0f);
+  dl = dl > far ? 0.0f : dl;
+  dh = dh > far ? 0.0f : dh;
+  *lo = dl * dl;
+  *hi = dh * dh;
 }
 
 // The t-th space of colour c, in the order of

@@ -99,6 +99,7 @@ int batch_read(hmc_batch* b, std::vector<ApplyState>& st, std::vector<unsigned l
   constexpr uint32_t words = sizeof(ApplyState) / 8;
   BHIPCHK(b, b->rb.read(b->sts, nullptr, words, words, b->R, st.data(), nullptr, b->stream));
   BHIPCHK(b, b->rb.read(b->w.acc_slots, nullptr, 1, 1, b->R, acc.data(), nullptr, b->stream));
+  settled_resident(b->device, b->stream);
   for (uint32_t r = 0; r < b->R; ++r) {
     if (st[r].error & kErrBarrier)
       return bfail(b, HMC_ERR_DEVICE, "a neighbour wait of the persistent apply timed out (replica " +
@@ -401,6 +402,7 @@ bool batch_regions(hmc_batch* b, int cus) {
     if (launch_resident(b->device, fn, chunk * 8, best_threads, args, best_lds, b->stream) != hipSuccess ||
         hipStreamSynchronize(b->stream) != hipSuccess)
       return false;
+    settled_resident(b->device, b->stream);
   }
   std::vector<ApplyState> st(R);
   if (hipMemcpy(st.data(), b->sts, R * sizeof(ApplyState), hipMemcpyDeviceToHost) != hipSuccess) return false;
@@ -626,6 +628,7 @@ int hmc_batch_run_translate(hmc_batch* b, const uint64_t* step0, const uint32_t*
     if (!(max_distance[r] > 0.0) || !draws_end(b->dim, max_distance[r]))
       return bfail(b, HMC_ERR_INVALID, "max_distance must be > 0 (in 2D its square too, and finite)");
   BHIPCHK(b, hipSetDevice(b->device));
+  const ResidentCall call{b->device, b->stream};
   b->kT = kT;
   BHIPCHK(b, hipMemcpyAsync(b->dstep, step0, b->R * sizeof(uint64_t), hipMemcpyHostToDevice, b->stream));
   BHIPCHK(b, hipMemcpyAsync(b->dseed, seeds, b->R * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
@@ -745,6 +748,7 @@ int hmc_batch_autotune(hmc_batch* b, const uint64_t* step0, const uint32_t* seed
       return bfail(b, HMC_ERR_INVALID, "max_distance must be > 0 (in 2D its square too, and finite)");
   if (!b->tiled) return bfail(b, HMC_ERR_UNSUPPORTED, "the batch does not run on LDS tiles");
   BHIPCHK(b, hipSetDevice(b->device));
+  const ResidentCall call{b->device, b->stream};
   hipStream_t s = b->stream;
   const uint32_t R = b->R;
   b->kT = kT;

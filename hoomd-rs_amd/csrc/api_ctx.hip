@@ -222,6 +222,7 @@ void collect_events(hmc_ctx* c, std::vector<std::pair<hipEvent_t, hipEvent_t>>& 
 
 int read_state(hmc_ctx* c, ApplyState* out, bool check_errors) {
   HIPCHK(c, c->rb.state(c->st, c->w.acc_slots, out, c->stream));
+  settled_resident(c->device, c->stream);
   if (c->profiling) {
     collect_events(c, c->pass_events, c->pass_ms, c->pass_n);
     collect_events(c, c->build_events, c->build_ms, c->build_n);
@@ -459,6 +460,7 @@ bool persist_probe(hmc_ctx* c) {
   (void)hipMemsetAsync(c->w.mbox, 0, fbytes, c->stream);
   (void)hipMemsetAsync(&c->st->error, 0, sizeof(uint32_t), c->stream);
   (void)hipStreamSynchronize(c->stream);
+  settled_resident(c->device, c->stream);
   return ok;
 }
 
@@ -1494,6 +1496,7 @@ static int apply_one(hmc_ctx* c, uint64_t step, uint32_t substep, uint32_t seed,
   if (move == 1 && c->g.model != HMC_CONVEX_POLYHEDRON)
     return fail(c, HMC_ERR_UNSUPPORTED, "rotation moves need oriented bodies");
   HIPCHK(c, hipSetDevice(c->device));
+  const ResidentCall call{c->device, c->stream};
   ApplyState before;
   int rc = read_state(c, &before);
   if (rc) return rc;
@@ -1548,6 +1551,7 @@ int hmc_run(hmc_ctx* c, uint64_t step0, uint32_t seed, double kT, const hmc_move
       return fail(c, HMC_ERR_UNSUPPORTED, "rotation moves need oriented bodies");
   }
   HIPCHK(c, hipSetDevice(c->device));
+  const ResidentCall call{c->device, c->stream};
   ApplyState before;
   int rc = read_state(c, &before);
   if (rc) return rc;

@@ -181,11 +181,19 @@ inline SdfGrid sdf_grid(uint32_t n) {
 
 inline uint32_t grid_for(uint64_t n, uint32_t block) { return (uint32_t)((n + block - 1) / block); }
 
-// A persistent apply's launch (resident.hip).  forget_resident: before a stream that
-// such launches used ends or captures, its work complete.  resident_order: whether
-// the device's order names a stream.
+// A persistent apply's launch (resident.hip).  settled_resident: the host has waited
+// for stream s, which is no longer in flight.  ResidentCall: at the end of a call that may
+// launch, also an early one.  forget_resident: before a stream that such launches used
+// ends or captures, its work complete.  resident_order: whether the device's order
+// names a stream.
 hipError_t launch_resident(int device, const void* fn, uint32_t blocks, uint32_t threads, void** args, size_t lds,
                            hipStream_t s);
+void settled_resident(int device, hipStream_t s);
+struct ResidentCall {
+  int device;
+  hipStream_t s;
+  ~ResidentCall();
+};
 void forget_resident(int device, hipStream_t s);
 bool resident_order(int device);
 hipEvent_t take_event(hmc_ctx* c);

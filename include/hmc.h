@@ -425,6 +425,12 @@ int hmc_debug_form(const hmc_ctx* ctx, uint32_t* out);
  * device, for the work of the last one's stream) names a stream, else 0. */
 int hmc_debug_order(int device);
 
+/* Test hook: the lock between processes that persistent launches hold, on a file of
+ * the caller's: op 0 opens lock `key` of the file at `path` (the process has one at a
+ * time), 1 waits for it, 2 gives it up, 3 tells whether another process waits.
+ * Returns 1 for done or yes, else 0. */
+int hmc_debug_turn(const char* path, uint64_t key, int op);
+
 /* Evaluate the library's device math on n inputs: kind 0 cbrt, 1 log,
  * 2 exp, 5 the sine and 6 the cosine of one sincos call (the device's
  * restatements of the glibc functions Rust's std calls on Linux), 3 sqrt,

@@ -40,7 +40,7 @@ EXPORTS = ["hmc_create", "hmc_set_state", "hmc_get_state", "hmc_clone_with_bound
            "hmc_apply_rotate",
            "hmc_set_orientations", "hmc_get_orientations", "hmc_run_translate", "hmc_total_energy",
            "hmc_total_energy_noalloc", "hmc_run", "hmc_moved_since", "hmc_get_bodies", "hmc_debug_regions",
-           "hmc_debug_form", "hmc_debug_order", "hmc_debug_turn",
+           "hmc_debug_form", "hmc_debug_order", "hmc_debug_turn", "hmc_debug_region_rule",
            "hmc_trace_enable", "hmc_trace_read", "hmc_get_stats", "hmc_profile_enable", "hmc_profile_read",
            "hmc_debug_math", "hmc_debug_normals", "hmc_debug_convex", "hmc_debug_convex_axes", "hmc_last_error",
            "hmc_destroy",
@@ -167,6 +167,8 @@ def lib():
         L.hmc_debug_regions.argtypes = [vp, C.POINTER(C.c_uint32), C.c_uint64, C.POINTER(C.c_uint64)]
         L.hmc_debug_form.argtypes = [vp, C.POINTER(C.c_uint32)]
         L.hmc_debug_order.argtypes = [C.c_int]
+        L.hmc_debug_region_rule.argtypes = [C.c_int, C.c_int, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
+        L.hmc_debug_region_rule.restype = C.c_uint32
         L.hmc_debug_turn.argtypes = [C.c_char_p, C.c_uint64, C.c_int]
         u64p = C.POINTER(C.c_uint64)
         L.hmc_sdf.argtypes = [vp, C.c_double, C.c_double, C.c_uint32, u64p, u64p]

@@ -1809,6 +1809,13 @@ int hmc_debug_form(const hmc_ctx* c, uint32_t* out) {
   return HMC_OK;
 }
 
+uint32_t hmc_debug_region_rule(int dim, int kind, const int32_t* a, const int32_t* rl) {
+  if (!a || (dim != 2 && dim != 3)) return UINT32_MAX;
+  if (kind == 0) return pass_distance((uint32_t)a[0], (uint32_t)a[1]);
+  if (!rl) return UINT32_MAX;
+  return dim == 2 ? halo_list<2>(a, rl) : halo_list<3>(a, rl);
+}
+
 int hmc_debug_order(int device) { return resident_order(device) ? 1 : 0; }
 
 int hmc_profile_enable(hmc_ctx* c, int on) {

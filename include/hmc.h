@@ -421,6 +421,13 @@ int hmc_debug_regions(hmc_ctx* ctx, uint32_t* out, uint64_t cap, uint64_t* n);
  * of persistent hard shapes. */
 int hmc_debug_form(const hmc_ctx* ctx, uint32_t* out);
 
+/* Test hook: the rules of the regions of a persistent apply.  kind 0: how many passes
+ * before pass a[0] the last one lies whose colour differs from its on every axis of the
+ * set a[1] (what a region waits for); 1: the pass (modulo 2^dim) before which the cell at
+ * a, counted from the region's first space, is reloaded from a neighbour by a region of
+ * rl spaces (UINT32_MAX: no halo cell). */
+uint32_t hmc_debug_region_rule(int dim, int kind, const int32_t* a, const int32_t* rl);
+
 /* Test hook: 1 when the device's order of persistent launches (each waits, on the
  * device, for the work of the last one's stream) names a stream, else 0. */
 int hmc_debug_order(int device);

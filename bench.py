@@ -327,7 +327,7 @@ def other_workloads(hmc, wl, cpu=True, only=None, fp64=True):
             fl = fpt * t_prof / pn
             ach = fl / (ms * 1e-3) / 1e12
             r["roofline"] = {"bound": "valu_fp64", "achieved": ach, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-                             "frac": ach / PEAK_FP64_TFLOPS, "traffic": None, "kernel": "k_pass_convex",
+                             "frac": ach / PEAK_FP64_TFLOPS, "traffic": None, "kernel": "k_apply_convex",
                              "avg_launch_ms": ms, "algorithmic_flops_per_launch": fl, "launches": pn,
                              "flops_per_trial": fpt}
         sim.close()
@@ -368,7 +368,7 @@ def other_workloads(hmc, wl, cpu=True, only=None, fp64=True):
     if want("c5"):
         # C5: 256 replicas of hard spheres (FCC, N 2,048 .. 62,500, packing
         # fractions 0.30 .. 0.54), seeds 42 + r, d = 0.08; mixed precision
-        # runs persistent applies (one cooperative launch per group of
+        # runs persistent applies (one launch per group of
         # replicas per step), FP64 the per-colour tile passes (one graph per
         # step)
         systems = wl.batched_replicas()

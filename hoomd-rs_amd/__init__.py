@@ -220,10 +220,9 @@ class GpuParallelSweep:
         derives them as wrap(body + 0).  lds_tiles=False runs every trial from
         global memory (same decisions).  graphs=False makes run() launch every
         apply directly instead of replaying a captured hipGraph (same results).
-        persistent=False keeps mixed-precision hard shapes on one launch per
-        colour pass instead of one persistent launch per apply (same results;
-        the persistent launch needs cooperative launch support and a region
-        shape whose workgroups all fit on the device at once).
+        persistent=False keeps one launch per colour pass instead of one
+        persistent launch per apply (same results; the persistent launch needs
+        a region shape whose workgroups all fit on the device at once).
         fp32_error=True (mixed precision) also measures in FP64 -- LJ: every
         trial's dH; hard spheres: every pair within 1.01 sigma, on the
         per-colour tile passes -- and records the largest FP32 error and its

@@ -337,7 +337,8 @@ bool batch_regions(hmc_batch* b, int cus) {
       if (!ok) continue;
       // the fewest rounds, then the most threads: lanes beyond the trials stage and
       // reload.  (64 replicas of 864 to 32,000 bodies, us per step: 247 with 128
-      // threads, 970 with 64 and the same 64 trials per region.)
+      // threads, 970 with 64 and the same 64 trials per region; 398 with
+      // the regions and counters before.)
       if (best.empty() || load.size() < best_groups || (load.size() == best_groups && threads > best_threads)) {
         std::vector<uint32_t> t0(load.size(), 0);
         for (size_t k = 1; k < load.size(); ++k) t0[k] = t0[k - 1] + load[k - 1];
@@ -560,10 +561,9 @@ int hmc_batch_create(uint32_t n_replicas, const hmc_config* cfgs, hmc_batch** ou
     }
     // mixed precision in 3D: persistent applies, one launch per step
     // (HMC_FLAG_PER_COLOUR keeps the per-colour tile passes)
-    int cus = 0, coop = 0;
+    int cus = 0;
     if (b->tiled && b->dim == 3 && b->precision == HMC_MIXED && !(cfgs[0].flags & HMC_FLAG_PER_COLOUR) &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) == hipSuccess && cus > 0 &&
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, b->device) == hipSuccess && coop)
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) == hipSuccess && cus > 0)
       choose_batch_regions(b, cus);
   }
   *out = b;

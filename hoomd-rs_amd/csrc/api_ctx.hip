@@ -81,8 +81,8 @@ int launch_apply(hmc_ctx* c, int from_args, int advance, uint64_t step, uint32_t
     c->build_events.push_back({e0, e1});
   }
   if (c->persist) {
-    // one persistent launch runs the apply: hard shapes (mixed precision) or
-    // isotropic pair energies (FP32 energies with the FP64 layout)
+    // one persistent launch runs the apply: hard shapes, isotropic pair energies
+    // (FP64, or FP32 energies with the FP64 layout) or convex polyhedra
     hipEvent_t p0 = nullptr, p1 = nullptr;
     if (prof) {
       p0 = take_event(c);
@@ -233,7 +233,7 @@ int read_state(hmc_ctx* c, ApplyState* out, bool check_errors) {
   return HMC_OK;
 }
 
-// The same in FP64, for the persistent apply's FP64 box-relative test (E the
+// contact_band (below) in FP64, for the persistent apply's FP64 box-relative test (E the
 // bound on its displacement, three fused roundings of d^2 and the reference's).
 bool contact_band64(double E, double sigma, double sigma2, double edge2, int D, double* lo, double* hi) {
   const double dref = 1.01 * sigma;
@@ -336,17 +336,6 @@ bool choose_tiles(const Geometry& g, int D, double occ, size_t vt, int cus, Tile
   return found;
 }
 
-// Region shape of the persistent apply (k_apply_tile).  A region is 2 T
-// spaces per axis; its box (the region and a one-space halo, 2 T + 2 spaces)
-// must span at most shape - 2 spaces.  entry: bytes of a staged site (in FP64
-// about 600,000 spheres fit the device; larger systems take the per-colour
-// passes).  Every region must be resident at once,
-// so a shape qualifies only if all its workgroups fit on the device (LDS: the
-// box's offsets and a site capacity of 1.1x its expected count plus 64).
-// Among those the fewest lanes per workgroup win -- a colour pass lasts as
-// long as one workgroup's trials -- then the least staging (C2: 500 regions of
-// 5 x 5 x 10 colour spaces; 510 of 3 x 5 x 17, whose boxes and halos are a
-// tenth larger, took 7% longer).
 void fill_halo_lists(TileCfg* tc, int D) {
   int32_t rl[3] = {1, 1, 1};
   for (int a = 0; a < D; ++a) rl[a] = (int32_t)(2 * tc->T[a]);
@@ -363,14 +352,24 @@ void fill_halo_lists(TileCfg* tc, int D) {
   for (int q = 0; q < kHaloLists; ++q) tc->hoff[q + 1] = tc->hoff[q] + cnt[q];
 }
 
-// Region shape of a persistent hard-shape apply: the fewest threads, then the
-// least staging over all regions.  Where one region per compute unit suffices
-// (with 64 lanes' trials each), about as many regions as that gives, at least
-// three quarters: their boxes are smaller, and staging and reloading a box is
-// much of a small system's apply.  Measured us per apply, least staging alone and
-// so: 400 disks 49.7 (4 regions) and 45.3 (100), 1,024 48.3 (4) and 42.9 (256),
-// 4,000 spheres 143 (8) and 119 (256), 13,500 146 (27) and 129 (216), 70,304 143
-// (147) and 141 (196); with the most regions 83,000 in FP64 took 149 instead of 145.
+// Region shape of a persistent hard-shape apply (k_apply_tile), for occ bodies per
+// space.  A region is 2 T spaces per axis; its box (the region and a one-space halo,
+// 2 T + 2 spaces) must span at most shape - 2 spaces.  entry: bytes of a staged site
+// (in FP64 about 600,000 spheres fit the device; larger systems take the per-colour
+// passes).  Every region must be resident at once, so a shape qualifies only if all
+// its workgroups fit on the device (LDS: the box's offsets and a site capacity of 1.1
+// times its expected count plus 64).
+//
+// Among those the fewest threads -- a colour pass lasts as long as one workgroup's
+// trials -- then the least staging over all regions (1,000,188 spheres: 500 regions of
+// 5 x 5 x 10 colour spaces; 510 of 3 x 5 x 17, whose boxes and halos are a tenth larger,
+// took 7% longer).  Where one region per compute unit suffices (with 64 lanes' trials
+// each), about as many regions as that gives, at least three quarters: their boxes are
+// smaller, and staging and reloading a box is much of a small system's apply.  Measured
+// us per apply, least staging alone and so: 400 disks 49.7 (4 regions) and 45.3 (100),
+// 1,024 48.3 (4) and 42.9 (256), 4,000 spheres 143 (8) and 119 (256), 13,500 146 (27) and
+// 129 (216), 70,304 143 (147) and 141 (196); with the most regions 83,000 in FP64 took 149
+// instead of 145.
 bool choose_regions(const Geometry& g, int D, double occ, size_t entry, int cus, TileCfg* out) {
   uint32_t lim[3] = {1, 1, 1};
   const uint32_t cap[3] = {16, 16, 32};
@@ -464,16 +463,14 @@ bool persist_probe(hmc_ctx* c) {
   return ok;
 }
 
-// Workgroup size of k_apply_lj for a region of `trials` trials: one
-// half-wavefront per trial up to eight, in 1, 2 or 4 wavefronts (a count
-// that divides the four SIMDs of a CU, so that the wavefronts of several
-// workgroups on one CU spread evenly; with five, two workgroups did not
-// always fit on a CU that the occupancy count said holds them).
+// Workgroup size of k_apply_lj for a region of `trials` trials, whose lanes share a
+// pass's trials: 1, 2 or 4 wavefronts (a count that divides the four SIMDs of a CU, so
+// that the wavefronts of several workgroups on one CU spread evenly; with five, two
+// workgroups did not always fit on a CU that the occupancy count said holds them).
 static uint32_t lj_region_threads(uint32_t trials) { return trials <= 2 ? 64u : (trials <= 4 ? 128u : 256u); }
 
 // Region shape of the persistent isotropic apply (k_apply_lj): as
-// choose_regions, with at most 12 trials (half-wavefronts taking one or two
-// each) and a site capacity of 1.1x
+// choose_regions, with at most 12 trials and a site capacity of 1.1x
 // the box's expected count plus 128.  Among the shapes whose workgroups all
 // fit on the device at once (two waves per SIMD, the kernel's register
 // budget; the host checks the real occupancy): the least staging over all
@@ -856,11 +853,10 @@ bool sites_apart(const Geometry& g, const double* body, const double* site, uint
 static bool plan_hard(const hmc_ctx* c, double occ, RegionPlan* out) {
   const Geometry& g = c->g;
   const int D = g.dim;
-  int cus = 0, coop = 0;
+  int cus = 0;
   // (the FP32 error report runs the per-colour passes)
   if (!c->tiled || !fits_fp32(g.sigma) || (c->cfg.flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR)) ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0 ||
-      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop)
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0)
     return false;
   TileCfg pc{};
   const size_t entry = c->cfg.precision == HMC_MIXED ? sizeof(float4) : sizeof(double4);
@@ -923,19 +919,19 @@ static uint32_t pass_lanes(const Geometry& g, double cand) {
 // The same in one persistent launch per apply (k_apply_iso) where the neighbour
 // scan reaches one space out and a wavefront per 64 / lanes spaces of a colour is
 // resident.  With more than 64 candidates per trial 64 lanes share them (442,368
-// LJ bodies at density 0.8: 2261 us per step; with 16 lanes 3053, with 8 5553).
+// LJ bodies at density 0.8: 2241 us per step, one launch per colour; with 16 lanes
+// and persistent 2978, with 8 5513).
 // With fewer, 64 lanes while that is at most four wavefronts per compute unit, 16
 // while the regions are resident, else 8: overlap penalty, us per step with 64, 16
-// and 8 lanes, 6,912 bodies 171, 187, 214; 16,384 206, 195, 221; 55,296 418 (not
-// resident), 229, 234; 131,072 765, 302 (neither resident), 290.
+// and 8 lanes, 6,912 bodies 132, 143, 175; 16,384 169 (8.6 per unit), 157, 182;
+// 55,296 222 (not resident), 185, 195; 131,072 294, 295 (neither resident), 253.
 static bool plan_iso(const hmc_ctx* c, double cand, RegionPlan* out) {
   const Geometry& g = c->g;
-  int cus = 0, coop = 0;
+  int cus = 0;
   for (int a = 0; a < g.dim; ++a)
     if (g.reach[a] != 1) return false;
   if ((c->cfg.flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS)) ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0 ||
-      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) != hipSuccess || !coop)
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || cus <= 0)
     return false;
   const bool many = cand > 64.0;
   for (uint32_t lanes : {64u, 16u, 8u}) {
@@ -1135,10 +1131,9 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
   // apply (k_apply_lj) when every axis has at least six spaces and the
   // neighbour scan reaches one space out.
   if (lj_mixed && !(cfg_in->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_FP32_ERROR | HMC_FLAG_GLOBAL_PASS))) {
-    int cus = 0, coop = 0;
+    int cus = 0;
     TileCfg pc{};
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
         choose_regions_lj(g, D, (double)cfg->n_bodies / (double)spaces, cus, &pc)) {
       fill_halo_lists(&pc, D);
       // Per-axis bound E on the FP32 displacement of two staged entries
@@ -1192,10 +1187,9 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
   // spaces of a colour is resident.
   if (convex && g.reach[0] == 1 && g.reach[1] == 1 && g.reach[2] == 1 &&
       !(cfg_in->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS))) {
-    int cus = 0, coop = 0, per_cu = 0;
+    int cus = 0, per_cu = 0;
     TileCfg pc{};
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0 &&
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, persist_kernel(c), kCvApply, 0) == hipSuccess &&
         choose_regions_wave(g, kCvTrials, (uint32_t)per_cu * (uint32_t)cus, &pc)) {
       if (!adopt(c, {pc, kCvApply, (uint32_t)per_cu, 0u})) {
@@ -1207,11 +1201,11 @@ int hmc_create(const hmc_config* cfg_in, hmc_ctx** out) {
   // A small system with isotropic pair energies in FP64: whole applies by one
   // workgroup, where the system fits its LDS (about 1,400 bodies) and a colour
   // has at most 32 spaces.  Measured us per step, this and a persistent launch of
-  // a wavefront per trial (k_apply_iso): 108 LJ bodies at density 0.8 292 and
-  // 727, 864 648 and 1133, 1,372 1251 and 1900; 400 LJ disks (16 trials a pass) 131
-  // and 199, 256 overlap-penalty bodies (27 trials) 118 and 155; beyond the line
-  // 900 LJ disks (49 trials) 203 and 153, 500 overlap-penalty bodies (64) 194 and
-  // 153.
+  // a wavefront per trial (k_apply_iso): 108 LJ bodies at density 0.8 277 and
+  // 673, 864 631 and 1106, 1,372 1214 and 1880; 400 LJ disks (16 trials a pass) 117
+  // and 164, 256 overlap-penalty bodies (27 trials) 106 and 119; beyond the line
+  // 900 LJ disks (49 trials) 194 and 124, 500 overlap-penalty bodies (64) 190 and
+  // 119.
   if (lj && !lj_mixed && g.n_bodies && g.n_bodies < 5000 && g.per_colour <= 32 && !(cfg->flags & (HMC_FLAG_PER_COLOUR | HMC_FLAG_GLOBAL_PASS))) {
     const SmallLds l = SmallLds::of(g);
     const void* fn = D == 2 ? (const void*)k_apply_small<2> : (const void*)k_apply_small<3>;

@@ -127,7 +127,9 @@ int total_energy_into(hmc_ctx* c, double* part, double* total, double* bound) {
 // ------------------------------------------- static scratch of the no-alloc --
 // hmc_total_energy_noalloc keeps the block partials of the total energy in
 // this array instead of a per-call allocation: 4 kNoAllocBlocks + 4 doubles
-// (1 MiB + 32 B), the partials of up to 8,388,608 bodies.  Each GPU the
+// (1 MiB + 32 B); a block's lanes take as many bodies in turn as that needs
+// (energy_per).  The entry point's limit of 8,388,608 bodies, 256 per block, is part
+// of its description: what it refuses does not follow that division.  Each GPU the
 // library runs on holds its own copy until the process ends.  In host code
 // the array's name is only a host-side stand-in: kernels receive the device
 // address taken once per device by noalloc_setup.  Calls on one GPU share it
@@ -302,8 +304,7 @@ int hmc_total_energy_noalloc(hmc_ctx* c, double* energy, double* bound) {
   if (!c->have_state) return fail(c, HMC_ERR_STATE, "hmc_set_state was not called");
   if (grid_for(c->g.n_bodies, kEnergyBlock) > kNoAllocBlocks)
     return fail(c, HMC_ERR_INVALID,
-                "hmc_total_energy_noalloc: more than 8,388,608 bodies (the static scratch holds the partials of "
-                "32,768 blocks of 256); use hmc_total_energy");
+                "hmc_total_energy_noalloc: more than 8,388,608 bodies; use hmc_total_energy");
   if (c->device < 0 || c->device >= kNoAllocDevices || !g_scratch[c->device])
     return fail(c, HMC_ERR_DEVICE, "hmc_total_energy_noalloc: the scratch of this device was not set up");
   HIPCHK(c, hipSetDevice(c->device));

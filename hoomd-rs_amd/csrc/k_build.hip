@@ -328,7 +328,8 @@ __global__ void __launch_bounds__(256) k_scan_lookback(Geometry g, ApplyState* s
 // and the block that scans a space's count also orders its bodies.  The origin is
 // drawn by every block of the first kernel; the second's last block stores the
 // new apply state, once all blocks before it have published, and so read the old.
-// Measured us per apply, before and now: 16,384 disks 76.4 and 70.8, 4,000 spheres
+// Measured us per apply, before and now (both with launches of the apply 20 us
+// dearer than launch_resident's): 16,384 disks 76.4 and 70.8, 4,000 spheres
 // 172 and 163, 83,000 in FP64 172 and 165, 1,000,188 259 and 253 (the kernels 5.1
 // and 7.4 us at 16,384 disks, 22.7 and 20.7 at 1,000,188 spheres, where the random
 // 4-byte writes of the counts and buckets bound them).

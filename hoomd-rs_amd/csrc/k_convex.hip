@@ -609,9 +609,10 @@ __global__ void __launch_bounds__(kBlock, 3) k_pass_convex(Geometry g, ApplyStat
 // neighbours its next trials read (region_wait), after their proposals.
 // One launch per pass spent most of its time on the launch, on fetching the
 // code anew (55 KB) and on the slowest wavefront of the whole device: 262,144
-// cubes at packing fraction 0.55 (10,648 trials per pass) took 2421 us per step
-// and take 1821, 2,744 cubes 1321 and 923.  Regions of four wavefronts took
-// 1949 (a pass of a region is as long as its slowest wavefront), of two 1911.
+// cubes at packing fraction 0.55 (10,648 trials per pass) took 2431 us per step
+// (two applies) and take 1755, 2,744 cubes 2853 and 1665.  With regions of one, two
+// and four wavefronts the first took 1821, 1911 and 1949 when launches were 20 us
+// dearer (a pass of a region is as long as its slowest wavefront).
 // Bound by the chain of a pass: proposal 8, XenoCollide of the slowest pair 15,
 // candidates 9, waits 20 thousand cycles of 60.
 template <bool MIXED>

@@ -5,9 +5,9 @@
 // trial and a launch per pass (48 us per pass of 17,576 trials) spent its time on
 // the chain of one trial, with 20 of 64 lanes in use and eleven wavefronts per
 // slot one after another.  Measured us per step, before and now: 131,072
-// overlap-penalty bodies 1058 and 276, 16,384 300 and 195; LJ at density 0.8,
-// 2,048 bodies 5311 and 2888, 131,072 2464 and 1467, 442,368 (one launch per
-// colour) 3015 and 2261.  Bound by the latency of a pass's chain (start slots,
+// overlap-penalty bodies 1049 and 254, 16,384 288 and 157; LJ at density 0.8,
+// 2,048 bodies 5270 and 2887, 131,072 2445 and 1447, 442,368 (one launch per
+// colour) 3012 and 2239.  Bound by the latency of a pass's chain (start slots,
 // body, proposal, candidates, decision), about 11 us.
 #include "persist.hpp"
 

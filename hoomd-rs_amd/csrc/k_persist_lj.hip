@@ -22,7 +22,7 @@
 // and initial FP32 displacements give r^2; membership r^2 < r_cut^2 is
 // decided in FP32 only outside a band around r_cut^2 that bounds the FP32
 // error of r^2 against the reference's FP64 value, and the pair energies are
-// FP32 (lj_energy32f).  The decision stands when the FP32 dH, with a
+// FP32 (s2 = sigma^2 rcp(r^2) and its powers, as in lj_energy32).  The decision stands when the FP32 dH, with a
 // rigorous bound on its distance to the reference's FP64 dH, decides the
 // Metropolis test; otherwise (a candidate in the membership band, a site
 // without images, or a bound that straddles the decision) the trial is

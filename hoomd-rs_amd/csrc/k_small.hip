@@ -4,7 +4,7 @@
 // 864 LJ bodies are 64 spaces: a colour pass is 8 trials, and an apply 112 of
 // them. One launch per pass cost 15 us each, of which the trials' arithmetic is
 // little; regions with halos (k_apply_lj) need six spaces per axis. Here a
-// barrier separates the passes: 1.79 ms per apply became 0.64 (5.7 us a pass, the
+// barrier separates the passes: 1.81 ms per apply became 0.63 (5.6 us a pass, the
 // pair distances of its trials on one compute unit's four SIMDs; the proposals
 // are 0.5 us of it).
 //

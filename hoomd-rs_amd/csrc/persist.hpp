@@ -53,11 +53,10 @@ namespace hmc {
 // The FP64 sites that neighbours read are written with device-scope stores;
 // every wave waits for its stores to complete before the progress word is
 // stored, and neighbours read the sites with device-scope loads (no cache
-// writeback or invalidation).  Every region is resident (launch_resident), and the region whose pass is lowest never waits for one ahead of
-// it, so all of them finish.  Waits are bounded: past the bound the state's
+// writeback or invalidation).  Every region is resident (launch_resident), and
+// the region whose pass is lowest never waits for one ahead of it, so all of them finish.  Waits are bounded: past the bound the state's
 // error word is set and the wait returns, so every wave still ends.
 //
-// Measured on C2's hard spheres (500 regions, 16 passes): see k_apply_tile.
 // The counters that all 26 neighbours incremented every pass, which this
 // replaces, made every pass last as long as the slowest of 27 regions.
 // wave_publish: by the wavefront that made all of the pass's stores.

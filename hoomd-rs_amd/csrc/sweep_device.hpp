@@ -615,7 +615,6 @@ __device__ __forceinline__ typename CellCopy<PREC>::type stage_entry(const Geome
   }
 }
 
-// Persistent apply: words between region mailboxes (256 B: separate channels)
 constexpr uint32_t kMailboxStride = 64;       // words between region mailboxes (256 B: separate channels)
 constexpr int kStageRows = 4;                 // rows per half-wave staged together by the persistent apply
 
@@ -749,15 +748,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 // computed *a (A in FP32) gives |e - e_exact| <= 48 u *a with room to spare.
 __device__ __forceinline__ float lj_energy32(float sig2, float eps4, float shift, double r2, float* a) {
   const float s2 = sig2 * __builtin_amdgcn_rcpf((float)r2);
-  const float s4 = s2 * s2, s8 = s4 * s4;
-  const float s12 = s4 * s8, s6 = s2 * s4;
-  *a = eps4 * (s12 + s6) + fabsf(shift);
-  return eps4 * (s12 - s6) - shift;
-}
-// The same from an FP32 r^2 (the conversion of r^2 it skips is within the
-// bound above).
-__device__ __forceinline__ float lj_energy32f(float sig2, float eps4, float shift, float r2, float* a) {
-  const float s2 = sig2 * __builtin_amdgcn_rcpf(r2);
   const float s4 = s2 * s2, s8 = s4 * s4;
   const float s12 = s4 * s8, s6 = s2 * s4;
   *a = eps4 * (s12 + s6) + fabsf(shift);

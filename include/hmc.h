@@ -13,6 +13,20 @@
  * Conventions: every function returns an int status (HMC_OK == 0, negative on
  * error) and never throws; positions are row-major (n_bodies x dim) doubles;
  * a context is single-threaded (one caller at a time, like &mut self).
+ *
+ * Persistent applies.  Their workgroups wait for one another on the device, so all
+ * of them must be resident together:
+ *  - a wait is bounded (about 0.2 s).  A kernel of another library or stream that
+ *    holds part of the device for longer than that turns the apply into HMC_ERR_DEVICE,
+ *    with some of its moves already stored: discard the context.  Beside such work use
+ *    HMC_FLAG_PER_COLOUR (same results);
+ *  - contexts and batches of one process wait for each other on the device;
+ *  - processes that use one device take turns, by a record lock on the driver's device
+ *    file (/dev/kfd) from a process's first persistent launch until its calls have
+ *    returned, or until another process waits.  A process that is stopped inside a call
+ *    keeps the others waiting; processes with device files of their own (containers
+ *    with separate /dev trees) are not ordered: give them HMC_FLAG_PER_COLOUR;
+ *  - where the lock cannot be had, the library takes one launch per colour.
  */
 #ifndef HMC_H
 #define HMC_H
@@ -291,7 +305,9 @@ int hmc_grand_canonical_apply(hmc_ctx** ctx, uint64_t step, uint32_t substep, ui
  * (step, substep, seed) = microstate.counter(); kT = macrostate.temperature();
  * max_distance = Translate::maximum_distance.  On return *substeps_used holds
  * the number of colour cycles: the caller increments the microstate substep by
- * that much, as the reference's apply does. */
+ * that much, as the reference's apply does.  In 2D a max_distance whose square is
+ * zero or infinite in FP64 is HMC_ERR_INVALID, here and wherever a move size is
+ * given: the reference's rejection loop does not end with it (distribution.rs:39-70). */
 int hmc_apply_translate(hmc_ctx* ctx, uint64_t step, uint32_t substep, uint32_t seed, double kT,
                         double max_distance, hmc_count* out, uint32_t* substeps_used);
 
@@ -365,12 +381,13 @@ int hmc_total_energy(hmc_ctx* ctx, double* energy, double* bound);
 
 /* hmc_total_energy without allocating: no counterpart in the reference; for
  * callers that cannot allocate device memory (code under graph capture,
- * tight serving loops, harnesses that forbid hipMalloc).  Same kernels and
- * the same *energy and *bound, bit for bit; the block partials live in a
+ * tight serving loops, harnesses that forbid hipMalloc).  Same kernels (two
+ * calls, of either function, agree within *bound: the order of the bodies in a
+ * cell is that of atomic counters); the block partials live in a
  * static device array of the library (1 MiB per GPU, held until the process
  * ends) instead of a per-call allocation.  HMC_ERR_INVALID above 8,388,608
- * bodies.  Calls that overlap on one GPU (several contexts on several
- * threads or streams) race on that array. */
+ * bodies, a limit of this function.  Calls that overlap on one GPU (several
+ * contexts on several threads or streams) race on that array. */
 int hmc_total_energy_noalloc(hmc_ctx* ctx, double* energy, double* bound);
 
 /* PairwiseCutoff::delta_energy_insert (hoomd-interaction/src/pairwise_cutoff.rs:1017-1025,
